@@ -31,6 +31,7 @@
 // the row-fragment read and the transposing read (UniFrags).
 #include <type_traits>
 
+#include "item_order.h"
 #include "kernels.h"
 #include "tile_core.h"
 
@@ -53,6 +54,13 @@ __device__ __forceinline__ void static_for(F&& f) {
 constexpr int waitcnt_vm(int n) { return (n & 0xF) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 // vmcnt(63) expcnt(7) lgkmcnt(N)
 constexpr int waitcnt_lgkm(int n) { return 0xF | (3 << 14) | (7 << 4) | ((n & 0xF) << 8); }
+
+// The lane id, computed here (no register has to carry it to this place).
+__device__ __forceinline__ int opaque_lane() {
+  int lane = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
 
 // 256-byte rows (head_dim 64 and 96 leave the tail of a row unused), 16-byte
 // chunks XOR-swizzled per row with a pattern
@@ -111,7 +119,7 @@ constexpr int kBwdStages = 3;  // streamed tile pairs resident in LDS (4 measure
 // dQ: resident q, do rows; streams K, V.
 //   S^T = K Q^T,  dP^T = V dO^T,  dS = P o (dP - Delta),  dQ^T += K^T dS^T
 template <typename T, int D>
-__device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int bid) {
+__device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, const int hr, const int rt, const int wave) {
   using G = RowGeom<D>;
   using F = UniFrags<D>;
   constexpr int NW = 8, BM = 32 * NW, TN = 64, NS = kBwdStages;
@@ -122,36 +130,12 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int bid) {
   constexpr int IPT = 2 * IPW;                    // loads per streamed tile and wave
   constexpr int OROWB = D * 2 + 16;               // epilogue staging row
 
-  const int tid = threadIdx.x;
-  int lane = tid & 63;
-  // An opaque copy per item: what is derived from the lane id (fragment
-  // addresses, load offsets) is then recomputed for every item instead of
-  // being held in registers across the whole item loop, where it was spilled.
-  asm volatile("" : "+v"(lane));
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // What is derived from the lane id (fragment addresses, load offsets) is
+  // recomputed for every item instead of being held in registers across the
+  // whole item loop, where it was spilled.
+  const int lane = opaque_lane();
 
-  const int heads_r = p.hq;
   const int gqa = p.hq / p.hkv;
-  // Work item -> (sequence, resident head, resident tile).  Consecutive ids go
-  // round-robin to the 8 XCDs (private L2 each): give every XCD whole
-  // (sequence, head) units so the streamed tensors of a unit stay in one L2,
-  // and walk a unit's tiles from the one that streams most to the one that
-  // streams least (causal: the last q tile).
-  const int n_units = p.batch * heads_r;
-  int unit, slot;
-  {
-    if ((n_units & 7) == 0) {
-      const int sl = bid >> 3;
-      unit = (sl / p.n_rtiles) * 8 + (bid & 7);
-      slot = sl % p.n_rtiles;
-    } else {
-      unit = bid / p.n_rtiles;
-      slot = bid % p.n_rtiles;
-    }
-  }
-  const int rt = p.n_rtiles - 1 - slot;
-  const int hr = unit % heads_r;
-  const int b = unit / heads_r;
 
   int len;
   int64_t start;  // first row of the sequence in packed tensors
@@ -165,7 +149,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int bid) {
   }
   const int64_t bsel = p.cu ? 0 : b;
   const int r0 = rt * BM;
-  if (r0 >= len) return;
+  if (rt < 0 || r0 >= len) return;
 
   F fr;
   const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd);
@@ -506,7 +490,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int bid) {
 // the fp32 P, :578): the score wave works one streamed tile AHEAD of the grad
 // wave, so the barrier that ends a tile step is the only synchronisation.
 template <typename T, int D>
-__device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid, const int n_rt) {
+__device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, const int hr, const int rt, const int wave) {
   using G = RowGeom<D>;
   using F = UniFrags<D>;
   constexpr int NP = 4, BM = 32 * NP, TN = 64, NS = kBwdStages;
@@ -518,28 +502,11 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid,
   constexpr uint32_t PBUF = NS * STAGEB;       // P exchange: [2 tile slots][NP pairs][2 blocks][2 KiB]
   constexpr uint32_t PSLOT = NP * 2 * 2048;
 
-  const int tid = threadIdx.x;
-  int lane = tid & 63;
-  asm volatile("" : "+v"(lane));
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = opaque_lane();
   const int pr = wave & 3;            // 32-row group of the item
   const bool grad = wave >= 4;        // role of this wave
 
   const int gqa = p.hq / p.hkv;
-  const int n_units = p.batch * p.hkv;
-  int unit, slot;
-  if ((n_units & 7) == 0) {
-    const int sl = bid >> 3;
-    unit = (sl / n_rt) * 8 + (bid & 7);
-    slot = sl % n_rt;
-  } else {
-    unit = bid / n_rt;
-    slot = bid % n_rt;
-  }
-  const int rt = slot;  // causal: the first key tile streams most
-  const int hr = unit % p.hkv;
-  const int b = unit / p.hkv;
-
   int len;
   int64_t start;
   if (p.cu) {
@@ -552,7 +519,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid,
   }
   const int64_t bsel = p.cu ? 0 : b;
   const int r0 = rt * BM;
-  if (r0 >= len) return;
+  if (rt < 0 || r0 >= len) return;
 
   F fr;
   const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd);
@@ -654,11 +621,12 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid,
       drip_on = 0;
       if (grad) return;
       const int last = len - 1 - iss_s0;  // >= 0
+      const int ln = opaque_lane();
 #pragma unroll
       for (int t = 0; t < kSlabs; ++t) {
         const int inst = pr + NP * t;
-        const int r = RPI * inst + drow;
-        const int c = dslot ^ F::swz(r);
+        const int r = RPI * inst + ln / F::SLOTS;
+        const int c = (ln % F::SLOTS) ^ F::swz(r);
         const int64_t rr = min(r, last);
         const uint32_t slab = (uint32_t)__builtin_amdgcn_readfirstlane(iss_base + inst * 1024);
         if (G::NCH == 16 || c < G::NCH) {
@@ -669,7 +637,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid,
         }
       }
       if (wave < 2) {
-        const int64_t rr = min(lane, last);
+        const int64_t rr = min(ln, last);
         const uint32_t slab = (uint32_t)__builtin_amdgcn_readfirstlane(iss_base + 2 * TILEB + (wave == 0 ? 0 : 256));
         asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
                      : : "v"((const char*)al + rr * pitchl), "s"(slab) : "memory");
@@ -943,9 +911,11 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid,
         bool need_mask = sblk + 32 > len || !rows_full;
         if (causal) need_mask = need_mask || sblk < r0w + 31;
         if (need_mask) {
+          const int ln = opaque_lane();
+          const int rrow = r0w + (ln & 31);
 #pragma unroll
           for (int r = 0; r < 16; ++r) {
-            const int srow = sblk + 16 * (r >> 3) + 8 * fr.lh + (r & 7);
+            const int srow = sblk + 16 * (r >> 3) + 8 * (ln >> 5) + (r & 7);
             const bool ok = srow < len && rrow < len && (!causal || rrow <= srow);
             S[r] = ok ? S[r] : -INFINITY;
           }
@@ -1054,21 +1024,22 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid,
   T* outp = grad ? reinterpret_cast<T*>(p.dk) + bsel * p.dk_sb + start * p.dk_ss + hr * p.dk_sh
                  : reinterpret_cast<T*>(p.dv) + bsel * p.dv_sb + start * p.dv_ss + hr * p.dv_sh;
   const int64_t o_ss = grad ? p.dk_ss : p.dv_ss;
+  const int ln = opaque_lane();
   unsigned char* stg = smem_bwd + wave * 32 * OROWB;
 #pragma unroll
   for (int db = 0; db < G::NDB; ++db)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      const int d = 32 * db + 8 * g + 4 * fr.lh;
+      const int d = 32 * db + 8 * g + 4 * (ln >> 5);
       i32x2 w;
       w[0] = (int)Elem<T>::pack2(acc[db][4 * g] * oscale, acc[db][4 * g + 1] * oscale);
       w[1] = (int)Elem<T>::pack2(acc[db][4 * g + 2] * oscale, acc[db][4 * g + 3] * oscale);
-      *reinterpret_cast<i32x2*>(stg + fr.lq * OROWB + d * 2) = w;
+      *reinterpret_cast<i32x2*>(stg + (ln & 31) * OROWB + d * 2) = w;
     }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < (32 * G::NCH + 63) / 64; ++i) {
-    const int idx = lane + 64 * i;
+    const int idx = ln + 64 * i;
     const int row = idx / G::NCH, ch = idx % G::NCH;
     if (((32 * G::NCH) % 64 == 0 || idx < 32 * G::NCH) && r0w + row < len) {
       const i32x4 val = *reinterpret_cast<const i32x4*>(stg + row * OROWB + ch * 16);
@@ -1077,66 +1048,84 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int bid,
   }
 }
 
+// Persistent launch, as in the forward pass: at most one workgroup per CU, each
+// walking the work items of its rounds (a fresh 512-thread workgroup with this
+// much LDS starts several microseconds after its predecessor ends; order of the
+// items: item_order.h).  The ids are kept in LDS behind the tiles (`LIST`): held
+// in registers across the items they cost the dK + dV kernel spills inside its
+// tile loop.
+constexpr int kListBytes = 3 * kMaxRounds * 4;
+template <int ROWS, bool FROM_END, uint32_t LIST, typename Item>
+__device__ __forceinline__ void walk_items(const BwdParams& p, const int n_items, const int heads, const int heads_kv,
+                                           const int n_rt, Item&& item) {
+  typedef __attribute__((address_space(3))) int lds_int;
+  lds_int* list = (lds_int*)(uintptr_t)((uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd) + LIST);
+  const int grid = gridDim.x;
+  if (threadIdx.x < kMaxRounds) {
+    const ItemId ids = items_of_rounds<ROWS, FROM_END>(p.cu, p.batch, p.max_seqlen, n_rt, heads, heads_kv,
+                                                       heads / heads_kv, p.by_level, n_items, grid);
+    list[threadIdx.x] = ids.t;
+    list[kMaxRounds + threadIdx.x] = ids.b;
+    list[2 * kMaxRounds + threadIdx.x] = ids.h;
+  }
+  __syncthreads();
+  const int n_rounds = (n_items + grid - 1) / grid;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  for (int round = 0; round < n_rounds; ++round) {
+    const int rt = __builtin_amdgcn_readfirstlane(list[round]);
+    const int b = __builtin_amdgcn_readfirstlane(list[kMaxRounds + round]);
+    const int h = __builtin_amdgcn_readfirstlane(list[2 * kMaxRounds + round]);
+    item(b, h, rt, wave);
+    if (round + 1 < n_rounds) __syncthreads();  // the next item's tiles overwrite the staging area
+  }
+}
+
+constexpr uint32_t kDqLds = kBwdStages * (2 * 64 * 256 + 1024);
+constexpr uint32_t kDkdvLds = kDqLds + 2 * 4 * 2 * 2048;  // tile ring + P exchange
+
 template <typename T, int D>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt) {
-  const int grid = gridDim.x;
-  int round = 0;
-  for (int base = 0; base < n_items; base += grid, ++round) {
-    int w = blockIdx.x;
-    if ((round & 1) && (grid & 7) == 0) w = (((grid >> 3) - 1 - (w >> 3)) << 3) | (w & 7);
-    const int bid = base + w;
-    if (bid < n_items) bwd_dkdv_item<T, D>(p, bid, n_rt);
-    if (base + grid < n_items) __syncthreads();
-  }
+  walk_items<128, true, kDkdvLds>(p, n_items, p.hkv, p.hkv, n_rt, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
+    bwd_dkdv_item<T, D>(p, b, hr, rt, wave);
+  });
 }
 
-// Persistent launch, as in the forward pass: at most one workgroup per CU, each
-// walking the work item ids id, id + grid, ... (a fresh 512-thread workgroup
-// with this much LDS starts several microseconds after its predecessor ends);
-// odd rounds run back to front within an XCD so that a workgroup that drew an
-// item that streams many tiles draws one that streams few next.
 template <typename T, int D>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 bwd_dq_kernel(const BwdParams p, const int n_items) {
-  const int grid = gridDim.x;
-  int round = 0;
-  for (int base = 0; base < n_items; base += grid, ++round) {
-    int w = blockIdx.x;
-    if ((round & 1) && (grid & 7) == 0) w = (((grid >> 3) - 1 - (w >> 3)) << 3) | (w & 7);
-    const int bid = base + w;
-    if (bid < n_items) bwd_dq_item<T, D>(p, bid);
-    if (base + grid < n_items) __syncthreads();  // the next item's tiles overwrite the staging area
-  }
+  walk_items<256, false, kDqLds>(p, n_items, p.hq, p.hkv, p.n_rtiles, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
+    bwd_dq_item<T, D>(p, b, hr, rt, wave);
+  });
 }
 
 template <typename T, int D>
-int launch_dq(const BwdParams& p, hipStream_t s) {
-  constexpr size_t lds = kBwdStages * (2 * 64 * 256 + 1024);
-  static_assert(lds >= 8 * 32 * (D * 2 + 16), "epilogue staging must fit the tile ring");
+int launch_dq(const BwdParams& p0, hipStream_t s) {
+  BwdParams p = p0;
+  constexpr size_t lds = kDqLds + kListBytes;
+  static_assert(kDqLds >= 8 * 32 * (D * 2 + 16), "epilogue staging must fit the tile ring");
   auto kern = bwd_dq_kernel<T, D>;
   static LdsLimitOnce lds_once;
   if (const int e = raise_lds_limit(lds_once, reinterpret_cast<const void*>(kern), (int)lds)) return e;
   const long long items = (long long)p.n_rtiles * p.hq * p.batch;
-  long long grid = items;
-  const int cus = device_cu_count();
-  if (cus > 0 && grid > cus) grid = cus;  // one workgroup per CU is resident (LDS)
+  const long long grid = persistent_grid(items, device_cu_count());  // one workgroup per CU is resident (LDS)
+  p.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items);
   return (int)hipGetLastError();
 }
 
 template <typename T, int D>
-int launch_dkdv(const BwdParams& p, hipStream_t s) {
-  constexpr size_t lds = kBwdStages * (2 * 64 * 256 + 1024) + 2 * 4 * 2 * 2048;  // tile ring + P exchange
-  static_assert(lds >= 8 * 32 * (D * 2 + 16), "epilogue staging must fit");
+int launch_dkdv(const BwdParams& p0, hipStream_t s) {
+  BwdParams p = p0;
+  constexpr size_t lds = kDkdvLds + kListBytes;
+  static_assert(kDqLds >= 8 * 32 * (D * 2 + 16), "epilogue staging must fit");
   auto kern = bwd_dkdv_kernel<T, D>;
   static LdsLimitOnce lds_once;
   if (const int e = raise_lds_limit(lds_once, reinterpret_cast<const void*>(kern), (int)lds)) return e;
   const int n_rt = (p.max_seqlen + 127) / 128;
   const long long items = (long long)n_rt * p.hkv * p.batch;
-  long long grid = items;
-  const int cus = device_cu_count();
-  if (cus > 0 && grid > cus) grid = cus;  // one workgroup per CU is resident (LDS)
+  const long long grid = persistent_grid(items, device_cu_count());  // one workgroup per CU is resident (LDS)
+  p.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items, n_rt);
   return (int)hipGetLastError();
 }

@@ -1,0 +1,176 @@
+// Order of the work items of a causal launch whose sequences differ in length.
+//
+// The persistent kernels deal item ids to the workgroups by a fixed rule, so a
+// launch is as long as its most loaded workgroup.  With ids numbered sequence
+// by sequence the items of a round differ by the spread of the lengths, and
+// ids that lie past the end of a short sequence leave their workgroup idle: on
+// five sequences of 517 to 3400 tokens (32 heads) the busiest of 256 workgroups
+// had 1.4 times the mean work with 8 kv-heads and twice the mean with 32.
+//
+// Here the items that exist are numbered LEVEL by level: level t holds the t-th
+// tile of every sequence that has one, and the levels are walked from the last
+// to the first.  A causal tile costs t + 1 tiles of keys whatever its sequence
+// (counted from the sequence's start for queries, from its end for keys), so
+// the numbering runs from the longest item to the shortest, and dealing it out
+// in alternating directions leaves the workgroups within a few per cent of one
+// another (1.07 in both cases above) without a shared counter and without the
+// lengths being known on the host.
+//
+// What the order costs is sharing: items that run side by side on an XCD read
+// the same K / V from its L2 only if they belong to one (sequence, kv-head).
+// With one query head per kv-head and sixteen sequences of 2048 tokens every
+// item of a level has K / V of its own, and the forward took 702 instead of
+// 595 us, four sequences of 8192 (two sharers) 2085 instead of 1919.  So
+//  - in launches of six rounds or more `block` adjacent levels of a sequence
+//    stay together, as many as make four sharers with the query heads of the
+//    group (eight from twelve rounds up: a level more or less weighs little), and
+//  - equal lengths, which the unit-by-unit order deals out evenly, keep that
+//    order from four rounds up.
+#pragma once
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+namespace mi {
+
+// Sequences a walk can hold: one per lane of a wavefront.
+constexpr int kLevelMaxBatch = 64;
+// Rounds from which the unit-by-unit order is even enough for equal lengths
+// (below: up to 1.8 times the level order's load on the busiest workgroup, for
+// instance one sequence of 3000 tokens with 32 heads of its own, a round and a
+// half of 256-row items: 121 against 83 us forward, 402 against 328 backward).
+constexpr int kLevelEvenRounds = 4;
+
+// Is a launch numbered by level?  (A single round of workgroups takes as long as
+// its longest item in any order.  cu == null: a batched call, equal lengths.)
+inline bool number_by_level(const int32_t* cu, bool causal, int batch, long long items, long long grid) {
+  if (!causal || batch > kLevelMaxBatch || items <= grid) return false;
+  return cu != nullptr || items < kLevelEvenRounds * grid;
+}
+
+// A workgroup's item of one round: sequence, head and tile (-1: none).
+struct ItemId {
+  int b, h, t;
+};
+
+// Rounds of one workgroup: one item per lane of a wavefront.
+constexpr int kMaxRounds = 64;
+
+// Workgroups of a persistent launch of `items` ids: `resident` run at once, and
+// as many generations of them as leave each no more than kMaxRounds rounds.
+inline long long persistent_grid(long long items, long long resident) {
+  if (resident <= 0 || items <= resident) return items;
+  const long long rounds = (items + resident - 1) / resident;
+  return resident * ((rounds + kMaxRounds - 1) / kMaxRounds);
+}
+
+// All items of a workgroup, one per lane (round = lane): the searches and
+// divisions of all of them at once, in vector code ahead of the item loop,
+// instead of a chain of scalar code at every item boundary.  Odd rounds are walked back to
+// front within each XCD (id & 7 is kept), so that the workgroup that drew a
+// long item in one round draws a short one in the next.
+//
+// Not by level: consecutive ids go round-robin to the 8 XCDs, each with a
+// private L2; every XCD is given whole (sequence, kv-head) units, so that the
+// K / V of a unit stay in one L2, and a unit's tiles run from the longest item
+// to the shortest.  FROM_END: the first tile of a sequence costs most (keys,
+// which every later query streams past), else the last.  heads_kv: heads per
+// sequence that share nothing (units); heads / heads_kv items of a unit run
+// side by side on each of its tiles.
+template <int ROWS, bool FROM_END>
+__device__ __forceinline__ ItemId items_of_rounds(const int32_t* cu, const int batch, const int max_seqlen,
+                                                  const int n_tiles, const int heads, const int heads_kv,
+                                                  const int sharing, const bool level_order, const int n_items,
+                                                  const int grid) {
+  const int lane = threadIdx.x & 63;
+  const int round = lane;
+  int w = blockIdx.x;
+  if ((round & 1) && (grid & 7) == 0) w = (((grid >> 3) - 1 - (w >> 3)) << 3) | (w & 7);
+  const long long id = (long long)round * grid + w;
+  const bool any = id < n_items;
+  const uint32_t bid = any ? (uint32_t)id : 0u;   // (unsigned: the shorter divisions)
+  // x = q d + r.  All divisors are wave-uniform and ids below 2^22 need no more
+  // than a float reciprocal: with x < 2^22 exact in fp32 and v_rcp_f32 within
+  // 1 ulp the product is off by less than one, which one step either way mends.
+  const bool small = n_items < (1 << 22);
+  auto divmod = [&](uint32_t x, uint32_t d, uint32_t& q, uint32_t& r) __attribute__((always_inline)) {
+    if (small) {
+      q = (uint32_t)((float)x * __builtin_amdgcn_rcpf((float)d));
+      r = x - q * d;
+      if ((int)r < 0) {
+        --q;
+        r += d;
+      } else if (r >= d) {
+        ++q;
+        r -= d;
+      }
+    } else {
+      q = x / d;
+      r = x % d;
+    }
+  };
+  uint32_t group, rest;
+  divmod((uint32_t)heads, (uint32_t)heads_kv, group, rest);
+  ItemId it = {0, 0, -1};
+  if (level_order) {
+    int tiles = 0;  // of sequence `lane`
+    if (lane < batch) {
+      const int len = cu ? min(cu[lane + 1] - cu[lane], max_seqlen) : max_seqlen;
+      tiles = len > 0 ? (len + ROWS - 1) / ROWS : 0;
+    }
+    int total = tiles;
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) total += __shfl_xor(total, m, 64);
+    total = __builtin_amdgcn_readfirstlane(total);
+    const int tiles0 = __builtin_amdgcn_readfirstlane(tiles);
+    const bool even = __builtin_amdgcn_ballot_w64(lane < batch && tiles != tiles0) == 0;
+    if (!(cu && even && total * heads >= kLevelEvenRounds * grid)) {
+      const int sharers = total * heads >= 12 * grid ? 8 : total * heads >= 6 * grid ? 4 : 1;
+      int block = 1;  // adjacent levels of a sequence that stay together
+      while (block * sharing < sharers) block *= 2;
+      uint32_t pair, r;
+      divmod(bid, (uint32_t)heads, pair, r);
+      const int n = any ? (int)pair : -1;  // (sequence, tile) pair in the order below
+      int at = 0;                                             // pairs before the ones being looked at
+      for (int first = (n_tiles - 1) / block * block; first >= 0; first -= block) {
+        uint64_t live = __builtin_amdgcn_ballot_w64(tiles > first);
+        while (live) {
+          const int seq = __builtin_ctzll(live);
+          live &= live - 1;
+          const int all = __builtin_amdgcn_readlane(tiles, seq);
+          const int own = min(all - first, block);
+          const int k = n - at;
+          if (k >= 0 && k < own) {
+            it.b = seq;
+            it.t = FROM_END ? all - first - own + k : first + own - 1 - k;
+          }
+          at += own;
+        }
+        if (__builtin_amdgcn_ballot_w64(n >= at) == 0) break;
+      }
+      // the kv-head runs fastest: ids eight apart, which share an XCD, then read
+      // the same K / V whenever the head counts are multiples of eight
+      uint32_t member, kvh;
+      divmod(r, (uint32_t)heads_kv, member, kvh);
+      it.h = (int)(kvh * group + member);
+      return it;
+    }
+  }
+  const uint32_t per_unit = (uint32_t)n_tiles * group;
+  uint32_t unit, s, tile, member, b, kvh;
+  if (((batch * heads_kv) & 7) == 0) {
+    divmod(bid >> 3, per_unit, unit, s);
+    unit = unit * 8 + (bid & 7);
+  } else {
+    divmod(bid, per_unit, unit, s);
+  }
+  divmod(s, group, tile, member);
+  divmod(unit, (uint32_t)heads_kv, b, kvh);
+  const int t = FROM_END ? (int)tile : n_tiles - 1 - (int)tile;
+  it.b = (int)b;
+  it.h = (int)(kvh * group + member);
+  const int len = cu ? min(cu[it.b + 1] - cu[it.b], max_seqlen) : max_seqlen;
+  it.t = any && t * ROWS < len ? t : -1;
+  return it;
+}
+
+}  // namespace mi

@@ -27,6 +27,7 @@ struct PrefillParams {
   int32_t n_items;   // logical workgroups = n_qtiles * hq * batch (set by the launcher)
   int32_t causal;
   int32_t dense_form;             // dense only: 0 chosen per launch, 1 256-row items, 2 128-row items
+  int32_t by_level;               // dense only: items numbered by level (item_order.h; set by the launcher)
   int32_t win_local, win_global;  // -1 => off
   float scale;                    // log2 domain
 };
@@ -81,6 +82,7 @@ struct BwdParams {
   const int32_t* cu;  // null => batched
   int32_t batch, hq, hkv, max_seqlen;
   int32_t n_rtiles;   // ceil(max_seqlen / 256): resident tiles of the dQ kernel
+  int32_t by_level;   // items numbered by level (item_order.h; set by the launcher)
   int32_t causal;
   float scale;        // log2 domain
   float scale_nat;    // natural base (= scale * ln 2)

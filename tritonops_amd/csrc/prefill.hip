@@ -22,6 +22,7 @@
 // every tile); Q is read once (:155 re-reads it per tile).
 #include <type_traits>
 
+#include "item_order.h"
 #include "kernels.h"
 #include "tile_core.h"
 
@@ -43,29 +44,9 @@ struct ItemGeo {
   int64_t q_off, k_off, v_off, o_off, lse_off;
 };
 
-// Work item id -> geometry; false when the q tile (BM rows) starts past the end
-// of its sequence.  Consecutive ids are dealt round-robin to the 8 XCDs, each
-// with a private L2: give every XCD whole (sequence, kv-head) units so their
-// K/V stay in one L2, and walk the q tiles of a unit from the longest (last)
-// to the shortest.
-template <int BM>
-__device__ __forceinline__ bool item_geo(const PrefillParams& p, const int bid, ItemGeo& g) {
-  const int gqa = p.hq / p.hkv;
-  const int per_unit = p.n_qtiles * gqa;
-  const int n_units = p.batch * p.hkv;
-  int unit, s;
-  if ((n_units & 7) == 0) {
-    const int xcd = bid & 7, slot = bid >> 3;
-    unit = (slot / per_unit) * 8 + xcd;
-    s = slot % per_unit;
-  } else {
-    unit = bid / per_unit;
-    s = bid % per_unit;
-  }
-  g.qt = p.n_qtiles - 1 - s / gqa;
-  g.b = unit / p.hkv;
-  g.kvh = unit % p.hkv;
-  g.h = g.kvh * gqa + s % gqa;
+// The rest of an item's geometry from its sequence g.b, q-head g.h and q tile g.qt.
+__device__ __forceinline__ void finish_geo(const PrefillParams& p, ItemGeo& g) {
+  g.kvh = g.h / (p.hq / p.hkv);
   if (p.cu) {
     const int start = p.cu[g.b];
     // (a sequence longer than the caller's bound is cut at the bound: the grid covers no row beyond it)
@@ -83,7 +64,45 @@ __device__ __forceinline__ bool item_geo(const PrefillParams& p, const int bid, 
     g.o_off = g.b * p.o_sb;
     g.lse_off = g.b * p.lse_sb;
   }
+}
+
+// Work item id -> geometry; false when the q tile (BM rows) starts past the end
+// of its sequence.  Consecutive ids are dealt round-robin to the 8 XCDs, each
+// with a private L2: give every XCD whole (sequence, kv-head) units so their
+// K/V stay in one L2, and walk the q tiles of a unit from the longest (last)
+// to the shortest.  (One launch per item; the persistent kernels work their
+// items out in items_of_rounds(), item_order.h.)
+template <int BM>
+__device__ __forceinline__ bool item_geo(const PrefillParams& p, const int bid, ItemGeo& g) {
+  const int gqa = p.hq / p.hkv;
+  const int per_unit = p.n_qtiles * gqa;
+  const int n_units = p.batch * p.hkv;
+  int unit, s;
+  if ((n_units & 7) == 0) {
+    const int xcd = bid & 7, slot = bid >> 3;
+    unit = (slot / per_unit) * 8 + xcd;
+    s = slot % per_unit;
+  } else {
+    unit = bid / per_unit;
+    s = bid % per_unit;
+  }
+  g.qt = p.n_qtiles - 1 - s / gqa;
+  g.b = unit / p.hkv;
+  g.h = (unit % p.hkv) * gqa + s % gqa;
+  finish_geo(p, g);
   return g.qt * BM < g.len;
+}
+// The next item of a persistent workgroup: `ids` holds the items of all rounds,
+// one per lane, `left` the rounds that have one and are still to come.
+__device__ __forceinline__ bool next_geo(const PrefillParams& p, const ItemId& ids, uint64_t& left, ItemGeo& g) {
+  if (left == 0) return false;
+  const int at = __builtin_ctzll(left);
+  left &= left - 1;
+  g.qt = __builtin_amdgcn_readlane(ids.t, at);
+  g.b = __builtin_amdgcn_readlane(ids.b, at);
+  g.h = __builtin_amdgcn_readlane(ids.h, at);
+  finish_geo(p, g);
+  return true;
 }
 
 // K and V of one (sequence, kv-head): first token, as pointers and as 64-bit
@@ -724,7 +743,8 @@ sparse_kernel(const PrefillParams p) {
 // next).  Odd rounds are walked back to front within each XCD (id & 7 is
 // kept): ids run from the longest q tile of a unit to the shortest, so the
 // workgroup that drew a long tile in one round draws a short one in the next,
-// which balances causal work without a shared counter.
+// which balances causal work without a shared counter.  (The ids and their
+// order: item_order.h.)
 //
 // Item boundary: once every wave is done with the tiles of an item, the
 // workgroup requests Q and the first NS-1 tiles of its NEXT item (stages
@@ -775,31 +795,23 @@ dense_kernel(const PrefillParams p) {
     float* lp;  // LSE row of this head, or null
     KvSrc<T> kv;
   };
-  const int grid = gridDim.x;
-  int round = 0, base = 0;
+  const ItemId ids = items_of_rounds<BM, false>(p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv, p.hq / p.hkv,
+                                                p.by_level, p.n_items, gridDim.x);
+  uint64_t left = __builtin_amdgcn_ballot_w64(ids.t >= 0);
   // advance to the next item of this workgroup that has rows; false when there is none
   auto next_item = [&](Item& it) __attribute__((always_inline)) -> bool {
-    while (base < p.n_items) {
-      int w = blockIdx.x;
-      if ((round & 1) && (grid & 7) == 0) w = (((grid >> 3) - 1 - (w >> 3)) << 3) | (w & 7);
-      const int bid = base + w;
-      base += grid;
-      ++round;
-      ItemGeo g;
-      if (bid < p.n_items && item_geo<BM>(p, bid, g)) {
-        it.len = g.len;
-        it.q0 = g.qt * BM;
-        it.n_tiles = (g.len + TN - 1) / TN;
-        if (causal) it.n_tiles = min(it.n_tiles, (it.q0 + BM + TN - 1) / TN);
-        it.qp = reinterpret_cast<const T*>(p.q) + g.q_off + g.h * p.q_sh;
-        it.op = reinterpret_cast<T*>(p.o) + g.o_off + g.h * p.o_sh;
-        it.lp = p.lse ? p.lse + g.lse_off + g.h * p.lse_sh : nullptr;
-        it.kv = DMA::source(reinterpret_cast<const T*>(p.k) + g.k_off + g.kvh * p.k_sh,
-                            reinterpret_cast<const T*>(p.v) + g.v_off + g.kvh * p.v_sh, g.len);
-        return true;
-      }
-    }
-    return false;
+    ItemGeo g;
+    if (!next_geo(p, ids, left, g)) return false;
+    it.len = g.len;
+    it.q0 = g.qt * BM;
+    it.n_tiles = (g.len + TN - 1) / TN;
+    if (causal) it.n_tiles = min(it.n_tiles, (it.q0 + BM + TN - 1) / TN);
+    it.qp = reinterpret_cast<const T*>(p.q) + g.q_off + g.h * p.q_sh;
+    it.op = reinterpret_cast<T*>(p.o) + g.o_off + g.h * p.o_sh;
+    it.lp = p.lse ? p.lse + g.lse_off + g.h * p.lse_sh : nullptr;
+    it.kv = DMA::source(reinterpret_cast<const T*>(p.k) + g.k_off + g.kvh * p.k_sh,
+                        reinterpret_cast<const T*>(p.v) + g.v_off + g.kvh * p.v_sh, g.len);
+    return true;
   };
   // Q^T operands of an item (lane (query lq, half lh) holds d = 16c + 8lh .. +7)
   // and its first tile (tiles 1 and 2 follow from request_tile1 / 2); nothing waits here
@@ -1240,38 +1252,30 @@ dense_short_kernel(const PrefillParams p) {
   auto key_of = [](const Item& it, int j) __attribute__((always_inline)) -> int {
     return WIN ? (j + (j >= it.n_sink ? it.skip : 0)) * TN : j * TN;
   };
-  const int grid = gridDim.x;
   const int wl = p.win_local, wg = p.win_global;
-  int round = 0, base = 0;
+  const ItemId ids = items_of_rounds<BM, false>(p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv, p.hq / p.hkv,
+                                                p.by_level, p.n_items, gridDim.x);
+  uint64_t left = __builtin_amdgcn_ballot_w64(ids.t >= 0);
   auto next_item = [&](Item& it) __attribute__((always_inline)) -> bool {
-    while (base < p.n_items) {
-      int w = blockIdx.x;
-      if ((round & 1) && (grid & 7) == 0) w = (((grid >> 3) - 1 - (w >> 3)) << 3) | (w & 7);
-      const int bid = base + w;
-      base += grid;
-      ++round;
-      ItemGeo g;
-      if (bid < p.n_items && item_geo<BM>(p, bid, g)) {
-        it.len = g.len;
-        it.q0 = g.qt * BM;
-        it.n_tiles = (g.len + TN - 1) / TN;
-        if (causal) it.n_tiles = min(it.n_tiles, (it.q0 + BM + TN - 1) / TN);
-        it.n_sink = it.skip = 0;
-        if (WIN) {
-          const int t0 = max(it.q0 - wl + 1, 0) / TN;  // tile of the first key inside the local window of the item's first row
-          it.n_sink = min((wg + TN - 1) / TN, t0);
-          it.skip = t0 - it.n_sink;
-          it.n_tiles -= it.skip;
-        }
-        it.qp = reinterpret_cast<const T*>(p.q) + g.q_off + g.h * p.q_sh;
-        it.op = reinterpret_cast<T*>(p.o) + g.o_off + g.h * p.o_sh;
-        it.lp = p.lse ? p.lse + g.lse_off + g.h * p.lse_sh : nullptr;
-        it.kv = DMA::source(reinterpret_cast<const T*>(p.k) + g.k_off + g.kvh * p.k_sh,
-                            reinterpret_cast<const T*>(p.v) + g.v_off + g.kvh * p.v_sh, g.len);
-        return true;
-      }
+    ItemGeo g;
+    if (!next_geo(p, ids, left, g)) return false;
+    it.len = g.len;
+    it.q0 = g.qt * BM;
+    it.n_tiles = (g.len + TN - 1) / TN;
+    if (causal) it.n_tiles = min(it.n_tiles, (it.q0 + BM + TN - 1) / TN);
+    it.n_sink = it.skip = 0;
+    if (WIN) {
+      const int t0 = max(it.q0 - wl + 1, 0) / TN;  // tile of the first key inside the local window of the item's first row
+      it.n_sink = min((wg + TN - 1) / TN, t0);
+      it.skip = t0 - it.n_sink;
+      it.n_tiles -= it.skip;
     }
-    return false;
+    it.qp = reinterpret_cast<const T*>(p.q) + g.q_off + g.h * p.q_sh;
+    it.op = reinterpret_cast<T*>(p.o) + g.o_off + g.h * p.o_sh;
+    it.lp = p.lse ? p.lse + g.lse_off + g.h * p.lse_sh : nullptr;
+    it.kv = DMA::source(reinterpret_cast<const T*>(p.k) + g.k_off + g.kvh * p.k_sh,
+                        reinterpret_cast<const T*>(p.v) + g.v_off + g.kvh * p.v_sh, g.len);
+    return true;
   };
   // Q^T operands of an item and its first tile; tiles 1 to 3 follow from
   // request_tile<1..3>.  Nothing waits here (loads from inline assembly, see dense_kernel).
@@ -1645,8 +1649,8 @@ int launch_short(const PrefillParams& p, long long items, int cus, hipStream_t s
   PrefillParams pp = p;
   pp.n_qtiles = (p.max_seqlen + kShortRows - 1) / kShortRows;
   pp.n_items = (int)items;
-  long long grid = items;
-  if (cus > 0 && grid > (long long)per_cu * cus) grid = (long long)per_cu * cus;
+  const long long grid = persistent_grid(items, (long long)per_cu * cus);
+  pp.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(kShortRows * 2), lds, s, pp);
   return (int)hipGetLastError();
 }
@@ -1685,8 +1689,8 @@ int launch_one(const PrefillParams& p, hipStream_t s) {
     // in-kernel.  (The sparse kernel keeps one launch per q tile: four small
     // workgroups share a CU and cover each other's start-up, and walking ids
     // in-kernel measured slower there.)
-    const int cus = device_cu_count();
-    if (cus > 0 && grid > cus) grid = cus;
+    grid = persistent_grid(items, device_cu_count());
+    pp.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(NW * 64), lds, s, pp);
   return (int)hipGetLastError();
