@@ -41,9 +41,9 @@ _NS = "_ZN2mi12_GLOBAL__N_1"
 KERNELS = {
     "dense_causal": _NS + "12dense_kernelIDF16bLi128EEEvNS_13PrefillParamsE",
     "c1_dense_noncausal_small": _NS + "18dense_short_kernelIDF16bLi64ELb0EEEvNS_13PrefillParamsE",
-    "gqa_decode": _NS + "21decode_splitkv_kernelIDF16bLi128EEEvNS_12DecodeParamsE",
+    "gqa_decode": _NS + "21decode_splitkv_kernelIDF16bLi128ELi1ELb0EEEvNS_12DecodeParamsE",
     "block_sparse": _NS + "13sparse_kernelIDF16bLi128EEEvNS_13PrefillParamsE",
-    "sparse_decode": _NS + "21decode_splitkv_kernelIDF16bLi128EEEvNS_12DecodeParamsE",
+    "sparse_decode": _NS + "21decode_splitkv_kernelIDF16bLi128ELi1ELb1EEEvNS_12DecodeParamsE",
     "dense_causal_bwd": " + ".join(_NS + n for n in (
         "13bwd_dq_kernelIDF16bLi128EEEvNS_9BwdParamsEi",
         "15bwd_dkdv_kernelIDF16bLi128EEEvNS_9BwdParamsEii")),
