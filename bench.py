@@ -50,7 +50,7 @@ KERNELS = {
     "rmsnorm": " + ".join(_NS + n for n in (
         "18rms_fwd_vec_kernelIDF16bfLi2ELi4EEEvNS_9RmsParamsE", "18rms_bwd_vec_kernelIDF16bfLi2ELi4EEEvNS_9RmsParamsE",
         "19rms_dw_stage_kernelILi4EEEvPKfPfii", "20rms_dw_reduce_kernelIfEEvPKfPT_ii")),
-    "fused_xent": _NS + "16xent_gemm_kernelIDF16bLb0EEEvNS_10XentParamsE",
+    "fused_xent": _NS + "16xent_gemm_kernelIDF16bLb0ELb0EEEvNS_10XentParamsE",
 }
 # the reference's own call forms run on the kernels of the configurations above
 KERNELS["dense_causal_packed"] = KERNELS["dense_causal"]

@@ -411,7 +411,7 @@ int mi_rmsnorm_bwd(const mi_rmsnorm_args *args, void *stream);
  * cross_entropy_fused_fwd_lse_kernel (cross_entropy_triton/cross_entropy.py:
  * 276-352, :43-183) and the element-wise kernel of its backward
  * (cross_entropy_fused_bwd_kernel, :185-266):
- *   logits[t,n] = sum_d x[t,d] w[n,d]             (never written by the forward)
+ *   logits[t,n] = sum_d x[t,d] w[n,d]             (written only by mi_xent_fwd_keep)
  *   lse[t]      = log sum_n exp(logits[t,n])       fp32, saved for the backward
  *   loss[t]     = lse[t] - logits[t, y[t]]         fp32
  *   dlogits[t,n] = dloss[t] (exp(logits[t,n] - lse[t]) - [n == y[t]])
@@ -460,6 +460,18 @@ typedef struct mi_xent_bwd_args {
 } mi_xent_bwd_args;
 
 int mi_xent_bwd_dlogits(const mi_xent_bwd_args *args, void *stream);
+
+/* The same pair with the logits kept in between: mi_xent_fwd_keep is mi_xent_fwd
+ * that also writes the fp32 logits to `kept` (mi_xent_kept_bytes(tokens, vocab)
+ * of device memory, 16-byte aligned), and mi_xent_kept_dlogits turns them into
+ * the dlogits that mi_xent_bwd_dlogits computes from x and w.  `kept` is opaque:
+ * 256 x 256 tiles in the kernels' register order.  mi_xent_kept_dlogits leaves
+ * it unchanged; for the tokens from a multiple t of 256 on, pass
+ * kept + mi_xent_kept_bytes(t, vocab) bytes and advance y, lse and dloss by t.
+ * Of its args x, w, dim and the row strides are not used. */
+size_t mi_xent_kept_bytes(int64_t tokens, int64_t vocab);
+int mi_xent_fwd_keep(const mi_xent_args *args, void *kept, void *stream);
+int mi_xent_kept_dlogits(const mi_xent_bwd_args *args, const void *kept, void *stream);
 
 /* In place over a block of logits [rows, vocab] (row stride ld, elements):
  * logits[t,n] <- dloss[t] (exp(logits[t,n] - lse[t]) - [n == y[t]]), the

@@ -1,0 +1,173 @@
+"""The fused cross-entropy whose forward keeps its logits for the backward:
+the same values as computing them again, bit for bit, and the oracle's."""
+import ctypes as C
+import math
+
+import pytest
+import torch
+
+from oracle import xent_oracle as xo
+
+
+def _inputs(T, D, N, dtype, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn((T, D), generator=g).to(dtype)
+    w = (torch.randn((N, D), generator=g) * 3.0 / math.sqrt(D)).to(dtype)
+    y = torch.randint(0, N, (T,), generator=g)
+    return x, w, y, torch.rand(T, generator=g) + 0.5
+
+
+def _both(x, w, y, go):
+    import tritonops_amd as ta
+
+    res = []
+    for keep in (False, True):
+        xg, wg = x.cuda().requires_grad_(True), w.cuda().requires_grad_(True)
+        loss = ta.CrossEntropyFusedFunction.apply(xg, wg, y.cuda(), keep)
+        assert len(loss.grad_fn.saved_tensors) == (5 if keep else 4)
+        res.append((loss.detach(),) + torch.autograd.grad(loss, (xg, wg), go.cuda()))
+    return res
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,D,N", [
+    (1, 128, 1),             # one token, one class
+    (31, 128, 129),          # one token short of a unit; one row in a tile's second half
+    (33, 200, 128),          # padded hidden size; the tile's second half empty
+    (256, 128, 256),         # exactly one tile
+    (257, 128, 264),         # a token tile of one token; rows that end on a 16-byte piece
+    (320, 256, 4096 + 37),   # several ranges; rows that no 16-byte piece fits
+])
+def test_kept_logits_give_the_recomputed_gradients(dtype, T, D, N):
+    x, w, y, go = _inputs(T, D, N, dtype)
+    if T > 30:
+        y[3], y[4] = -100, N + 5  # labels outside the vocabulary
+    again, kept = _both(x, w, y, go)
+    for a, b in zip(again, kept):
+        assert torch.equal(a, b)
+    if T > 30:
+        return
+    dx, dw = xo.linear_cross_entropy_backward(go, x, w, y)
+    # dlogits are rounded to the storage type once and the sums over them again: two roundings of at most 2^-8
+    # (bf16) relative to terms no larger than the sum of magnitudes, here one row
+    assert (kept[1].cpu().double() - dx).abs().max() <= 2e-2 * max(1.0, dx.abs().max().item())
+    assert (kept[2].cpu().double() - dw).abs().max() <= 2e-2 * max(1.0, dw.abs().max().item())
+
+
+@pytest.mark.gpu
+def test_infinite_and_nan_inputs_like_recomputed():
+    x, w, y, go = _inputs(64, 128, 300, torch.bfloat16)
+    x[2, 5], x[3, 7], w[17, 3] = float("inf"), float("nan"), 1e30
+    again, kept = _both(x, w, y, go)
+    for a, b in zip(again, kept):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
+
+
+@pytest.mark.gpu
+def test_rows_in_blocks_and_a_second_backward(monkeypatch):
+    import tritonops_amd as ta
+    from tritonops_amd import xent
+
+    x, w, y, go = _inputs(1200, 128, 700, torch.bfloat16)
+    monkeypatch.setattr(xent, "BWD_ROWS", 512)
+    again, kept = _both(x, w, y.to(torch.int32), go)
+    for a, b in zip(again, kept):
+        assert torch.equal(a, b)
+    xg, wg = x.cuda().requires_grad_(True), w.cuda().requires_grad_(True)
+    loss = ta.CrossEntropyFusedFunction.apply(xg, wg, y.cuda(), True)
+    first = torch.autograd.grad(loss, (xg, wg), go.cuda(), retain_graph=True)
+    second = torch.autograd.grad(loss, (xg, wg), go.cuda())
+    for a, b in zip(first, second):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_when_the_logits_are_kept(monkeypatch):
+    import tritonops_amd as ta
+    from tritonops_amd import xent
+
+    x, w, y, _ = _inputs(40, 1024, 300, torch.bfloat16)
+    x, w, y = x.cuda(), w.cuda(), y.cuda()
+
+    def saved(xx, ww):
+        loss = ta.cross_entropy_fused_triton(xx, ww, y)
+        return len(loss.grad_fn.saved_tensors)
+
+    wg = w.clone().requires_grad_(True)
+    assert saved(x, wg) == 5
+    assert saved(x[:, :1016], wg[:, :1016]) == 4        # rows too short to pay
+    with torch.autograd.graph.save_on_cpu():             # hooks on saved tensors
+        assert not xent._keeps_logits(x, wg)
+    with torch.no_grad():
+        assert not xent._keeps_logits(x, wg)
+    assert not xent._keeps_logits(x, w)
+    monkeypatch.setattr(xent, "KEEP_BYTES", 2 * 256 * 256 * 4 - 1)
+    assert saved(x, wg) == 4
+    monkeypatch.setattr(xent, "KEEP_BYTES", 2 * 256 * 256 * 4)
+    assert saved(x, wg) == 5
+
+
+@pytest.mark.gpu
+def test_replays_of_a_captured_step():
+    import tritonops_amd as ta
+
+    x, w, y, go = _inputs(300, 1024, 1000, torch.bfloat16)
+    xg, wg = x.cuda().requires_grad_(True), w.cuda().requires_grad_(True)
+    y, go = y.cuda(), go.cuda()
+
+    def step():
+        loss = ta.cross_entropy_fused_triton(xg, wg, y)
+        return (loss.detach(),) + torch.autograd.grad(loss, (xg, wg), go)
+
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        step()
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = step()
+    for i in range(3):
+        with torch.no_grad():
+            xg.copy_(torch.roll(xg, 1, 0))
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, step()):
+            assert torch.equal(a, b), i
+
+
+def test_kept_entry_points_validate():
+    from tritonops_amd import _lib
+
+    lib = _lib.load()
+
+    def name(rc):
+        return lib.mi_status_name(rc).decode()
+
+    assert lib.mi_xent_kept_bytes(0, 10) == lib.mi_xent_kept_bytes(10, 0) == 0
+    assert lib.mi_xent_kept_bytes(257, 256) == 2 * 256 * 256 * 4
+    a = _lib.XentArgs()
+    a.struct_size, a.dtype, a.tokens, a.dim, a.vocab = C.sizeof(a), _lib.MI_DTYPE_BF16, 4, 128, 16
+    assert name(lib.mi_xent_fwd_keep(None, C.c_void_p(16), None)) == "MI_ERR_NULL_POINTER"
+    assert name(lib.mi_xent_fwd_keep(C.byref(a), None, None)) == "MI_ERR_NULL_POINTER"
+    assert name(lib.mi_xent_fwd_keep(C.byref(a), C.c_void_p(24), None)) == "MI_ERR_ALIGNMENT"
+    a.tokens = 0
+    assert lib.mi_xent_fwd_keep(C.byref(a), None, None) == 0
+    b = _lib.XentBwdArgs()
+    b.struct_size, b.dtype, b.tokens, b.vocab, b.ld = C.sizeof(b), _lib.MI_DTYPE_BF16, 4, 16, 16
+    some = C.c_void_p(64)
+    assert name(lib.mi_xent_kept_dlogits(C.byref(b), some, None)) == "MI_ERR_NULL_POINTER"
+    b.y = b.lse = b.dloss = b.dlogits = 64
+    assert name(lib.mi_xent_kept_dlogits(C.byref(b), None, None)) == "MI_ERR_NULL_POINTER"
+    assert name(lib.mi_xent_kept_dlogits(C.byref(b), C.c_void_p(72), None)) == "MI_ERR_ALIGNMENT"
+    b.ld = 15
+    assert name(lib.mi_xent_kept_dlogits(C.byref(b), some, None)) == "MI_ERR_STRIDE"
+    b.ld = b.vocab = 2 ** 31 - 1
+    b.tokens = 65
+    assert name(lib.mi_xent_kept_dlogits(C.byref(b), some, None)) == "MI_ERR_SHAPE"
+    b.dtype = _lib.MI_DTYPE_F32
+    assert name(lib.mi_xent_kept_dlogits(C.byref(b), some, None)) == "MI_ERR_DTYPE"
+    b.struct_size = 1
+    assert name(lib.mi_xent_kept_dlogits(C.byref(b), some, None)) == "MI_ERR_STRUCT_SIZE"
+    assert name(lib.mi_xent_kept_dlogits(None, some, None)) == "MI_ERR_NULL_POINTER"

@@ -166,6 +166,9 @@ EXPORTS = {
     "mi_rmsnorm_bwd_workspace_bytes": (_sz, [C.POINTER(RmsNormArgs)]),
     "mi_xent_fwd": (C.c_int, [C.POINTER(XentArgs), _vp]),
     "mi_xent_fwd_workspace_bytes": (_sz, [C.POINTER(XentArgs)]),
+    "mi_xent_kept_bytes": (_sz, [C.c_int64, C.c_int64]),
+    "mi_xent_fwd_keep": (C.c_int, [C.POINTER(XentArgs), _vp, _vp]),
+    "mi_xent_kept_dlogits": (C.c_int, [C.POINTER(XentBwdArgs), _vp, _vp]),
     "mi_xent_dlogits": (C.c_int, [C.POINTER(XentGradArgs), _vp]),
     "mi_xent_bwd_dlogits": (C.c_int, [C.POINTER(XentBwdArgs), _vp]),
     "mi_decode_num_splits": (C.c_int, [C.POINTER(DecodeArgs)]),

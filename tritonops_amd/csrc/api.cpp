@@ -294,7 +294,7 @@ size_t mi_xent_fwd_workspace_bytes(const mi_xent_args* a) {
   return (size_t)a->tokens * (size_t)mi::xent_choose_splits(a->tokens, a->vocab, 256) * 2 * sizeof(float);
 }
 
-int mi_xent_fwd(const mi_xent_args* a, void* stream) {
+static int xent_fwd(const mi_xent_args* a, float* kept, void* stream, const char* what) {
   int rc = xent_validate(a);
   if (rc) return rc;
   if (a->tokens == 0) return MI_OK;
@@ -306,8 +306,48 @@ int mi_xent_fwd(const mi_xent_args* a, void* stream) {
   p.n_split = mi::xent_choose_splits(a->tokens, a->vocab, 256);
   p.lse_part = static_cast<float*>(a->workspace);
   p.tgt_part = p.lse_part + (size_t)a->tokens * p.n_split;
-  p.lse = a->lse; p.loss = a->loss;
-  return launch_status(mi::launch_xent_fwd(p, a->dtype, false, static_cast<hipStream_t>(stream)), "mi_xent_fwd");
+  p.lse = a->lse; p.loss = a->loss; p.kept = kept;
+  return launch_status(mi::launch_xent_fwd(p, a->dtype, false, static_cast<hipStream_t>(stream)), what);
+}
+
+int mi_xent_fwd(const mi_xent_args* a, void* stream) { return xent_fwd(a, nullptr, stream, "mi_xent_fwd"); }
+
+size_t mi_xent_kept_bytes(int64_t tokens, int64_t vocab) {
+  return tokens <= 0 || vocab <= 0 ? 0 : mi::xent_kept_bytes(tokens, vocab);
+}
+
+int mi_xent_fwd_keep(const mi_xent_args* a, void* kept, void* stream) {
+  if (a && a->tokens > 0) {
+    if (!kept) return fail(MI_ERR_NULL_POINTER, "kept must be non-NULL");
+    if (!aligned16(kept)) return fail(MI_ERR_ALIGNMENT, "kept must be 16-byte aligned");
+  }
+  return xent_fwd(a, static_cast<float*>(kept), stream, "mi_xent_fwd_keep");
+}
+
+int mi_xent_kept_dlogits(const mi_xent_bwd_args* a, const void* kept, void* stream) {
+  if (!a) return fail(MI_ERR_NULL_POINTER, "args is NULL");
+  if (a->struct_size != sizeof(mi_xent_bwd_args))
+    return fail(MI_ERR_STRUCT_SIZE, "mi_xent_bwd_args.struct_size %u != %zu", a->struct_size, sizeof(mi_xent_bwd_args));
+  if (a->dtype != MI_DTYPE_BF16 && a->dtype != MI_DTYPE_F16) return fail(MI_ERR_DTYPE, "dtype %d is not bf16 / f16", a->dtype);
+  if (a->tokens < 0 || a->vocab <= 0)
+    return fail(MI_ERR_SHAPE, "tokens %d must be >= 0 and vocab %d positive", a->tokens, a->vocab);
+  if (a->labels_i64 != 0 && a->labels_i64 != 1) return fail(MI_ERR_SHAPE, "labels_i64 must be 0 or 1");
+  if (a->tokens == 0) return MI_OK;
+  if (!kept || !a->y || !a->lse || !a->dloss || !a->dlogits)
+    return fail(MI_ERR_NULL_POINTER, "kept, y, lse, dloss and dlogits must be non-NULL");
+  if (!aligned16(kept)) return fail(MI_ERR_ALIGNMENT, "kept must be 16-byte aligned");
+  if (a->ld < a->vocab) return fail(MI_ERR_STRIDE, "ld %lld < vocab", (long long)a->ld);
+  if (((long long)a->tokens + 63) / 64 * (((long long)a->vocab + 255) / 256) > 0x7fffff)
+    return fail(MI_ERR_SHAPE, "tokens %d x vocab %d: more than 2^23 - 1 blocks of 64 x 256", a->tokens, a->vocab);
+  mi::XentParams p;
+  std::memset(&p, 0, sizeof(p));
+  p.y = a->y; p.y_is_i64 = a->labels_i64;
+  p.T = a->tokens; p.N = a->vocab;
+  p.lse = const_cast<float*>(a->lse); p.dloss = a->dloss;
+  p.kept = static_cast<float*>(const_cast<void*>(kept));
+  p.dlogits = a->dlogits; p.dl_ld = a->ld;
+  p.dl_vec = aligned16(a->dlogits) && a->ld % 8 == 0;
+  return launch_status(mi::launch_xent_kept_dlogits(p, a->dtype, static_cast<hipStream_t>(stream)), "mi_xent_kept_dlogits");
 }
 
 int mi_xent_bwd_dlogits(const mi_xent_bwd_args* a, void* stream) {

@@ -107,6 +107,7 @@ struct XentParams {
   float *lse, *loss;   // [T]: outputs of the forward; lse is an input of the gradient launch
   const float* dloss;  // [T], gradient launch
   void* dlogits;       // [T, N] row stride dl_ld (elements), gradient launch
+  float* kept;         // xent_kept_bytes(T, N): logits as the forward's accumulators hold them, or null
   int64_t dl_ld;
   int32_t dl_vec;      // dlogits rows can be written in 16-byte pieces
   int64_t x_st, w_st;
@@ -198,6 +199,8 @@ int launch_rms_bwd(const RmsParams& p, int x_dtype, int w_dtype, bool vec, int n
 // Fused linear + cross-entropy.  D a multiple of 64, rows 16-byte aligned.
 int xent_choose_splits(long long tokens, int vocab, int num_cus);
 int launch_xent_fwd(const XentParams& p, int dtype, bool grad, hipStream_t s);  // forward: partials + combine
+size_t xent_kept_bytes(long long tokens, long long vocab);
+int launch_xent_kept_dlogits(const XentParams& p, int dtype, hipStream_t s);
 int launch_xent_dlogits(const XentGradParams& p, int dtype, hipStream_t s);
 
 // Query rows per workgroup of the two prefill kernels.

@@ -3,7 +3,7 @@
 // Replaces cross_entropy_fused_fwd_lse_kernel and cross_entropy_fused_bwd_kernel
 // of cross_entropy_triton/cross_entropy.py:43-183, :185-266 and the host
 // combine in CrossEntropyFusedFunction.forward (:337-339):
-//   logits[t, n] = sum_d x[t, d] w[n, d]        never written to memory
+//   logits[t, n] = sum_d x[t, d] w[n, d]        written to memory only by the keeping form
 //   lse[t]  = log sum_n exp(logits[t, n])
 //   loss[t] = lse[t] - logits[t, y[t]]
 //   dlogits[t, n] = do[t] (exp(logits[t, n] - lse[t]) - [n == y[t]])   (:255-265)
@@ -43,8 +43,19 @@ constexpr int kXTileN = 256;   // vocabulary rows per tile
 constexpr int kXStepK = 64;    // elements of D per step
 constexpr int kXSlabB = 256 * kXStepK * 2;  // one slab: 32 KiB
 constexpr int kXLdsBytes = 4 * kXSlabB;     // W stage 0, W stage 1, X stage 0, X stage 1
+typedef float xf32x4 __attribute__((ext_vector_type(4)));
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
+
+// Kept logits: a unit is the 32 tokens x 128 vocabulary rows that one wavefront
+// holds in four accumulators, 16 x 64 pieces of four floats in register order:
+// piece (4 rb + g4, lane) holds the logits of token lane % 32 and vocabulary
+// rows 32 rb + 8 g4 + 4 (lane / 32) + 0..3.  Units of a 256 x 256 tile follow
+// each other as [wave][cb].  Returns the offset of a unit in floats.
+constexpr int kXUnit = 32 * 128;
+__device__ __forceinline__ int64_t kept_unit(int t_tile, int n_tile, int tiles_n, int wave, int cb) {
+  return ((((int64_t)t_tile * tiles_n + n_tile) * 8 + wave) * 2 + cb) * kXUnit;
+}
 
 // GRAD = false: forward (partial lse and target logit per token and range).
 // GRAD = true: the same product with the epilogue of the backward pass: every
@@ -52,7 +63,17 @@ constexpr float kLn2 = 0.6931471805599453f;
 // straight from the fp32 accumulators and written to dlogits[t, n] in the
 // storage dtype (the reference rounds the logits to the storage dtype first,
 // cross_entropy.py:374,255-265, which costs accuracy when logits are large).
-template <typename T, bool GRAD>
+// KEEP (forward only): every tile's fp32 accumulators are also written out as
+// they lie in the registers, one 1-KiB row of 64 lanes x 16 bytes per store
+// (kept_unit above), for xent_kept_dlogits_kernel: the backward then reads 4
+// bytes per logit instead of running the product again.  The stores of a tile
+// drain before its next step's loads count as landed, and all workgroups reach
+// the end of a tile together, so they cost what 4 bytes per logit cost at 5 to
+// 6 TB/s: 6.99 -> 7.70 ms at 8192 x 4096 x 128256 (rows of 32 bytes per token
+// would be row-major, and far slower: short pieces of many rows per store).  Without the non-temporal hint
+// 7.74 ms there, but 1.40 instead of 1.15 ms at 4096 x 1024 x 128256, and at
+// dim 512 it costs three times as much.
+template <typename T, bool KEEP, bool GRAD>
 __global__ void __launch_bounds__(512) xent_gemm_kernel(const XentParams p) {
   typedef __attribute__((address_space(3))) const i32x4 lds_i32x4;
   const int tid = threadIdx.x;
@@ -292,6 +313,29 @@ __global__ void __launch_bounds__(512) xent_gemm_kernel(const XentParams p) {
         }
       }
     } else if (nw < p.N) {
+      if (KEEP) {
+        // rows past the vocabulary are written too (their logits are never used), tokens past the end are not
+        // (the lane's offset and the addresses are formed here, not carried through the main loop)
+        const int nt = (p.N + kXTileN - 1) / kXTileN;
+        int t0v = t0;
+        uint32_t off = (uint32_t)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)) * 16;
+        asm volatile("" : "+s"(t0v), "+v"(off));
+#pragma unroll
+        for (int cb = 0; cb < 2; ++cb) {
+          unsigned char* base = reinterpret_cast<unsigned char*>(p.kept + kept_unit(t_tile, n0 / kXTileN, nt, wave, cb));
+          if (t0v + 64 * wt + 32 * cb + (int)((off >> 4) & 31) < p.T) {
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+              for (int g4 = 0; g4 < 4; ++g4) {
+                const xf32x4 v = {acc[rb][cb][4 * g4], acc[rb][cb][4 * g4 + 1], acc[rb][cb][4 * g4 + 2],
+                                  acc[rb][cb][4 * g4 + 3]};
+                __builtin_nontemporal_store(v, reinterpret_cast<xf32x4*>(base + (4 * rb + g4) * 1024 + off));
+                __builtin_amdgcn_sched_barrier(0);
+              }
+          }
+        }
+      }
       if (nw + 128 > p.N) {  // the tile that crosses the end of the vocabulary
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb)
@@ -437,6 +481,73 @@ __global__ void __launch_bounds__(256) xent_dlogits_kernel(const XentGradParams 
   }
 }
 
+// dlogits from the kept logits of the forward: a wavefront reads one unit
+// (contiguous, 16 KiB), applies dloss[t] (exp(logit - lse[t]) - [n == y[t]]) to
+// the same fp32 values and in the same order as the epilogue of the GRAD
+// kernel, turns the unit through LDS and writes 32 pieces of 256-byte rows.
+// A workgroup is the 64 tokens x 256 vocabulary rows of two wavefronts of the
+// product.  HBM-bound: 4 bytes in and 2 out per logit: 1.12 ms (5.6 TB/s) at
+// 8192 x 128256, where the GRAD kernel takes 7.12 at dim 4096.
+template <typename T>
+__global__ void __launch_bounds__(256) xent_kept_dlogits_kernel(const XentParams p) {
+  __shared__ __attribute__((aligned(16))) unsigned char stage[4][32 * 256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lq = lane & 31, lh = lane >> 5;
+  const int wv = wave & 1, cb = wave >> 1;
+  const int nt = (p.N + kXTileN - 1) / kXTileN;
+  const int n_tile = blockIdx.x % nt, q = blockIdx.x / nt;  // q: 64-token group
+  const int t_tile = q >> 2, wt = q & 3;
+  const int t0 = q * 64 + cb * 32;                          // first token of the unit
+  const int nw = n_tile * kXTileN + 128 * wv;
+  if (t0 < p.T && nw < p.N) {
+    const xf32x4* src = reinterpret_cast<const xf32x4*>(p.kept + kept_unit(t_tile, n_tile, nt, 4 * wv + wt, cb)) + lane;
+    const bool live = t0 + lq < p.T;
+    const int tok = live ? t0 + lq : p.T - 1;
+    xf32x4 in[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) in[i] = live ? __builtin_nontemporal_load(src + i * 64) : (xf32x4){0.f, 0.f, 0.f, 0.f};
+    const float lse2 = p.lse[tok] * kLog2e, gl = p.dloss[tok];
+    const long long y = p.y_is_i64 ? reinterpret_cast<const long long*>(p.y)[tok]
+                                   : (long long)reinterpret_cast<const int*>(p.y)[tok];
+    const long long rel64 = y - nw;
+    const int rel = rel64 >= 0 && rel64 < 128 ? (int)rel64 : -1;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int nl = 8 * i + 4 * lh;
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float pr = exp2f(in[i][j] * kLog2e - lse2);
+        v[j] = gl * (pr - (rel == nl + j ? 1.f : 0.f));
+      }
+      const i32x2 pk = {(int)Elem<T>::pack2(v[0], v[1]), (int)Elem<T>::pack2(v[2], v[3])};
+      const uint32_t slot = (uint32_t)(nl >> 2) ^ ((lq & 15) << 1);  // 8-byte slots, pairs swizzled by the row
+      *reinterpret_cast<i32x2*>(&stage[wave][lq * 256 + slot * 8]) = pk;
+    }
+  }
+  __syncthreads();
+  if (t0 < p.T && nw < p.N) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4), ch = lane & 15;
+      const uint32_t slot = (uint32_t)(2 * ch) ^ ((r & 15) << 1);
+      const i32x4 val = *reinterpret_cast<const i32x4*>(&stage[wave][r * 256 + slot * 8]);
+      const int n = nw + 8 * ch;
+      if (t0 + r < p.T && n < p.N) {
+        T* dst = reinterpret_cast<T*>(p.dlogits) + (int64_t)(t0 + r) * p.dl_ld + n;
+        if (p.dl_vec && n + 8 <= p.N) {
+          __builtin_nontemporal_store(val, reinterpret_cast<i32x4*>(dst));
+        } else {
+          const T* e = reinterpret_cast<const T*>(&val);
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (n + j < p.N) dst[j] = e[j];
+        }
+      }
+    }
+  }
+}
+
 }  // namespace
 
 // Vocabulary ranges for `tokens` rows: as many as keep one round of workgroups
@@ -451,9 +562,9 @@ int xent_choose_splits(long long tokens, int vocab, int num_cus) {
 }
 
 namespace {
-template <typename T, bool GRAD>
+template <typename T, bool KEEP, bool GRAD>
 int launch_gemm(const XentParams& p, unsigned grid, hipStream_t s) {
-  auto kern = xent_gemm_kernel<T, GRAD>;
+  auto kern = xent_gemm_kernel<T, KEEP, GRAD>;
   static LdsLimitOnce lds_once;
   if (const int e = raise_lds_limit(lds_once, reinterpret_cast<const void*>(kern), kXLdsBytes)) return e;
   hipLaunchKernelGGL(kern, dim3(grid), dim3(512), kXLdsBytes, s, p);
@@ -471,11 +582,30 @@ int launch_xent_fwd(const XentParams& p0, int dtype, bool grad, hipStream_t s) {
   const unsigned grid = (unsigned)((blocks * 32 + 255) / 256 * 256);
   int rc;
   if (dtype == 0)
-    rc = grad ? launch_gemm<__bf16, true>(p, grid, s) : launch_gemm<__bf16, false>(p, grid, s);
+    rc = grad     ? launch_gemm<__bf16, false, true>(p, grid, s)
+         : p.kept ? launch_gemm<__bf16, true, false>(p, grid, s)
+                  : launch_gemm<__bf16, false, false>(p, grid, s);
   else
-    rc = grad ? launch_gemm<_Float16, true>(p, grid, s) : launch_gemm<_Float16, false>(p, grid, s);
+    rc = grad     ? launch_gemm<_Float16, false, true>(p, grid, s)
+         : p.kept ? launch_gemm<_Float16, true, false>(p, grid, s)
+                  : launch_gemm<_Float16, false, false>(p, grid, s);
   if (rc || grad) return rc;
   hipLaunchKernelGGL(xent_combine_kernel, dim3((unsigned)((p.T + 255) / 256)), dim3(256), 0, s, p);
+  return (int)hipGetLastError();
+}
+
+size_t xent_kept_bytes(long long tokens, long long vocab) {
+  const size_t tiles = (size_t)((tokens + kXTileT - 1) / kXTileT) * (size_t)((vocab + kXTileN - 1) / kXTileN);
+  return tiles * kXTileT * kXTileN * sizeof(float);
+}
+
+int launch_xent_kept_dlogits(const XentParams& p, int dtype, hipStream_t s) {
+  // the C entry bounds the grid
+  const unsigned grid = (unsigned)(((p.T + 63) / 64) * (long long)((p.N + kXTileN - 1) / kXTileN));
+  if (dtype == 0)
+    hipLaunchKernelGGL(xent_kept_dlogits_kernel<__bf16>, dim3(grid), dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL(xent_kept_dlogits_kernel<_Float16>, dim3(grid), dim3(256), 0, s, p);
   return (int)hipGetLastError();
 }
 

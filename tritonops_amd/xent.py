@@ -1,10 +1,11 @@
 """Fused linear + cross-entropy with the names of the reference's
 cross_entropy_triton/cross_entropy.py, on the HIP kernels of libmi_attn.so
-(no Triton, no fallback).  The forward never materialises the logits; the
-backward follows the reference's scheme in blocks of rows, with the logits GEMM
-and the element-wise kernel fused into one launch (the dlogits come straight
-from fp32 accumulators) and the two plain gradient GEMMs left to the BLAS
-library behind torch.mm."""
+(no Triton, no fallback).  The backward follows the reference's scheme in blocks
+of rows, with the two plain gradient GEMMs left to the BLAS library behind
+torch.mm.  Its dlogits come from the forward's fp32 logits where those are kept
+(KEEP_BYTES below), and from one launch that computes the logits again and
+applies the element-wise step to the fp32 accumulators where they are not: in a
+plain cross_entropy_fused_fwd / _bwd pair the logits are never materialised."""
 import ctypes as C
 
 import torch
@@ -16,6 +17,16 @@ _TAGS = {torch.bfloat16: _lib.MI_DTYPE_BF16, torch.float16: _lib.MI_DTYPE_F16}
 # Rows of logits that the backward materialises at a time (the reference uses
 # 2048, cross_entropy.py:367; a 288 GB device holds far larger blocks).
 BWD_ROWS = 16384
+# The forward of a call that will be differentiated keeps its fp32 logits where
+# that is at most KEEP_BYTES (of 288 GB, from the forward to the backward) and
+# the rows have at least KEEP_DIM elements: 8 bytes per logit go through memory
+# once instead of 2 * dim operations.  Forward + backward, recomputed -> kept:
+# dim 4096, 8192 tokens x 128256: 28.0 -> 22.8 ms; dim 1024, 4096 x 128256:
+# 4.60 -> 4.27; dim 768, 4096 x 50257: 1.84 -> 1.75; dim 512, 8192 x 128256:
+# 4.96 -> 5.25; dim 256, 8192 x 32000: 0.82 -> 0.97.
+KEEP_BYTES = 8 << 30
+KEEP_DIM = 1024
+_saved_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
 
 
 def _tag(t):
@@ -50,6 +61,12 @@ def cross_entropy_fused_fwd(x, w, y):
     """(loss, lse), both fp32 [T]: lse[t] = logsumexp_n(x[t] . w[n]),
     loss[t] = lse[t] - x[t] . w[y[t]] — forward of CrossEntropyFusedFunction
     (cross_entropy.py:276-352)."""
+    return _fwd(x, w, y, False)[:2]
+
+
+def _fwd(x, w, y, keep):
+    """(loss, lse, kept): kept is the logits for _kept_dlogits, None unless
+    `keep` is set and there is memory for them."""
     _require_gpu(x, w, y)
     lib = _lib.load()
     if x.ndim != 2 or w.ndim != 2:
@@ -75,8 +92,17 @@ def cross_entropy_fused_fwd(x, w, y):
     nbytes = lib.mi_xent_fwd_workspace_bytes(C.byref(a))
     ws = torch.empty(max(nbytes, 16), device=x.device, dtype=torch.uint8)
     a.workspace, a.workspace_bytes = _ptr(ws), nbytes
-    _lib.check(lib.mi_xent_fwd(C.byref(a), _stream()))
-    return loss, lse
+    kept = None
+    if keep and T and N:
+        try:
+            kept = torch.empty(lib.mi_xent_kept_bytes(T, N) // 4, device=x.device, dtype=torch.float32)
+        except torch.OutOfMemoryError:
+            pass
+    if kept is None:
+        _lib.check(lib.mi_xent_fwd(C.byref(a), _stream()))
+    else:
+        _lib.check(lib.mi_xent_fwd_keep(C.byref(a), _ptr(kept), _stream()))
+    return loss, lse, kept
 
 
 def cross_entropy_dlogits_(logits, lse, dloss, y):
@@ -121,22 +147,45 @@ def cross_entropy_dlogits(x, w, y, lse, dloss):
     return dl
 
 
+def _kept_dlogits(kept, first, y, lse, dloss, N, dl):
+    """dl [rows, N] <- dlogits of the rows from `first` on (a multiple of 256),
+    from the logits that _fwd kept; the values of cross_entropy_dlogits."""
+    lib = _lib.load()
+    a = _lib.XentBwdArgs()
+    a.struct_size = C.sizeof(a)
+    a.dtype = _tag(dl)
+    a.tokens, a.vocab = dl.shape[0], N
+    a.labels_i64 = 1 if y.dtype == torch.int64 else 0
+    a.y, a.lse, a.dloss = _ptr(y), _ptr(lse), _ptr(dloss)
+    a.dlogits, a.ld = _ptr(dl), N
+    at = C.c_void_p(kept.data_ptr() + lib.mi_xent_kept_bytes(first, N))
+    _lib.check(lib.mi_xent_kept_dlogits(C.byref(a), at, _stream()))
+    return dl
+
+
 def cross_entropy_fused_bwd(grad_o, x, w, y, lse, rows_per_block=None):
     """(grad_x, grad_w) in the dtypes of x and w — backward of
     CrossEntropyFusedFunction (cross_entropy.py:355-420): per block of rows,
     dlogits from the fused GEMM kernel, then the two gradient GEMMs."""
+    return _bwd(grad_o, x, w, y, lse, None, rows_per_block or BWD_ROWS)
+
+
+def _bwd(grad_o, x, w, y, lse, kept, step):
     _require_gpu(grad_o, x, w, y, lse)
     T = x.shape[0]
     y = _labels(y, T)
     g = grad_o.reshape(-1).to(torch.float32).contiguous()
     lse = lse.contiguous()
-    step = rows_per_block or BWD_ROWS
     grad_x = torch.empty_like(x)
     grad_w = None
     for s in range(0, T, step):
         e = min(s + step, T)
         xc = x[s:e]
-        dl = cross_entropy_dlogits(xc, w, y[s:e], lse[s:e], g[s:e])
+        if kept is None:
+            dl = cross_entropy_dlogits(xc, w, y[s:e], lse[s:e], g[s:e])
+        else:
+            dl = torch.empty((e - s, w.shape[0]), device=x.device, dtype=x.dtype)
+            _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl)
         torch.mm(dl, w, out=grad_x[s:e])
         if grad_w is None:
             grad_w = torch.mm(dl.t(), xc)
@@ -147,24 +196,38 @@ def cross_entropy_fused_bwd(grad_o, x, w, y, lse, rows_per_block=None):
     return grad_x, grad_w
 
 
+def _keeps_logits(x, w):
+    """Whether the forward keeps its logits for the backward (see KEEP_BYTES)."""
+    if not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+        return False
+    if x.ndim != 2 or w.ndim != 2 or x.shape[1] < KEEP_DIM:
+        return False
+    # hooks on saved tensors (activation checkpointing, offloading to the host) would copy or drop them
+    if _saved_hooks is None or _saved_hooks(False) is not None:
+        return False
+    return _lib.load().mi_xent_kept_bytes(x.shape[0], w.shape[0]) <= KEEP_BYTES
+
+
 class CrossEntropyFusedFunction(torch.autograd.Function):
-    """Drop-in for the reference's autograd Function (cross_entropy.py:270-420)."""
+    """Drop-in for the reference's autograd Function (cross_entropy.py:270-420).
+    `keep_logits`: the backward reads the forward's logits instead of computing
+    them again; the results are the same."""
 
     @staticmethod
-    def forward(ctx, x, w, y):
+    def forward(ctx, x, w, y, keep_logits=False):
         if y.ndim != 1 and y.shape[-1] != 1:
             raise ValueError("y must be a 1D tensor.")
-        loss, lse = cross_entropy_fused_fwd(x, w, y)
-        ctx.save_for_backward(x, w, y, lse)
+        loss, lse, kept = _fwd(x, w, y, keep_logits)
+        ctx.save_for_backward(x, w, y, lse, *(() if kept is None else (kept,)))
         return loss
 
     @staticmethod
     def backward(ctx, grad_o):
-        x, w, y, lse = ctx.saved_tensors
-        grad_x, grad_w = cross_entropy_fused_bwd(grad_o, x, w, y, lse)
-        return grad_x, grad_w, None
+        x, w, y, lse, *kept = ctx.saved_tensors
+        grad_x, grad_w = _bwd(grad_o, x, w, y, lse, kept[0] if kept else None, BWD_ROWS)
+        return grad_x, grad_w, None, None
 
 
 def cross_entropy_fused_triton(x, w, y):
     """loss [T] fp32 of softmax cross-entropy over x @ w^T (cross_entropy.py:423-425)."""
-    return CrossEntropyFusedFunction.apply(x, w, y)
+    return CrossEntropyFusedFunction.apply(x, w, y, _keeps_logits(x, w))
