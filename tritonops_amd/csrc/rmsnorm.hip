@@ -14,8 +14,13 @@
 // thread's element positions in registers over all its rows; dw is reduced in
 // two deterministic stages (every workgroup writes one fp32 partial row, a
 // second kernel adds the partial rows).  Rows that cannot be read in 16-byte
-// chunks (dim not a multiple of the chunk, unaligned rows, more than 4096
-// chunks) take an element-wise path with one partial row per wavefront.
+// chunks (dim not a multiple of the chunk, unaligned rows) are read into
+// registers element by element, each load 64 neighbouring elements: forward
+// and backward of 134083 x 1001 bf16 took 469 and 661 us as two passes over
+// the row with the dw sums in memory, 101 and 217 us (5.3 and 3.7 TB/s) now.
+// Only rows of more than 4096 elements that are not chunks, or of more chunks
+// than a workgroup's registers hold, still go that way, with one partial row
+// per wavefront.
 #include <type_traits>
 
 #include "kernels.h"
@@ -35,21 +40,32 @@ __device__ __forceinline__ float wave_sum(float v) {
 // element type tags: 0 bf16, 1 f16, 2 f32
 constexpr int kMaxJ = 16;  // 16-byte chunks a lane keeps in registers per row
 
-// EPC elements per 16-byte chunk
-template <typename T>
+// EPC elements per chunk: 16 bytes, or (WIDE = false) a single element, which
+// rows of any width, alignment and stride can be read in.
+template <typename T, bool WIDE>
 struct Chunk {
   static constexpr int EPC = 16 / sizeof(T);
-  i32x4 raw;
+  typedef i32x4 Raw;
+  Raw raw;
   __device__ __forceinline__ float at(int e) const { return (float)reinterpret_cast<const T*>(&raw)[e]; }
   __device__ __forceinline__ void set(int e, float v) { reinterpret_cast<T*>(&raw)[e] = (T)v; }
 };
+template <typename T>
+struct Chunk<T, false> {
+  static constexpr int EPC = 1;
+  typedef T Raw;
+  Raw raw;
+  __device__ __forceinline__ float at(int) const { return (float)raw; }
+  __device__ __forceinline__ void set(int, float v) { raw = (T)v; }
+};
 
-// One row's 16-byte chunks of a thread: chunk j is row chunk t + GROUP*j, where
+// One row's chunks of a thread: chunk j is row chunk t + GROUP*j, where
 // GROUP threads (one wavefront, or the four of a workgroup) share the row.
-template <typename T, int J, int GROUP>
+template <typename T, int J, int GROUP, bool WIDE>
 struct RowRegs {
-  static constexpr int EPC = Chunk<T>::EPC;
-  Chunk<T> c[J];
+  typedef Chunk<T, WIDE> C;
+  static constexpr int EPC = C::EPC;
+  C c[J];
   // STREAM: the row is not read again soon (non-temporal hint)
   template <bool STREAM = false>
   __device__ __forceinline__ void load(const T* row, int t, int nch) {
@@ -57,11 +73,31 @@ struct RowRegs {
     for (int j = 0; j < J; ++j) {
       const int ch = t + GROUP * j;
       if (ch < nch) {
-        const i32x4* src = reinterpret_cast<const i32x4*>(row + ch * EPC);
+        const typename C::Raw* src = reinterpret_cast<const typename C::Raw*>(row + ch * EPC);
         c[j].raw = STREAM ? __builtin_nontemporal_load(src) : *src;
       }
     }
   }
+};
+
+// The weights of a thread's positions: kept for all rows where a chunk is one
+// element (each would be a load of its own again), read from the cache with
+// the row otherwise.
+template <typename TW, int J, int GROUP, int EPC, bool KEPT>
+struct WeightRegs {
+  const TW* w;
+  int t;
+  __device__ __forceinline__ WeightRegs(const TW* w_, int t_, int) : w(w_), t(t_) {}
+  __device__ __forceinline__ float at(int j, int e) const { return (float)w[(t + GROUP * j) * EPC + e]; }
+};
+template <typename TW, int J, int GROUP>
+struct WeightRegs<TW, J, GROUP, 1, true> {
+  float v[J];
+  __device__ __forceinline__ WeightRegs(const TW* w, int t, int nch) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) v[j] = t + GROUP * j < nch ? (float)w[t + GROUP * j] : 0.f;
+  }
+  __device__ __forceinline__ float at(int j, int) const { return v[j]; }
 };
 
 // Sum over the GROUP threads that share a row.  WPR == 4: the wavefront sums
@@ -84,22 +120,23 @@ __device__ __forceinline__ float group_sum(float v, float (*xs)[4], int& par, in
 // WPR wavefronts (1 or 4) own a row at a time and walk rows slot, slot +
 // n_slots, ...; the next row is requested before the current one is reduced
 // and scaled (J <= 8: two rows fit in registers).
-template <typename T, typename TW, int J, int WPR>
+template <typename T, typename TW, int J, int WPR, bool WIDE>
 __global__ void __launch_bounds__(256) rms_fwd_vec_kernel(const RmsParams p) {
-  constexpr int EPC = Chunk<T>::EPC;
+  typedef Chunk<T, WIDE> C;
+  constexpr int EPC = C::EPC;
   constexpr int GROUP = 64 * WPR;
-  constexpr bool PF = J <= 8;
+  constexpr bool PF = !WIDE || J <= 8;
   __shared__ float xs[2][4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t = WPR == 1 ? lane : (int)threadIdx.x;
   const int slot = WPR == 1 ? blockIdx.x * 4 + wave : (int)blockIdx.x;
   const int n_slots = WPR == 1 ? gridDim.x * 4 : (int)gridDim.x;
-  const TW* w = reinterpret_cast<const TW*>(p.w);
   const int D = p.dim;
   const int nch = D / EPC;
+  const WeightRegs<TW, J, GROUP, EPC, !WIDE> w(reinterpret_cast<const TW*>(p.w), t, nch);
   const T* xb = reinterpret_cast<const T*>(p.x);
   int par = 0;
-  RowRegs<T, J, GROUP> cur, nxt;
+  RowRegs<T, J, GROUP, WIDE> cur, nxt;
   if (PF && slot < p.rows) cur.load(xb + (int64_t)slot * p.x_st, t, nch);
   for (int64_t row = slot; row < p.rows; row += n_slots) {
     if (PF) {
@@ -121,10 +158,10 @@ __global__ void __launch_bounds__(256) rms_fwd_vec_kernel(const RmsParams p) {
     for (int j = 0; j < J; ++j) {
       const int ch = t + GROUP * j;
       if (ch < nch) {
-        Chunk<T> o;
+        C o;
 #pragma unroll
-        for (int e = 0; e < EPC; ++e) o.set(e, cur.c[j].at(e) * r * (float)w[ch * EPC + e]);
-        __builtin_nontemporal_store(o.raw, reinterpret_cast<i32x4*>(y + ch * EPC));
+        for (int e = 0; e < EPC; ++e) o.set(e, cur.c[j].at(e) * r * w.at(j, e));
+        __builtin_nontemporal_store(o.raw, reinterpret_cast<typename C::Raw*>(y + ch * EPC));
       }
     }
     if (t == 0) p.rsqrt[row] = r;
@@ -160,20 +197,21 @@ __global__ void __launch_bounds__(256) rms_fwd_elem_kernel(const RmsParams p) {
 // n_slots, ...; every thread keeps the dw contributions of its element
 // positions in registers and the workgroup writes ONE fp32 partial row (WPR ==
 // 1: the four wavefronts cover the same positions and add theirs through LDS).
-template <typename T, typename TW, int J, int WPR>
+template <typename T, typename TW, int J, int WPR, bool WIDE>
 __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
-  constexpr int EPC = Chunk<T>::EPC;
+  typedef Chunk<T, WIDE> C;
+  constexpr int EPC = C::EPC;
   constexpr int GROUP = 64 * WPR;
-  constexpr bool PF = J <= 4;  // two (x, dy) row pairs in registers
+  constexpr bool PF = !WIDE || J <= 4;  // two (x, dy) row pairs in registers
   __shared__ float xs[2][4];
   __shared__ float red[WPR == 1 ? 4 : 1][64][EPC + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t = WPR == 1 ? lane : (int)threadIdx.x;
   const int slot = WPR == 1 ? blockIdx.x * 4 + wave : (int)blockIdx.x;
   const int n_slots = WPR == 1 ? gridDim.x * 4 : (int)gridDim.x;
-  const TW* w = reinterpret_cast<const TW*>(p.w);
   const int D = p.dim;
   const int nch = D / EPC;
+  const WeightRegs<TW, J, GROUP, EPC, !WIDE> w(reinterpret_cast<const TW*>(p.w), t, nch);
   const T* xb = reinterpret_cast<const T*>(p.x);
   const T* db = reinterpret_cast<const T*>(p.dy);
   int par = 0;
@@ -182,7 +220,13 @@ __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
   for (int j = 0; j < J; ++j)
 #pragma unroll
     for (int e = 0; e < EPC; ++e) dwacc[j][e] = 0.f;
-  RowRegs<T, J, GROUP> cx, cd, nx, nd;
+  // element by element an owner may walk many rows: their sums are folded away every eight rows, which keeps
+  // the fp32 error at that of short sums (33563 x 3999 in fp32: 2.0e-7 without it, dw against 64 bits)
+  float dwold[WIDE ? 1 : J];
+  int walked = 0;
+#pragma unroll
+  for (int j = 0; j < (WIDE ? 1 : J); ++j) dwold[j] = 0.f;
+  RowRegs<T, J, GROUP, WIDE> cx, cd, nx, nd;
   if (PF && slot < p.rows) {
     cx.template load<true>(xb + (int64_t)slot * p.x_st, t, nch);
     cd.template load<true>(db + (int64_t)slot * p.dy_st, t, nch);
@@ -205,7 +249,7 @@ __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
       const int ch = t + GROUP * j;
       if (ch < nch) {
 #pragma unroll
-        for (int e = 0; e < EPC; ++e) dot += cd.c[j].at(e) * (float)w[ch * EPC + e] * cx.c[j].at(e);
+        for (int e = 0; e < EPC; ++e) dot += cd.c[j].at(e) * w.at(j, e) * cx.c[j].at(e);
       }
     }
     dot = group_sum<WPR>(dot, xs, par, wave, lane);
@@ -214,20 +258,31 @@ __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
     for (int j = 0; j < J; ++j) {
       const int ch = t + GROUP * j;
       if (ch < nch) {
-        Chunk<T> o;
+        C o;
 #pragma unroll
         for (int e = 0; e < EPC; ++e) {
           const float xv = cx.c[j].at(e), dv = cd.c[j].at(e);
-          o.set(e, dv * (float)w[ch * EPC + e] * r - xv * k);
+          o.set(e, dv * w.at(j, e) * r - xv * k);
           dwacc[j][e] += dv * xv * r;
         }
-        __builtin_nontemporal_store(o.raw, reinterpret_cast<i32x4*>(dx + ch * EPC));
+        __builtin_nontemporal_store(o.raw, reinterpret_cast<typename C::Raw*>(dx + ch * EPC));
       }
     }
     if (PF) {
       cx = nx;
       cd = nd;
     }
+    if (!WIDE && (++walked & 7) == 0) {
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        dwold[WIDE ? 0 : j] += dwacc[j][0];
+        dwacc[j][0] = 0.f;
+      }
+    }
+  }
+  if (!WIDE) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) dwacc[j][0] += dwold[WIDE ? 0 : j];
   }
   float* part = p.dw_part + (int64_t)blockIdx.x * D;
   if (WPR > 1) {
@@ -357,43 +412,57 @@ int reduce_dw(const RmsParams& p, int n_parts, int max_parts, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-// Shape of the 16-byte path: rows of up to 128 chunks are owned by one
-// wavefront (1 or 2 chunks per lane), longer ones by a workgroup of four.
-constexpr int kWaveRowChunks = 128;
+// Shapes of the chunked path.  16-byte chunks: rows of up to 128 are owned by
+// one wavefront (1 or 2 chunks per lane), longer ones by a workgroup of four.
+// Single elements: a wavefront owns rows of up to 1024, a workgroup up to 4096.
+constexpr int kWaveRowChunks = 128, kWaveRowElems = 1024, kMaxRowElems = 4096;
 constexpr int kMaxRowWorkgroups = 1024;
 
 template <typename F>
-void by_shape(int nch, F&& f) {
+void by_shape(bool wide, int nch, F&& f) {
   using std::integral_constant;
-  if (nch <= 64)
-    f(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+  using std::true_type;
+  using std::false_type;
+  if (!wide) {
+    if (nch <= 256)
+      f(integral_constant<int, 4>{}, integral_constant<int, 1>{}, false_type{});
+    else if (nch <= 512)
+      f(integral_constant<int, 8>{}, integral_constant<int, 1>{}, false_type{});
+    else if (nch <= kWaveRowElems)
+      f(integral_constant<int, 16>{}, integral_constant<int, 1>{}, false_type{});
+    else if (nch <= 2048)
+      f(integral_constant<int, 8>{}, integral_constant<int, 4>{}, false_type{});
+    else
+      f(integral_constant<int, 16>{}, integral_constant<int, 4>{}, false_type{});
+  } else if (nch <= 64)
+    f(integral_constant<int, 1>{}, integral_constant<int, 1>{}, true_type{});
   else if (nch <= kWaveRowChunks)
-    f(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+    f(integral_constant<int, 2>{}, integral_constant<int, 1>{}, true_type{});
   else if (nch <= 256)
-    f(integral_constant<int, 1>{}, integral_constant<int, 4>{});
+    f(integral_constant<int, 1>{}, integral_constant<int, 4>{}, true_type{});
   else if (nch <= 512)
-    f(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+    f(integral_constant<int, 2>{}, integral_constant<int, 4>{}, true_type{});
   else if (nch <= 1024)
-    f(integral_constant<int, 4>{}, integral_constant<int, 4>{});
+    f(integral_constant<int, 4>{}, integral_constant<int, 4>{}, true_type{});
   else if (nch <= 2048)
-    f(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+    f(integral_constant<int, 8>{}, integral_constant<int, 4>{}, true_type{});
   else
-    f(integral_constant<int, kMaxJ>{}, integral_constant<int, 4>{});
+    f(integral_constant<int, kMaxJ>{}, integral_constant<int, 4>{}, true_type{});
 }
 
-// workgroups of the 16-byte path (= partial dw rows of the backward pass)
-inline unsigned vec_grid(const RmsParams& p, int nch, int n_waves) {
-  if (nch <= kWaveRowChunks) return (unsigned)(n_waves / 4);
+// workgroups of the chunked path (= partial dw rows of the backward pass)
+inline unsigned vec_grid(const RmsParams& p, bool wide, int nch, int n_waves) {
+  if (nch <= (wide ? kWaveRowChunks : kWaveRowElems)) return (unsigned)(n_waves / 4);
   return (unsigned)(p.rows < kMaxRowWorkgroups ? p.rows : kMaxRowWorkgroups);
 }
 
 template <typename T, typename TW>
-int launch_fwd_t(const RmsParams& p, bool vec, int n_waves, hipStream_t s) {
-  if (vec) {
-    const int nch = p.dim / Chunk<T>::EPC;
-    by_shape(nch, [&](auto jc, auto wc) {
-      hipLaunchKernelGGL((rms_fwd_vec_kernel<T, TW, decltype(jc)::value, decltype(wc)::value>),
-                         dim3(vec_grid(p, nch, n_waves)), dim3(256), 0, s, p);
+int launch_fwd_t(const RmsParams& p, bool wide, int n_waves, hipStream_t s) {
+  if (wide || p.dim <= kMaxRowElems) {
+    const int nch = wide ? p.dim / (16 / (int)sizeof(T)) : p.dim;
+    by_shape(wide, nch, [&](auto jc, auto wc, auto wide_c) {
+      hipLaunchKernelGGL((rms_fwd_vec_kernel<T, TW, decltype(jc)::value, decltype(wc)::value, decltype(wide_c)::value>),
+                         dim3(vec_grid(p, wide, nch, n_waves)), dim3(256), 0, s, p);
     });
   } else {
     hipLaunchKernelGGL((rms_fwd_elem_kernel<T, TW>), dim3((unsigned)(n_waves / 4)), dim3(256), 0, s, p);
@@ -401,17 +470,17 @@ int launch_fwd_t(const RmsParams& p, bool vec, int n_waves, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-// Partial dw rows: one per workgroup (16-byte path) or one per wavefront; never more than n_waves.
+// Partial dw rows: one per workgroup (chunked path) or one per wavefront; never more than n_waves.
 template <typename T, typename TW>
-int launch_bwd_t(const RmsParams& p, bool vec, int n_waves, hipStream_t s) {
+int launch_bwd_t(const RmsParams& p, bool wide, int n_waves, hipStream_t s) {
   int n_parts = n_waves;
-  if (vec) {
-    const int nch = p.dim / Chunk<T>::EPC;
-    const unsigned grid = vec_grid(p, nch, n_waves);
+  if (wide || p.dim <= kMaxRowElems) {
+    const int nch = wide ? p.dim / (16 / (int)sizeof(T)) : p.dim;
+    const unsigned grid = vec_grid(p, wide, nch, n_waves);
     n_parts = (int)grid;
-    by_shape(nch, [&](auto jc, auto wc) {
-      hipLaunchKernelGGL((rms_bwd_vec_kernel<T, TW, decltype(jc)::value, decltype(wc)::value>), dim3(grid),
-                         dim3(256), 0, s, p);
+    by_shape(wide, nch, [&](auto jc, auto wc, auto wide_c) {
+      hipLaunchKernelGGL((rms_bwd_vec_kernel<T, TW, decltype(jc)::value, decltype(wc)::value, decltype(wide_c)::value>),
+                         dim3(grid), dim3(256), 0, s, p);
     });
   } else {
     hipLaunchKernelGGL((rms_bwd_elem_kernel<T, TW>), dim3((unsigned)(n_waves / 4)), dim3(256), 0, s, p);
