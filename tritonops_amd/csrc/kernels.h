@@ -190,7 +190,8 @@ int launch_attn_bwd(const BwdParams& p, int dtype, int head_dim, hipStream_t s);
 // can be read in 16-byte chunks (dim a multiple of the chunk, aligned rows,
 // at most 4096 chunks).  `n_waves` = rms_partial_rows(): wavefronts of the
 // launch and upper bound of the partial dw rows the backward pass writes.
-// The backward workspace holds rms_partial_rows() + kRmsStageRows fp32 rows of `dim`.
+// The backward workspace holds rms_partial_rows() + kRmsStageRows fp32 rows of `dim`; the latter
+// are part of the size that callers were given and are not used any more.
 constexpr int kRmsStageRows = 32;
 int rms_partial_rows(long long rows, int num_cus);
 int launch_rms_fwd(const RmsParams& p, int x_dtype, int w_dtype, bool vec, int n_waves, hipStream_t s);

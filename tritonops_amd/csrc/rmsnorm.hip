@@ -342,73 +342,82 @@ __global__ void __launch_bounds__(256) rms_bwd_elem_kernel(const RmsParams p) {
   }
 }
 
-// First stage of the dw sum: out[y][d] = sum of the rows i = y (mod gridDim.y)
-// of in[n_in][D].  A workgroup covers 64 x V columns with 4 row slices.
-template <int V>
-__global__ void __launch_bounds__(256) rms_dw_stage_kernel(const float* in, float* out, int n_in, int D) {
-  __shared__ float red[4][64][V + 1];
-  const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
-  const int col = (blockIdx.x * 64 + lane) * V;
-  float acc[V];
+// dw[d] = sum of in[n_in][D] over the rows, in one launch: a workgroup covers
+// CL x V columns with 256 / CL row slices, whose sums meet by lane exchanges and
+// through LDS in a fixed order.  1024 rows of 4096: 5 us (two launches, 32 rows
+// in between, took 5 + 4 and the gap between them).
+template <typename TW, int V, int CL>
+__global__ void __launch_bounds__(256) rms_dw_sum_kernel(const float* in, TW* dw, int n_in, int D) {
+  __shared__ float red[4][CL][V];
+  constexpr int NS = 256 / CL;
+  const int c = threadIdx.x % CL, slice = threadIdx.x / CL;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = (blockIdx.x * CL + c) * V;
+  float a4[4][V];  // four sums per column: short ones, whose loads do not wait for each other
 #pragma unroll
-  for (int e = 0; e < V; ++e) acc[e] = 0.f;
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int e = 0; e < V; ++e) a4[u][e] = 0.f;
   if (col < D) {
-    for (int i = blockIdx.y + gridDim.y * slice; i < n_in; i += gridDim.y * 4) {
+    auto add = [&](int i, int u) __attribute__((always_inline)) {
       const float* src = in + (int64_t)i * D + col;
       if (V == 4) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(src);
 #pragma unroll
-        for (int e = 0; e < V; ++e) acc[e] += v[e];
+        for (int e = 0; e < V; ++e) a4[u][e] += v[e];
       } else {
-        acc[0] += src[0];
+        a4[u][0] += src[0];
       }
+    };
+    int i = slice;
+    if (V == 4) {
+      // few rows to a slice: the bound is looked at per row (1048576 x 64, whole backward: 75 against 82 us)
+#pragma unroll 2
+      for (; i < n_in; i += 4 * NS) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          if (i + u * NS >= n_in) break;
+          add(i + u * NS, u);
+        }
+      }
+    } else {
+      // many: batches of sixteen loads (262144 x 511: 189 against 207 us)
+#pragma unroll 4
+      for (; i + 3 * NS < n_in; i += 4 * NS) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) add(i + u * NS, u);
+      }
+      for (; i < n_in; i += NS) add(i, 0);
     }
   }
+  float acc[V];
 #pragma unroll
-  for (int e = 0; e < V; ++e) red[slice][lane][e] = acc[e];
+  for (int e = 0; e < V; ++e) acc[e] = (a4[0][e] + a4[1][e]) + (a4[2][e] + a4[3][e]);
+#pragma unroll
+  for (int e = 0; e < V; ++e) {
+#pragma unroll
+    for (int m = 32; m >= CL; m >>= 1) acc[e] += __shfl_xor(acc[e], m, 64);
+    if (lane < CL) red[wave][c][e] = acc[e];
+  }
   __syncthreads();
-  if (slice == 0 && col < D) {
-#pragma unroll
-    for (int e = 0; e < V; ++e)
-      out[(int64_t)blockIdx.y * D + col + e] = (red[0][lane][e] + red[1][lane][e]) + (red[2][lane][e] + red[3][lane][e]);
+  if (threadIdx.x < CL * V) {
+    const int cc = threadIdx.x / V, e = threadIdx.x % V;
+    const int d = (blockIdx.x * CL + cc) * V + e;
+    if (d < D) dw[d] = (TW)((red[0][cc][e] + red[1][cc][e]) + (red[2][cc][e] + red[3][cc][e]));
   }
 }
 
-// Last stage: dw[d] = sum of in[n_in][D] over the rows, 64 columns x 4 row slices per workgroup
+// Adds the n_parts partial rows at p.dw_part into p.dw
 template <typename TW>
-__global__ void __launch_bounds__(256) rms_dw_reduce_kernel(const float* in, TW* dw, int n_in, int D) {
-  __shared__ float red[4][64];
-  const int col = threadIdx.x & 63, slice = threadIdx.x >> 6;
-  const int d = blockIdx.x * 64 + col;
-  float s = 0.f;
-  if (d < D)
-    for (int i = slice; i < n_in; i += 4) s += in[(int64_t)i * D + d];
-  red[slice][col] = s;
-  __syncthreads();
-  if (slice == 0 && d < D) dw[d] = (TW)((red[0][col] + red[1][col]) + (red[2][col] + red[3][col]));
-}
-
-// Adds n_parts partial rows at p.dw_part into p.dw; more than kStageRows of
-// them go through kStageRows intermediate rows kept behind the `max_parts`
-// rows of the workspace.
-template <typename TW>
-int reduce_dw(const RmsParams& p, int n_parts, int max_parts, hipStream_t s) {
+int reduce_dw(const RmsParams& p, int n_parts, hipStream_t s) {
   const float* in = p.dw_part;
-  if (n_parts > kRmsStageRows) {
-    float* mid = p.dw_part + (int64_t)max_parts * p.dim;
-    const bool v4 = p.dim % 4 == 0 && reinterpret_cast<uintptr_t>(p.dw_part) % 16 == 0;
-    const dim3 grid((unsigned)((p.dim + (v4 ? 255 : 63)) / (v4 ? 256 : 64)), kRmsStageRows);
-    if (v4)
-      hipLaunchKernelGGL((rms_dw_stage_kernel<4>), grid, dim3(256), 0, s, in, mid, n_parts, p.dim);
-    else
-      hipLaunchKernelGGL((rms_dw_stage_kernel<1>), grid, dim3(256), 0, s, in, mid, n_parts, p.dim);
-    int rc = (int)hipGetLastError();
-    if (rc) return rc;
-    in = mid;
-    n_parts = kRmsStageRows;
-  }
-  hipLaunchKernelGGL((rms_dw_reduce_kernel<TW>), dim3((unsigned)((p.dim + 63) / 64)), dim3(256), 0, s, in,
-                     reinterpret_cast<TW*>(p.dw), n_parts, p.dim);
+  TW* dw = reinterpret_cast<TW*>(p.dw);
+  if (p.dim % 4 == 0 && reinterpret_cast<uintptr_t>(in) % 16 == 0)
+    hipLaunchKernelGGL((rms_dw_sum_kernel<TW, 4, 4>), dim3((unsigned)((p.dim + 15) / 16)), dim3(256), 0, s, in, dw, n_parts,
+                       p.dim);
+  else
+    hipLaunchKernelGGL((rms_dw_sum_kernel<TW, 1, 16>), dim3((unsigned)((p.dim + 15) / 16)), dim3(256), 0, s, in, dw, n_parts,
+                       p.dim);
   return (int)hipGetLastError();
 }
 
@@ -487,7 +496,7 @@ int launch_bwd_t(const RmsParams& p, bool wide, int n_waves, hipStream_t s) {
   }
   int rc = (int)hipGetLastError();
   if (rc) return rc;
-  return reduce_dw<TW>(p, n_parts, n_waves, s);
+  return reduce_dw<TW>(p, n_parts, s);
 }
 
 template <typename F>

@@ -65,7 +65,7 @@ def rmsnorm_bwd(dy, x, weight, rsqrt, eps):
     wk = wk.contiguous()
     x2, dy2 = _rows(x), _rows(dy.to(x.dtype))
     dx = torch.empty((x2.shape[0], x2.shape[1]), device=x.device, dtype=x.dtype)
-    dw = torch.zeros_like(wk)
+    dw = torch.empty_like(wk) if x2.shape[0] else torch.zeros_like(wk)  # without rows the library leaves it alone
     a = _args(x2, wk, eps)
     a.rsqrt = _ptr(rsqrt)
     a.dy, a.dx, a.dw = _ptr(dy2), _ptr(dx), _ptr(dw)
