@@ -41,7 +41,7 @@ def _inputs(rows, dim, dt, wdt, seed=0):
 
 @pytest.mark.parametrize("rows,dim", [
     (5, 1), (4099, 7), (129, 255), (300, 257), (4097, 511), (33, 513), (5, 1023), (4100, 1025), (3, 2047), (1025, 2049),
-    (1500, 4095), (7, 4097)])
+    (1500, 4095), (7, 4097), (1100, 5001), (3, 8191), (3, 8193)])
 @pytest.mark.parametrize("dt,wdt", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float32),
                                     (torch.float32, torch.float32)])
 def test_element_wise_rows(rows, dim, dt, wdt):

@@ -7,8 +7,8 @@
 //   dx_td = dy_td w_d r_t - x_td r_t^3 (sum_d dy_td w_d x_td) / D   (:199-212)
 //   dw_d  = sum_t dy_td x_td r_t                  (:213; the reference adds
 //           per-tile sums with atomics, :215)
-// A row is owned by one wavefront (short rows) or by the four wavefronts of a
-// workgroup (long rows) and is read once, with 16-byte loads, into registers;
+// A row is owned by part of a wavefront, by one, or by the four wavefronts of a
+// workgroup and is read once, with 16-byte loads, into registers;
 // the owners walk the rows with a fixed stride and request the next row before
 // they work on the current one.  The backward pass keeps the dw sums of each
 // thread's element positions in registers over all its rows; dw is reduced in
@@ -18,9 +18,11 @@
 // registers element by element, each load 64 neighbouring elements: forward
 // and backward of 134083 x 1001 bf16 took 469 and 661 us as two passes over
 // the row with the dw sums in memory, 101 and 217 us (5.3 and 3.7 TB/s) now.
-// Only rows of more than 4096 elements that are not chunks, or of more chunks
+// Only rows of more than 8192 elements that are not chunks, or of more chunks
 // than a workgroup's registers hold, still go that way, with one partial row
-// per wavefront.
+// per wavefront.  Rows of up to 32 chunks share a wavefront: with one row each,
+// 8 of 64 lanes worked on a head of 64 (1048576 rows: 252 and 411 us, now 42
+// and 75, 6.3 and 5.4 TB/s).
 #include <type_traits>
 
 #include "kernels.h"
@@ -31,9 +33,11 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
+// sum over aligned groups of LANES lanes
+template <int LANES = 64>
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  for (int m = LANES / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
   return v;
 }
 
@@ -100,14 +104,14 @@ struct WeightRegs<TW, J, GROUP, 1, true> {
   __device__ __forceinline__ float at(int j, int) const { return v[j]; }
 };
 
-// Sum over the GROUP threads that share a row.  WPR == 4: the wavefront sums
+// Sum over the GROUP threads that share a row.  GROUP == 256: the wavefront sums
 // meet in LDS; `xs` is double-buffered by row parity, so one barrier per row is
 // enough (a wavefront can only overwrite a slot after every other wavefront
 // has passed the barrier of the row in between).
-template <int WPR>
+template <int GROUP>
 __device__ __forceinline__ float group_sum(float v, float (*xs)[4], int& par, int wave, int lane) {
-  v = wave_sum(v);
-  if (WPR > 1) {
+  v = wave_sum<(GROUP < 64 ? GROUP : 64)>(v);
+  if (GROUP > 64) {
     if (lane == 0) xs[par][wave] = v;
     __syncthreads();
     v = (xs[par][0] + xs[par][1]) + (xs[par][2] + xs[par][3]);
@@ -117,20 +121,20 @@ __device__ __forceinline__ float group_sum(float v, float (*xs)[4], int& par, in
 }
 
 // ---------------------------------------------------------------- forward
-// WPR wavefronts (1 or 4) own a row at a time and walk rows slot, slot +
-// n_slots, ...; the next row is requested before the current one is reduced
+// GROUP threads (part of a wavefront, one, or a workgroup) own a row at a time
+// and walk rows slot, slot + n_slots, ...; the next row is requested before the current one is reduced
 // and scaled (J <= 8: two rows fit in registers).
-template <typename T, typename TW, int J, int WPR, bool WIDE>
+template <typename T, typename TW, int J, int GROUP, bool WIDE>
 __global__ void __launch_bounds__(256) rms_fwd_vec_kernel(const RmsParams p) {
   typedef Chunk<T, WIDE> C;
   constexpr int EPC = C::EPC;
-  constexpr int GROUP = 64 * WPR;
-  constexpr bool PF = !WIDE || J <= 8;
+  constexpr int ROWS = 256 / GROUP;  // rows a workgroup has in hand
+  constexpr bool PF = J <= (WIDE ? 8 : 16);
   __shared__ float xs[2][4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t = WPR == 1 ? lane : (int)threadIdx.x;
-  const int slot = WPR == 1 ? blockIdx.x * 4 + wave : (int)blockIdx.x;
-  const int n_slots = WPR == 1 ? gridDim.x * 4 : (int)gridDim.x;
+  const int t = (int)threadIdx.x % GROUP;
+  const int slot = (int)blockIdx.x * ROWS + (int)threadIdx.x / GROUP;
+  const int n_slots = (int)gridDim.x * ROWS;
   const int D = p.dim;
   const int nch = D / EPC;
   const WeightRegs<TW, J, GROUP, EPC, !WIDE> w(reinterpret_cast<const TW*>(p.w), t, nch);
@@ -151,7 +155,7 @@ __global__ void __launch_bounds__(256) rms_fwd_vec_kernel(const RmsParams p) {
 #pragma unroll
         for (int e = 0; e < EPC; ++e) ss += cur.c[j].at(e) * cur.c[j].at(e);
       }
-    ss = group_sum<WPR>(ss, xs, par, wave, lane);
+    ss = group_sum<GROUP>(ss, xs, par, wave, lane);
     const float r = 1.0f / sqrtf(p.eps + ss / (float)D);
     T* y = reinterpret_cast<T*>(p.y) + row * p.y_st;
 #pragma unroll
@@ -193,22 +197,21 @@ __global__ void __launch_bounds__(256) rms_fwd_elem_kernel(const RmsParams p) {
 }
 
 // --------------------------------------------------------------- backward
-// WPR wavefronts (1 or 4) own a row at a time and walk rows slot, slot +
-// n_slots, ...; every thread keeps the dw contributions of its element
-// positions in registers and the workgroup writes ONE fp32 partial row (WPR ==
-// 1: the four wavefronts cover the same positions and add theirs through LDS).
-template <typename T, typename TW, int J, int WPR, bool WIDE>
+// GROUP threads (part of a wavefront, one, or a workgroup) own a row at a time
+// and walk rows slot, slot + n_slots, ...; every thread keeps the dw contributions of its element
+// positions in registers and the workgroup writes ONE fp32 partial row.
+template <typename T, typename TW, int J, int GROUP, bool WIDE>
 __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
   typedef Chunk<T, WIDE> C;
   constexpr int EPC = C::EPC;
-  constexpr int GROUP = 64 * WPR;
-  constexpr bool PF = !WIDE || J <= 4;  // two (x, dy) row pairs in registers
+  constexpr int ROWS = 256 / GROUP;  // rows a workgroup has in hand
+  constexpr bool PF = J <= (WIDE ? 4 : 16);  // two (x, dy) row pairs in registers
   __shared__ float xs[2][4];
-  __shared__ float red[WPR == 1 ? 4 : 1][64][EPC + 1];
+  __shared__ float red[GROUP <= 64 ? 4 : 1][64][EPC + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t = WPR == 1 ? lane : (int)threadIdx.x;
-  const int slot = WPR == 1 ? blockIdx.x * 4 + wave : (int)blockIdx.x;
-  const int n_slots = WPR == 1 ? gridDim.x * 4 : (int)gridDim.x;
+  const int t = (int)threadIdx.x % GROUP;
+  const int slot = (int)blockIdx.x * ROWS + (int)threadIdx.x / GROUP;
+  const int n_slots = (int)gridDim.x * ROWS;
   const int D = p.dim;
   const int nch = D / EPC;
   const WeightRegs<TW, J, GROUP, EPC, !WIDE> w(reinterpret_cast<const TW*>(p.w), t, nch);
@@ -252,7 +255,7 @@ __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
         for (int e = 0; e < EPC; ++e) dot += cd.c[j].at(e) * w.at(j, e) * cx.c[j].at(e);
       }
     }
-    dot = group_sum<WPR>(dot, xs, par, wave, lane);
+    dot = group_sum<GROUP>(dot, xs, par, wave, lane);
     const float k = r * r * r * dot / (float)D;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -285,7 +288,7 @@ __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
     for (int j = 0; j < J; ++j) dwacc[j][0] += dwold[WIDE ? 0 : j];
   }
   float* part = p.dw_part + (int64_t)blockIdx.x * D;
-  if (WPR > 1) {
+  if (GROUP > 64) {
     // every thread owns its positions of the workgroup's partial row
 #pragma unroll
     for (int j = 0; j < J; ++j) {
@@ -296,14 +299,20 @@ __global__ void __launch_bounds__(256) rms_bwd_vec_kernel(const RmsParams p) {
       }
     }
   } else {
-    // the four wavefronts cover the same positions: add through LDS, one chunk position at a time
+    // the groups of a wavefront and the four wavefronts cover the same positions: add by lane exchanges and
+    // through LDS, one chunk position at a time
 #pragma unroll
     for (int j = 0; j < J; ++j) {
 #pragma unroll
-      for (int e = 0; e < EPC; ++e) red[wave][lane][e] = dwacc[j][e];
+      for (int e = 0; e < EPC; ++e) {
+        float v = dwacc[j][e];
+#pragma unroll
+        for (int m = 32; m >= GROUP; m >>= 1) v += __shfl_xor(v, m, 64);
+        red[wave][lane][e] = v;
+      }
       __syncthreads();
-      if (wave == 0) {
-        const int ch = lane + 64 * j;
+      if (wave == 0 && lane < GROUP) {
+        const int ch = lane + GROUP * j;
         if (ch < nch) {
 #pragma unroll
           for (int e = 0; e < EPC; ++e)
@@ -421,46 +430,52 @@ int reduce_dw(const RmsParams& p, int n_parts, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-// Shapes of the chunked path.  16-byte chunks: rows of up to 128 are owned by
-// one wavefront (1 or 2 chunks per lane), longer ones by a workgroup of four.
-// Single elements: a wavefront owns rows of up to 1024, a workgroup up to 4096.
-constexpr int kWaveRowChunks = 128, kWaveRowElems = 1024, kMaxRowElems = 4096;
-constexpr int kMaxRowWorkgroups = 1024;
+// Shapes of the chunked path: GROUP threads with J chunks each.  16-byte
+// chunks: rows of up to 32 are owned by 8, 16 or 32 lanes, up to 128 by a
+// wavefront, longer ones by a workgroup.  Single elements: a wavefront owns rows
+// of up to 1024, a workgroup up to 8192.
+constexpr int kWaveRowChunks = 128, kWaveRowElems = 1024, kMaxRowElems = 8192;
+constexpr int kMaxRowWorkgroups = 1024, kMaxPartRowWorkgroups = 2048;
 
 template <typename F>
 void by_shape(bool wide, int nch, F&& f) {
   using std::integral_constant;
   using std::true_type;
   using std::false_type;
+  auto go = [&](auto j, auto group, auto w) { f(j, group, w); };
+#define MI_RMS_SHAPE(J, GROUP, W) go(integral_constant<int, J>{}, integral_constant<int, GROUP>{}, W{})
   if (!wide) {
-    if (nch <= 256)
-      f(integral_constant<int, 4>{}, integral_constant<int, 1>{}, false_type{});
-    else if (nch <= 512)
-      f(integral_constant<int, 8>{}, integral_constant<int, 1>{}, false_type{});
-    else if (nch <= kWaveRowElems)
-      f(integral_constant<int, 16>{}, integral_constant<int, 1>{}, false_type{});
-    else if (nch <= 2048)
-      f(integral_constant<int, 8>{}, integral_constant<int, 4>{}, false_type{});
-    else
-      f(integral_constant<int, 16>{}, integral_constant<int, 4>{}, false_type{});
-  } else if (nch <= 64)
-    f(integral_constant<int, 1>{}, integral_constant<int, 1>{}, true_type{});
-  else if (nch <= kWaveRowChunks)
-    f(integral_constant<int, 2>{}, integral_constant<int, 1>{}, true_type{});
-  else if (nch <= 256)
-    f(integral_constant<int, 1>{}, integral_constant<int, 4>{}, true_type{});
-  else if (nch <= 512)
-    f(integral_constant<int, 2>{}, integral_constant<int, 4>{}, true_type{});
-  else if (nch <= 1024)
-    f(integral_constant<int, 4>{}, integral_constant<int, 4>{}, true_type{});
-  else if (nch <= 2048)
-    f(integral_constant<int, 8>{}, integral_constant<int, 4>{}, true_type{});
-  else
-    f(integral_constant<int, kMaxJ>{}, integral_constant<int, 4>{}, true_type{});
+    if (nch <= 256) MI_RMS_SHAPE(4, 64, false_type);
+    else if (nch <= 512) MI_RMS_SHAPE(8, 64, false_type);
+    else if (nch <= kWaveRowElems) MI_RMS_SHAPE(16, 64, false_type);
+    else if (nch <= 2048) MI_RMS_SHAPE(8, 256, false_type);
+    else if (nch <= 4096) MI_RMS_SHAPE(16, 256, false_type);
+    else MI_RMS_SHAPE(32, 256, false_type);
+  } else {
+    if (nch <= 8) MI_RMS_SHAPE(1, 8, true_type);
+    else if (nch <= 16) MI_RMS_SHAPE(1, 16, true_type);
+    else if (nch <= 32) MI_RMS_SHAPE(1, 32, true_type);
+    else if (nch <= 64) MI_RMS_SHAPE(1, 64, true_type);
+    else if (nch <= kWaveRowChunks) MI_RMS_SHAPE(2, 64, true_type);
+    else if (nch <= 256) MI_RMS_SHAPE(1, 256, true_type);
+    else if (nch <= 512) MI_RMS_SHAPE(2, 256, true_type);
+    else if (nch <= 1024) MI_RMS_SHAPE(4, 256, true_type);
+    else if (nch <= 2048) MI_RMS_SHAPE(8, 256, true_type);
+    else MI_RMS_SHAPE(kMaxJ, 256, true_type);
+  }
+#undef MI_RMS_SHAPE
 }
 
-// workgroups of the chunked path (= partial dw rows of the backward pass)
+// Workgroups of the chunked path (= partial dw rows of the backward pass, so
+// never more than n_waves, which is at least the number of rows up to 4096).
+// Part-wavefront rows keep only 16 bytes per lane and row in flight: eight
+// workgroups per CU instead of four.
 inline unsigned vec_grid(const RmsParams& p, bool wide, int nch, int n_waves) {
+  if (wide && nch <= 32) {
+    const int rows_wg = 256 / (nch <= 8 ? 8 : nch <= 16 ? 16 : 32);
+    const int64_t wgs = (p.rows + rows_wg - 1) / rows_wg;
+    return (unsigned)(wgs < kMaxPartRowWorkgroups ? wgs : kMaxPartRowWorkgroups);
+  }
   if (nch <= (wide ? kWaveRowChunks : kWaveRowElems)) return (unsigned)(n_waves / 4);
   return (unsigned)(p.rows < kMaxRowWorkgroups ? p.rows : kMaxRowWorkgroups);
 }
