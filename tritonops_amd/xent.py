@@ -129,10 +129,13 @@ def cross_entropy_dlogits(x, w, y, lse, dloss):
     accumulators (replaces the logits GEMM + element-wise kernel of
     cross_entropy.py:374, :185-266, which round the logits to x's dtype first)."""
     _require_gpu(x, w, y, lse, dloss)
+    return _dlogits(x, w, y, lse, dloss, torch.empty((x.shape[0], w.shape[0]), device=x.device, dtype=x.dtype))
+
+
+def _dlogits(x, w, y, lse, dloss, dl):
     lib = _lib.load()
     T, N = x.shape[0], w.shape[0]
     xp, wp = _pad_dim(x), _pad_dim(w)
-    dl = torch.empty((T, N), device=x.device, dtype=x.dtype)
     a = _lib.XentBwdArgs()
     a.struct_size = C.sizeof(a)
     a.dtype = _tag(x)
@@ -142,9 +145,19 @@ def cross_entropy_dlogits(x, w, y, lse, dloss):
     a.x_stride = xp.stride(0) if T > 1 else xp.shape[1]
     a.w_stride = wp.stride(0) if N > 1 else wp.shape[1]
     a.lse, a.dloss = _ptr(lse), _ptr(dloss)
-    a.dlogits, a.ld = _ptr(dl), N
+    a.dlogits, a.ld = _ptr(dl), dl.stride(0) if T > 1 else N
     _lib.check(lib.mi_xent_bwd_dlogits(C.byref(a), _stream()))
     return dl
+
+
+def _dlogits_rows(rows, N, like):
+    """Room for dlogits [rows, N] as the two gradient products read them best:
+    rows start on 16-byte boundaries, which an odd vocabulary's own pitch does
+    not give, neither to the 16-byte stores of the kernels that write them nor
+    to the library's loads.  Forward + backward, 8192 tokens x 2048 x 50257:
+    5.31 -> 4.81 ms with padded rows, 1000 x 1024 x 50257: 0.75 -> 0.69."""
+    ld = N if N % 8 == 0 else -(-N // 64) * 64
+    return torch.empty((rows, ld), device=like.device, dtype=like.dtype)[:, :N]
 
 
 def _kept_dlogits(kept, first, y, lse, dloss, N, dl):
@@ -157,7 +170,7 @@ def _kept_dlogits(kept, first, y, lse, dloss, N, dl):
     a.tokens, a.vocab = dl.shape[0], N
     a.labels_i64 = 1 if y.dtype == torch.int64 else 0
     a.y, a.lse, a.dloss = _ptr(y), _ptr(lse), _ptr(dloss)
-    a.dlogits, a.ld = _ptr(dl), N
+    a.dlogits, a.ld = _ptr(dl), dl.stride(0) if dl.shape[0] > 1 else N
     at = C.c_void_p(kept.data_ptr() + lib.mi_xent_kept_bytes(first, N))
     _lib.check(lib.mi_xent_kept_dlogits(C.byref(a), at, _stream()))
     return dl
@@ -181,10 +194,10 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
     for s in range(0, T, step):
         e = min(s + step, T)
         xc = x[s:e]
+        dl = _dlogits_rows(e - s, w.shape[0], x)
         if kept is None:
-            dl = cross_entropy_dlogits(xc, w, y[s:e], lse[s:e], g[s:e])
+            _dlogits(xc, w, y[s:e], lse[s:e], g[s:e], dl)
         else:
-            dl = torch.empty((e - s, w.shape[0]), device=x.device, dtype=x.dtype)
             _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl)
         torch.mm(dl, w, out=grad_x[s:e])
         if grad_w is None:
