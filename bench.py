@@ -48,8 +48,9 @@ KERNELS = {
         "13bwd_dq_kernelIDF16bLi128EEEvNS_9BwdParamsEi",
         "15bwd_dkdv_kernelIDF16bLi128EEEvNS_9BwdParamsEii")),
     "rmsnorm": " + ".join(_NS + n for n in (
-        "18rms_fwd_vec_kernelIDF16bfLi2ELi4EEEvNS_9RmsParamsE", "18rms_bwd_vec_kernelIDF16bfLi2ELi4EEEvNS_9RmsParamsE",
-        "19rms_dw_stage_kernelILi4EEEvPKfPfii", "20rms_dw_reduce_kernelIfEEvPKfPT_ii")),
+        "18rms_fwd_vec_kernelIDF16bfLi2ELi256ELb1EEEvNS_9RmsParamsE",
+        "18rms_bwd_vec_kernelIDF16bfLi2ELi256ELb1EEEvNS_9RmsParamsE",
+        "17rms_dw_sum_kernelIfLi4ELi4EEEvPKfPT_ii")),
     "fused_xent": _NS + "16xent_gemm_kernelIDF16bLb0ELb0EEEvNS_10XentParamsE",
 }
 # the reference's own call forms run on the kernels of the configurations above
