@@ -51,6 +51,24 @@ def test_every_partition_meets_the_oracle(i, dtype):
     assert torch.equal(got, again)
 
 
+@pytest.mark.parametrize("lens,split", [([3000, 700], 64), ([5000], 64), (LONG[:1] * 8, 512), (LONG * 6, 2048)],
+                         ids=["chunks", "wavefronts", "one_wavefront", "ranges"])
+def test_nan_in_a_key_makes_its_heads_nan(lens, split):
+    """One key row that holds NaN: the query heads of its kv-head are NaN however many
+    chunks were merged, and nothing else is touched."""
+    import tritonops_amd as ta
+
+    B, L = len(lens), max(lens)
+    q, k, v = randn((B, 8, 128), 1).cuda(), randn((B, L, 2, 128), 2).cuda(), randn((B, L, 2, 128), 3).cuda()
+    sl = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    want = ta.flash_attention_decoding(q, k, v, None, seq_lens=sl, split_tokens=split)
+    k[0, 1777, 1, 5] = float("nan")
+    got, lse = ta.flash_attention_decoding(q, k, v, None, seq_lens=sl, split_tokens=split, return_lse=True)
+    assert got[0, 4:].isnan().all() and lse[0, 4:].isnan().all()
+    got[0, 4:] = want[0, 4:]
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("split_blocks", [1, 2, 5])
 @pytest.mark.parametrize("D", [64, 96, 128])
 def test_lists_of_few_chunks(D, split_blocks):

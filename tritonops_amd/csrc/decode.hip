@@ -307,7 +307,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
     const float l_tot = sum_with_other_half(l);
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if (lc.lq < gqa) {
-      if (lc.lh == 0) p.part_lse[slot] = l_tot > 0.f ? m + fast_log2(l_tot) : -INFINITY;
+      if (lc.lh == 0) p.part_lse[slot] = l_tot == 0.f ? -INFINITY : m + fast_log2(l_tot);  // NaN stays NaN
       float* po = p.part_o + slot * D;
 #pragma unroll
       for (int db = 0; db < G::NDB; ++db)
@@ -351,7 +351,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
     }
     const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
     if (lc.lq < gqa) {
-      if (lc.lh == 0 && wave == 0) p.part_lse[slot] = l_tot > 0.f ? M + fast_log2(l_tot) : -INFINITY;
+      if (lc.lh == 0 && wave == 0) p.part_lse[slot] = l_tot == 0.f ? -INFINITY : M + fast_log2(l_tot);
       float* po = p.part_o + slot * D;
 #pragma unroll
       for (int i = 0; i < QUADS / NW; ++i) {
@@ -504,7 +504,9 @@ decode_splitkv_kernel(const DecodeParams p) {
 // lanes take a slot, 8 slots of head_dim 128 at a time, instead of one thread
 // per column walking all slots one after the other: 9.2 -> 4.0 us for 2 sequences of 28
 // chunks, 8.3 -> 6.1 us for 64 of about 13 (32 heads of 128).
-// Slots marked -inf hold nothing; what lies in them is not used.
+// Slots marked -inf hold nothing; what lies in them is not used.  A NaN among a
+// chunk's scores arrives as a NaN log-sum-exp and makes the result NaN, however
+// the sequence was divided.
 constexpr int kMergeThreads = 256;
 template <typename T>
 __global__ void __launch_bounds__(kMergeThreads)
@@ -533,8 +535,7 @@ decode_merge_kernel(const DecodeParams p, int D) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) M = fmaxf(M, __shfl_xor(M, m, 64));
   float den = 0.f;
-  if (M > -INFINITY)
-    for (int c = lane; c < nvalid; c += 64) den += fast_exp2(pl[c] - M);
+  for (int c = lane; c < nvalid; c += 64) den += pl[c] == -INFINITY ? 0.f : fast_exp2(pl[c] - M);
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) den += __shfl_xor(den, m, 64);
 
@@ -562,8 +563,8 @@ decode_merge_kernel(const DecodeParams p, int D) {
     float sum = 0.f;
     for (int g = 0; g < groups; ++g) sum += col[g * D];
     T* op = reinterpret_cast<T*>(p.o) + b * p.o_sb + h * p.o_sh;
-    op[d] = (T)(den > 0.f ? sum / den : 0.f);
-    if (d == 0 && p.lse) p.lse[(int64_t)b * p.hq + h] = den > 0.f ? M + fast_log2(den) : -INFINITY;
+    op[d] = (T)(den == 0.f ? 0.f : sum / den);
+    if (d == 0 && p.lse) p.lse[(int64_t)b * p.hq + h] = den == 0.f ? -INFINITY : M + fast_log2(den);
   }
 }
 
