@@ -1063,7 +1063,7 @@ __device__ __forceinline__ void walk_items(const BwdParams& p, const int n_items
   const int grid = gridDim.x;
   if (threadIdx.x < kMaxRounds) {
     const ItemId ids = items_of_rounds<ROWS, FROM_END>(p.cu, p.batch, p.max_seqlen, n_rt, heads, heads_kv,
-                                                       heads / heads_kv, p.by_level, n_items, grid);
+                                                       p.by_level, n_items, grid);
     list[threadIdx.x] = ids.t;
     list[kMaxRounds + threadIdx.x] = ids.b;
     list[2 * kMaxRounds + threadIdx.x] = ids.h;

@@ -44,9 +44,8 @@ struct ItemGeo {
   int64_t q_off, k_off, v_off, o_off, lse_off;
 };
 
-// The rest of an item's geometry from its sequence g.b, q-head g.h and q tile g.qt.
+// The rest of an item's geometry from its sequence g.b, heads g.h and g.kvh and q tile g.qt.
 __device__ __forceinline__ void finish_geo(const PrefillParams& p, ItemGeo& g) {
-  g.kvh = g.h / (p.hq / p.hkv);
   if (p.cu) {
     const int start = p.cu[g.b];
     // (a sequence longer than the caller's bound is cut at the bound: the grid covers no row beyond it)
@@ -88,7 +87,8 @@ __device__ __forceinline__ bool item_geo(const PrefillParams& p, const int bid, 
   }
   g.qt = p.n_qtiles - 1 - s / gqa;
   g.b = unit / p.hkv;
-  g.h = (unit % p.hkv) * gqa + s % gqa;
+  g.kvh = unit % p.hkv;
+  g.h = g.kvh * gqa + s % gqa;
   finish_geo(p, g);
   return g.qt * BM < g.len;
 }
@@ -101,6 +101,7 @@ __device__ __forceinline__ bool next_geo(const PrefillParams& p, const ItemId& i
   g.qt = __builtin_amdgcn_readlane(ids.t, at);
   g.b = __builtin_amdgcn_readlane(ids.b, at);
   g.h = __builtin_amdgcn_readlane(ids.h, at);
+  g.kvh = __builtin_amdgcn_readlane(ids.kvh, at);
   finish_geo(p, g);
   return true;
 }
@@ -795,7 +796,7 @@ dense_kernel(const PrefillParams p) {
     float* lp;  // LSE row of this head, or null
     KvSrc<T> kv;
   };
-  const ItemId ids = items_of_rounds<BM, false>(p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv, p.hq / p.hkv,
+  const ItemId ids = items_of_rounds<BM, false>(p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv,
                                                 p.by_level, p.n_items, gridDim.x);
   uint64_t left = __builtin_amdgcn_ballot_w64(ids.t >= 0);
   // advance to the next item of this workgroup that has rows; false when there is none
@@ -1253,7 +1254,7 @@ dense_short_kernel(const PrefillParams p) {
     return WIN ? (j + (j >= it.n_sink ? it.skip : 0)) * TN : j * TN;
   };
   const int wl = p.win_local, wg = p.win_global;
-  const ItemId ids = items_of_rounds<BM, false>(p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv, p.hq / p.hkv,
+  const ItemId ids = items_of_rounds<BM, false>(p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv,
                                                 p.by_level, p.n_items, gridDim.x);
   uint64_t left = __builtin_amdgcn_ballot_w64(ids.t >= 0);
   auto next_item = [&](Item& it) __attribute__((always_inline)) -> bool {
