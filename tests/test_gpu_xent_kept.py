@@ -82,6 +82,51 @@ def test_rows_in_blocks_and_a_second_backward(monkeypatch):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("rows", [1, 255, 256, 257, 1000, 1024, 16384])
+def test_row_blocks_of_kept_logits_start_on_whole_tiles(monkeypatch, rows):
+    """Whatever number of rows the backward takes at a time.  (On the CPU: only where
+    the blocks lie, with a stand-in for the kernel.)"""
+    from tritonops_amd import xent
+
+    blocks = []
+
+    def kept_dlogits(kept, first, y, lse, dloss, N, dl):
+        blocks.append((first, dl.shape[0]))
+        return dl.zero_()
+
+    monkeypatch.setattr(xent, "_require_gpu", lambda *ts: None)
+    monkeypatch.setattr(xent, "_kept_dlogits", kept_dlogits)
+    x, w, y, go = _inputs(1001, 16, 8, torch.float32)
+    xent._bwd(go, x, w, y, torch.zeros(1001), object(), rows)
+    assert all(first % 256 == 0 for first, _ in blocks)
+    assert blocks[0][0] == 0 and sum(n for _, n in blocks) == 1001
+    assert all(a + n == b for (a, n), (b, _) in zip(blocks, blocks[1:]))
+    assert max(n for _, n in blocks) <= max(rows, 256)
+
+
+def test_kept_rows_that_start_inside_a_tile_are_refused():
+    from tritonops_amd import xent
+
+    with pytest.raises(ValueError):
+        xent._kept_dlogits(torch.zeros(1), 1000, None, None, None, 8, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [100, 1000])
+def test_rows_in_blocks_that_are_no_whole_tiles(monkeypatch, rows):
+    from tritonops_amd import xent
+
+    x, w, y, go = _inputs(1001, 128, 700, torch.bfloat16)
+    monkeypatch.setattr(xent, "BWD_ROWS", rows)
+    again, kept = _both(x, w, y, go)
+    assert torch.equal(again[0], kept[0])
+    # both divide the rows in other blocks: dx is rounded once to bf16 (2^-8 of a value that the order of its fp32
+    # sum has moved across a rounding point), dw once per block of rows, eleven of them at 100
+    dx, dw = xo.linear_cross_entropy_backward(go, x, w, y)
+    for got, want, tol in ((kept[1], dx, 2e-2), (kept[2], dw, 4e-2)):
+        assert (got.cpu().double() - want).abs().max() <= tol * max(1.0, want.abs().max().item())
+
+
 @pytest.mark.gpu
 def test_when_the_logits_are_kept(monkeypatch):
     import tritonops_amd as ta

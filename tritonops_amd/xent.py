@@ -17,6 +17,9 @@ _TAGS = {torch.bfloat16: _lib.MI_DTYPE_BF16, torch.float16: _lib.MI_DTYPE_F16}
 # Rows of logits that the backward materialises at a time (the reference uses
 # 2048, cross_entropy.py:367; a 288 GB device holds far larger blocks).
 BWD_ROWS = 16384
+# Kept logits lie in tiles of this many tokens: a block of rows read from them
+# starts on a tile (BWD_ROWS is rounded down to whole tiles there, to one at least).
+_KEPT_ROWS = 256
 # The forward of a call that will be differentiated keeps its fp32 logits where
 # that is at most KEEP_BYTES (of 288 GB, from the forward to the backward) and
 # the rows have at least KEEP_DIM elements: 8 bytes per logit go through memory
@@ -161,8 +164,10 @@ def _dlogits_rows(rows, N, like):
 
 
 def _kept_dlogits(kept, first, y, lse, dloss, N, dl):
-    """dl [rows, N] <- dlogits of the rows from `first` on (a multiple of 256),
+    """dl [rows, N] <- dlogits of the rows from `first` on (a multiple of _KEPT_ROWS),
     from the logits that _fwd kept; the values of cross_entropy_dlogits."""
+    if first % _KEPT_ROWS:
+        raise ValueError("rows of kept logits start at a multiple of %d, not at %d" % (_KEPT_ROWS, first))
     lib = _lib.load()
     a = _lib.XentBwdArgs()
     a.struct_size = C.sizeof(a)
@@ -189,6 +194,8 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
     y = _labels(y, T)
     g = grad_o.reshape(-1).to(torch.float32).contiguous()
     lse = lse.contiguous()
+    if kept is not None and step % _KEPT_ROWS:
+        step = max(step - step % _KEPT_ROWS, _KEPT_ROWS)
     grad_x = torch.empty_like(x)
     grad_w = None
     for s in range(0, T, step):
