@@ -239,11 +239,12 @@ int mi_attn_fwd_blocksparse(const mi_attn_sparse_args *args, void *stream);
  * reference fetches it once per query head, flash_attn_decoding.py:42-45,
  * 264-268); any ratio G is accepted.
  *
- * Pass 1 splits each sequence into at most ceil(max_seqlen / split_tokens)
- * chunks (dense; where they begin follows from the lengths of the batch, so that
- * all workgroups have the same work) or chunks of `split_blocks` listed blocks
- * (sparse); a workgroup writes a chunk's fp32 partial output and its base-2 LSE
- * for one kv-head into the workspace.  Pass 2 merges the partials (flash_attn_decoding.py:171-208).
+ * Pass 1 splits each sequence into chunks of `split_tokens` tokens (dense) or
+ * `split_blocks` listed blocks (sparse); a workgroup writes a chunk's fp32
+ * partial output and its base-2 LSE for one kv-head into the workspace.  Pass 2
+ * merges the partials (flash_attn_decoding.py:171-208).  A row's bits follow from
+ * its own query, keys, values and length and from the split: the other sequences
+ * of the batch have no part in them.
  * seq_lens[b] == 0 gives an all-zero output row (flash_attn_decoding.py:49-50,
  * 151,197-210).
  *
@@ -300,8 +301,7 @@ typedef struct mi_decode_args {
   int32_t head_dim;              /* 64, 96 or 128                              */
   float scale_log2;
   /* split-KV */
-  int32_t split_tokens;          /* dense: sets the chunks per sequence (above),*/
-                                 /* multiple of 64                             */
+  int32_t split_tokens;          /* dense: tokens per chunk, multiple of 64    */
   void *workspace;               /* device, mi_decode_workspace_bytes() bytes  */
   size_t workspace_bytes;
   /* block-sparse (all ignored when block_idx == NULL) */

@@ -1,8 +1,7 @@
-"""How a decoding launch divides its work: chunks of one sequence, tile ranges that
-run across sequences (csrc/decode.hip, decode_splitkv_kernel), one, two or four
-wavefronts to a chunk, and slots of the workspace that stay empty.  The workspace
-comes out of memory that held NaN, so a slot that is used without having been
-written shows."""
+"""How a decoding launch divides its work (csrc/decode.hip): chunks of split_tokens
+tokens or split_blocks blocks, one, two or four wavefronts to a chunk, and slots of
+the workspace that stay empty.  The workspace comes out of memory that held NaN, so
+a slot that is used without having been written shows."""
 import pytest
 import torch
 
@@ -15,12 +14,12 @@ TOL = 2e-2
 LONG = [3000, 0, 1, 31, 32, 33, 4095, 2048, 0, 700]
 CASES = [
     # lens, Hq, Hkv, D, split_tokens, max_seq_len
-    (LONG, 32, 8, 128, 64, None),         # many slots: equal chunks of four tiles and more
-    (LONG * 6, 32, 8, 128, 2048, None),   # two slots to a sequence: ranges, bounded by the slots
-    (LONG * 6, 64, 32, 96, 512, None),    # ranges, several rounds' worth of sequences
+    (LONG, 32, 8, 128, 64, None),         # many slots of two tiles
+    (LONG * 6, 32, 8, 128, 2048, None),   # two slots to a sequence
+    (LONG * 6, 64, 32, 96, 512, None),    # several rounds of chunks
     (LONG * 13, 16, 16, 64, 256, None),   # 130 sequences: the search steps over the batch
     (LONG, 8, 8, 64, 4096, None),         # one slot: whole sequences
-    ([5000], 4, 1, 128, 64, None),        # one sequence, 4 wavefronts to a chunk
+    ([5000], 4, 1, 128, 64, None),        # one sequence, two wavefronts to a chunk of two tiles
     ([8192], 80, 2, 128, 1024, None),     # two slices of query heads
     ([1, 2], 8, 2, 96, None, 4096),       # one tile each under a large bound
     ([0, 0, 0], 8, 2, 64, None, 512),     # nothing at all
@@ -85,3 +84,58 @@ def test_lists_of_few_chunks(D, split_blocks):
                                              block_indices=idx.cuda(), block_counts=cnt.cuda(),
                                              split_blocks=split_blocks)
     assert_close(got, want, TOL)
+
+
+def _rows(lens, Hq, Hkv, D, room):
+    B = len(lens)
+    return (randn((B, Hq, D), 5).cuda(), randn((B, room, Hkv, D), 6).cuda(), randn((B, room, Hkv, D), 7).cuda(),
+            torch.tensor(lens, dtype=torch.int32, device="cuda"))
+
+
+@pytest.mark.parametrize("split", [None, 64, 512, 4096])
+def test_a_row_does_not_depend_on_the_lengths_of_its_neighbours(split):
+    """The same bits for a row whatever the other sequences of the batch hold, and (where
+    the caller says how long a chunk is) alone."""
+    import tritonops_amd as ta
+
+    lens = [3000, 4095, 1, 700, 2049, 32]
+    q, k, v, sl = _rows(lens, 32, 8, 128, 4096)
+    o, lse = ta.flash_attention_decoding(q, k, v, None, seq_lens=sl, split_tokens=split, return_lse=True)
+    for i in range(len(lens)):
+        for others in (4096, 5, 0):
+            ln = torch.full_like(sl, others)
+            ln[i] = lens[i]
+            o2, lse2 = ta.flash_attention_decoding(q, k, v, None, seq_lens=ln, split_tokens=split, return_lse=True)
+            assert torch.equal(o2[i], o[i]) and torch.equal(lse2[i], lse[i]), (i, others)
+        if split:
+            one = slice(i, i + 1)
+            o1, lse1 = ta.flash_attention_decoding(q[one], k[one], v[one], None, seq_lens=sl[one], split_tokens=split,
+                                                   return_lse=True)
+            assert torch.equal(o1[0], o[i]) and torch.equal(lse1[0], lse[i]), i
+
+
+@pytest.mark.parametrize("D", [64, 96, 128])
+@pytest.mark.parametrize("length", [4096, 3937, 33])
+def test_bits_do_not_depend_on_the_number_of_wavefronts(D, length):
+    """A launch of few chunks puts four wavefronts to a chunk, one of many chunks two or one
+    (up to 2048 wavefronts are resident): chunks of 256 tokens and of four blocks, 8 kv-heads."""
+    import tritonops_amd as ta
+
+    q, k, v, sl = _rows([length], 32, 8, D, 4096)
+    blocks = torch.arange(0, (length + 63) // 64, 2, dtype=torch.int32, device="cuda").expand(1, 8, -1)
+
+    def dense(B):
+        r = lambda t: t.expand(B, *t.shape[1:])
+        return ta.flash_attention_decoding(r(q), r(k), r(v), None, seq_lens=r(sl).contiguous(), split_tokens=256,
+                                           return_lse=True)
+
+    def listed(B):
+        r = lambda t: t.expand(B, *t.shape[1:])
+        return ta.flash_attention_sparse_decoding(r(q), r(k), r(v), None, seq_lens=r(sl).contiguous(),
+                                                  block_indices=r(blocks), split_blocks=4, return_lse=True)
+
+    for call in (dense, listed):
+        want = call(1)
+        for B in (3, 8, 40):
+            for got, w in zip(call(B), want):
+                assert torch.equal(got, w.expand_as(got)), (call.__name__, B)

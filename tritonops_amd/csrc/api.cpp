@@ -602,14 +602,17 @@ size_t mi_decode_workspace_bytes(const mi_decode_args* a) {
 }
 
 int mi_decode_choose_split_tokens(int batch, int heads_kv, int max_seqlen, int num_cus) {
-  // The dense kernel deals the live chunks to one resident round of wavefronts
-  // (8 per CU).  Chunks of about half a round's share keep every wavefront's
+  // The dense kernel deals the live chunks to one resident round of workgroups
+  // (8 wavefronts per CU).  The bound stands in for the lengths, which the host
+  // does not know, and no length has a part in the choice, so that a row's
+  // chunks do not move with its neighbours.  Chunks of about half a round's share keep every wavefront's
   // fixed costs (first tile, partial results, merge) small against its stream;
   // beyond 2048 tokens nothing is gained, and the shortest chunk worth a
   // partial result is 512 tokens, or 256 where that still leaves a sequence in
   // no more than 32 chunks for the merge (measured on 1 to 64 sequences of 8k,
-  // 32k and 128k tokens: 1 to 4 sequences of 8k take 29 to 36 us with chunks of
-  // 256 tokens against 36 to 43 us with 512, one sequence of 32k 63 against 55).
+  // 32k and 128k tokens, one wavefront to a chunk: 1 to 4 sequences of 8k take 29
+  // to 36 us with chunks of 256 tokens against 36 to 43 us with 512, one sequence
+  // of 32k 63 against 55).
   if (batch <= 0 || heads_kv <= 0 || max_seqlen <= 0) return 64;
   if (num_cus <= 0) num_cus = 256;
   const long long work = (long long)batch * heads_kv * max_seqlen;  // tokens x kv-heads

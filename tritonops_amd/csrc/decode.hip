@@ -6,11 +6,12 @@
 // twins in flash_attn_triton/flash_attn_decoding_sparse.py:10-127,:131-219.
 //
 // Pass 1: a work item is a (chunk, kv-head, sequence) triple and is handled
-// by one workgroup of NW wavefronts: one where the items fill the chip, two or
-// four, which share a chunk's tiles and merge in LDS, where they do not.  The
-// block-list form launches one workgroup per item; the dense form launches one
-// resident round (8 wavefronts per CU) and divides the tiles that the batch
-// really has among its workgroups (decode_splitkv_kernel).
+// by one workgroup of NW wavefronts.  A sequence's chunks follow from its own
+// length and split_tokens (split_blocks) alone, and a chunk's tiles are worked on
+// in order whatever NW is, so a row's bits depend neither on the other sequences
+// of the batch nor on the launch.  The block-list form launches one workgroup
+// per item; the dense form launches one resident round (8 wavefronts per CU)
+// and deals the live chunks of a ragged batch to them round-robin.
 // The G = hq/hkv query heads that share the kv-head sit in the first G of the 32
 // query columns of the same S^T = K.Q^T / O^T = V^T.P^T MFMA pipeline the
 // prefill kernel uses, so each K/V byte is fetched once for the whole group
@@ -20,11 +21,13 @@
 // item of its own: KV is then fetched once per slice.  KV streams global -> registers -> wave-private LDS in 32-key tiles
 // with fully coalesced 16-byte loads (non-temporal: every byte is used once);
 // as soon as a tile has arrived, each register is written to LDS and refilled
-// with its part of the tile after next.  No barriers are needed because a
-// single wave's LDS operations execute in order.  Partials are fp32 (the reference
-// rounds them to the input dtype, :249-251).
+// with its part of the tile after next.  With one wavefront no barriers are
+// needed because a single wave's LDS operations execute in order; several take
+// the tiles of a chunk in steps of NW, a tile each, between two barriers.
+// Partials are fp32 (the reference rounds them to the input dtype, :249-251).
 // Pass 2: per (sequence, q-head) merge  o = sum_c o_c 2^(lse_c - lse).
 #include <atomic>
+#include <type_traits>
 
 #include "kernels.h"
 #include "tile_core.h"
@@ -57,36 +60,50 @@ __device__ __forceinline__ WindowList window_list(int len, int wg, int wl) {
   return w;
 }
 
-// Bytes of LDS a wavefront owns: its K / V tile, and behind the tile loop of a
-// workgroup of several wavefronts its accumulators, running max and row sum.
+// LDS of a workgroup: the K tiles of its wavefronts, then their V tiles.
 template <int D>
 constexpr int wave_lds() {
   using F = PaddedFrags<D>;
   return kDecTile * (F::KROWB + F::VROWB);
 }
 
+// Barrier between the wavefronts of a workgroup that orders LDS accesses only:
+// the loads of the next tiles stay in flight across it.
+template <int NW>
+__device__ __forceinline__ void lds_barrier() {
+  if constexpr (NW > 1) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  }
+}
+
 // One work item: chunk `split` of (sequence b, kv-head kvh) for the 32 query
 // heads of the group that start at head g0 of it (slice kvs % gslices; a group
-// of up to 32 heads is one slice).  Dense form: the chunk is the n_dense tiles
-// from tile t_dense on, `split` is the slot of the partial result, and the
-// slots from fill_from on (fill_from >= 0: this chunk is the sequence's last)
-// are marked empty for the merge.
+// of up to 32 heads is one slice).
+//
+// NW > 1: the wavefronts fetch NW tiles at a time, one each, every wavefront
+// works out all their scores and probabilities and 1 / NW of the output columns
+// (blocks of 32, wave + NW j).  What is computed, and in which order, is what one wavefront computes,
+// bit for bit; matrix and vector units have room for the repeated scores (memory
+// is the bound), and the output needs no merge between wavefronts.
 template <typename T, int D, int NW, bool LIST>
-__device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char* smem_all, const int split, const int kvs,
-                                            const int b, const int t_dense, const int n_dense, const int fill_from) {
+__device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char* smem, const int split, const int kvs,
+                                            const int b) {
   const int kvh = kvs / p.gslices;
   const int g0 = (kvs % p.gslices) * 32;
   using G = RowGeom<D>;
   using F = PaddedFrags<D>;
   constexpr int KTILEB = kDecTile * F::KROWB;
   constexpr int NCHUNK = kDecTile * G::NCH;
+  constexpr int VTILEB = kDecTile * F::VROWB;
   constexpr int LOADS = (NCHUNK + 63) / 64;
+  constexpr int NB = (G::NDB + NW - 1) / NW;  // output blocks of a wavefront
 
   const int lane = threadIdx.x & 63;
   const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  unsigned char* smem = smem_all + wave * wave_lds<D>();
   unsigned char* sK = smem;
-  unsigned char* sV = smem + KTILEB;
+  unsigned char* sV = smem + NW * KTILEB;
 
   const int len = p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
   const int gqa_all = p.hq / p.hkv;
@@ -115,12 +132,9 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
     n_tiles = 2 * min(total - b0, p.split_blocks);
     n_listed = max(0, min(cnt - b0, p.split_blocks));
   } else {
-    t_begin = t_dense * kDecTile;
-    n_tiles = n_dense;
+    t_begin = split * p.split_tokens;
+    n_tiles = (min(len - t_begin, p.split_tokens) + kDecTile - 1) / kDecTile;
   }
-  // this wavefront's share of the chunk's tiles
-  const int i_begin = NW == 1 ? 0 : wave * n_tiles / NW;
-  const int i_end = NW == 1 ? n_tiles : (wave + 1) * n_tiles / NW;
   // sparse: entry i/2 of the chunk; entries behind the listed ones are the
   // implicit last block, and a LISTED last block is dropped when the implicit
   // one exists (base -1 => the whole tile is masked)
@@ -165,9 +179,9 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
     }
   }
 
-  f32x16 O[G::NDB];
+  f32x16 O[NB];
 #pragma unroll
-  for (int db = 0; db < G::NDB; ++db) O[db] = (f32x16){0};
+  for (int j = 0; j < NB; ++j) O[j] = (f32x16){0};
   float m = -INFINITY, l = 0.f;
 
   // The loads of tile t + 1 fly while tile t is worked on.  (Registers for a
@@ -226,8 +240,8 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
     const int idx = lane + i * 64;
     if (NCHUNK % 64 != 0 && idx >= NCHUNK) return;
     const int row = idx / G::NCH, ch = idx % G::NCH;
-    F::store_k(sK, row, ch, kreg[i]);
-    F::store_v(sV, row, ch, vreg[i]);
+    F::store_k(sK + wave * KTILEB, row, ch, kreg[i]);
+    F::store_v(sV + wave * VTILEB, row, ch, vreg[i]);
   };
   // where a tile comes from: uniform addresses of its first K / V row and the
   // last row that may be read
@@ -249,253 +263,153 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
   };
 
   const int wl = LIST ? p.win_local : -1, wg = p.win_global;
-  // Tile t is worked on from LDS while tile t + 1 is in flight into the
-  // registers.  When it has arrived, every register is written to LDS and
-  // refilled at once with its part of tile t + 2, so that the next loads leave
-  // as early as possible; the address of tile t + 2 (block list and page
-  // look-ups) is prepared before tile t is worked on.
-  int base_cur = 0, base_nxt = 0;
-  TileSrc src = {0, 0, 0};  // the second tile, then the tile two ahead of the compute
-  if (NW == 1 || i_begin < i_end) {
-    base_cur = tile_base(i_begin);
-    const TileSrc t0 = tile_src(base_cur);
+  // A step is NW tiles, tile `wave` of each fetched by this wavefront.  Step t is
+  // worked on from LDS while the tiles of step t + 1 are in flight into the
+  // registers.  When they have arrived, every register is written to LDS and
+  // refilled at once with its part of step t + 2, so that the next loads leave
+  // as early as possible; the addresses of step t + 2 (block list and page
+  // look-ups) are prepared before step t is worked on.
+  auto step_bases = [&](int i0, int (&base)[NW]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_pair(i, t0);
-    base_nxt = i_begin + 1 < i_end ? tile_base(i_begin + 1) : 0;
-    src = tile_src(base_nxt);
+    for (int j = 0; j < NW; ++j) base[j] = i0 + j < n_tiles ? tile_base(i0 + j) : 0;
+  };
+  int cur[NW], nxt[NW];
+  step_bases(0, cur);
+  step_bases(NW, nxt);
+  TileSrc src = tile_src(wave < n_tiles ? tile_base(wave) : 0);  // the first tile, the second, then the one two ahead of the compute
+  if (wave < n_tiles) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) load_pair(i, src);
+    if (NW + wave < n_tiles) src = tile_src(tile_base(NW + wave));
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       store_one(i);
-      if (i_begin + 1 < i_end) load_pair(i, src);
+      if (NW + wave < n_tiles) load_pair(i, src);
     }
   }
-  for (int it = i_begin; it < i_end; ++it) {
-    const int base = base_cur;
-    base_cur = base_nxt;
-    const bool refill = it + 2 < i_end;
-    if (refill) {
-      base_nxt = tile_base(it + 2);
-      src = tile_src(base_nxt);
+  for (int i0 = 0; i0 < n_tiles; i0 += NW) {
+    lds_barrier<NW>();
+    const bool refill = i0 + 2 * NW + wave < n_tiles;
+    int nn[NW];
+    step_bases(i0 + 2 * NW, nn);
+    if (refill) src = tile_src(tile_base(i0 + 2 * NW + wave));
+    if (NW == 1 || wave < G::NDB) {
+      // (scores of tiles behind the chunk's last are computed and not used)
+      f32x16 S[NW];
+      qk_scores<T, D, NW>(sK, lc, Qf, S);
+      auto tile = [&](auto tc) __attribute__((always_inline)) {
+        constexpr int t = decltype(tc)::value;
+        if (NW > 1 && i0 + t >= n_tiles) return;
+        const int base = cur[t];
+        bool need_mask = base + kDecTile > len || base < 0;
+        if (wl >= 0) need_mask = need_mask || !((base + kDecTile - 1 < wg) || (base >= len - wl));
+        auto allowed = [&](int key_in_tile) -> bool {
+          const int key = base + key_in_tile;
+          bool ok = key < len && base >= 0;
+          if (wl >= 0) ok = ok && (key < wg || key >= len - wl);
+          return ok;
+        };
+        f32x16 S1[1] = {S[t]};
+        uint32_t P[1][8];
+        softmax_tile<T, D, 1>(S1, lc.lh, O, m, l, p.scale, need_mask, allowed, P);
+        pv_accumulate<T, D, 1, NW>(sV + t * VTILEB + wave * 64, lc, P, O);
+      };
+      using std::integral_constant;  // (a loop of this size is not unrolled, and S and cur went to scratch)
+      tile(integral_constant<int, 0>{});
+      if constexpr (NW > 1) tile(integral_constant<int, 1>{});
+      if constexpr (NW > 2) tile(integral_constant<int, 2>{}), tile(integral_constant<int, 3>{});
     }
-    bool need_mask = base + kDecTile > len || base < 0;
-    if (wl >= 0) need_mask = need_mask || !((base + kDecTile - 1 < wg) || (base >= len - wl));
-    auto allowed = [&](int key_in_tile) -> bool {
-      const int key = base + key_in_tile;
-      bool ok = key < len && base >= 0;
-      if (wl >= 0) ok = ok && (key < wg || key >= len - wl);
-      return ok;
-    };
-    compute_tile<T, D, 1>(sK, sV, lc, Qf, O, m, l, p.scale, need_mask, allowed);
-    if (it + 1 < i_end) {
+    lds_barrier<NW>();
+    if (i0 + NW + wave < n_tiles) {
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
         store_one(i);
         if (refill) load_pair(i, src);
       }
     }
+#pragma unroll
+    for (int j = 0; j < NW; ++j) {
+      cur[j] = nxt[j];
+      nxt[j] = nn[j];
+    }
   }
 
-  // slot of query head h: row (b, h), column `split`
-  const int64_t row0 = (int64_t)b * p.hq + kvh * gqa_all + g0;
-  if (fill_from >= 0 && wave == 0) {
-    const int n_fill = p.n_splits - fill_from;
-    for (int i = lane; i < n_fill * gqa; i += 64)
-      p.part_lse[(row0 + i % gqa) * p.n_splits + fill_from + i / gqa] = -INFINITY;
-  }
-  const int64_t slot = (row0 + lc.lq) * p.n_splits + split;
-  if constexpr (NW == 1) {
-    const float l_tot = sum_with_other_half(l);
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (lc.lq < gqa) {
-      if (lc.lh == 0) p.part_lse[slot] = l_tot == 0.f ? -INFINITY : m + fast_log2(l_tot);  // NaN stays NaN
-      float* po = p.part_o + slot * D;
+  const float l_tot = sum_with_other_half(l);
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  if (lc.lq < gqa) {
+    const int h = kvh * gqa_all + g0 + lc.lq;
+    const int64_t slot = ((int64_t)b * p.hq + h) * p.n_splits + split;
+    // (a NaN sum stays NaN)
+    if (lc.lh == 0 && wave == 0) p.part_lse[slot] = l_tot == 0.f ? -INFINITY : m + fast_log2(l_tot);
+    float* po = p.part_o + slot * D;
 #pragma unroll
-      for (int db = 0; db < G::NDB; ++db)
+    for (int j = 0; j < NB; ++j) {
+      const int db = wave + NW * j;
+      if (G::NDB % NW != 0 && db >= G::NDB) break;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          float4 w = {O[db][4 * g] * inv, O[db][4 * g + 1] * inv, O[db][4 * g + 2] * inv,
-                      O[db][4 * g + 3] * inv};
-          *reinterpret_cast<float4*>(po + 32 * db + 8 * g + 4 * lc.lh) = w;
-        }
-    }
-  } else {
-    // The wavefronts' partial results meet in LDS, each in the tile it no
-    // longer needs: quad j of a lane at [j][lane], then max and sum per lane.
-    // A wavefront then writes every NW-th quad of the merged row.
-    constexpr int QUADS = 4 * G::NDB;
-    static_assert(QUADS * 64 * 16 + 2 * 64 * 4 <= wave_lds<D>(), "accumulators fit a wavefront's tile");
-    float4* mine = reinterpret_cast<float4*>(smem);
-#pragma unroll
-    for (int db = 0; db < G::NDB; ++db)
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        mine[(4 * db + g) * 64 + lane] =
-            (float4){O[db][4 * g], O[db][4 * g + 1], O[db][4 * g + 2], O[db][4 * g + 3]};
-    float* ml = reinterpret_cast<float*>(smem + QUADS * 64 * 16);
-    const float l_wave = sum_with_other_half(l);
-    ml[lane] = m;
-    ml[64 + lane] = l_wave;
-    __syncthreads();
-    float mw[NW], lw[NW], M = -INFINITY, l_tot = 0.f;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float* o = reinterpret_cast<const float*>(smem_all + w * wave_lds<D>() + QUADS * 64 * 16);
-      mw[w] = o[lane];
-      lw[w] = o[64 + lane];
-      M = fmaxf(M, mw[w]);
-    }
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      mw[w] = mw[w] == -INFINITY ? 0.f : fast_exp2(mw[w] - M);  // factor of wavefront w
-      l_tot += lw[w] * mw[w];
-    }
-    const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-    if (lc.lq < gqa) {
-      if (lc.lh == 0 && wave == 0) p.part_lse[slot] = l_tot == 0.f ? -INFINITY : M + fast_log2(l_tot);
-      float* po = p.part_o + slot * D;
-#pragma unroll
-      for (int i = 0; i < QUADS / NW; ++i) {
-        const int j = i * NW + wave;
-        float4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-          const float4 x = reinterpret_cast<const float4*>(smem_all + w * wave_lds<D>())[j * 64 + lane];
-          acc.x += x.x * mw[w];
-          acc.y += x.y * mw[w];
-          acc.z += x.z * mw[w];
-          acc.w += x.w * mw[w];
-        }
-        *reinterpret_cast<float4*>(po + 8 * j + 4 * lc.lh) =
-            (float4){acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+      for (int g = 0; g < 4; ++g) {
+        float4 w = {O[j][4 * g] * inv, O[j][4 * g + 1] * inv, O[j][4 * g + 2] * inv, O[j][4 * g + 3] * inv};
+        *reinterpret_cast<float4*>(po + 32 * db + 8 * g + 4 * lc.lh) = w;
       }
     }
-    __syncthreads();  // the next item's tiles go where these results are read from
   }
 }
 
 // Block-list form: one workgroup per (chunk, kv-head, sequence), grid
-// (n_splits, hkv, batch).
-//
-// Dense form: bound by memory, so the launch is one resident round and ends
-// well only if every wavefront has the same number of bytes to fetch.  What the
-// batch really holds is known on the device alone; with total, the 32-key tiles
-// of all sequences, and R workgroups for each (kv-head, 32-head slice):
-//  - chunks: every sequence in equal chunks of about c tiles, one chunk to a
-//    workgroup, c = total / (R - sequences) rounded up, so that there are no
-//    more chunks than workgroups; c is at least kMinChunk tiles and large enough
-//    for the sequence's n_splits slots;
-//  - ranges: the tiles of all sequences in a row, W = total / R of them to a
-//    workgroup, which writes a partial result for each sequence it touches;
-//    a sequence of n tiles meets at most (n - 2) / W + 2 ranges, which W keeps
-//    within n_splits.
-// Chunks start one stream per workgroup, ranges about 1 + sequences / R, a tile
-// or two of latency each: chunks are taken where they cost no more than that.
-// 64 sequences of 16k to 32k tokens, 8 kv-heads of 128: 1187 us when chunks of
-// a fixed 2048 tokens were dealt out (3.2 of them to a wavefront, so four to
-// some), 1066 us = 6.3 TB/s in ranges.  Two sequences of 6k to 8k tokens: 19.8 us
-// with 448 wavefronts of eight tiles, 16.2 us with four wavefronts to a chunk.
-constexpr int kMinChunk = 4;
+// (n_splits, hkv, batch).  Dense form: the live chunks of all sequences (a
+// sequence of length L has ceil(L / split_tokens) of them) are numbered
+// consecutively and dealt round-robin to gridDim.x workgroups, one resident
+// round of the chip, so that ragged batches leave no tail of half-empty rounds:
+// every workgroup gets the same number of chunks, give or take one.
 template <typename T, int D, int NW, bool LIST>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 decode_splitkv_kernel(const DecodeParams p) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[NW * wave_lds<D>()];
   if constexpr (LIST) {
-    decode_item<T, D, NW, true>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z, 0, 0, -1);
+    decode_item<T, D, NW, true>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z);
     return;
   }
   const int lane = threadIdx.x & 63;
-  auto tiles_of = [&](int b) -> int {
+  auto chunks_of = [&](int b) -> int {
     if (b >= p.batch) return 0;
     const int len = p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
-    const long long most = (long long)p.n_splits * p.split_tokens;
-    return len > 0 ? (int)((min((long long)len, most) + kDecTile - 1) / kDecTile) : 0;
+    return len > 0 ? min((len - 1) / p.split_tokens + 1, p.n_splits) : 0;
   };
-  const int tiles_lane = tiles_of(lane);  // the first 64 sequences, which most batches end within
-  auto tiles_at = [&](int b0) __attribute__((always_inline)) -> int { return b0 == 0 ? tiles_lane : tiles_of(b0 + lane); };
-  int total = 0, longest = 0, live = 0;
-  for (int b0 = 0; b0 < p.batch; b0 += 64) {
-    const int t = tiles_at(b0);
-    int sum = t, top = t;
+  auto chunks_up_to = [&](int n) __attribute__((always_inline)) -> int {  // inclusive scan over the lanes
 #pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-      sum += __shfl_xor(sum, m, 64);
-      top = max(top, __shfl_xor(top, m, 64));
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(n, d, 64);
+      if (lane >= d) n += up;
     }
-    total += sum;
-    longest = max(longest, top);
-    live += __builtin_popcountll(__builtin_amdgcn_ballot_w64(t > 0));
-  }
-  total = __builtin_amdgcn_readfirstlane(total);
-  longest = __builtin_amdgcn_readfirstlane(longest);
-  if (total == 0) return;
-  const int kv_slices = p.hkv * p.gslices;  // (kv-head, 32-head slice of its group) pairs
-  const int R = max(1, (int)gridDim.x / kv_slices);
-  int c = max(kMinChunk, (longest + p.n_splits - 1) / p.n_splits);
-  if (R > live) c = max(c, (total + R - live - 1) / (R - live));
-  int W = (total + R - 1) / R;
-  if (p.n_splits > 1) W = max(W, (longest - 2) / (p.n_splits - 1) + 1);
-  const bool ranges = p.n_splits > 1 && (R <= live || c > W + 2);
-
-  // The sequence that owns element x of a numbering in which sequence b has
-  // count(tiles of b) elements, the number of its first one and its tiles.
-  struct Found {
-    int b, first, tiles;
+    return n;
   };
-  auto locate = [&](int x, auto count) __attribute__((always_inline)) -> Found {
+  // the first 64 sequences, which most batches end within: looked at once
+  const int n_first = chunks_of(lane);
+  const int incl_first = chunks_up_to(n_first);
+  const uint32_t kv_slices = p.hkv * p.gslices;  // (kv-head, 32-head slice of its group) pairs
+  // (every item has a slot of at least 64 floats in the workspace: ids stay far below 2^32)
+  for (uint32_t g = blockIdx.x;; g += gridDim.x) {
+    const int t = (int)(g / kv_slices), kvs = (int)(g % kv_slices);
+    // the sequence that owns live chunk t, and the number of its first chunk
+    int b = -1, first = 0;
     for (int b0 = 0, seen = 0; b0 < p.batch; b0 += 64) {
-      const int t = tiles_at(b0);
-      const int n = count(t);
-      int incl = n;
-#pragma unroll
-      for (int d = 1; d < 64; d <<= 1) {
-        const int up = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += up;
+      int n = n_first, incl = incl_first;
+      if (b0 != 0) {
+        n = chunks_of(b0 + lane);
+        incl = chunks_up_to(n);
       }
-      const int before = seen + incl - n;  // elements ahead of this lane's sequence
-      const unsigned long long hit = __builtin_amdgcn_ballot_w64(n > 0 && x >= before && x < before + n);
+      const int before = seen + incl - n;  // live chunks ahead of this lane's sequence
+      const unsigned long long hit = __builtin_amdgcn_ballot_w64(n > 0 && t >= before && t < before + n);
       if (hit) {
-        const int src = __builtin_ctzll(hit);
-        return {b0 + src, __builtin_amdgcn_readlane(before, src), __builtin_amdgcn_readlane(t, src)};
+        const int at = __builtin_ctzll(hit);
+        b = b0 + at;
+        first = __builtin_amdgcn_readlane(before, at);
+        break;
       }
       seen += __builtin_amdgcn_readlane(incl, 63);
     }
-    return {-1, 0, 0};  // x lies behind the last element
-  };
-  auto chunks_of = [&](int tiles) -> int { return (tiles + c - 1) / c; };
-  // One call of decode_item for both: its code is long.  (Every item has a slot
-  // of at least 64 floats in the workspace: ids stay far below 2^32.)
-  uint32_t g = blockIdx.x;
-  int x = (int)(g / (uint32_t)kv_slices), kvs = (int)(g % (uint32_t)kv_slices);
-  long long pos = (long long)x * W;  // ranges: next tile of range x
-  while (true) {
-    int split, b, t0 = 0, n = 0, parts = 0;
-    if (ranges) {
-      if (pos >= total) break;
-      const Found f = locate((int)pos, [](int t) { return t; });
-      const int first_range = f.first / W;
-      b = f.b;
-      t0 = (int)pos - f.first;
-      n = min(min((x + 1) * W, total) - (int)pos, f.tiles - t0);
-      split = x - first_range;
-      parts = (f.first + f.tiles - 1) / W - first_range + 1;
-      pos += n;
-    } else {
-      const Found f = locate(x, chunks_of);
-      if (f.b < 0) break;
-      b = f.b;
-      split = x - f.first;
-      parts = chunks_of(f.tiles);
-      const int q = f.tiles / parts, r = f.tiles % parts;
-      t0 = split * q + min(split, r);
-      n = q + (split < r ? 1 : 0);
-    }
-    decode_item<T, D, NW, false>(p, smem, split, kvs, b, t0, n, split == parts - 1 ? parts : -1);
-    if (!ranges || pos >= min((long long)(x + 1) * W, (long long)total)) {
-      g += gridDim.x;
-      x = (int)(g / (uint32_t)kv_slices);
-      kvs = (int)(g % (uint32_t)kv_slices);
-      pos = (long long)x * W;
-    }
+    if (b < 0) return;  // behind the last live chunk
+    decode_item<T, D, NW, false>(p, smem, t - first, kvs, b);
   }
 }
 
@@ -504,9 +418,8 @@ decode_splitkv_kernel(const DecodeParams p) {
 // lanes take a slot, 8 slots of head_dim 128 at a time, instead of one thread
 // per column walking all slots one after the other: 9.2 -> 4.0 us for 2 sequences of 28
 // chunks, 8.3 -> 6.1 us for 64 of about 13 (32 heads of 128).
-// Slots marked -inf hold nothing; what lies in them is not used.  A NaN among a
-// chunk's scores arrives as a NaN log-sum-exp and makes the result NaN, however
-// the sequence was divided.
+// A NaN among a chunk's scores arrives as a NaN log-sum-exp and makes the
+// result NaN.
 constexpr int kMergeThreads = 256;
 template <typename T>
 __global__ void __launch_bounds__(kMergeThreads)
@@ -515,7 +428,7 @@ decode_merge_kernel(const DecodeParams p, int D) {
   const int h = blockIdx.x, b = blockIdx.y;
   const int lane = threadIdx.x & 63;
   const int len = p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
-  int nvalid = p.n_splits;
+  int nvalid;  // slots that pass 1 wrote
   if (p.list_mode != 0) {
     const int kvh = h / (p.hq / p.hkv);
     int cnt;
@@ -523,9 +436,11 @@ decode_merge_kernel(const DecodeParams p, int D) {
       cnt = min(window_list(len, p.win_global, p.win_local).cnt, p.max_blocks);
     else
       cnt = p.block_cnt ? min(p.block_cnt[b * p.hkv + kvh], p.max_blocks) : p.max_blocks;
-    nvalid = min((cnt + p.add_last + p.split_blocks - 1) / p.split_blocks, p.n_splits);
+    nvalid = (cnt + p.add_last + p.split_blocks - 1) / p.split_blocks;
+  } else {
+    nvalid = len > 0 ? (len - 1) / p.split_tokens + 1 : 0;
   }
-  if (len <= 0) nvalid = 0;
+  nvalid = len > 0 ? max(0, min(nvalid, p.n_splits)) : 0;
   const int64_t slot0 = ((int64_t)b * p.hq + h) * p.n_splits;
   const float* pl = p.part_lse + slot0;
 
@@ -583,7 +498,11 @@ int launch_waves(const DecodeParams& p, long long slots, long long resident, hip
 
 // Wavefronts per chunk: as many as leave the launch within one resident round
 // (8 wavefronts per CU), so that a call with few chunks still has eight streams
-// in flight on every CU.  (A list's chunk has two tiles per block.)
+// in flight on every CU; where one wavefront to a chunk fills the round, the
+// barriers of the others cost more than they give.  Whole call, one / two / four
+// wavefronts, head_dim 128, 8 kv-heads: 8192 tokens 21.0 / 17.6 / 15.4 us, two
+// sequences of 6k to 8k 22.6 / 20.5 / 20.5, one of 131072 99.7 / 96.8 / 110.9,
+// 64 of 16k to 32k 1104 / 1157 / 1262.  (A list's chunk has two tiles per block.)
 template <typename T, int D>
 int launch_split(const DecodeParams& p, hipStream_t s) {
   const long long slots = (long long)p.n_splits * p.hkv * p.gslices * p.batch;

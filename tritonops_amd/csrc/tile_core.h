@@ -258,11 +258,10 @@ __device__ __forceinline__ void qk_scores(Tile sK, const Frags& fr,
 // 16-bit probabilities (P[kb][i] = keys 2i, 2i+1 of the lane's 16 keys in block
 // kb), l has this lane's share of the row sum added, and O / l / m have been
 // rescaled if the row max outgrew the slack.
-template <typename T, int D, int NKB, typename MaskF>
-__device__ __forceinline__ void softmax_tile(f32x16 (&S)[NKB], int lh, f32x16 (&O)[RowGeom<D>::NDB], float& m,
+template <typename T, int D, int NKB, int NB, typename MaskF>
+__device__ __forceinline__ void softmax_tile(f32x16 (&S)[NKB], int lh, f32x16 (&O)[NB], float& m,
                                              float& l, float scale, bool need_mask, MaskF allowed,
                                              uint32_t (&P)[NKB][8]) {
-  using G = RowGeom<D>;
   if (need_mask) {
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb)
@@ -289,7 +288,7 @@ __device__ __forceinline__ void softmax_tile(f32x16 (&S)[NKB], int lh, f32x16 (&
     const float alpha = fast_exp2(m - ((m_new == -INFINITY) ? 0.f : m_new));
     l *= alpha;
 #pragma unroll
-    for (int db = 0; db < G::NDB; ++db) O[db] *= alpha;
+    for (int j = 0; j < NB; ++j) O[j] *= alpha;
     m = m_new;
   }
   const float m_use = (m == -INFINITY) ? 0.f : m;  // nothing but masked keys so far
@@ -307,42 +306,19 @@ __device__ __forceinline__ void softmax_tile(f32x16 (&S)[NKB], int lh, f32x16 (&
   l += rs;
 }
 
-// O^T += V^T P^T for one tile.
-template <typename T, int D, int NKB, typename Frags, typename Tile>
-__device__ __forceinline__ void pv_accumulate(Tile sV, const Frags& fr,
-                                              const uint32_t (&P)[NKB][8], f32x16 (&O)[RowGeom<D>::NDB]) {
-  using G = RowGeom<D>;
+// O^T += V^T P^T for one tile: NB blocks of 32 columns, every STEP-th one.
+template <typename T, int D, int NKB, int STEP, int NB, typename Frags, typename Tile>
+__device__ __forceinline__ void pv_accumulate(Tile sV, const Frags& fr, const uint32_t (&P)[NKB][8], f32x16 (&O)[NB]) {
 #pragma unroll
   for (int kk = 0; kk < 2 * NKB; ++kk) {
     const int kb = kk >> 1, o4 = (kk & 1) * 4;
     const i32x4 pf = {(int)P[kb][o4], (int)P[kb][o4 + 1], (int)P[kb][o4 + 2], (int)P[kb][o4 + 3]};
 #pragma unroll
-    for (int db = 0; db < G::NDB; ++db) {
-      const i32x4 vf = fr.load_v(sV, kk, db);
-      O[db] = Elem<T>::mfma(vf, pf, O[db]);
+    for (int j = 0; j < NB; ++j) {
+      const i32x4 vf = fr.load_v(sV, kk, STEP * j);
+      O[j] = Elem<T>::mfma(vf, pf, O[j]);
     }
   }
-}
-
-// One KV tile of NKB*32 keys against the wave's 32 queries.
-//   sK, sV : LDS tiles holding the keys of this tile, in the layout of Frags
-//            (pointers for PaddedFrags, byte offsets for SwizzledFrags)
-//   Qf     : B operands of Q^T, chunk c covers d = 16c .. 16c+15
-//   O      : O^T accumulators, block db covers d = 32db .. 32db+31
-//   m      : reference max of the exponent, scaled base-2 domain (-inf at
-//            start); within kRescaleSlack of the true running max
-//   l      : this lane's share of the running row sum (the other half of the
-//            sum lives in lane l^32; add them at the end)
-//   allowed(key_in_tile) is consulted only when need_mask is true.
-template <typename T, int D, int NKB, typename Frags, typename Tile, typename MaskF>
-__device__ __forceinline__ void compute_tile(Tile sK, Tile sV, const Frags& fr, const i32x4 (&Qf)[RowGeom<D>::KSTEPS],
-                                             f32x16 (&O)[RowGeom<D>::NDB], float& m, float& l,
-                                             float scale, bool need_mask, MaskF allowed) {
-  f32x16 S[NKB];
-  uint32_t P[NKB][8];
-  qk_scores<T, D, NKB>(sK, fr, Qf, S);
-  softmax_tile<T, D, NKB>(S, fr.lh, O, m, l, scale, need_mask, allowed, P);
-  pv_accumulate<T, D, NKB>(sV, fr, P, O);
 }
 
 }  // namespace mi

@@ -621,9 +621,12 @@ def flash_attention_decoding(q, k, v, cu_seq_lens, qk_scale=None, *, seq_lens=No
     [B,maxL,Hkv,D] (any strides, e.g. a transposed view of [B,Hkv,L,D]);
     cu_seq_lens [B+1] supplies only the lengths (:46-48); `qk_scale` natural
     base, default D^-0.5 (:236-237).  Returns o [B,Hq,D]; rows with length 0
-    are zero.  Extensions: `seq_lens` [B] instead of cu_seq_lens, `max_seq_len`
-    and `split_tokens` to size the launch, `return_lse` (base-2, [B,Hq]), and
-    two more KV-cache layouts: kv_layout="packed" — k, v [1,T,Hkv,D] with
+    are zero.  Extensions: `seq_lens` [B] instead of cu_seq_lens; `max_seq_len`,
+    which bounds the lengths (default: the room of the cache), and `split_tokens`,
+    the tokens of a chunk (default: chosen from batch, kv-heads and that bound; a
+    bound near the lengths gives the better chunks) - a row's bits follow from its
+    own inputs and these, not from the lengths of its neighbours; `return_lse`
+    (base-2, [B,Hq]); and two more KV-cache layouts: kv_layout="packed" — k, v [1,T,Hkv,D] with
     sequence b in rows cu_seq_lens[b]:cu_seq_lens[b+1], what the reference's
     decode oracle consumes (:357-359); kv_layout="paged" — k, v are page pools
     [num_pages, page_size, Hkv, D] and page_table [B, max_pages] int32 maps a
