@@ -139,3 +139,22 @@ def test_bits_do_not_depend_on_the_number_of_wavefronts(D, length):
         for B in (3, 8, 40):
             for got, w in zip(call(B), want):
                 assert torch.equal(got, w.expand_as(got)), (call.__name__, B)
+
+
+@pytest.mark.parametrize("split", [64, 256, 2048])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_values_that_are_not_finite_reach_the_result(value, split):
+    """A value that is infinite or NaN under a key whose probability underflows is
+    0 * inf = NaN, whether its chunk holds keys of weight too or is all underflow."""
+    import tritonops_amd as ta
+
+    q, k, v, sl = _rows([2000], 8, 2, 128, 2048)
+    q.fill_(4.0)
+    k.fill_(-4.0)
+    k[0, 700:1000] = 4.0  # 522 binades above the others
+    want = ta.flash_attention_decoding(q, k, v, None, seq_lens=sl, split_tokens=split)
+    v[0, 10, 1, 5] = value
+    got = ta.flash_attention_decoding(q, k, v, None, seq_lens=sl, split_tokens=split)
+    assert got[0, 4:, 5].isnan().all()
+    got[0, 4:, 5] = want[0, 4:, 5]
+    assert torch.equal(got, want)

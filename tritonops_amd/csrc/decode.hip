@@ -413,20 +413,23 @@ decode_splitkv_kernel(const DecodeParams p) {
   }
 }
 
-// Merge: a workgroup per (query head, sequence).  Bound by latency (a few KiB
-// per workgroup), so the log-sum-exps are read by all lanes at once and D / 4
-// lanes take a slot, 8 slots of head_dim 128 at a time, instead of one thread
-// per column walking all slots one after the other: 9.2 -> 4.0 us for 2 sequences of 28
-// chunks, 8.3 -> 6.1 us for 64 of about 13 (32 heads of 128).
+// Merge: a workgroup per (query head, sequence), a thread per output column.
+// Bound by latency (a few KiB per workgroup), so the weights are formed by all
+// lanes at once and the partial results requested kMergeBatch slots at a time;
+// they are added slot by slot, in the order of the sequence.  (Eight slots side
+// by side, then the sums of the eight: no faster, whole call 20.9 against 20.2 us
+// for 2 sequences of 28 chunks, 35.8 against 34.3 for one of 64.)
 // A NaN among a chunk's scores arrives as a NaN log-sum-exp and makes the
-// result NaN.
-constexpr int kMergeThreads = 256;
+// result NaN; so does a NaN or infinity among its values, whatever the weight
+// of the chunk.
+constexpr int kMergeThreads = 128, kMergeBatch = 32;
 template <typename T>
 __global__ void __launch_bounds__(kMergeThreads)
 decode_merge_kernel(const DecodeParams p, int D) {
-  __shared__ float4 part[kMergeThreads];
+  __shared__ float weight[2][kMergeThreads];
+  __shared__ float top[kMergeThreads / 64];
   const int h = blockIdx.x, b = blockIdx.y;
-  const int lane = threadIdx.x & 63;
+  const int d = threadIdx.x;
   const int len = p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
   int nvalid;  // slots that pass 1 wrote
   if (p.list_mode != 0) {
@@ -444,43 +447,43 @@ decode_merge_kernel(const DecodeParams p, int D) {
   const int64_t slot0 = ((int64_t)b * p.hq + h) * p.n_splits;
   const float* pl = p.part_lse + slot0;
 
-  // every wavefront forms the maximum and the sum of weights for itself
   float M = -INFINITY;
-  for (int c = lane; c < nvalid; c += 64) M = fmaxf(M, pl[c]);
+  for (int c = d; c < nvalid; c += kMergeThreads) M = fmaxf(M, pl[c]);
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) M = fmaxf(M, __shfl_xor(M, m, 64));
-  float den = 0.f;
-  for (int c = lane; c < nvalid; c += 64) den += pl[c] == -INFINITY ? 0.f : fast_exp2(pl[c] - M);
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) den += __shfl_xor(den, m, 64);
+  if ((d & 63) == 0) top[d >> 6] = M;
+  __syncthreads();
+  M = fmaxf(top[0], top[1]);
 
-  const int quads = D / 4, groups = kMergeThreads / quads;
-  const int grp = threadIdx.x / quads, d4 = threadIdx.x % quads;
-  float4 acc = {0.f, 0.f, 0.f, 0.f};
-  if (M > -INFINITY && grp < groups) {
-    const float4* po = reinterpret_cast<const float4*>(p.part_o + slot0 * D) + d4;
-#pragma unroll 4
-    for (int c = grp; c < nvalid; c += groups) {
-      const float4 x = po[(int64_t)c * quads];
-      const float w = fast_exp2(pl[c] - M);
-      acc.x += w > 0.f ? w * x.x : 0.f;
-      acc.y += w > 0.f ? w * x.y : 0.f;
-      acc.z += w > 0.f ? w * x.z : 0.f;
-      acc.w += w > 0.f ? w * x.w : 0.f;
+  float den = 0.f, acc = 0.f;
+  const float* po = p.part_o + slot0 * D + min(d, D - 1);
+  for (int c0 = 0, par = 0; c0 < nvalid; c0 += kMergeThreads, par ^= 1) {
+    if (c0 + d < nvalid) {
+      const float e = pl[c0 + d];
+      weight[par][d] = e == -INFINITY ? 0.f : fast_exp2(e - M);
+    }
+    __syncthreads();  // (the other buffer is read until the next one)
+    const int n = min(nvalid - c0, kMergeThreads);
+    for (int c1 = 0; c1 < n; c1 += kMergeBatch) {
+      float x[kMergeBatch];
+#pragma unroll
+      for (int i = 0; i < kMergeBatch; ++i)
+        x[i] = po[(int64_t)(c0 + min(c1 + i, n - 1)) * D];
+#pragma unroll
+      for (int i = 0; i < kMergeBatch; ++i) {
+        // (selects: a branch would pull the load down to it)
+        const bool live = c1 + i < n;
+        const float w = weight[par][min(c1 + i, n - 1)];
+        den = live ? den + w : den;
+        acc = live ? fmaf(w, x[i], acc) : acc;
+      }
     }
   }
-  part[threadIdx.x] = acc;
-  __syncthreads();
-  if (threadIdx.x < D) {
-    // column d: element d % 4 of quad d / 4, summed over the groups
-    const int d = threadIdx.x;
-    const float* col = reinterpret_cast<const float*>(part) + d;
-    float sum = 0.f;
-    for (int g = 0; g < groups; ++g) sum += col[g * D];
+  if (d < D) {
     T* op = reinterpret_cast<T*>(p.o) + b * p.o_sb + h * p.o_sh;
-    op[d] = (T)(den == 0.f ? 0.f : sum / den);
-    if (d == 0 && p.lse) p.lse[(int64_t)b * p.hq + h] = den == 0.f ? -INFINITY : M + fast_log2(den);
+    op[d] = (T)(den == 0.f ? 0.f : acc / den);
   }
+  if (d == 0 && p.lse) p.lse[(int64_t)b * p.hq + h] = den == 0.f ? -INFINITY : M + fast_log2(den);
 }
 
 template <typename T, int D, int NW>
