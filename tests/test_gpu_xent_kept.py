@@ -154,6 +154,71 @@ def test_when_the_logits_are_kept(monkeypatch):
 
 
 @pytest.mark.gpu
+def test_all_live_graphs_share_one_budget(monkeypatch):
+    import tritonops_amd as ta
+    from tritonops_amd import xent
+
+    x, w, y, _ = _inputs(40, 1024, 300, torch.bfloat16)
+    x, w, y = x.cuda(), w.cuda().requires_grad_(True), y.cuda()
+    one = 2 * 256 * 256 * 4
+    assert not xent._kept_live
+    monkeypatch.setattr(xent, "KEEP_BYTES", 3 * one - 1)
+
+    def call(**kw):
+        return ta.cross_entropy_fused_triton(x, w, y, **kw)
+
+    def saved(loss):  # (a call in its argument holds the graph until this returns)
+        return len(loss.grad_fn.saved_tensors)
+
+    losses = [call(), call(), call()]
+    assert [saved(a) for a in losses] == [5, 5, 4]
+    losses[0].sum().backward(retain_graph=True)          # still held
+    assert saved(call()) == 4
+    losses[0].sum().backward()                           # given back by the backward pass ...
+    again = call()
+    assert saved(again) == 5 and saved(call()) == 4
+    del losses[1]                                        # ... and with a graph that has none
+    assert saved(call()) == 5
+    forced = call(keep_logits=True)                      # the caller's own choice, which counts as well
+    assert saved(forced) == 5 and saved(call(keep_logits=True)) == 5 and saved(call()) == 4
+    del again, forced, losses
+    assert not xent._kept_live and saved(call()) == 5
+    assert saved(call(keep_logits=False)) == 4
+
+
+@pytest.mark.gpu
+def test_little_free_memory_means_no_kept_logits(monkeypatch):
+    import tritonops_amd as ta
+    from tritonops_amd import xent
+
+    x, w, y, _ = _inputs(40, 1024, 300, torch.bfloat16)
+    x, w, y = x.cuda(), w.cuda().requires_grad_(True), y.cuda()
+    need = 4 * (2 * 256 * 256 * 4 + 40 * 300 * 2)
+
+    def saved(**kw):
+        loss = ta.cross_entropy_fused_triton(x, w, y, **kw)
+        return len(loss.grad_fn.saved_tensors)
+
+    assert xent._free_bytes(x.device) > need
+    monkeypatch.setattr(xent, "_free_bytes", lambda device: need - 1)
+    assert saved() == 5                                  # a few hundred KiB are not asked about
+    monkeypatch.setattr(xent, "KEEP_UNASKED", 0)
+    assert saved() == 4 and saved(keep_logits=True) == 5
+    monkeypatch.setattr(xent, "_free_bytes", lambda device: need)
+    assert saved() == 5
+    out_of_memory = torch.OutOfMemoryError("no memory")
+
+    def empty(*size, **kw):
+        if size == (2 * 256 * 256,):
+            raise out_of_memory
+        return torch_empty(*size, **kw)
+
+    torch_empty = torch.empty
+    monkeypatch.setattr(xent.torch, "empty", empty)
+    assert saved() == 4 and saved(keep_logits=True) == 4 and not xent._kept_live
+
+
+@pytest.mark.gpu
 def test_replays_of_a_captured_step():
     import tritonops_amd as ta
 

@@ -7,6 +7,8 @@ torch.mm.  Its dlogits come from the forward's fp32 logits where those are kept
 applies the element-wise step to the fp32 accumulators where they are not: in a
 plain cross_entropy_fused_fwd / _bwd pair the logits are never materialised."""
 import ctypes as C
+import threading
+import weakref
 
 import torch
 
@@ -20,15 +22,24 @@ BWD_ROWS = 16384
 # Kept logits lie in tiles of this many tokens: a block of rows read from them
 # starts on a tile (BWD_ROWS is rounded down to whole tiles there, to one at least).
 _KEPT_ROWS = 256
-# The forward of a call that will be differentiated keeps its fp32 logits where
-# that is at most KEEP_BYTES (of 288 GB, from the forward to the backward) and
-# the rows have at least KEEP_DIM elements: 8 bytes per logit go through memory
+# The forward of a call that will be differentiated keeps its fp32 logits (unless
+# its caller says otherwise, keep_logits) where the rows have at least KEEP_DIM
+# elements and all graphs that are alive hold at most KEEP_BYTES of them on the
+# device, this call included: 8 bytes per logit go through memory
 # once instead of 2 * dim operations.  Forward + backward, recomputed -> kept:
 # dim 4096, 8192 tokens x 128256: 28.0 -> 22.8 ms; dim 1024, 4096 x 128256:
 # 4.60 -> 4.27; dim 768, 4096 x 50257: 1.84 -> 1.75; dim 512, 8192 x 128256:
 # 4.96 -> 5.25; dim 256, 8192 x 32000: 0.82 -> 0.97.
 KEEP_BYTES = 8 << 30
 KEEP_DIM = 1024
+# From KEEP_UNASKED bytes in all on, the memory is asked first: kept logits and the
+# backward's block of dlogits take at most a quarter of what is free (to the
+# allocator or in its cache), so that what the program allocates next still fits.
+KEEP_UNASKED = 256 << 20
+# Kept logits that are alive: token -> (device, bytes).  An entry leaves when its
+# tensor is freed, from whichever thread that happens in (one dict operation, no lock).
+_kept_live = {}
+_kept_lock = threading.Lock()
 _saved_hooks = getattr(torch._C._autograd, "_top_saved_tensors_default_hooks", None)
 
 
@@ -67,9 +78,44 @@ def cross_entropy_fused_fwd(x, w, y):
     return _fwd(x, w, y, False)[:2]
 
 
+def _free_bytes(device):
+    """Device memory that an allocation could get.  (The nested form of the
+    allocator's figures: 6 us, the flat one takes 260.)"""
+    stats = torch.cuda.memory_stats_as_nested_dict(device)
+    reserved, used = (stats[k]["all"]["current"] if k in stats else 0 for k in ("reserved_bytes", "allocated_bytes"))
+    return torch.cuda.mem_get_info(device)[0] + reserved - used
+
+
+def _alloc_kept(T, N, device, esize, always):
+    """Room for the logits of [T, N], or None: where the automatic choice (not
+    `always`) finds too many of them alive or too little memory free, and where the
+    allocation fails."""
+    nbytes = _lib.load().mi_xent_kept_bytes(T, N)
+    token = object()
+    with _kept_lock:
+        if not always:
+            live = nbytes + sum(n for d, n in list(_kept_live.values()) if d == device)
+            if live > KEEP_BYTES:
+                return None
+            # (a capture repeats what its program ran before it, and its pool is not in these figures)
+            if live > KEEP_UNASKED and not torch.cuda.is_current_stream_capturing() \
+                    and 4 * (nbytes + min(T, BWD_ROWS) * N * esize) > _free_bytes(device):
+                return None
+        _kept_live[token] = (device, nbytes)
+    try:
+        kept = torch.empty(nbytes // 4, device=device, dtype=torch.float32)
+    except BaseException as e:
+        _kept_live.pop(token, None)
+        if not isinstance(e, torch.OutOfMemoryError):
+            raise
+        return None
+    weakref.finalize(kept, _kept_live.pop, token, None).atexit = False
+    return kept
+
+
 def _fwd(x, w, y, keep):
-    """(loss, lse, kept): kept is the logits for _kept_dlogits, None unless
-    `keep` is set and there is memory for them."""
+    """(loss, lse, kept): kept is the logits for _kept_dlogits, or None; `keep`:
+    False never, True where there is memory for them, None within the budget."""
     _require_gpu(x, w, y)
     lib = _lib.load()
     if x.ndim != 2 or w.ndim != 2:
@@ -96,11 +142,8 @@ def _fwd(x, w, y, keep):
     ws = torch.empty(max(nbytes, 16), device=x.device, dtype=torch.uint8)
     a.workspace, a.workspace_bytes = _ptr(ws), nbytes
     kept = None
-    if keep and T and N:
-        try:
-            kept = torch.empty(lib.mi_xent_kept_bytes(T, N) // 4, device=x.device, dtype=torch.float32)
-        except torch.OutOfMemoryError:
-            pass
+    if keep is not False and T and N:
+        kept = _alloc_kept(T, N, x.device, x.element_size(), bool(keep))
     if kept is None:
         _lib.check(lib.mi_xent_fwd(C.byref(a), _stream()))
     else:
@@ -217,7 +260,7 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
 
 
 def _keeps_logits(x, w):
-    """Whether the forward keeps its logits for the backward (see KEEP_BYTES)."""
+    """Whether the forward may keep its logits for the backward (see KEEP_BYTES)."""
     if not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
         return False
     if x.ndim != 2 or w.ndim != 2 or x.shape[1] < KEEP_DIM:
@@ -231,7 +274,8 @@ def _keeps_logits(x, w):
 class CrossEntropyFusedFunction(torch.autograd.Function):
     """Drop-in for the reference's autograd Function (cross_entropy.py:270-420).
     `keep_logits`: the backward reads the forward's logits instead of computing
-    them again; the results are the same."""
+    them again; the results are the same.  True: wherever there is memory for them;
+    None: within KEEP_BYTES."""
 
     @staticmethod
     def forward(ctx, x, w, y, keep_logits=False):
@@ -248,6 +292,14 @@ class CrossEntropyFusedFunction(torch.autograd.Function):
         return grad_x, grad_w, None, None
 
 
-def cross_entropy_fused_triton(x, w, y):
-    """loss [T] fp32 of softmax cross-entropy over x @ w^T (cross_entropy.py:423-425)."""
-    return CrossEntropyFusedFunction.apply(x, w, y, _keeps_logits(x, w))
+def cross_entropy_fused_triton(x, w, y, *, keep_logits=None):
+    """loss [T] fp32 of softmax cross-entropy over x @ w^T (cross_entropy.py:423-425).
+
+    `keep_logits`: whether the fp32 logits (4 bytes each) stay in memory from the
+    forward to the backward, which then does not compute them again; loss and
+    gradients are the same bits either way.  None: where that is the faster way and
+    KEEP_BYTES and the free memory allow it.  False: never, no more memory than the
+    reference's scheme takes.  True: always where the allocation succeeds."""
+    if keep_logits is None:
+        keep_logits = None if _keeps_logits(x, w) else False
+    return CrossEntropyFusedFunction.apply(x, w, y, keep_logits)
