@@ -153,6 +153,28 @@ def test_when_the_logits_are_kept(monkeypatch):
     assert saved(x, wg) == 5
 
 
+@pytest.mark.parametrize("getter,want", [
+    (lambda ignore: None, True), (lambda ignore: ("pack", "unpack"), False), (lambda: None, True),
+    (lambda: ("pack", "unpack"), False), (lambda a, b: None, False), (None, False)],
+    ids=["none", "hooks", "none_no_argument", "hooks_no_argument", "other_signature", "no_getter"])
+def test_the_getter_of_saved_tensor_hooks_may_differ(monkeypatch, getter, want):
+    """torch's getter is private: without it, or with a signature that is not known, nothing is kept."""
+    from tritonops_amd import xent
+
+    monkeypatch.setattr(xent, "_saved_hooks", getter)
+    x, w = torch.zeros((4, 1024)), torch.zeros((8, 1024), requires_grad=True)
+    assert xent._keeps_logits(x, w) is want
+
+
+def test_the_getter_of_this_torch():
+    from tritonops_amd import xent
+
+    x, w = torch.zeros((4, 1024)), torch.zeros((8, 1024), requires_grad=True)
+    assert xent._keeps_logits(x, w) is True
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        assert xent._keeps_logits(x, w) is False
+
+
 @pytest.mark.gpu
 def test_all_live_graphs_share_one_budget(monkeypatch):
     import tritonops_amd as ta

@@ -259,14 +259,26 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
     return grad_x, grad_w
 
 
+def _saved_hooks_set():
+    """Whether hooks on saved tensors (activation checkpointing, offloading to the host),
+    which would copy or drop kept logits, are or may be in force."""
+    if _saved_hooks is None:
+        return True
+    for args in ((False,), ()):  # torch has had the getter with and without its argument
+        try:
+            return _saved_hooks(*args) is not None
+        except TypeError:
+            pass
+    return True
+
+
 def _keeps_logits(x, w):
     """Whether the forward may keep its logits for the backward (see KEEP_BYTES)."""
     if not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
         return False
     if x.ndim != 2 or w.ndim != 2 or x.shape[1] < KEEP_DIM:
         return False
-    # hooks on saved tensors (activation checkpointing, offloading to the host) would copy or drop them
-    if _saved_hooks is None or _saved_hooks(False) is not None:
+    if _saved_hooks_set():
         return False
     return _lib.load().mi_xent_kept_bytes(x.shape[0], w.shape[0]) <= KEEP_BYTES
 
