@@ -1,10 +1,11 @@
 """The host model of the kernels' walks (tests/host_model/walk_model.cpp), built with
 AddressSanitizer and UndefinedBehaviorSanitizer and run on the CPU.
 
-The model restates, without any device code, the work-item map and persistent
-schedule of the dense forward kernel, its four-stage tile ring (and the five-stage ring of its short form) with the counted
+The model restates, without any device code, the order of the persistent kernels'
+work items, the dense forward kernel's four-stage tile ring (and the five-stage ring of its short form) with the counted
 vector-memory waits and barriers, the running-reference softmax, the window
-form's block list and the dealing of decode chunks, and checks their invariants
+form's block list, the dealing of decode chunks and their merge, and the tiles
+that several wavefronts of a decode chunk share, and checks their invariants
 over thousands of ragged shapes.  Each of its deliberate-mistake modes breaks one
 of those protocols; the model has to notice every one of them.
 """
@@ -33,6 +34,14 @@ MISTAKES = {
     13: "window walk: a wave's positions are counted in keys, not in positions of the walk",
     14: "window walk: the sink tiles are not cut at the first tile of the band",
     15: "window walk: a tile at the window's lower edge is taken for unmasked",
+    16: "level order: levels that stay together are left one at a time",
+    17: "level order: key tiles are counted from the start of a sequence",
+    18: "one generation of workgroups however many rounds there are",
+    19: "a quotient by reciprocal is not mended",
+    20: "decode: the search steps over 64 sequences without counting their chunks",
+    21: "decode: the merge walks every slot of the bound",
+    22: "decode: no barrier between the last reads of a step and the next step's stores",
+    23: "decode: the refill behind a store fetches the next step again",
 }
 
 
@@ -57,7 +66,7 @@ def test_walks_hold_their_invariants(model):
     r = _run(model)
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
     assert "host model ok" in r.stdout
-    for part in ("dense walk", "block-sparse walk", "softmax reference point", "decode lists and chunks", "window walk"):
+    for part in ("item order", "dense walk", "block-sparse walk", "softmax reference point", "decode lists and chunks", "window walk"):
         assert part in r.stdout
 
 
