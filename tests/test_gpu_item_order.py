@@ -68,3 +68,54 @@ def test_batched_call_of_a_few_rounds(B, H, S, D):
         assert torch.equal(o[:1, h:h + 5], o1), h
         for a, b in zip(grads, torch.autograd.grad(o1, part, do[:1, h:h + 5])):
             assert torch.equal(a[:1, h:h + 5], b), h
+
+
+def _gpu_randn(shape, seed, dt=torch.bfloat16):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(shape, generator=g, device="cuda", dtype=dt)
+
+
+# A workgroup holds the items of 64 rounds (one per lane); beyond that a launch has several generations of
+# workgroups.  256 compute units hold one workgroup of the 256-row forms and two of the 128-row form.
+@pytest.mark.parametrize("B,H,S,D", [(1100, 32, 16, 128), (130, 40, 1100, 64)])
+def test_more_rounds_than_a_wavefront_has_lanes(B, H, S, D):
+    """Batched (unit order): the bits of calls on parts of the batch."""
+    import tritonops_amd as ta
+
+    q, k, v, do = (_gpu_randn((B, H, S, D), i) for i in range(4))
+    sm = D ** -0.5 * ta.LOG2E
+    for form in ("256", "128"):
+        with ta.dense_form(form):
+            o, lse = ta.flash_attn_triton_fwd(q, k, v, None, sm)
+            for b in range(0, B, 50):
+                e = min(b + 50, B)
+                o1, lse1 = ta.flash_attn_triton_fwd(q[b:e], k[b:e], v[b:e], None, sm)
+                assert torch.equal(o[b:e], o1) and torch.equal(lse[b:e], lse1), (form, b)
+    grads = ta.flash_attn_triton_bwd(q, k, v, o, do, lse, None, sm)
+    for b in range(0, B, 50):
+        e = min(b + 50, B)
+        want = ta.flash_attn_triton_bwd(q[b:e], k[b:e], v[b:e], o[b:e], do[b:e], lse[b:e], None, sm)
+        for a, w in zip(grads, want):
+            assert torch.equal(a[b:e], w), b
+
+
+def test_more_rounds_by_level():
+    """Packed, with more heads than models have: the bits of calls on parts of the heads."""
+    import tritonops_amd as ta
+
+    lens, H, D = [1300, 1, 700, 256, 0, 900, 257, 128], 1100, 64
+    q, k, v, do = (_gpu_randn((1, sum(lens), H, D), i) for i in range(4))
+    cu = cu_from(torch.tensor(lens, dtype=torch.int32)).cuda()
+    sm = D ** -0.5 * ta.LOG2E
+    parts = [slice(h, min(h + 100, H)) for h in range(0, H, 100)]
+    for form in ("256", "128"):
+        with ta.dense_form(form):
+            o, lse = ta.flash_attn_triton_fwd(q, k, v, cu, sm)
+            for p in parts:
+                o1, lse1 = ta.flash_attn_triton_fwd(q[:, :, p], k[:, :, p], v[:, :, p], cu, sm)
+                assert torch.equal(o[:, :, p], o1) and torch.equal(lse[:, :, p], lse1), (form, p)
+    grads = ta.flash_attn_triton_bwd(q, k, v, o, do, lse, cu, sm)
+    for p in parts:
+        want = ta.flash_attn_triton_bwd(q[:, :, p], k[:, :, p], v[:, :, p], o[:, :, p], do[:, :, p], lse[:, :, p], cu, sm)
+        for a, w in zip(grads, want):
+            assert torch.equal(a[:, :, p], w), p

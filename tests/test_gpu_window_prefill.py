@@ -155,3 +155,25 @@ def test_no_lists_through_the_c_abi_and_its_refusals():
         outs.append((o, lse))
     assert_close(outs[0][0], outs[1][0], 1e-2)
     assert (outs[0][1] - outs[1][1]).abs().max().item() <= LSE_TOL
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,lw,gw", [(32, 8, 128, 2048, 128), (24, 24, 96, 2048, 0), (40, 8, 64, 300, 64)])
+def test_ragged_window_walk_of_several_rounds_equals_its_sequences(no_lists, Hq, Hkv, D, lw, gw):
+    """More items than resident workgroups: the items are numbered by level, and a sequence keeps
+    the bits of a call of its own, one kv-head at a time (a single round)."""
+    import tritonops_amd as ta
+
+    lens = [3000, 1, 2100, 700, 0, 2600, 129]
+    q, k, v, cu = _inputs(lens, Hq, Hkv, D)
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    o, lse = ta.flash_attn_sparse_triton(q, k, v, cu.cuda(), None, lw, gw)
+    at, group = 0, Hq // Hkv
+    for n in lens:
+        s = slice(at, at + n)
+        at += n
+        if not n:
+            continue
+        for kh in range(Hkv):
+            hs, ks = slice(kh * group, (kh + 1) * group), slice(kh, kh + 1)
+            o1, lse1 = ta.flash_attn_sparse_triton(q[:, s, hs], k[:, s, ks], v[:, s, ks], cu_from([n]).cuda(), None, lw, gw)
+            assert torch.equal(o[:, s, hs], o1) and torch.equal(lse[:, s, hs], lse1), (n, kh)

@@ -5,16 +5,25 @@
 // by sequence the items of a round differ by the spread of the lengths, and
 // ids that lie past the end of a short sequence leave their workgroup idle: on
 // five sequences of 517 to 3400 tokens (32 heads) the busiest of 256 workgroups
-// had 1.4 times the mean work with 8 kv-heads and twice the mean with 32.
+// had 1.4 times the mean work with 8 kv-heads and twice the mean with 32 (queries).
 //
 // Here the items that exist are numbered LEVEL by level: level t holds the t-th
 // tile of every sequence that has one, and the levels are walked from the last
 // to the first.  A causal tile costs t + 1 tiles of keys whatever its sequence
 // (counted from the sequence's start for queries, from its end for keys), so
 // the numbering runs from the longest item to the shortest, and dealing it out
-// in alternating directions leaves the workgroups within a few per cent of one
-// another (1.07 in both cases above) without a shared counter and without the
-// lengths being known on the host.
+// in alternating directions leaves the busiest workgroup with 1.08 times the
+// mean in both cases above without a shared counter and without the lengths
+// being known on the host.  The keys of the backward pass (128 rows to an item):
+// 1.61 -> 1.33 times the mean with 8 kv-heads, where 536 items make two rounds
+// and a few items of a third and the longest one alone is 1.2 times the mean,
+// 1.57 -> 1.09 with 32.
+//
+// The window walk's items cost a band each, not t + 1 tiles, until the local
+// window is filled; numbered by level it gains from the same balance: seven
+// sequences of 500 to 7000 tokens, 16 heads, local window 2048: 296 -> 225 us
+// with 4 kv-heads, 301 -> 234 with 16; six of 1024 to 12288, 32 heads: 964 -> 950
+// and 1038 -> 994.
 //
 // What the order costs is sharing: items that run side by side on an XCD read
 // the same K / V from its L2 only if they belong to one (sequence, kv-head).

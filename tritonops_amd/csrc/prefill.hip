@@ -1609,7 +1609,10 @@ constexpr size_t prefill_lds_bytes() {
 // are fitted to HIP-event timings of both forms on 1 to 48 sequences of 256 to
 // 8192 tokens with 12, 20 and 32 heads, causal and not: against the faster
 // form of each launch the choice costs 0.7 % in the geometric mean (always the
-// long form: 8.5 %, always the short form: 2.5 %).
+// long form: 8.5 %, always the short form: 2.5 %).  That fit is of items numbered
+// unit by unit; with causal launches of few rounds numbered by level (item_order.h)
+// the same choice costs 1.0 % over 216 such launches (long 5.7 %, short 1.0 %),
+// 0.3 % over those without a mask and 1.7 % over the causal ones (5.1 %, 1.3 %).
 inline double short_form_cost(long long n, int cus) {
   const long long grid = (long long)kShortPerCu * cus;
   const long long q = n / grid, r = n % grid;

@@ -20,10 +20,12 @@ LOG2E = 1.4426950408889634
 # flash_attn_sparse_triton's window form runs either on block lists built on the
 # host (the block-list kernel, as every other mask) or without lists: the library
 # then walks each 128-row item's sink tiles and band with the dense kernel's
-# pipeline.  The second is 5 to 9 % faster for local windows of 2048 tokens or more
-# at head_dim 96 / 128 (B1 H16 S32768: 0.586 against 0.615 ms at 2048, 0.995 against
-# 1.087 ms at 4096) and up to 11 % slower for short windows and at head_dim 64, so
-# the choice is made per call.  True / False force one of the two (tests).
+# pipeline.  Walk against lists, local window 1024 / 2048 / 4096 at head_dim 128:
+# 0.347 / 0.556 / 0.979 against 0.356 / 0.583 / 1.038 ms on one sequence of 32768
+# tokens (16 heads), 0.338 / 0.530 / 0.846 against 0.332 / 0.525 / 0.834 on four of
+# 8192; shorter windows 0 to 4 % slower, head_dim 64 3 to 18 % slower throughout.
+# The walk is taken where it gains more than it can lose.  True / False force one
+# of the two (tests).
 WINDOW_PREFILL_LISTS = None
 _WINDOW_WALK_MIN_LOCAL = 2048
 _CU_COUNT = {}
