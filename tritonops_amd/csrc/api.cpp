@@ -224,9 +224,7 @@ static int rms_validate(const mi_rmsnorm_args* a, bool backward) {
 // 16-byte chunk path: dim and row strides multiples of the chunk, 16-byte aligned bases, <= 16 chunks per lane
 static bool rms_vec_ok(const mi_rmsnorm_args* a, bool backward) {
   const int epc = 16 / rms_elem_bytes(a->x_dtype);
-  // chunks per row: 16 per thread of a workgroup; 8 in the backward pass, whose
-  // per-position dw sums share the registers
-  if (a->dim % epc || a->dim / epc > 256 * (backward ? 8 : 16)) return false;
+  if (a->dim % epc || a->dim / epc > 256 * (backward ? mi::kRmsMaxChunksBwd : mi::kRmsMaxChunks)) return false;
   if (!aligned16(a->x) || a->x_stride % epc) return false;
   if (!backward) return aligned16(a->y) && a->y_stride % epc == 0;
   return aligned16(a->dy) && aligned16(a->dx) && a->dy_stride % epc == 0 && a->dx_stride % epc == 0;

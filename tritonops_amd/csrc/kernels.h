@@ -193,6 +193,9 @@ int launch_attn_bwd(const BwdParams& p, int dtype, int head_dim, hipStream_t s);
 // The backward workspace holds rms_partial_rows() + kRmsStageRows fp32 rows of `dim`; the latter
 // are part of the size that callers were given and are not used any more.
 constexpr int kRmsStageRows = 32;
+// 16-byte chunks of a row that a thread of a workgroup keeps in registers at most; in the backward pass the
+// dw sums of its positions share them.
+constexpr int kRmsMaxChunks = 16, kRmsMaxChunksBwd = 8;
 int rms_partial_rows(long long rows, int num_cus);
 int launch_rms_fwd(const RmsParams& p, int x_dtype, int w_dtype, bool vec, int n_waves, hipStream_t s);
 int launch_rms_bwd(const RmsParams& p, int x_dtype, int w_dtype, bool vec, int n_waves, hipStream_t s);

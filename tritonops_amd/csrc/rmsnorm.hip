@@ -42,7 +42,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // element type tags: 0 bf16, 1 f16, 2 f32
-constexpr int kMaxJ = 16;  // 16-byte chunks a lane keeps in registers per row
 
 // EPC elements per chunk: 16 bytes, or (WIDE = false) a single element, which
 // rows of any width, alignment and stride can be read in.
@@ -437,7 +436,8 @@ int reduce_dw(const RmsParams& p, int n_parts, hipStream_t s) {
 constexpr int kWaveRowChunks = 128, kWaveRowElems = 1024, kMaxRowElems = 8192;
 constexpr int kMaxRowWorkgroups = 1024, kMaxPartRowWorkgroups = 2048;
 
-template <typename F>
+// MAX_J: 16-byte chunks that a thread holds at most (the C entry passes `wide` for no longer rows).
+template <int MAX_J, typename F>
 void by_shape(bool wide, int nch, F&& f) {
   using std::integral_constant;
   using std::true_type;
@@ -461,7 +461,7 @@ void by_shape(bool wide, int nch, F&& f) {
     else if (nch <= 512) MI_RMS_SHAPE(2, 256, true_type);
     else if (nch <= 1024) MI_RMS_SHAPE(4, 256, true_type);
     else if (nch <= 2048) MI_RMS_SHAPE(8, 256, true_type);
-    else MI_RMS_SHAPE(kMaxJ, 256, true_type);
+    else if constexpr (MAX_J > 8) MI_RMS_SHAPE(MAX_J, 256, true_type);
   }
 #undef MI_RMS_SHAPE
 }
@@ -484,7 +484,7 @@ template <typename T, typename TW>
 int launch_fwd_t(const RmsParams& p, bool wide, int n_waves, hipStream_t s) {
   if (wide || p.dim <= kMaxRowElems) {
     const int nch = wide ? p.dim / (16 / (int)sizeof(T)) : p.dim;
-    by_shape(wide, nch, [&](auto jc, auto wc, auto wide_c) {
+    by_shape<kRmsMaxChunks>(wide, nch, [&](auto jc, auto wc, auto wide_c) {
       hipLaunchKernelGGL((rms_fwd_vec_kernel<T, TW, decltype(jc)::value, decltype(wc)::value, decltype(wide_c)::value>),
                          dim3(vec_grid(p, wide, nch, n_waves)), dim3(256), 0, s, p);
     });
@@ -502,7 +502,7 @@ int launch_bwd_t(const RmsParams& p, bool wide, int n_waves, hipStream_t s) {
     const int nch = wide ? p.dim / (16 / (int)sizeof(T)) : p.dim;
     const unsigned grid = vec_grid(p, wide, nch, n_waves);
     n_parts = (int)grid;
-    by_shape(wide, nch, [&](auto jc, auto wc, auto wide_c) {
+    by_shape<kRmsMaxChunksBwd>(wide, nch, [&](auto jc, auto wc, auto wide_c) {
       hipLaunchKernelGGL((rms_bwd_vec_kernel<T, TW, decltype(jc)::value, decltype(wc)::value, decltype(wide_c)::value>),
                          dim3(grid), dim3(256), 0, s, p);
     });
