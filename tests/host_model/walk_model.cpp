@@ -44,7 +44,7 @@
 #include <vector>
 
 static int g_fail = 0;
-// 0: the kernels' protocols as they are.  1..23: one deliberate mistake each; the
+// 0: the kernels' protocols as they are.  1..24: one deliberate mistake each; the
 // run must then fail (tests/test_host_model.py checks that it does), which is
 // what shows that the checks below can tell a broken protocol from a sound one.
 static int g_mut = 0;
@@ -62,6 +62,7 @@ static int g_mut = 0;
 // item_order.h: number_by_level, persistent_grid, items_of_rounds.
 namespace order {
 constexpr int kLevelMaxBatch = 64, kLevelEvenRounds = 4, kMaxRounds = 64;
+constexpr int kLevelWorthRounds = 6, kLevelWorth = 120;
 
 struct Launch {
   std::vector<int> lens;  // per sequence
@@ -118,6 +119,42 @@ static void divmod(bool small, uint32_t x, uint32_t d, uint32_t& q, uint32_t& r)
   }
 }
 
+// Item `id` of the unit order.
+static void unit_item(const Launch& L, bool small, uint32_t id, uint32_t group, uint32_t& b, uint32_t& kvh, uint32_t& member, int& t) {
+  const uint32_t per_unit = (uint32_t)L.n_tiles * group;
+  uint32_t unit, s, tile;
+  if (((L.batch * L.heads_kv) & 7) == 0) {
+    divmod(small, id >> 3, per_unit, unit, s);
+    unit = unit * 8 + (id & 7);
+  } else {
+    divmod(small, id, per_unit, unit, s);
+  }
+  divmod(small, s, group, tile, member);
+  divmod(small, unit, L.heads_kv, b, kvh);
+  t = L.from_end ? (int)tile : L.n_tiles - 1 - (int)tile;
+}
+
+// What the unit order gives the busiest of 32 workgroups of the first XCD, against the mean of all.
+static double sampled_load(const Launch& L) {
+  const int grid = (int)L.grid, per_xcd = grid >> 3;
+  long long load[32] = {};
+  for (int lane = 0; lane < 64; ++lane) {
+    const int half = lane >> 5, slot = (lane & 31) * std::max(per_xcd >> 5, 1), at = half && g_mut != 24 ? per_xcd - 1 - slot : slot;
+    for (int r = 0; r < kMaxRounds && (long long)r * grid < L.n_items; r += 2) {
+      const long long id = (long long)(r + half) * grid + at * 8;
+      const bool live = slot < per_xcd && id < L.n_items;
+      uint32_t b, kvh, member;
+      int t;
+      unit_item(L, L.n_items < (1 << 22), live ? (uint32_t)id : 0u, L.heads / L.heads_kv, b, kvh, member, t);
+      CHECK(b < 64, "lane %u is asked for the tiles of a sequence", b);
+      if (live && t < L.tiles(b)) load[lane & 31] += L.from_end ? L.tiles(b) - t : t + 1;
+    }
+  }
+  double work = 0;
+  for (int b = 0; b < L.batch; ++b) work += 0.5 * L.tiles(b) * (L.tiles(b) + 1);
+  return work > 0 ? (double)*std::max_element(load, load + 32) * grid / (work * L.heads) : 0;
+}
+
 // Levels of a sequence that stay together, 0: unit by unit.
 static int level_block(const Launch& L) {
   if (!L.by_level) return 0;
@@ -128,17 +165,18 @@ static int level_block(const Launch& L) {
     even = even && L.tiles(b) == L.tiles(0);
   }
   if (L.packed && even && total * L.heads >= kLevelEvenRounds * L.grid) return 0;
+  if (total * L.heads >= kLevelWorthRounds * L.grid && (L.grid & 7) == 0 && sampled_load(L) * 100 <= kLevelWorth) return 0;
   const int sharers = total * L.heads >= 12 * L.grid ? 8 : total * L.heads >= 6 * L.grid ? 4 : 1;
   int block = 1;
   while (block * (L.heads / L.heads_kv) < sharers) block *= 2;
   return block;
 }
 
-// The items of workgroup wg, one per round: what lane `round` of a wavefront holds.
-static std::vector<ItemId> items(const Launch& L, int wg) {
+// The items of workgroup wg, one per round: what lane `round` of a wavefront holds (block: level_block).
+static std::vector<ItemId> items(const Launch& L, int wg, int block) {
   std::vector<ItemId> out(kMaxRounds);
   const bool small = L.n_items < (1 << 22);
-  const int grid = (int)L.grid, block = level_block(L);
+  const int grid = (int)L.grid;
   for (int round = 0; round < kMaxRounds; ++round) {
     int w = wg;
     if ((round & 1) && (grid & 7) == 0) w = (((grid >> 3) - (g_mut == 7 ? 0 : 1) - (w >> 3)) << 3) | (w & 7);
@@ -171,17 +209,9 @@ static std::vector<ItemId> items(const Launch& L, int wg) {
       it.kvh = (int)kvh;
       continue;
     }
-    const uint32_t per_unit = (uint32_t)L.n_tiles * group;
-    uint32_t unit, s, tile, member, b, kvh;
-    if (((L.batch * L.heads_kv) & 7) == 0) {
-      divmod(small, bid >> 3, per_unit, unit, s);
-      unit = unit * 8 + (bid & 7);
-    } else {
-      divmod(small, bid, per_unit, unit, s);
-    }
-    divmod(small, s, group, tile, member);
-    divmod(small, unit, L.heads_kv, b, kvh);
-    const int t = L.from_end ? (int)tile : L.n_tiles - 1 - (int)tile;
+    uint32_t member, b, kvh;
+    int t;
+    unit_item(L, small, bid, group, b, kvh, member, t);
     it.b = (int)b;
     it.h = (int)(kvh * group + member);
     it.kvh = (int)kvh;
@@ -208,9 +238,7 @@ static void check_all(const Launch& L) {
   const int block = level_block(L);
   std::vector<int> cost_of_id(L.n_items, -1);
   for (int wg = 0; wg < L.grid; ++wg) {
-    const std::vector<ItemId> own = items(L, wg);
-    for (int round = 0; round < kMaxRounds; ++round) {
-      const ItemId& it = own[round];
+    for (const ItemId& it : items(L, wg, block)) {
       if (it.t < 0) continue;
       check_in_range(L, it);
       const int at = base[it.b] + it.h * L.tiles(it.b) + it.t;
@@ -227,6 +255,18 @@ static void check_all(const Launch& L) {
       CHECK(cost_of_id[id] < least + block, "id %lld streams past %d tiles, one before it past %d", id, cost_of_id[id], least);
       least = std::min(least, cost_of_id[id]);
     }
+  // the load that decides between the orders is what the unit order gives these workgroups
+  if ((L.grid & 7) == 0 && L.grid <= 256 && L.batch <= kLevelMaxBatch) {
+    long long worst = 0;
+    double work = 0;
+    for (int wg = 0; wg < L.grid; wg += 8) {
+      long long load = 0;
+      for (const ItemId& it : items(L, wg, 0)) load += it.t >= 0 ? cost(L, it) : 0;
+      worst = std::max(worst, load);
+    }
+    for (int b = 0; b < L.batch; ++b) work += 0.5 * L.tiles(b) * (L.tiles(b) + 1);
+    if (work > 0) CHECK(std::fabs(sampled_load(L) - (double)worst * L.grid / (work * L.heads)) < 1e-9, "sampled load %.3f", sampled_load(L));
+  }
   long long missing = 0;
   for (unsigned char c : seen) missing += c == 0;
   CHECK(missing == 0, "%lld of %zu items are dealt to nobody (%lld ids, %lld workgroups)", missing, seen.size(), L.n_items, L.grid);
@@ -237,8 +277,9 @@ static void check_all(const Launch& L) {
 static double imbalance(const Launch& L, int resident) {
   std::vector<long long> load(resident, 0);
   long long total = 0;
+  const int block = level_block(L);
   for (int wg = 0; wg < L.grid; ++wg)
-    for (const ItemId& it : items(L, wg))
+    for (const ItemId& it : items(L, wg, block))
       if (it.t >= 0) {
         load[wg % resident] += cost(L, it);
         total += cost(L, it);
@@ -280,6 +321,7 @@ static void test(std::mt19937& rng) {
     }
   }
   // ids around 2^22, where the divisions change: sampled workgroups against the order written out
+  int by_level = 0;
   for (const int batch : {64, 65})
     for (const int heads : {2044, 2047, 2048, 2049})
       for (const bool from_end : {false, true}) {
@@ -291,7 +333,8 @@ static void test(std::mt19937& rng) {
         L.max_seqlen = 128 * n_tiles;
         L.plan(256);
         const int block = level_block(L);
-        CHECK((block != 0) == (batch == 64), "batch %d: block %d", batch, block);
+        by_level += block != 0;
+        CHECK(block == 0 || batch == 64, "batch %d: block %d", batch, block);
         std::vector<std::pair<int, int>> pairs;  // (sequence, tile)
         if (block)
           for (int first = (n_tiles - 1) / block * block; first >= 0; first -= block)
@@ -300,7 +343,7 @@ static void test(std::mt19937& rng) {
                 pairs.push_back({b, from_end ? L.tiles(b) - 1 - t : t});
         for (int rep = 0; rep < 40; ++rep) {
           const int wg = rep == 0 ? 0 : rep == 1 ? (int)L.grid - 1 : (int)(rng() % L.grid);
-          const std::vector<ItemId> own = items(L, wg);
+          const std::vector<ItemId> own = items(L, wg, block);
           for (const ItemId& it : own) {
             const long long id = it.id;
             if (it.t >= 0) check_in_range(L, it);
@@ -323,6 +366,7 @@ static void test(std::mt19937& rng) {
         }
         ++cases;
       }
+  CHECK(by_level > 4, "%d launches of 2^22 ids by level", by_level);
   // the batch of five sequences that the comment in item_order.h quotes, 256 workgroups
   std::printf("item order: %d launches; busiest workgroup / mean, by level (unit by unit):", cases);
   for (const int hkv : {8, 32})
@@ -509,9 +553,9 @@ static void execute(std::vector<std::vector<Step>>& prog, M& m, int ksteps) {
 }
 
 // The items of workgroup wg, as next_item() finds them.
-static std::vector<Item> items_of(const order::Launch& L, int wg, int tn) {
+static std::vector<Item> items_of(const order::Launch& L, int wg, int tn, int block) {
   std::vector<Item> out;
-  for (const order::ItemId& id : order::items(L, wg)) {
+  for (const order::ItemId& id : order::items(L, wg, block)) {
     if (id.t < 0) continue;
     Item it;
     it.id = (id.b * L.heads + id.h) * L.n_tiles + id.t;
@@ -526,8 +570,9 @@ static std::vector<Item> items_of(const order::Launch& L, int wg, int tn) {
 
 static void run(const Shape& s, const order::Launch& L, int ksteps, int ipw, int out_stores_full, Machine& m) {
   m.ipw2 = 2 * ipw;
+  const int block = order::level_block(L);
   for (int wg = 0; wg < L.grid; ++wg) {
-    const std::vector<Item> items = items_of(L, wg, TN);
+    const std::vector<Item> items = items_of(L, wg, TN, block);
     if (items.empty()) continue;
     m = Machine();
     m.ipw2 = 2 * ipw;
@@ -624,8 +669,9 @@ constexpr int NW = 4, NS = 5, TN = 32, BM = 128;
 using Machine = MachineT<NW, NS>;
 
 static void run(const Shape& s, const order::Launch& L, int ksteps, int ipw) {
+  const int block = order::level_block(L);
   for (int wg = 0; wg < L.grid; ++wg) {
-    const std::vector<Item> items = items_of(L, wg, TN);
+    const std::vector<Item> items = items_of(L, wg, TN, block);
     if (items.empty()) continue;
     Machine m;
     m.ipw2 = 2 * ipw;
@@ -1144,7 +1190,7 @@ int main(int argc, char** argv) {
   std::mt19937 rng(12345);
   // (a mistake that sits in another part is not looked for in these two, which take longest)
   const auto in = [](std::initializer_list<int> parts) { return std::find(parts.begin(), parts.end(), g_mut) != parts.end(); };
-  if (in({0, 7, 16, 17, 18, 19})) order::test(rng);
+  if (in({0, 7, 16, 17, 18, 19, 24})) order::test(rng);
   if (in({0, 1, 2, 3, 4, 8, 11, 12})) dense::test(rng);
   sparse::test(rng);
   softmax::test(rng);

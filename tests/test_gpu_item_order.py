@@ -119,3 +119,30 @@ def test_more_rounds_by_level():
         want = ta.flash_attn_triton_bwd(q[:, :, p], k[:, :, p], v[:, :, p], o[:, :, p], do[:, :, p], lse[:, :, p], cu, sm)
         for a, w in zip(grads, want):
             assert torch.equal(a[:, :, p], w), p
+
+
+@pytest.mark.parametrize("lens,H,D", [
+    ([random.Random(i).randint(490, 700) for i in range(48)], 16, 128),   # nine rounds and more, nearly even: unit order
+    ([8192, 5900, 7000], 16, 128),                                        # few and uneven: level order
+    ([8192, 8101, 8192, 8040], 8, 64),
+], ids=["many", "few", "alike"])
+def test_rounds_enough_for_either_order(lens, H, D):
+    """From six rounds up the kernels choose the order from the lengths: the bits of calls on one head."""
+    import tritonops_amd as ta
+
+    q, k, v, do = (_gpu_randn((1, sum(lens), H, D), i) for i in range(4))
+    cu = cu_from(torch.tensor(lens, dtype=torch.int32)).cuda()
+    sm = D ** -0.5 * ta.LOG2E
+    for form in ("256", "128"):
+        with ta.dense_form(form):
+            o, lse = ta.flash_attn_triton_fwd(q, k, v, cu, sm)
+            for h in range(H):
+                p = slice(h, h + 1)
+                o1, lse1 = ta.flash_attn_triton_fwd(q[:, :, p], k[:, :, p], v[:, :, p], cu, sm)
+                assert torch.equal(o[:, :, p], o1) and torch.equal(lse[:, :, p], lse1), (form, h)
+    grads = ta.flash_attn_triton_bwd(q, k, v, o, do, lse, cu, sm)
+    for h in range(H):
+        p = slice(h, h + 1)
+        want = ta.flash_attn_triton_bwd(q[:, :, p], k[:, :, p], v[:, :, p], o[:, :, p], do[:, :, p], lse[:, :, p], cu, sm)
+        for a, w in zip(grads, want):
+            assert torch.equal(a[:, :, p], w), h

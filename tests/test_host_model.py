@@ -42,6 +42,7 @@ MISTAKES = {
     21: "decode: the merge walks every slot of the bound",
     22: "decode: no barrier between the last reads of a step and the next step's stores",
     23: "decode: the refill behind a store fetches the next step again",
+    24: "choice of the order: odd rounds are sampled as if they ran forward",
 }
 
 

@@ -19,8 +19,9 @@
 // and a few items of a third and the longest one alone is 1.2 times the mean,
 // 1.57 -> 1.09 with 32.
 //
-// The window walk's items cost a band each, not t + 1 tiles, until the local
-// window is filled; numbered by level it gains from the same balance: seven
+// The window walk's items cost t + 1 tiles only until the local window is filled
+// and a band each from there; numbered by level (always: what the unit order would
+// cost it is not t + 1 either) it gains from the same balance: seven
 // sequences of 500 to 7000 tokens, 16 heads, local window 2048: 296 -> 225 us
 // with 4 kv-heads, 301 -> 234 with 16; six of 1024 to 12288, 32 heads: 964 -> 950
 // and 1038 -> 994.
@@ -32,9 +33,17 @@
 // 595 us, four sequences of 8192 (two sharers) 2085 instead of 1919.  So
 //  - in launches of six rounds or more `block` adjacent levels of a sequence
 //    stay together, as many as make four sharers with the query heads of the
-//    group (eight from twelve rounds up: a level more or less weighs little), and
+//    group (eight from twelve rounds up: a level more or less weighs little),
 //  - equal lengths, which the unit-by-unit order deals out evenly, keep that
-//    order from four rounds up.
+//    order from four rounds up, and
+//  - from six rounds up so do lengths that it deals out nearly evenly: many
+//    sequences even out over a workgroup's rounds.  The kernel works out what the
+//    busiest of 32 workgroups would get (about a microsecond) and takes the level
+//    order above kLevelWorth of the mean.  Level -> unit order: 48 sequences of
+//    490 to 700 tokens, 16 heads of their own (1.15 and 1.04 times the mean),
+//    forward 153 -> 146 us, backward 522 -> 502; four of 8040 to 8192, 32 heads
+//    (keys 1.00), backward 7059 -> 6616.  Where the level order stays, two
+//    sequences of 5900 to 8192 (1.57 and more), it is 1.3 to 1.4 times as fast.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -48,6 +57,13 @@ constexpr int kLevelMaxBatch = 64;
 // instance one sequence of 3000 tokens with 32 heads of its own, a round and a
 // half of 256-row items: 121 against 83 us forward, 402 against 328 backward).
 constexpr int kLevelEvenRounds = 4;
+// From kLevelWorthRounds rounds on, the load of the busiest workgroup in the unit
+// order, in hundredths of the mean, above which the level order pays for its
+// sharing: measured on 63 batches of 1 to 64 sequences, it loses up to 12 % where
+// that is 115 or less and gains 1 to 45 % from 123 on (launches of one workgroup
+// or two per CU).  Three workgroups to a CU share what their CU has left when one
+// of them is done: 124 to 130 still lost 2 to 3 %, 160 gained 22 (in fewer rounds).
+constexpr int kLevelWorthRounds = 6, kLevelWorth = 120, kLevelWorthThree = 135, kLevelAlways = 0;
 
 // Is a launch numbered by level?  (A single round of workgroups takes as long as
 // its longest item in any order.  cu == null: a batched call, equal lengths.)
@@ -88,7 +104,7 @@ inline long long persistent_grid(long long items, long long resident) {
 // which every later query streams past), else the last.  heads_kv: heads per
 // sequence that share nothing (units); heads / heads_kv items of a unit run
 // side by side on each of its tiles.
-template <int ROWS, bool FROM_END>
+template <int ROWS, bool FROM_END, int WORTH = kLevelWorth>
 __device__ __forceinline__ ItemId items_of_rounds(const int32_t* cu, const int batch, const int max_seqlen,
                                                   const int n_tiles, const int heads, const int heads_kv,
                                                   const bool level_order, const int n_items, const int grid) {
@@ -121,6 +137,20 @@ __device__ __forceinline__ ItemId items_of_rounds(const int32_t* cu, const int b
   };
   uint32_t group, rest;
   divmod((uint32_t)heads, (uint32_t)heads_kv, group, rest);
+  // item `id` of the unit order: sequence, kv-head, member of its group and slot of the unit's tiles
+  const uint32_t per_unit = (uint32_t)n_tiles * group;
+  auto unit_item = [&](uint32_t id, uint32_t& b, uint32_t& kvh, uint32_t& member, int& t) __attribute__((always_inline)) {
+    uint32_t unit, s, tile;
+    if (((batch * heads_kv) & 7) == 0) {
+      divmod(id >> 3, per_unit, unit, s);
+      unit = unit * 8 + (id & 7);
+    } else {
+      divmod(id, per_unit, unit, s);
+    }
+    divmod(s, group, tile, member);
+    divmod(unit, (uint32_t)heads_kv, b, kvh);
+    t = FROM_END ? (int)tile : n_tiles - 1 - (int)tile;
+  };
   ItemId it = {0, 0, 0, -1};
   if (level_order) {
     int tiles = 0;  // of sequence `lane`
@@ -134,7 +164,34 @@ __device__ __forceinline__ ItemId items_of_rounds(const int32_t* cu, const int b
     total = __builtin_amdgcn_readfirstlane(total);
     const int tiles0 = __builtin_amdgcn_readfirstlane(tiles);
     const bool even = __builtin_amdgcn_ballot_w64(lane < batch && tiles != tiles0) == 0;
-    if (!(cu && even && total * heads >= kLevelEvenRounds * grid)) {
+    bool by_unit = cu && even && total * heads >= kLevelEvenRounds * grid;
+    if (WORTH != kLevelAlways && !by_unit && total * heads >= kLevelWorthRounds * grid && (grid & 7) == 0) {
+      // what the unit order would give 32 workgroups of the first XCD, one to a lane, rounds of one parity to a
+      // half of the wavefront
+      const int per_xcd = grid >> 3, half = lane >> 5;
+      const int slot = (lane & 31) * max(per_xcd >> 5, 1);
+      const int at = half ? per_xcd - 1 - slot : slot;
+      int load = 0;
+      for (int r = 0; r < kMaxRounds && (long long)r * grid < n_items; r += 2) {
+        const long long id2 = (long long)(r + half) * grid + at * 8;
+        const bool live = slot < per_xcd && id2 < n_items;
+        uint32_t b2, kvh2, member2;
+        int t2;
+        unit_item(live ? (uint32_t)id2 : 0u, b2, kvh2, member2, t2);
+        const int all = __shfl(tiles, (int)b2, 64);
+        if (live && t2 < all) load += FROM_END ? all - t2 : t2 + 1;
+      }
+      load += __shfl_xor(load, 32, 64);
+      float work = 0.5f * (float)tiles * (float)(tiles + 1);  // of one head of sequence `lane`
+#pragma unroll
+      for (int m = 32; m >= 1; m >>= 1) {
+        load = max(load, __shfl_xor(load, m, 64));
+        work += __shfl_xor(work, m, 64);
+      }
+      by_unit = (float)load * (float)grid * 100.f <= (float)WORTH * work * (float)heads;
+      by_unit = __builtin_amdgcn_readfirstlane(by_unit);
+    }
+    if (!by_unit) {
       const int sharers = total * heads >= 12 * grid ? 8 : total * heads >= 6 * grid ? 4 : 1;
       int block = 1;  // adjacent levels of a sequence that stay together
       while (block * (int)group < sharers) block *= 2;
@@ -167,17 +224,9 @@ __device__ __forceinline__ ItemId items_of_rounds(const int32_t* cu, const int b
       return it;
     }
   }
-  const uint32_t per_unit = (uint32_t)n_tiles * group;
-  uint32_t unit, s, tile, member, b, kvh;
-  if (((batch * heads_kv) & 7) == 0) {
-    divmod(bid >> 3, per_unit, unit, s);
-    unit = unit * 8 + (bid & 7);
-  } else {
-    divmod(bid, per_unit, unit, s);
-  }
-  divmod(s, group, tile, member);
-  divmod(unit, (uint32_t)heads_kv, b, kvh);
-  const int t = FROM_END ? (int)tile : n_tiles - 1 - (int)tile;
+  uint32_t member, b, kvh;
+  int t;
+  unit_item(bid, b, kvh, member, t);
   it.b = (int)b;
   it.h = (int)(kvh * group + member);
   it.kvh = (int)kvh;

@@ -1254,8 +1254,8 @@ dense_short_kernel(const PrefillParams p) {
     return WIN ? (j + (j >= it.n_sink ? it.skip : 0)) * TN : j * TN;
   };
   const int wl = p.win_local, wg = p.win_global;
-  const ItemId ids = items_of_rounds<BM, false>(p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv,
-                                                p.by_level, p.n_items, gridDim.x);
+  const ItemId ids = items_of_rounds<BM, false, WIN ? kLevelAlways : short_per_cu(D) == 3 ? kLevelWorthThree : kLevelWorth>(
+      p.cu, p.batch, p.max_seqlen, p.n_qtiles, p.hq, p.hkv, p.by_level, p.n_items, gridDim.x);
   uint64_t left = __builtin_amdgcn_ballot_w64(ids.t >= 0);
   auto next_item = [&](Item& it) __attribute__((always_inline)) -> bool {
     ItemGeo g;
