@@ -91,9 +91,9 @@ inline long long persistent_grid(long long items, long long resident) {
 // All items of a workgroup, one per lane (round = lane): the searches and
 // divisions of all of them at once, in vector code ahead of the item loop,
 // instead of a chain of scalar code at every item boundary.  (The kv-head comes
-// along: dividing by the group again at each boundary cost 0.35 us on one
-// prompt of 1000 tokens, 23.9 against 23.5 us, and six registers at head_dim
-// 128.)  Odd rounds are walked back to
+// along: dividing by the group again at each boundary cost six registers at
+// head_dim 128; in time no more than runs differ, 23.9 against 23.5 us on one
+// prompt of 1000 tokens.)  Odd rounds are walked back to
 // front within each XCD (id & 7 is kept), so that the workgroup that drew a
 // long item in one round draws a short one in the next.
 //
