@@ -69,7 +69,7 @@ __device__ __forceinline__ int64_t kept_unit(int t_tile, int n_tile, int tiles_n
 // bytes per logit instead of running the product again.  The stores of a tile
 // drain before its next step's loads count as landed, and all workgroups reach
 // the end of a tile together, so they cost what 4 bytes per logit cost at 5 to
-// 6 TB/s: 6.99 -> 7.70 ms at 8192 x 4096 x 128256 (rows of 32 bytes per token
+// 6 TB/s: 6.49 -> 7.68 ms at 8192 x 4096 x 128256 (rows of 32 bytes per token
 // would be row-major, and far slower: short pieces of many rows per store).  Without the non-temporal hint
 // 7.74 ms there, but 1.40 instead of 1.15 ms at 4096 x 1024 x 128256, and at
 // dim 512 it costs three times as much.
@@ -193,39 +193,40 @@ __global__ void __launch_bounds__(512) xent_gemm_kernel(const XentParams p) {
   // One step = four 16-element sub-steps of 8 MFMAs.  The fragments of sub-step
   // s + 1 are read while the MFMAs of sub-step s issue; sched_barrier(0) pins
   // the slices (two reads, two MFMAs) so that the reads stay spread out.
-  auto compute = [&](int stage) __attribute__((always_inline)) {
-    i32x4 af[2][4], bf[2][2];
-    auto read_a = [&](int s, int rb) __attribute__((always_inline)) {
-      af[s & 1][rb] = *(lds_i32x4*)(uintptr_t)(a_addr[s] + stage * kXSlabB + rb * 4096);
-    };
-    auto read_b = [&](int s, int cb) __attribute__((always_inline)) {
-      bf[s & 1][cb] = *(lds_i32x4*)(uintptr_t)(b_addr[s] + stage * kXSlabB + cb * 4096);
-    };
-    read_b(0, 0);
-    read_b(0, 1);
+  i32x4 af[2][4], bf[2][2];
+  auto read_a = [&](int stage, int s, int rb) __attribute__((always_inline)) {
+    af[s & 1][rb] = *(lds_i32x4*)(uintptr_t)(a_addr[s] + stage * kXSlabB + rb * 4096);
+  };
+  auto read_b = [&](int stage, int s, int cb) __attribute__((always_inline)) {
+    bf[s & 1][cb] = *(lds_i32x4*)(uintptr_t)(b_addr[s] + stage * kXSlabB + cb * 4096);
+  };
+  auto read_first = [&](int stage) __attribute__((always_inline)) {
+    read_b(stage, 0, 0);
+    read_b(stage, 0, 1);
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) read_a(0, rb);
+    for (int rb = 0; rb < 4; ++rb) read_a(stage, 0, rb);
+  };
+  // sub-step s on the fragments in registers, those of sub-step sn of `stage` read along the way (sn < 0: none);
+  // first_load >= 0: every slice carries one load of the step that drip() is armed for
+  auto sub_step = [&](int s, int stage, int sn, int first_load) __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb) {
-        if (s + 1 < 4) {
-          if (rb == 0) {
-            read_b(s + 1, 0);
-            read_b(s + 1, 1);
-          } else if (rb == 1) {
-            read_a(s + 1, 0);
-            read_a(s + 1, 1);
-          } else if (rb == 2) {
-            read_a(s + 1, 2);
-            read_a(s + 1, 3);
-          }
+    for (int rb = 0; rb < 4; ++rb) {
+      if (sn >= 0) {
+        if (rb == 0) {
+          read_b(stage, sn, 0);
+          read_b(stage, sn, 1);
+        } else if (rb == 1) {
+          read_a(stage, sn, 0);
+          read_a(stage, sn, 1);
+        } else if (rb == 2) {
+          read_a(stage, sn, 2);
+          read_a(stage, sn, 3);
         }
-        acc[rb][0] = Elem<T>::mfma(af[s & 1][rb], bf[s & 1][0], acc[rb][0]);
-        acc[rb][1] = Elem<T>::mfma(af[s & 1][rb], bf[s & 1][1], acc[rb][1]);
-        if (4 * s + rb < 8) drip(4 * s + rb);   // the first eight slices carry one load each
-        __builtin_amdgcn_sched_barrier(0);
       }
+      acc[rb][0] = Elem<T>::mfma(af[s & 1][rb], bf[s & 1][0], acc[rb][0]);
+      acc[rb][1] = Elem<T>::mfma(af[s & 1][rb], bf[s & 1][1], acc[rb][1]);
+      if (first_load >= 0) drip(first_load + rb);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -382,35 +383,83 @@ __global__ void __launch_bounds__(512) xent_gemm_kernel(const XentParams p) {
       for (int cb = 0; cb < 2; ++cb) acc[rb][cb] = (f32x16){0};
   };
 
-  // ---- main loop: one barrier per step; the loads of step it + 1 fly during
-  // the products of step it.  D is a multiple of 128, so a tile is a whole
-  // number of step pairs.
-  int ck = 0, cn0 = tile_first * kXTileN;
-  int it = 0;
+  // ---- main loop: one barrier per step.  D is a multiple of 128, so a tile is
+  // a whole number of step pairs.
   arm(0, total > 0);
 #pragma unroll
   for (int k = 0; k < 8; ++k) drip(k);
   next();
-  auto step = [&](int stage) __attribute__((always_inline)) {
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    __syncthreads();
-    const bool more = ++it < total;
-    arm(stage ^ 1, more);
-    compute(stage);
-    if (more) next();
-  };
-  while (it < total) {
-    step(0);
-    step(1);
-    ck += 2;
-    if (ck == nk) {
-      finish_tile(cn0);
-      ck = 0;
-      cn0 += kXTileN;
+  if constexpr (GRAD) {
+    int ck = 0, cn0 = tile_first * kXTileN;
+    int it = 0;
+    // The loads of step it + 1 fly during the products of step it, and the stage
+    // that a tile's last step has left is the epilogue's staging area.
+    auto step = [&](int stage) __attribute__((always_inline)) {
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+      __syncthreads();
+      const bool more = ++it < total;
+      arm(stage ^ 1, more);
+      read_first(stage);
+      sub_step(0, stage, 1, 0);
+      sub_step(1, stage, 2, 4);
+      sub_step(2, stage, 3, -1);
+      sub_step(3, stage, -1, -1);
+      if (more) next();
+    };
+    while (it < total) {
+      step(0);
+      step(1);
+      ck += 2;
+      if (ck == nk) {
+        finish_tile(cn0);
+        ck = 0;
+        cn0 += kXTileN;
+      }
     }
+    return;
+  }
+  // The barrier of a step lies between its third and fourth sub-step: the step's
+  // last fragments are in registers by then, so its stage is free for the loads
+  // of step it + 2, and the fourth sub-step's MFMAs run while the first fragments
+  // of step it + 1 are read.  With the barrier at the top of a step all eight
+  // wavefronts wait for their first fragments together, with no MFMA in flight:
+  // 6875 -> 6490 us at 8192 x 4096 x 128256 (keeping the logits 7845 -> 7680),
+  // 937 -> 888 at 4096 x 2560 x 50257, 140 -> 134 at 1000 x 2048 x 32000, the
+  // same bits.  (All eight loads of a step behind the fourth sub-step: 6465 / 7750
+  // where 6412 / 7600 were measured for this split.)
+  arm(1, total > 1);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) drip(k);
+  next();
+  int sent = 2;              // steps whose loads have been sent, or are about to be
+  bool half_sent = false;    // drip() is armed and its loads 4 to 7 are still to go
+  arm(0, false);
+  __builtin_amdgcn_s_waitcnt(waitcnt_vm(8));
+  __syncthreads();
+  // `more`: the next step is of the same tile, its first fragments are read along the way
+  auto step = [&](int stage, bool more) __attribute__((always_inline)) {
+    sub_step(0, stage, 1, 4);
+    if (half_sent) next();
+    sub_step(1, stage, 2, -1);
+    sub_step(2, stage, 3, -1);
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0) & ~(15 << 8));  // fragments read, the loads of step it + 1 landed
+    __syncthreads();
+    half_sent = sent < total;
+    arm(stage, half_sent);
+    ++sent;
+    sub_step(3, stage ^ 1, more ? 0 : -1, 0);
+  };
+  for (int tile = 0; tile < tile_cnt; ++tile) {
+    read_first(0);
+    for (int k = 2; k < nk; k += 2) {
+      step(0, true);
+      step(1, true);
+    }
+    step(0, true);
+    step(1, false);
+    finish_tile((tile_first + tile) * kXTileN);
   }
 
-  if (GRAD) return;
   // ---- lane halves, then the two wavefronts that share tokens
 #pragma unroll
   for (int cb = 0; cb < 2; ++cb) {
