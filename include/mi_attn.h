@@ -472,6 +472,17 @@ int mi_xent_bwd_dlogits(const mi_xent_bwd_args *args, void *stream);
 size_t mi_xent_kept_bytes(int64_t tokens, int64_t vocab);
 int mi_xent_fwd_keep(const mi_xent_args *args, void *kept, void *stream);
 int mi_xent_kept_dlogits(const mi_xent_bwd_args *args, const void *kept, void *stream);
+/* The same with a second copy of the dlogits the other way round, for a BLAS that
+ * is faster on operands contiguous along the summed index: dlogits_t [vocab, ld_t]
+ * (16-byte aligned, ld_t a multiple of 8 and at least tokens rounded up to 64);
+ * its columns from `tokens` up to that multiple of 64 are zeroed. */
+int mi_xent_kept_dlogits_both(const mi_xent_bwd_args *args, const void *kept, void *dlogits_t, int64_t ld_t, void *stream);
+
+/* dst[c][r] = src[r][c] for 16-bit elements: src [rows, cols] with row stride
+ * ld_src, dst [cols, ld_dst]; cols, ld_src and ld_dst multiples of 8, both bases
+ * 16-byte aligned, ld_dst at least rows rounded up to 64; the columns of dst from
+ * `rows` up to that multiple of 64 are zeroed.  src and dst do not overlap. */
+int mi_transpose16(const void *src, int64_t rows, int64_t cols, int64_t ld_src, void *dst, int64_t ld_dst, void *stream);
 
 /* In place over a block of logits [rows, vocab] (row stride ld, elements):
  * logits[t,n] <- dloss[t] (exp(logits[t,n] - lse[t]) - [n == y[t]]), the

@@ -169,6 +169,8 @@ EXPORTS = {
     "mi_xent_kept_bytes": (_sz, [C.c_int64, C.c_int64]),
     "mi_xent_fwd_keep": (C.c_int, [C.POINTER(XentArgs), _vp, _vp]),
     "mi_xent_kept_dlogits": (C.c_int, [C.POINTER(XentBwdArgs), _vp, _vp]),
+    "mi_xent_kept_dlogits_both": (C.c_int, [C.POINTER(XentBwdArgs), _vp, _vp, _i64, _vp]),
+    "mi_transpose16": (C.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "mi_xent_dlogits": (C.c_int, [C.POINTER(XentGradArgs), _vp]),
     "mi_xent_bwd_dlogits": (C.c_int, [C.POINTER(XentBwdArgs), _vp]),
     "mi_decode_num_splits": (C.c_int, [C.POINTER(DecodeArgs)]),

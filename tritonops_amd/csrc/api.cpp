@@ -322,7 +322,8 @@ int mi_xent_fwd_keep(const mi_xent_args* a, void* kept, void* stream) {
   return xent_fwd(a, static_cast<float*>(kept), stream, "mi_xent_fwd_keep");
 }
 
-int mi_xent_kept_dlogits(const mi_xent_bwd_args* a, const void* kept, void* stream) {
+static int kept_dlogits(const mi_xent_bwd_args* a, const void* kept, bool both, void* dlogits_t, int64_t ld_t, void* stream,
+                        const char* what) {
   if (!a) return fail(MI_ERR_NULL_POINTER, "args is NULL");
   if (a->struct_size != sizeof(mi_xent_bwd_args))
     return fail(MI_ERR_STRUCT_SIZE, "mi_xent_bwd_args.struct_size %u != %zu", a->struct_size, sizeof(mi_xent_bwd_args));
@@ -335,6 +336,12 @@ int mi_xent_kept_dlogits(const mi_xent_bwd_args* a, const void* kept, void* stre
     return fail(MI_ERR_NULL_POINTER, "kept, y, lse, dloss and dlogits must be non-NULL");
   if (!aligned16(kept)) return fail(MI_ERR_ALIGNMENT, "kept must be 16-byte aligned");
   if (a->ld < a->vocab) return fail(MI_ERR_STRIDE, "ld %lld < vocab", (long long)a->ld);
+  if (both) {
+    if (!dlogits_t) return fail(MI_ERR_NULL_POINTER, "dlogits_t must be non-NULL");
+    if (!aligned16(dlogits_t)) return fail(MI_ERR_ALIGNMENT, "dlogits_t must be 16-byte aligned");
+    if (!mult8(ld_t) || ld_t < ((int64_t)a->tokens + 63) / 64 * 64)
+      return fail(MI_ERR_STRIDE, "ld_t %lld must be a multiple of 8 and at least %d tokens rounded up to 64", (long long)ld_t, a->tokens);
+  }
   if (((long long)a->tokens + 63) / 64 * (((long long)a->vocab + 255) / 256) > 0x7fffff)
     return fail(MI_ERR_SHAPE, "tokens %d x vocab %d: more than 2^23 - 1 blocks of 64 x 256", a->tokens, a->vocab);
   mi::XentParams p;
@@ -345,8 +352,31 @@ int mi_xent_kept_dlogits(const mi_xent_bwd_args* a, const void* kept, void* stre
   p.kept = static_cast<float*>(const_cast<void*>(kept));
   p.dlogits = a->dlogits; p.dl_ld = a->ld;
   p.dl_vec = aligned16(a->dlogits) && a->ld % 8 == 0;
-  return launch_status(mi::launch_xent_kept_dlogits(p, a->dtype, static_cast<hipStream_t>(stream)), "mi_xent_kept_dlogits");
+  p.dlogits_t = both ? dlogits_t : nullptr; p.dlt_ld = ld_t;
+  return launch_status(mi::launch_xent_kept_dlogits(p, a->dtype, static_cast<hipStream_t>(stream)), what);
 }
+
+int mi_xent_kept_dlogits(const mi_xent_bwd_args* a, const void* kept, void* stream) {
+  return kept_dlogits(a, kept, false, nullptr, 0, stream, "mi_xent_kept_dlogits");
+}
+
+int mi_xent_kept_dlogits_both(const mi_xent_bwd_args* a, const void* kept, void* dlogits_t, int64_t ld_t, void* stream) {
+  return kept_dlogits(a, kept, true, dlogits_t, ld_t, stream, "mi_xent_kept_dlogits_both");
+}
+
+int mi_transpose16(const void* src, int64_t rows, int64_t cols, int64_t ld_src, void* dst, int64_t ld_dst, void* stream) {
+  if (rows < 0 || cols < 0) return fail(MI_ERR_SHAPE, "rows %lld and cols %lld must not be negative", (long long)rows, (long long)cols);
+  if (rows == 0 || cols == 0) return MI_OK;
+  if (!src || !dst) return fail(MI_ERR_NULL_POINTER, "src and dst must be non-NULL");
+  if (!aligned16(src) || !aligned16(dst)) return fail(MI_ERR_ALIGNMENT, "src and dst must be 16-byte aligned");
+  if (cols % 8) return fail(MI_ERR_SHAPE, "cols %lld must be a multiple of 8", (long long)cols);
+  if (!mult8(ld_src) || !mult8(ld_dst) || ld_src < cols || ld_dst < (rows + 63) / 64 * 64)
+    return fail(MI_ERR_STRIDE, "row strides must be multiples of 8 elements, ld_src >= cols and ld_dst >= rows rounded up to 64");
+  if (rows > 0x3fffffffLL || cols > 0x3fffffffLL || (rows + 255) / 256 * ((cols + 63) / 64) > 0x7fffffLL)
+    return fail(MI_ERR_SHAPE, "%lld x %lld: more than 2^23 - 1 blocks of 256 x 64", (long long)rows, (long long)cols);
+  return launch_status(mi::launch_transpose16(src, rows, cols, ld_src, dst, ld_dst, static_cast<hipStream_t>(stream)), "mi_transpose16");
+}
+
 
 int mi_xent_bwd_dlogits(const mi_xent_bwd_args* a, void* stream) {
   if (!a) return fail(MI_ERR_NULL_POINTER, "args is NULL");

@@ -108,7 +108,8 @@ struct XentParams {
   const float* dloss;  // [T], gradient launch
   void* dlogits;       // [T, N] row stride dl_ld (elements), gradient launch
   float* kept;         // xent_kept_bytes(T, N): logits as the forward's accumulators hold them, or null
-  int64_t dl_ld;
+  void* dlogits_t;     // [N, dlt_ld], kept form: dlogits the other way round, dlt_ld = T rounded up to 64 at least, or null
+  int64_t dl_ld, dlt_ld;
   int32_t dl_vec;      // dlogits rows can be written in 16-byte pieces
   int64_t x_st, w_st;
   int32_t T, D, N;
@@ -206,6 +207,9 @@ int launch_xent_fwd(const XentParams& p, int dtype, bool grad, hipStream_t s);  
 size_t xent_kept_bytes(long long tokens, long long vocab);
 int launch_xent_kept_dlogits(const XentParams& p, int dtype, hipStream_t s);
 int launch_xent_dlogits(const XentGradParams& p, int dtype, hipStream_t s);
+// dst[c][r] = src[r][c], 16-bit elements: src [rows, cols] and dst [cols, ld_dst] with 16-byte aligned rows of
+// multiples of 8 elements, ld_dst >= rows rounded up to 64; columns of dst from `rows` up to that multiple are zeroed.
+int launch_transpose16(const void* src, int64_t rows, int64_t cols, int64_t ld_src, void* dst, int64_t ld_dst, hipStream_t s);
 
 // Query rows per workgroup of the two prefill kernels.
 constexpr int kDenseRows = 256;

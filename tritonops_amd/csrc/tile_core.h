@@ -114,6 +114,16 @@ __device__ __forceinline__ i32x4 read_tr_pair(const unsigned char* a0, const uns
   return out;
 }
 
+// 8 x 8 elements of 16 bits, in[row] -> out[column], within a lane's registers: one byte permute per output dword.
+__device__ __forceinline__ void transpose8x8(const i32x4 (&in)[8], i32x4 (&out)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+      out[j][m] = (int)__builtin_amdgcn_perm((uint32_t)in[2 * m + 1][j >> 1], (uint32_t)in[2 * m][j >> 1],
+                                             (j & 1) ? 0x07060302u : 0x05040100u);
+}
+
 // ---------------------------------------------------------------------------
 // Layout policy 1: padded rows.
 template <int D>

@@ -32,8 +32,24 @@ _KEPT_ROWS = 256
 # 4.96 -> 5.25; dim 256, 8192 x 32000: 0.82 -> 0.97.
 KEEP_BYTES = 8 << 30
 KEEP_DIM = 1024
-# From KEEP_UNASKED bytes in all on, the memory is asked first: kept logits and the
-# backward's block of dlogits take at most a quarter of what is free (to the
+# The two gradient products sum over the vocabulary and over the tokens; the library
+# is fastest where both operands are contiguous along the summed index.
+# grad_w = dlogits^T x: a transposed x costs little, a second copy of the dlogits, written
+# along with the first, 0.55 us per million.  Both from _TURN_ROWS rows and _TURN_DIM
+# columns on (product before -> after, cost: 8192 x 4096 x 128256: 7.85 -> 5.55, 0.61 ms;
+# 4096 x 2560 x 128256: 2.49 -> 1.90, 0.29; 1000 x 2560 x 50304: 302 -> 249, 29 us), with
+# fewer columns the copy costs what it saves (4096 x 1024 x 128256: 1.07 -> 0.82, 0.29 ms)
+# and x alone is turned, from _TURN_X_ROWS rows on (1.07 -> 0.94; 1000 rows: 329 -> 332 us).
+# grad_x = dlogits w: a transposed w costs the same whatever the number of rows: from
+# _TURN_W_ROWS rows on, where the result has at least _TURN_W_TILES tiles of 256 x 256
+# (8192 x 4096 x 128256: 6.25 -> 5.34, 0.40 ms; 8192 x 1024: 1.69 -> 1.39, 0.10;
+# 4096 x 2560: 2.88 -> 2.02, 0.26, but 4096 x 1024: 1.25 -> 1.34 and 2048 x 4096:
+# 1.62 -> 1.37, 0.40).
+_TURN_ROWS, _TURN_DIM = 256, 1536
+_TURN_X_ROWS, _TURN_X_DIM = 2048, 1024
+_TURN_W_ROWS, _TURN_W_TILES = 4096, 128
+# From KEEP_UNASKED bytes in all on, the memory is asked first: kept logits and what the
+# backward allocates for its products take at most a quarter of what is free (to the
 # allocator or in its cache), so that what the program allocates next still fits.
 KEEP_UNASKED = 256 << 20
 # Kept logits that are alive: token -> (device, bytes).  An entry leaves when its
@@ -86,10 +102,10 @@ def _free_bytes(device):
     return torch.cuda.mem_get_info(device)[0] + reserved - used
 
 
-def _alloc_kept(T, N, device, esize, always):
+def _alloc_kept(T, N, device, bwd_bytes, always):
     """Room for the logits of [T, N], or None: where the automatic choice (not
-    `always`) finds too many of them alive or too little memory free, and where the
-    allocation fails."""
+    `always`) finds too many of them alive or too little memory free for them and
+    the `bwd_bytes` of the backward, and where the allocation fails."""
     nbytes = _lib.load().mi_xent_kept_bytes(T, N)
     token = object()
     with _kept_lock:
@@ -99,7 +115,7 @@ def _alloc_kept(T, N, device, esize, always):
                 return None
             # (a capture repeats what its program ran before it, and its pool is not in these figures)
             if live > KEEP_UNASKED and not torch.cuda.is_current_stream_capturing() \
-                    and 4 * (nbytes + min(T, BWD_ROWS) * N * esize) > _free_bytes(device):
+                    and 4 * (nbytes + bwd_bytes) > _free_bytes(device):
                 return None
         _kept_live[token] = (device, nbytes)
     try:
@@ -143,7 +159,7 @@ def _fwd(x, w, y, keep):
     a.workspace, a.workspace_bytes = _ptr(ws), nbytes
     kept = None
     if keep is not False and T and N:
-        kept = _alloc_kept(T, N, x.device, x.element_size(), bool(keep))
+        kept = _alloc_kept(T, N, x.device, _bwd_bytes(x, w), bool(keep))
     if kept is None:
         _lib.check(lib.mi_xent_fwd(C.byref(a), _stream()))
     else:
@@ -206,9 +222,10 @@ def _dlogits_rows(rows, N, like):
     return torch.empty((rows, ld), device=like.device, dtype=like.dtype)[:, :N]
 
 
-def _kept_dlogits(kept, first, y, lse, dloss, N, dl):
+def _kept_dlogits(kept, first, y, lse, dloss, N, dl, dl_t=None):
     """dl [rows, N] <- dlogits of the rows from `first` on (a multiple of _KEPT_ROWS),
-    from the logits that _fwd kept; the values of cross_entropy_dlogits."""
+    from the logits that _fwd kept; the values of cross_entropy_dlogits.  dl_t [N, ld]
+    receives their transpose as well, its columns behind `rows` zeros."""
     if first % _KEPT_ROWS:
         raise ValueError("rows of kept logits start at a multiple of %d, not at %d" % (_KEPT_ROWS, first))
     lib = _lib.load()
@@ -220,8 +237,59 @@ def _kept_dlogits(kept, first, y, lse, dloss, N, dl):
     a.y, a.lse, a.dloss = _ptr(y), _ptr(lse), _ptr(dloss)
     a.dlogits, a.ld = _ptr(dl), dl.stride(0) if dl.shape[0] > 1 else N
     at = C.c_void_p(kept.data_ptr() + lib.mi_xent_kept_bytes(first, N))
-    _lib.check(lib.mi_xent_kept_dlogits(C.byref(a), at, _stream()))
+    if dl_t is None:
+        _lib.check(lib.mi_xent_kept_dlogits(C.byref(a), at, _stream()))
+    else:
+        _lib.check(lib.mi_xent_kept_dlogits_both(C.byref(a), at, _ptr(dl_t), dl_t.shape[1], _stream()))
     return dl
+
+
+def _can_turn(t):
+    """Whether mi_transpose16 takes t (2-D, 16-bit)."""
+    return (t.stride(1) == 1 and t.shape[1] % 8 == 0 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1]
+            and t.data_ptr() % 16 == 0)
+
+
+def _room_turned(t):
+    """Room for the transpose of t [r, c]: [c rounded up to 8, r rounded up to 64], or
+    None without memory for it."""
+    try:
+        return torch.empty((-(-t.shape[1] // 8) * 8, -(-t.shape[0] // 64) * 64), device=t.device, dtype=t.dtype)
+    except torch.OutOfMemoryError:
+        return None
+
+
+def _turn(t, out):
+    """out <- the transpose of t, its columns behind t's rows zeros."""
+    rows, cols = t.shape
+    _lib.check(_lib.load().mi_transpose16(_ptr(t), rows, cols, t.stride(0) if rows > 1 else max(cols, t.stride(0)),
+                                          _ptr(out), out.shape[1], _stream()))
+    return out
+
+
+def _turns_x(rows, x):
+    """(x, dlogits): which operands of grad_w a block of `rows` rows takes the other way round."""
+    if not _can_turn(x):
+        return False, False
+    both = rows >= _TURN_ROWS and x.shape[1] >= _TURN_DIM
+    return both or (rows >= _TURN_X_ROWS and x.shape[1] >= _TURN_X_DIM), both
+
+
+def _turns_w(rows, w):
+    """Whether grad_x of a block of `rows` rows sums over a contiguous vocabulary."""
+    return (rows >= _TURN_W_ROWS and -(-rows // 256) * -(-w.shape[1] // 256) >= _TURN_W_TILES
+            and w.shape[1] >= _TURN_X_DIM and _can_turn(w))
+
+
+def _bwd_bytes(x, w):
+    """What the backward allocates for its dlogits and products at a time."""
+    rows, N = min(x.shape[0], BWD_ROWS), w.shape[0]
+    n = rows * N
+    turn_x, turn_dl = _turns_x(rows, x)
+    n += rows * (turn_x * x.shape[1] + turn_dl * N)
+    if _turns_w(rows, w):
+        n += w.numel()
+    return n * x.element_size()
 
 
 def cross_entropy_fused_bwd(grad_o, x, w, y, lse, rows_per_block=None):
@@ -240,20 +308,38 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
     if kept is not None and step % _KEPT_ROWS:
         step = max(step - step % _KEPT_ROWS, _KEPT_ROWS)
     grad_x = torch.empty_like(x)
-    grad_w = None
+    grad_w = w_t = None
+    if _turns_w(min(T, step), w):
+        w_t = _room_turned(w)
+        if w_t is not None:
+            w_t = _turn(w, w_t)[:, :w.shape[0]].t()
     for s in range(0, T, step):
         e = min(s + step, T)
         xc = x[s:e]
         dl = _dlogits_rows(e - s, w.shape[0], x)
+        turn_x, turn_dl = _turns_x(e - s, xc)
+        x_t = _room_turned(xc) if turn_x else None
+        dl_t = _room_turned(dl) if turn_dl and x_t is not None else None
         if kept is None:
             _dlogits(xc, w, y[s:e], lse[s:e], g[s:e], dl)
-        else:
+            if dl_t is not None:  # (rows of dlogits are padded to whole pieces of 8, see _dlogits_rows)
+                _turn(dl.as_strided((e - s, dl_t.shape[0]), dl.stride()), dl_t)
+        elif dl_t is None:
             _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl)
-        torch.mm(dl, w, out=grad_x[s:e])
-        if grad_w is None:
-            grad_w = torch.mm(dl.t(), xc)
         else:
-            grad_w.addmm_(dl.t(), xc)
+            _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl, dl_t)
+        torch.mm(dl, w if w_t is None else w_t, out=grad_x[s:e])
+        d, v = dl.t(), xc
+        if x_t is not None:
+            v = _turn(xc, x_t).t()
+            if dl_t is None:
+                v = v[:e - s]
+            else:  # (the columns behind the rows are zeros in both)
+                d = dl_t[:w.shape[0]]
+        if grad_w is None:
+            grad_w = torch.mm(d, v)
+        else:
+            grad_w.addmm_(d, v)
     if grad_w is None:
         grad_w = torch.zeros_like(w)
     return grad_x, grad_w
