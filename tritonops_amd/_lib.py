@@ -222,6 +222,23 @@ def load():
     return lib
 
 
+_native = None
+
+
+def native():
+    """The native host calls (csrc/host_calls.cpp), loaded behind the library."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise ImportError("tritonops_amd/_native.so is missing or does not load (%s): build it with "
+                              "`python -m tritonops_amd.build`" % e) from e
+        _native = module
+    return _native
+
+
 def check(status):
     if status != 0:
         raise MiAttnError(status, load().mi_last_error().decode())

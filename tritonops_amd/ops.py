@@ -65,6 +65,19 @@ def _stream():
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+def _here():
+    """(current device, its current stream) as the native calls take them."""
+    dev = torch.cuda.current_device()
+    return dev, _raw_stream(dev) if _raw_stream is not None else torch.cuda.current_stream(dev).cuda_stream
+
+
+def _outputs(r):
+    """What a native call gave: its outputs, or the status of the C ABI."""
+    if type(r) is int:
+        _lib.check(r)
+    return r
+
+
 def _inner_contig(t):
     return t if t.stride(-1) == 1 else t.contiguous()
 
@@ -121,6 +134,14 @@ def _rows_to_cover(cu_seq_lens, max_seqlen, rows):
         return rows
     longest, first, last = hit[2]
     return 0 if (first == 0 and last == rows and longest <= max_seqlen) else rows
+
+
+def _cu_launch(cu_seq_lens, max_seq_len, rows):
+    """(max_seqlen, total_rows) of a packed call over `rows` rows; (0, 0) of a batched one."""
+    if cu_seq_lens is None:
+        return 0, 0
+    max_len = min(_max_len(cu_seq_lens, max_seq_len), rows)
+    return max_len, _rows_to_cover(cu_seq_lens, max_len, rows)
 
 
 _HEAD_DIMS = (64, 96, 128)
@@ -196,10 +217,34 @@ def dense_form(form):
         _dense_form.value = before
 
 
+def _native_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse, bhsd):
+    """(o, lse) of a plain call in native code, or None (host_calls.cpp); with `bhsd`
+    all tensors are [X, H, S, D], without it [X, S, H, D]."""
+    if not q.is_cuda or q.dim() != 4:
+        return None
+    max_len, rows = _cu_launch(cu_seq_lens, max_seq_len, q.shape[1])
+    return _outputs(_lib.native().dense_fwd(q, k, v, cu_seq_lens, max_len, rows, scale_log2, causal, want_lse, bhsd,
+                                            getattr(_dense_form, "value", _lib.MI_DENSE_FORM_AUTO), *_here()))
+
+
 def _dense_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse=True, bhsd=False):
     """q,k,v as [X, S, H, D] (see _fill_qkvo). Returns (o, lse[X, S, H]); with
     `bhsd` the outputs own [X, H, S, D] / [X, H, S] memory and are returned as
     [X, S, H, ...] views of it."""
+    if not bhsd:
+        out = _native_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse, False)
+        if out is not None:
+            return out
+    elif q.dim() == k.dim() == v.dim() == 4:
+        out = _native_fwd(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), cu_seq_lens, scale_log2, causal,
+                          max_seq_len, want_lse, True)
+        if out is not None:
+            return out[0].transpose(1, 2), out[1].transpose(1, 2) if want_lse else None
+    return _general_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse, bhsd)
+
+
+def _general_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse, bhsd):
+    """_dense_fwd for every form of its arguments."""
     _check_qkv(q, k, v)
     _require_gpu(q, k, v, cu_seq_lens)
     lib = _lib.load()
@@ -252,6 +297,17 @@ def _dense_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse=T
 def _dense_bwd(q, k, v, o, do, lse, cu_seq_lens, scale_log2, causal, max_seq_len):
     """q, k, v, o, do as [X, S, H, D] views, lse [X, S, H] (see _fill_qkvo).
     Returns dq, dk, dv shaped and laid out like q, k, v."""
+    if q.is_cuda and q.dim() == 4:
+        max_len, rows = _cu_launch(cu_seq_lens, max_seq_len, q.shape[1])
+        out = _outputs(_lib.native().dense_bwd(q, k, v, o, do, lse, cu_seq_lens, max_len, rows, scale_log2, causal,
+                                               *_here()))
+        if out is not None:
+            return out
+    return _general_bwd(q, k, v, o, do, lse, cu_seq_lens, scale_log2, causal, max_seq_len)
+
+
+def _general_bwd(q, k, v, o, do, lse, cu_seq_lens, scale_log2, causal, max_seq_len):
+    """_dense_bwd for every form of its arguments."""
     _check_qkv(q, k, v)
     if o.shape != q.shape or do.shape != q.shape:
         raise ValueError("o %s and do %s must have the shape of q %s" % (tuple(o.shape), tuple(do.shape), tuple(q.shape)))
@@ -401,8 +457,11 @@ def flash_attention(q, k, v, cu_seq_lens=None, *, causal=True, softmax_scale=Non
         o, lse = _FlashAttention.apply(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), None, scale, causal,
                                        None, True)
     else:
-        o, lse = _dense_fwd(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), None, scale, causal,
-                            None, return_lse, bhsd=True)
+        out = _native_fwd(q, k, v, None, scale, causal, None, return_lse, True)
+        if out is not None:
+            return out if return_lse else out[0]
+        o, lse = _general_fwd(q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), None, scale, causal,
+                              None, return_lse, True)
     o = o.transpose(1, 2)  # contiguous [B,H,S,D]
     if return_lse:
         return o, lse.transpose(1, 2)
@@ -425,6 +484,49 @@ def flash_attn_sparse_triton(q, k, v, cu_seqlens, softmax_scale=None, local_wind
     `csr_strides`); diagonal blocks are masked causally per token.
     A query with no allowed key gets o = 0 and lse = -inf.
     """
+    if q.is_cuda and q.dim() == 4 and q.shape[-1] in _HEAD_DIMS and q.numel() != 0:
+        packed = cu_seqlens is not None
+        max_len, rows = _cu_launch(cu_seqlens, max_seq_len, q.shape[1])
+        lists = _sparse_lists(q.shape[-1], max_len if packed else q.shape[2], local_window_size, global_window_size,
+                              block_mask, row_ptr, col_idx, csr_strides, q.device)
+        scale = (q.shape[-1] ** -0.5 if softmax_scale is None else float(softmax_scale)) * LOG2E
+        out = _outputs(_lib.native().sparse_fwd(q, k, v, cu_seqlens, max_len, rows, scale, not packed, lists[0], lists[1],
+                                                *lists[2], lists[3], lists[4], *_here()))
+        if out is not None:
+            return out
+    return _general_sparse(q, k, v, cu_seqlens, softmax_scale, local_window_size, global_window_size, block_mask,
+                           row_ptr, col_idx, csr_strides, max_seq_len)
+
+
+def _sparse_lists(D, max_len, local_window_size, global_window_size, block_mask, row_ptr, col_idx, csr_strides, device):
+    """(row_ptr, col_idx, strides, win_local, win_global) of a sparse forward: the caller's lists, those of its
+    mask or windows, or none where the library works the blocks out from the two windows."""
+    nqb = max((max_len + _masks.BLOCK - 1) // _masks.BLOCK, 1)
+    wl = wg = -1
+    if row_ptr is None:
+        if block_mask is None:
+            wl, wg = int(local_window_size), int(global_window_size)
+            if wl < 0 or wg < 0:
+                raise ValueError("window sizes must be >= 0")
+            wl, wg = min(wl, 2 ** 31 - 1), min(wg, 2 ** 31 - 1)   # (the C ABI takes 32-bit windows; longer than any sequence either way)
+            # The library works the blocks out from the two windows when it
+            # gets no lists.  (local_window_size 0 hides even the diagonal; that
+            # case always goes through lists.)
+            use_lists = WINDOW_PREFILL_LISTS
+            if use_lists is None:
+                use_lists = not (D >= 96 and wl >= _WINDOW_WALK_MIN_LOCAL)
+            if wl < 1 or use_lists:
+                row_ptr, col_idx, csr_strides = _masks.window_csr(nqb, wl, wg, device)
+        else:
+            row_ptr, col_idx, csr_strides = _masks.block_mask_to_csr(block_mask, device)
+        if row_ptr is not None and row_ptr.shape[-1] - 1 < nqb:
+            raise ValueError("block mask covers %d query blocks, sequences need %d" % (row_ptr.shape[-1] - 1, nqb))
+    return row_ptr, col_idx, csr_strides, wl, wg
+
+
+def _general_sparse(q, k, v, cu_seqlens, softmax_scale, local_window_size, global_window_size, block_mask, row_ptr,
+                    col_idx, csr_strides, max_seq_len):
+    """flash_attn_sparse_triton for every form of its arguments."""
     if cu_seqlens is not None:
         _check_qkv(q, k, v)
     else:
@@ -464,26 +566,8 @@ def flash_attn_sparse_triton(q, k, v, cu_seqlens, softmax_scale=None, local_wind
         qv, kv, vv, ov, lv = (t.transpose(1, 2) for t in (q, k, v, o, lse))
         batch = X
     scale = (D ** -0.5 if softmax_scale is None else float(softmax_scale)) * LOG2E
-    nqb = max((max_len + _masks.BLOCK - 1) // _masks.BLOCK, 1)
-    wl = wg = -1
-    if row_ptr is None:
-        if block_mask is None:
-            wl, wg = int(local_window_size), int(global_window_size)
-            if wl < 0 or wg < 0:
-                raise ValueError("window sizes must be >= 0")
-            wl, wg = min(wl, 2 ** 31 - 1), min(wg, 2 ** 31 - 1)   # (the C ABI takes 32-bit windows; longer than any sequence either way)
-            # The library works the blocks out from the two windows when it
-            # gets no lists.  (local_window_size 0 hides even the diagonal; that
-            # case always goes through lists.)
-            use_lists = WINDOW_PREFILL_LISTS
-            if use_lists is None:
-                use_lists = not (D >= 96 and wl >= _WINDOW_WALK_MIN_LOCAL)
-            if wl < 1 or use_lists:
-                row_ptr, col_idx, csr_strides = _masks.window_csr(nqb, wl, wg, q.device)
-        else:
-            row_ptr, col_idx, csr_strides = _masks.block_mask_to_csr(block_mask, q.device)
-        if row_ptr is not None and row_ptr.shape[-1] - 1 < nqb:
-            raise ValueError("block mask covers %d query blocks, sequences need %d" % (row_ptr.shape[-1] - 1, nqb))
+    row_ptr, col_idx, csr_strides, wl, wg = _sparse_lists(D, max_len, local_window_size, global_window_size, block_mask,
+                                                          row_ptr, col_idx, csr_strides, q.device)
     if q.numel() == 0:
         return o, lse
     a = _lib.AttnSparseArgs()
@@ -508,6 +592,28 @@ def _decode(q, k, v, cu_seq_lens, seq_lens, scale, max_seq_len, split_tokens, re
             block_idx=None, block_cnt=None, bi_strides=(0, 0), max_blocks=0, split_blocks=0,
             window=(-1, -1), include_last=False, kv_layout="batched", page_table=None, page_size=0,
             window_form=False):
+    if q.is_cuda and (max_seq_len is None or max_seq_len >= 0) \
+            and (block_idx is None or tuple(bi_strides) == block_idx.stride()[:2]):
+        listed = window_form or block_idx is not None
+        out = _outputs(_lib.native().decode(
+            q, k, v, cu_seq_lens, seq_lens, float(scale) * LOG2E, -1 if max_seq_len is None else int(max_seq_len),
+            int((split_blocks if listed else split_tokens) or 0), return_lse, _KV_LAYOUTS.get(kv_layout, -1),
+            page_table, int(page_size or 0), block_idx, block_cnt, int(max_blocks), window[0], window[1], window_form,
+            include_last, *_here()))
+        if out is not None:
+            return out if return_lse else out[0]
+    return _general_decode(q, k, v, cu_seq_lens, seq_lens, scale, max_seq_len, split_tokens, return_lse, block_idx,
+                           block_cnt, bi_strides, max_blocks, split_blocks, window, include_last, kv_layout, page_table,
+                           page_size, window_form)
+
+
+_KV_LAYOUTS = {"batched": _lib.MI_KV_BATCHED, "packed": _lib.MI_KV_PACKED, "paged": _lib.MI_KV_PAGED}
+
+
+def _general_decode(q, k, v, cu_seq_lens, seq_lens, scale, max_seq_len, split_tokens, return_lse, block_idx, block_cnt,
+                    bi_strides, max_blocks, split_blocks, window, include_last, kv_layout, page_table, page_size,
+                    window_form):
+    """_decode for every form of its arguments."""
     if q.dim() != 3 or k.dim() != 4:
         raise ValueError("decoding takes q [B, Hq, D] and k, v [B, maxL, Hkv, D] (or a packed / paged cache)")
     if v.shape != k.shape:
@@ -682,8 +788,12 @@ def flash_attention_sparse_decoding(q, k, v, cu_seq_lens, global_window_size=64,
         cap = gw // _masks.BLOCK + (lw + _masks.BLOCK - 1) // _masks.BLOCK + 1
         return _decode(q, k, v, cu_seq_lens, seq_lens, scale, None, None, return_lse, max_blocks=cap,
                        split_blocks=split_blocks or 0, window=(lw, gw), window_form=True, **layout)
-    lens = seq_lens if seq_lens is not None else (cu_seq_lens[1:] - cu_seq_lens[:-1])
-    lens = lens.to(torch.int32)
+    cu = lens = None
+    if seq_lens is None and cu_seq_lens.dtype == torch.int32 and cu_seq_lens.dim() == 1 and cu_seq_lens.is_contiguous():
+        cu = cu_seq_lens    # the kernels take the lengths from it
+    else:
+        lens = seq_lens if seq_lens is not None else (cu_seq_lens[1:] - cu_seq_lens[:-1])
+        lens = lens.to(torch.int32)
     if block_indices.dim() != 3 or block_indices.shape[0] != B or block_indices.shape[1] != Hkv \
             or block_indices.is_floating_point():
         raise ValueError("block_indices must be an integer tensor [B, Hkv, n], got %s %s"
@@ -700,9 +810,9 @@ def flash_attention_sparse_decoding(q, k, v, cu_seq_lens, global_window_size=64,
             raise ValueError("an empty block list needs include_last_block")
         # a non-NULL list address selects the block form even when only the implicit block is read
         idx = torch.zeros((B, Hkv, 1), device=q.device, dtype=torch.int32)
-        return _decode(q, k, v, None, lens, scale, None, None, return_lse, block_idx=idx, block_cnt=None,
+        return _decode(q, k, v, cu, lens, scale, None, None, return_lse, block_idx=idx, block_cnt=None,
                        bi_strides=(Hkv, 1), max_blocks=0, split_blocks=split_blocks or 0, include_last=True, **layout)
     # the block of the newest token is appended (and de-duplicated) by the kernel
-    return _decode(q, k, v, None, lens, scale, None, None, return_lse, block_idx=idx, block_cnt=cnt,
+    return _decode(q, k, v, cu, lens, scale, None, None, return_lse, block_idx=idx, block_cnt=cnt,
                    bi_strides=(Hkv * n, n), max_blocks=n, split_blocks=split_blocks or 0,
                    include_last=bool(include_last_block), **layout)

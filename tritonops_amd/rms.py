@@ -7,7 +7,7 @@ from torch import nn
 from torch.autograd import Function
 
 from . import _lib
-from .ops import _ptr, _require_gpu, _stream
+from .ops import _here, _outputs, _ptr, _require_gpu, _stream
 
 _TAGS = {torch.bfloat16: _lib.MI_DTYPE_BF16, torch.float16: _lib.MI_DTYPE_F16, torch.float32: _lib.MI_DTYPE_F32}
 
@@ -40,6 +40,15 @@ def rmsnorm_fwd(x, weight, eps):
     """y = x / sqrt(mean(x^2) + eps) * weight over the last dimension; returns
     (y, rsqrt) with rsqrt fp32 [rows] — forward of RMSNormTritonFunction
     (common/rms.py:223-287)."""
+    if x.is_cuda:
+        out = _outputs(_lib.native().rms_fwd(x, weight, eps, *_here()))
+        if out is not None:
+            return out
+    return _general_fwd(x, weight, eps)
+
+
+def _general_fwd(x, weight, eps):
+    """rmsnorm_fwd for every form of its arguments."""
     _require_gpu(x, weight)
     lib = _lib.load()
     if x.shape[-1] != weight.shape[0]:
@@ -59,6 +68,15 @@ def rmsnorm_fwd(x, weight, eps):
 def rmsnorm_bwd(dy, x, weight, rsqrt, eps):
     """(dx, dweight) — backward of RMSNormTritonFunction (common/rms.py:289-355);
     dweight is reduced deterministically (the reference uses atomics, :215)."""
+    if x.is_cuda:
+        out = _outputs(_lib.native().rms_bwd(dy, x, weight, rsqrt, eps, *_here()))
+        if out is not None:
+            return out
+    return _general_bwd(dy, x, weight, rsqrt, eps)
+
+
+def _general_bwd(dy, x, weight, rsqrt, eps):
+    """rmsnorm_bwd for every form of its arguments."""
     _require_gpu(dy, x, weight, rsqrt)
     lib = _lib.load()
     wk = weight if (weight.dtype == x.dtype or weight.dtype == torch.float32) else weight.to(x.dtype)
