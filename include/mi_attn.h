@@ -332,6 +332,10 @@ size_t mi_decode_workspace_bytes(const mi_decode_args *args);
  * units for the given problem; host only. */
 int mi_decode_choose_split_tokens(int batch, int heads_kv, int max_seqlen,
                                   int num_cus);
+/* The same for callers whose workspace grows with the call: shorter chunks, so
+ * that a call takes 12 % less time in the mean, for up to four times the partial
+ * results (mi_decode_noalloc holds a fixed amount of them: take the former). */
+int mi_decode_choose_split(int batch, int heads_kv, int max_seqlen, int num_cus);
 /* Heuristic chunk length in listed blocks for the block-list form: the largest
  * number of chunks per (sequence, kv-head) whose wavefronts are all resident
  * at once on `num_cus` compute units (a second, partly filled round of

@@ -653,6 +653,29 @@ int mi_decode_choose_split_tokens(int batch, int heads_kv, int max_seqlen, int n
   return (int)tokens;
 }
 
+int mi_decode_choose_split(int batch, int heads_kv, int max_seqlen, int num_cus) {
+  // As above, for a caller whose workspace grows with the call.  The kernel puts
+  // two or four wavefronts to a chunk where there are few, so chunks may be as
+  // short as 64 tokens: the smallest power of two that leaves no more than ten
+  // chunks to a CU if every sequence were as long as the bound, and no more of
+  // them than the merge adds up in the time that shorter chunks save (32 of 64
+  // tokens, 128 of 128, 256 of 256).  Whole call in us, chunk of the function
+  // above -> this one, lengths half the bound to the bound unless given: 1 x 1024,
+  // 8 kv-heads 256 -> 64: 13.2 -> 9.4; 8 x 2048 256 -> 64: 20.2 -> 16.6; 64 x 128
+  // to 512 of 1024 512 -> 256: 33.4 -> 28.8; 1 x 8192 256 -> 128: 14.4 -> 11.5;
+  // 32 x 8192, 2 kv-heads 512 -> 256: 48.8 -> 45.4; 4 x 32768, 16 kv-heads of 64
+  // 2048 -> 1024: 92 -> 79; 64 x 2048 to 8192 of 16384, 2 kv-heads 2048 -> 1024:
+  // 90 -> 71.  Over 175 calls of 1 to 64 sequences, bounds 64 to 131072, 2 to 16
+  // kv-heads, 12 % less in the mean.  (Beyond 2048 tokens nothing is gained, and
+  // chunks of no power of two are slower than either neighbour.)
+  if (batch <= 0 || heads_kv <= 0 || max_seqlen <= 0) return 64;
+  if (num_cus <= 0) num_cus = 256;
+  const long long work = (long long)batch * heads_kv * max_seqlen;  // tokens x kv-heads
+  long long tokens = max_seqlen <= 2048 ? 64 : max_seqlen <= 16384 ? 128 : max_seqlen <= 65536 ? 256 : 512;
+  while (tokens < 2048 && tokens * 10 * num_cus < work) tokens *= 2;
+  return (int)tokens;
+}
+
 int mi_decode_choose_split_blocks(int batch, int heads_kv, int total_blocks, int num_cus) {
   // One wavefront per (chunk, kv-head, sequence), 8 wavefronts resident per
   // compute unit: use as many chunks as fit in one resident round.

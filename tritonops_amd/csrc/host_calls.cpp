@@ -481,7 +481,7 @@ PyObject* decode(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   const int slices = (int)((hq / hkv + 31) / 32);  // 32 query heads each
   if (!listed) {
     a.split_tokens = split ? (int32_t)split
-                           : mi_decode_choose_split_tokens(a.batch, a.heads_kv * slices, a.max_seqlen, mi_device_cu_count());
+                           : mi_decode_choose_split(a.batch, a.heads_kv * slices, a.max_seqlen, mi_device_cu_count());
   } else {
     a.split_tokens = 64;
     a.window_form = window_form;

@@ -698,7 +698,7 @@ def _general_decode(q, k, v, cu_seq_lens, seq_lens, scale, max_seq_len, split_to
     a.scale_log2 = float(scale) * LOG2E
     gslices = (Hq // Hkv + 31) // 32   # wavefronts per (chunk, kv-head): 32 query heads each
     if block_idx is None and not window_form:
-        a.split_tokens = int(split_tokens) if split_tokens else lib.mi_decode_choose_split_tokens(
+        a.split_tokens = int(split_tokens) if split_tokens else lib.mi_decode_choose_split(
             B, Hkv * gslices, a.max_seqlen, _num_cus(lib))
     else:
         a.split_tokens = 64
