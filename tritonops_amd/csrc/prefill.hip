@@ -1182,12 +1182,11 @@ dense_kernel(const PrefillParams p) {
 // dense_kernel keeps one 8-wave workgroup per CU, two wavefronts per SIMD, and
 // a work item is one chain of latencies (geometry, Q and first tiles, the exact
 // first half, the tile loop, normalise, stage, store).  Two uses:
-//  - launches with at most one 128-row item per CU (short prompts, few heads):
-//    twice as many CUs work, each on a chain half as long.  10 to 17 % faster
-//    than dense_kernel at head_dim 128 on every such launch measured (1 to 4
-//    sequences of 256 to 4096 tokens, 8 and 32 heads, causal and not); with
-//    more items than CUs the two forms are within 5 % of each other at head_dim
-//    96 and 128 (two waves per SIMD either way) and dense_kernel stays ahead.
+//  - head_dim 128 and launches of few rounds (up to three items per CU): items
+//    half as long spread more evenly, 1 to 14 % faster (launch_one); with more
+//    items the two forms are within 5 % of each other at head_dim 96 and 128 (two
+//    waves per SIMD either way) and dense_kernel stays ahead.  (At most one item
+//    per CU: dense_pair_kernel.)
 //  - head_dim 64: the softmax arithmetic outweighs the matrix work there (56
 //    vector instructions against 8 MFMAs per 32 x 32 block of scores) and a
 //    wave's registers (O, S, Q^T, P: 163 in all) leave room for a third
@@ -1591,6 +1590,328 @@ dense_short_kernel(const PrefillParams p) {
   }
 }
 
+constexpr int kPairStages = 8;
+template <int D>
+constexpr int kPairLdsBytes = 2 * kPairStages * kShortTileKeys * SwizzledFrags<D>::ROWB + 2 * 4 * (2048 + 256) + 4 * 256;
+
+// Dense forward, paired form: work items of 128 query rows on workgroups of eight
+// wavefronts, one item to a workgroup, for launches with at most one item per CU.
+//
+// Such a launch is as long as its longest item's chain of key tiles (a prompt of
+// 1000 tokens: 32 tiles of 32 keys), and a lone wavefront per SIMD spends about
+// 1300 clocks on a tile, 512 of them in MFMAs: scores, softmax and output follow
+// one another in one instruction stream.  Here two wavefronts share 32 rows.  The
+// SCORE wavefront holds Q^T, forms S(h+1) = K(h+1) Q^T with the softmax of S(h)
+// between its MFMAs, and leaves the packed probabilities, 2 KB, in LDS; the OUTPUT
+// wavefront reads them one position later (two buffers, published by the barrier
+// that every position has) and forms O += V(h)^T P(h)^T.  They sit on one SIMD,
+// and each has half the MFMAs of a tile.  When the score wavefront moves a row's
+// reference point it leaves the factor for O beside the probabilities.  What is
+// computed, and in which order, is what the other forms compute, bit for bit.
+// 4000 tokens, 8 heads: 62.6 us (short form 68.2, long 79.0), at head_dim 96 56.4
+// (82.3, 80.8); 2000 tokens, 16 heads of 64: 27.4 (31.8, 33.4); one prompt of 1000
+// tokens, 32 heads: 22.7 (24.2, 26.6).  A position takes 0.46 us at head_dim 128: a
+// lone wavefront issues one instruction in about six clocks, and the score
+// wavefront has about 130 of them, which is why it loads nothing itself (0.52 us
+// when it did) and why neither fewer MFMAs nor no exponentials shorten it much.
+//
+// The output wavefronts, which have fewer instructions to issue, load the tiles
+// into a ring of eight stages: tile p + 6 is requested at the top of position p into
+// the stage of tile p - 2, whose V was read in position p - 1; at the top of
+// position h tiles up to h + 2 have landed and up to three may still fly.
+template <typename T, int D>
+__global__ void __launch_bounds__(kShortRows * 4) dense_pair_kernel(const PrefillParams p) {
+  constexpr int NW = kShortRows / 32, NS = kPairStages, TN = kShortTileKeys;
+  static_assert(NW == 4 && NS == 8 && TN == 32, "the positions are unrolled over the stages");
+  using G = RowGeom<D>;
+  using F = SwizzledFrags<D>;
+  using DMA = TileDma<T, D, NW, NS, TN>;
+  constexpr int BM = 32 * NW;
+  constexpr int TILEB = DMA::TILEB, VBASE = DMA::VBASE, IPW = DMA::IPW;
+  constexpr int EXB = 2048 + 256;                // probabilities and factors of 32 rows x 32 keys
+  constexpr int EXBASE = 2 * NS * TILEB, INVBASE = EXBASE + 2 * NW * EXB;
+  static_assert(INVBASE + NW * 256 == kPairLdsBytes<D>, "LDS of a workgroup");
+
+  // Items level by level, the last (longest) tile of every sequence first: where there are more of them than CUs the
+  // short ones follow the long ones.  The kv-head runs fastest: ids eight apart, which share an XCD, then share K / V.
+  ItemGeo g;
+  {
+    const int per_level = p.hq * p.batch, gqa = p.hq / p.hkv;
+    int r = blockIdx.x % per_level;
+    g.qt = p.n_qtiles - 1 - blockIdx.x / per_level;
+    g.kvh = r % p.hkv;
+    r /= p.hkv;
+    g.h = g.kvh * gqa + r % gqa;
+    g.b = r / gqa;
+    finish_geo(p, g);
+    if (g.qt * BM >= g.len) return;
+  }
+  const int lane = threadIdx.x & 63;
+  const int wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wave8 & 3;                    // 32-row block of the item
+  const bool scores = wave8 < 4;
+  F fr;
+  fr.init(lane, (uint32_t)(uintptr_t)smem, VBASE);
+  const int len = g.len, causal = p.causal, q0 = g.qt * BM;
+  const float scale = p.scale;
+  int n_tiles = (len + TN - 1) / TN;
+  if (causal) n_tiles = min(n_tiles, (q0 + BM) / TN);
+  const int q0w = q0 + 32 * wave, qrow = q0w + fr.lq;
+  const int row_lim = causal ? min(qrow, len - 1) : len - 1;
+  int H_w = causal ? min(n_tiles, q0w / 32 + 1) : n_tiles;  // tiles this wavefront's rows see
+  if (q0w >= len) H_w = 0;
+  unsigned char* const ex = smem + EXBASE + wave * EXB;
+  float* const inv_at = reinterpret_cast<float*>(smem + INVBASE + wave * 256) + lane;
+
+  // ---- tile loads (output wavefronts): IPW of K and IPW of V per wavefront and
+  // tile, each 1 KiB of LDS, "scalar base + 32-bit lane offset" (TileDma's
+  // layout); the last tile's rows past the end re-read the last row.
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem) + wave * 1024;
+  const uint32_t k_pitch = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(p.k_ss * 2));
+  const uint32_t v_pitch = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(p.v_ss * 2));
+  // tile `next` of K and of V
+  uint64_t k_next = DMA::uniform64((uint64_t)(uintptr_t)(reinterpret_cast<const T*>(p.k) + g.k_off + g.kvh * p.k_sh));
+  uint64_t v_next = DMA::uniform64((uint64_t)(uintptr_t)(reinterpret_cast<const T*>(p.v) + g.v_off + g.kvh * p.v_sh));
+  const int last_tile = (len - 1) / TN;
+  uint32_t k_off[IPW], v_off[IPW], k_last[IPW], v_last[IPW];
+  uint64_t k_live[IPW], v_live[IPW];
+#pragma unroll
+  for (int t = 0; t < IPW; ++t) {
+    const int r = DMA::RPI * (wave + NW * t) + lane / F::SLOTS, rl = min(r, len - 1 - last_tile * TN);
+    const int kc = (lane % F::SLOTS) ^ F::swz_k(r), vc = (lane % F::SLOTS) ^ F::swz_v(r);
+    k_off[t] = (uint32_t)r * k_pitch + kc * 16;
+    k_last[t] = (uint32_t)rl * k_pitch + kc * 16;
+    v_off[t] = (uint32_t)r * v_pitch + vc * 16;
+    v_last[t] = (uint32_t)rl * v_pitch + vc * 16;
+    k_live[t] = DMA::uniform64(__builtin_amdgcn_ballot_w64(kc < G::NCH));
+    v_live[t] = DMA::uniform64(__builtin_amdgcn_ballot_w64(vc < G::NCH));
+  }
+  // the next tile, j, into its stage
+  auto send = [&](int j) __attribute__((always_inline)) {
+    const bool on = j < n_tiles, last = j == last_tile;
+    const uint32_t at = lds0 + (uint32_t)(j & (NS - 1)) * TILEB;
+#pragma unroll
+    for (int t = 0; t < IPW; ++t) {
+      DMA::dma16m(on ? k_live[t] : 0ull, k_next, last ? k_last[t] : k_off[t], at + t * NW * 1024);
+      DMA::dma16m(on ? v_live[t] : 0ull, v_next, last ? v_last[t] : v_off[t], at + VBASE + t * NW * 1024);
+    }
+    k_next += (uint64_t)TN * k_pitch;
+    v_next += (uint64_t)TN * v_pitch;
+  };
+  // top of position h, output wavefronts
+  auto top = [&](int h) __attribute__((always_inline)) {
+    if (h + 5 < n_tiles)
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm(3 * 2 * IPW));
+    else
+      __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    __syncthreads();
+  };
+  // from the address of a fragment of tile j to that of the same fragment of tile j + 1
+  auto step_of = [&](int j) __attribute__((always_inline)) -> uint32_t {
+    return (j & (NS - 1)) == NS - 1 ? (uint32_t)(-(NS - 1) * TILEB) : (uint32_t)TILEB;
+  };
+  if (scores) {
+    i32x4 Qf[G::KSTEPS];
+    {
+      const T* qr = reinterpret_cast<const T*>(p.q) + g.q_off + g.h * p.q_sh + (int64_t)min(qrow, len - 1) * p.q_ss + 8 * fr.lh;
+#pragma unroll
+      for (int c = 0; c < G::KSTEPS; ++c) Qf[c] = *reinterpret_cast<const i32x4*>(qr + 16 * c);
+    }
+    float m = -INFINITY, m_neg = 0.f, l = 0.f;
+    f32x16 S[2];
+    constexpr int KR = G::KSTEPS < 4 ? G::KSTEPS : 4;
+    i32x4 kf[KR];
+    const int first_masked = causal ? min(q0w, len) / TN : len / TN;  // the first tile that crosses the diagonal or the end
+    auto mask_tile = [&](int h, f32x16& Sx) __attribute__((always_inline)) {
+      if (h >= first_masked) {
+        const int t = row_lim - h * TN - 8 * fr.lh;
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (16 * (r >> 3) + (r & 7) > t) Sx[r] = -INFINITY;
+      }
+    };
+    constexpr float kRowSumLimit = 4096.f;   // as in dense_kernel
+    // the reference point moved to the true maximum: the factor for what was summed before
+    auto exact_fix = [&](const f32x16& Sx, uint32_t (&P)[8], float& rs) __attribute__((always_inline)) -> float {
+      float mx = Sx[0];
+#pragma unroll
+      for (int r = 1; r < 16; ++r) mx = fmaxf(mx, Sx[r]);
+      mx = max_with_other_half(mx);
+      const float m_new = fmaxf(m, mx * scale);
+      const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+      const float alpha = fast_exp2(m - m_safe);
+      l *= alpha;
+      m = m_new;
+      m_neg = -m_safe;
+      rs = 0.f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float p0 = fast_exp2(fmaf(Sx[2 * i], scale, -m_safe));
+        const float p1 = fast_exp2(fmaf(Sx[2 * i + 1], scale, -m_safe));
+        rs += p0 + p1;
+        P[i] = Elem<T>::pack2(p0, p1);
+      }
+      return alpha;
+    };
+    typedef __attribute__((address_space(3))) const i32x4 lds_i32x4;
+    // addresses of the K fragments to be read next: those of step c < KR are a tile ahead of the others
+    uint32_t ka[G::KSTEPS];
+#pragma unroll
+    for (int c = 0; c < G::KSTEPS; ++c) ka[c] = fr.k_a[c] + (c < KR ? 2 : 1) * TILEB;
+    auto body = [&](auto parity, int h) __attribute__((always_inline)) {
+      constexpr int J = decltype(parity)::value;
+      f32x16& Sc = S[J];
+      f32x16& Sn = S[J ^ 1];
+      uint32_t P[8];
+      const uint32_t step1 = step_of(h + 1), step2 = step_of(h + 2);
+      float rs = 0.f, u0 = fmaf(Sc[0], scale, m_neg), u1 = fmaf(Sc[1], scale, m_neg), p0, p1;
+      unsigned char* e = ex + J * NW * EXB;
+      auto leave = [&](int half) __attribute__((always_inline)) {
+        *reinterpret_cast<i32x4*>(e + 1024 * half + lane * 16) =
+            (i32x4){(int)P[4 * half], (int)P[4 * half + 1], (int)P[4 * half + 2], (int)P[4 * half + 3]};
+      };
+      // (for the last tile of a wavefront Sn holds scores of stale LDS contents that are never used)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        if (c < G::KSTEPS) {
+          const f32x16 acc = (c == 0) ? (f32x16){0} : Sn;
+          Sn = Elem<T>::mfma(kf[c % KR], Qf[c], acc);
+          const int f = c + KR < G::KSTEPS ? c + KR : c % KR;   // the fragment that takes this one's place
+          kf[c % KR] = *(lds_i32x4*)(uintptr_t)ka[f];
+          ka[f] += f < KR ? step2 : step1;
+        }
+        if (c > 0) {   // sum and pack of the pair before
+          rs = c == 1 ? p0 + p1 : rs + (p0 + p1);
+          P[c - 1] = Elem<T>::pack2(p0, p1);
+        }
+        p0 = fast_exp2(u0);
+        p1 = fast_exp2(u1);
+        if (c < 7) {
+          u0 = fmaf(Sc[2 * c + 2], scale, m_neg);
+          u1 = fmaf(Sc[2 * c + 3], scale, m_neg);
+        }
+        if (c == 5) leave(0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      rs += p0 + p1;
+      P[7] = Elem<T>::pack2(p0, p1);
+      float alpha = 1.f;
+      if (__builtin_amdgcn_ballot_w64(!(rs <= kRowSumLimit)) != 0) {
+        alpha = exact_fix(Sc, P, rs);
+        leave(0);
+      }
+      leave(1);
+      l += rs;
+      *reinterpret_cast<float*>(e + 2048 + lane * 4) = alpha;
+      mask_tile(h + 1, Sn);
+    };
+    __syncthreads();
+    if (H_w > 0) {  // the first tile's scores and exact maximum
+      f32x16 acc = (f32x16){0};
+#pragma unroll
+      for (int c = 0; c < G::KSTEPS; ++c) acc = Elem<T>::mfma(fr.load_k(0u, 0, c), Qf[c], acc);
+      S[0] = acc;
+      mask_tile(0, S[0]);
+      uint32_t P[8];
+      float rs;
+      exact_fix(S[0], P, rs);
+#pragma unroll
+      for (int c = 0; c < KR; ++c) kf[c] = fr.load_k(1u * TILEB, 0, c);
+      for (int h = 0;;) {
+        body(ic<0>{}, h);
+        if (++h >= H_w) break;
+        __syncthreads();
+        body(ic<1>{}, h);
+        if (++h >= H_w) break;
+        __syncthreads();
+      }
+    }
+    for (int h = max(H_w, 1); h < n_tiles; ++h) __syncthreads();
+    const float l_tot = sum_with_other_half(l);
+    *inv_at = l_tot > 0.f ? 1.f / l_tot : 0.f;
+    if (p.lse && fr.lh == 0 && qrow < len)
+      p.lse[g.lse_off + g.h * p.lse_sh + (int64_t)qrow * p.lse_ss] = l_tot > 0.f ? m + fast_log2(l_tot) : -INFINITY;
+    __syncthreads();
+    return;
+  }
+
+#pragma unroll
+  for (int j = 0; j < 6; ++j) send(j);
+  f32x16 O[G::NDB];
+#pragma unroll
+  for (int db = 0; db < G::NDB; ++db) O[db] = (f32x16){0};
+  i32x4 vf[2][G::NDB];
+  uint32_t va[G::NDB][2];  // where the next tile's fragments are
+#pragma unroll
+  for (int db = 0; db < G::NDB; ++db) va[db][0] = fr.v_a[db][0], va[db][1] = fr.v_a[db][1];
+  // Position h: the output of tile h - 1, and on the way the fragments of V(h) (landed: tiles up to h + 2 have) and the
+  // loads of tile h + 6.  (Position n_tiles, which the score wavefronts end with a barrier of their own, reads stale
+  // ones.  Positions without output are loops of their own: where paths with and without MFMAs join, the accumulators
+  // are copied at every position.)
+  auto read_v = [&](int kk, int db) __attribute__((always_inline)) {
+    vf[kk][db] = read_tr_at(va[db][0] + kk * 16 * F::ROWB, va[db][1] + kk * 16 * F::ROWB);
+  };
+  top(0);
+  send(6);
+#pragma unroll
+  for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+    for (int db = 0; db < G::NDB; ++db) read_v(kk, db);
+#pragma unroll
+  for (int db = 0; db < G::NDB; ++db) va[db][0] += TILEB, va[db][1] += TILEB;
+  for (int h = 1; h <= H_w; ++h) {
+    top(h);
+    const unsigned char* e = ex + ((h & 1) ^ 1) * NW * EXB;
+    i32x4 pf[2];
+    pf[0] = *reinterpret_cast<const i32x4*>(e + lane * 16);
+    const float alpha = *reinterpret_cast<const float*>(e + 2048 + lane * 4);
+    pf[1] = *reinterpret_cast<const i32x4*>(e + 1024 + lane * 16);
+    send(h + 6);
+    const uint32_t step = step_of(h);
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+      for (int db = 0; db < G::NDB; ++db) O[db] *= alpha;
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int db = 0; db < G::NDB; ++db) {
+        O[db] = Elem<T>::mfma(vf[kk][db], pf[kk], O[db]);
+        read_v(kk, db);
+        if (kk == 1) va[db][0] += step, va[db][1] += step;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  }
+  for (int h = H_w + 1; h <= n_tiles; ++h) {
+    top(h);
+    send(h + 6);
+  }
+  // normalise, transpose through the wavefront's own K stage (no score wavefront reads K any more), coalesced stores
+  const float inv = *inv_at;
+  unsigned char* stage = smem + wave * TILEB;
+  constexpr int SLOTS = F::SLOTS;
+#pragma unroll
+  for (int db = 0; db < G::NDB; ++db)
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+      const int c = 4 * db + gq;
+      i32x2 w;
+      w[0] = (int)Elem<T>::pack2(O[db][4 * gq] * inv, O[db][4 * gq + 1] * inv);
+      w[1] = (int)Elem<T>::pack2(O[db][4 * gq + 2] * inv, O[db][4 * gq + 3] * inv);
+      *reinterpret_cast<i32x2*>(stage + fr.lq * F::ROWB + ((c ^ (fr.lq & (SLOTS - 1))) << 4) + 8 * fr.lh) = w;
+    }
+  asm volatile("" ::: "memory");
+  T* op = reinterpret_cast<T*>(p.o) + g.o_off + g.h * p.o_sh;
+#pragma unroll
+  for (int i = 0; i < 32 * SLOTS / 64; ++i) {
+    const int idx = lane + 64 * i;
+    const int row = idx / SLOTS, ch = idx % SLOTS;
+    if (ch < G::NCH && q0w + row < len)
+      *reinterpret_cast<i32x4*>(op + (int64_t)(q0w + row) * p.o_ss + ch * 8) =
+          *reinterpret_cast<const i32x4*>(stage + row * F::ROWB + ((ch ^ (row & (SLOTS - 1))) << 4));
+  }
+}
+
 template <int D, int NW, int NS, int TN>
 constexpr size_t prefill_lds_bytes() {
   const size_t pipe = (size_t)NS * 2 * TN * SwizzledFrags<D>::ROWB;
@@ -1638,7 +1959,6 @@ inline double short_form_cost(long long n, int cus) {
 }
 inline bool short_form_pays(long long n128, long long n256, int cus) {
   if (cus <= 0) return false;
-  if (n128 <= cus) return true;   // a CU per workgroup: twice as many CUs busy as with 256-row items
   return short_form_cost(n128, cus) < 2.3 * (double)((n256 + cus - 1) / cus);
 }
 
@@ -1659,6 +1979,18 @@ int launch_short(const PrefillParams& p, long long items, int cus, hipStream_t s
   return (int)hipGetLastError();
 }
 
+// One 128-row item to a workgroup: p.n_qtiles counts tiles of that height.
+template <typename T, int D>
+int launch_pair(const PrefillParams& p, long long items, hipStream_t s) {
+  auto kern = dense_pair_kernel<T, D>;
+  static LdsLimitOnce lds_once;
+  if (const int e = raise_lds_limit(lds_once, reinterpret_cast<const void*>(kern), kPairLdsBytes<D>)) return e;
+  PrefillParams pp = p;
+  pp.n_qtiles = (p.max_seqlen + kShortRows - 1) / kShortRows;
+  hipLaunchKernelGGL(kern, dim3((unsigned)items), dim3(kShortRows * 4), kPairLdsBytes<D>, s, pp);
+  return (int)hipGetLastError();
+}
+
 template <typename T, int D, bool SPARSE>
 int launch_one(const PrefillParams& p, hipStream_t s) {
   if constexpr (!SPARSE) {
@@ -1666,10 +1998,16 @@ int launch_one(const PrefillParams& p, hipStream_t s) {
     const long long n = (long long)((p.max_seqlen + kShortRows - 1) / kShortRows) * p.hq * p.batch;
     bool short_form = p.dense_form == 2;
     if (p.dense_form == 0) {
+      // A CU per 128-row item; one sequence up to half as many more, whose short items follow the long ones: 1500 tokens,
+      // 32 heads 29.9 us (short form 32.8, long 35.3), 1516 without a mask 31.3 (35.0, 37.5).  Two rounds of it lose
+      // where the items are alike: 6 x 471 tokens, 16 heads of 64, no mask 18.1 (13.8, 13.0).
+      if (cus > 0 && (n <= cus || (p.batch == 1 && 2 * n <= 3 * cus))) return launch_pair<T, D>(p, n, s);
       if (D == 64)
         short_form = short_form_pays(n, (long long)p.n_qtiles * p.hq * p.batch, cus);
-      else
-        short_form = cus > 0 && n <= cus;   // a CU per 128-row item
+      else if (D == 128)
+        // few rounds: 12 x 300 tokens, 16 heads 20.8 us against 24.1, 700 + 300 + 900, 32 heads 24.5 against 26.6, 6 x 736
+        // without a mask 43.0 against 45.9, 4 x 858 40.7 against 42.2; level from three rounds on, behind in many
+        short_form = n <= 3LL * cus;
     }
     if (short_form) return launch_short<T, D>(p, n, cus, s);
   }

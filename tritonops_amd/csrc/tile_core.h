@@ -114,6 +114,16 @@ __device__ __forceinline__ i32x4 read_tr_pair(const unsigned char* a0, const uns
   return out;
 }
 
+// the same from LDS addresses
+__device__ __forceinline__ i32x4 read_tr_at(uint32_t a0, uint32_t a1) {
+  s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)a0);
+  s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(uintptr_t)a1);
+  i32x2 l2 = __builtin_bit_cast(i32x2, lo);
+  i32x2 h2 = __builtin_bit_cast(i32x2, hi);
+  i32x4 out = {l2[0], l2[1], h2[0], h2[1]};
+  return out;
+}
+
 // 8 x 8 elements of 16 bits, in[row] -> out[column], within a lane's registers: one byte permute per output dword.
 __device__ __forceinline__ void transpose8x8(const i32x4 (&in)[8], i32x4 (&out)[8]) {
 #pragma unroll
