@@ -482,6 +482,29 @@ int mi_xent_kept_dlogits(const mi_xent_bwd_args *args, const void *kept, void *s
  * its columns from `tokens` up to that multiple of 64 are zeroed. */
 int mi_xent_kept_dlogits_both(const mi_xent_bwd_args *args, const void *kept, void *dlogits_t, int64_t ld_t, void *stream);
 
+/* grad_x [tokens, dim] = dlogits [tokens, vocab] w [vocab, dim], fp32 sums, for
+ * results too small to fill the chip with their tiles: the vocabulary is divided
+ * into n_split ranges (mi_xent_grad_x_splits picks their number), whose fp32
+ * partial tiles go to the workspace and are added up in order.  All bases 16-byte
+ * aligned, all strides multiples of 8 elements, ld and w_stride up to 2^22;
+ * elements of dlogits rows from vocab up to its next multiple of 8 are read and
+ * not used. */
+typedef struct mi_xent_grad_x_args {
+  uint32_t struct_size;
+  int32_t dtype;                 /* of dlogits, w and grad_x                   */
+  int32_t tokens, dim, vocab;    /* dim a multiple of 8, vocab at least 64     */
+  int32_t n_split;
+  const void *dlogits, *w;
+  void *grad_x;
+  int64_t ld, w_stride, grad_x_stride;
+  void *workspace;
+  size_t workspace_bytes;
+} mi_xent_grad_x_args;
+
+int mi_xent_grad_x_splits(int64_t tokens, int64_t dim, int64_t vocab, int num_cus);
+size_t mi_xent_grad_x_workspace_bytes(int64_t tokens, int64_t dim, int n_split);
+int mi_xent_grad_x(const mi_xent_grad_x_args *args, void *stream);
+
 /* dst[c][r] = src[r][c] for 16-bit elements: src [rows, cols] with row stride
  * ld_src, dst [cols, ld_dst]; cols, ld_src and ld_dst multiples of 8, both bases
  * 16-byte aligned, ld_dst at least rows rounded up to 64; the columns of dst from

@@ -129,6 +129,16 @@ class XentGradArgs(C.Structure):
     ]
 
 
+class XentGradXArgs(C.Structure):
+    _fields_ = [
+        ("struct_size", _u32), ("dtype", _i32),
+        ("tokens", _i32), ("dim", _i32), ("vocab", _i32), ("n_split", _i32),
+        ("dlogits", _vp), ("w", _vp), ("grad_x", _vp),
+        ("ld", _i64), ("w_stride", _i64), ("grad_x_stride", _i64),
+        ("workspace", _vp), ("workspace_bytes", _sz),
+    ]
+
+
 class DecodeArgs(C.Structure):
     _fields_ = [
         ("struct_size", _u32), ("dtype", _i32),
@@ -170,6 +180,9 @@ EXPORTS = {
     "mi_xent_fwd_keep": (C.c_int, [C.POINTER(XentArgs), _vp, _vp]),
     "mi_xent_kept_dlogits": (C.c_int, [C.POINTER(XentBwdArgs), _vp, _vp]),
     "mi_xent_kept_dlogits_both": (C.c_int, [C.POINTER(XentBwdArgs), _vp, _vp, _i64, _vp]),
+    "mi_xent_grad_x_splits": (C.c_int, [_i64, _i64, _i64, C.c_int]),
+    "mi_xent_grad_x_workspace_bytes": (_sz, [_i64, _i64, C.c_int]),
+    "mi_xent_grad_x": (C.c_int, [C.POINTER(XentGradXArgs), _vp]),
     "mi_transpose16": (C.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "mi_xent_dlogits": (C.c_int, [C.POINTER(XentGradArgs), _vp]),
     "mi_xent_bwd_dlogits": (C.c_int, [C.POINTER(XentBwdArgs), _vp]),

@@ -15,7 +15,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(HERE, "libmi_attn.so")
-SOURCES = ["api.cpp", "bench_timing.cpp", "prefill.hip", "decode.hip", "bwd.hip", "rmsnorm.hip", "xent.hip", "transpose.hip"]
+SOURCES = ["api.cpp", "bench_timing.cpp", "prefill.hip", "decode.hip", "bwd.hip", "rmsnorm.hip", "xent.hip", "xent_grad.hip", "transpose.hip"]
 NATIVE_SRC = os.path.join(CSRC, "host_calls.cpp")
 NATIVE_PATH = os.path.join(HERE, "_native.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

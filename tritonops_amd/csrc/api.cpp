@@ -364,6 +364,45 @@ int mi_xent_kept_dlogits_both(const mi_xent_bwd_args* a, const void* kept, void*
   return kept_dlogits(a, kept, true, dlogits_t, ld_t, stream, "mi_xent_kept_dlogits_both");
 }
 
+int mi_xent_grad_x_splits(int64_t tokens, int64_t dim, int64_t vocab, int num_cus) {
+  return mi::xent_gradx_splits(tokens, dim, vocab, num_cus);
+}
+
+size_t mi_xent_grad_x_workspace_bytes(int64_t tokens, int64_t dim, int n_split) {
+  return tokens <= 0 || dim <= 0 || n_split <= 0 ? 0 : mi::xent_gradx_bytes(tokens, dim, n_split);
+}
+
+int mi_xent_grad_x(const mi_xent_grad_x_args* a, void* stream) {
+  if (!a) return fail(MI_ERR_NULL_POINTER, "args is NULL");
+  if (a->struct_size != sizeof(mi_xent_grad_x_args))
+    return fail(MI_ERR_STRUCT_SIZE, "mi_xent_grad_x_args.struct_size %u != %zu", a->struct_size, sizeof(mi_xent_grad_x_args));
+  if (a->dtype != MI_DTYPE_BF16 && a->dtype != MI_DTYPE_F16) return fail(MI_ERR_DTYPE, "dtype %d is not bf16 / f16", a->dtype);
+  if (a->tokens < 0 || a->dim <= 0 || a->dim % 8 || a->vocab < 64)
+    return fail(MI_ERR_SHAPE, "tokens %d must be >= 0, dim %d a positive multiple of 8, vocab %d at least 64", a->tokens, a->dim, a->vocab);
+  if (a->tokens == 0) return MI_OK;
+  if (!a->dlogits || !a->w || !a->grad_x || !a->workspace)
+    return fail(MI_ERR_NULL_POINTER, "dlogits, w, grad_x and workspace must be non-NULL");
+  if (!aligned16(a->dlogits) || !aligned16(a->w) || !aligned16(a->grad_x) || !aligned16(a->workspace))
+    return fail(MI_ERR_ALIGNMENT, "dlogits, w, grad_x and workspace must be 16-byte aligned");
+  if (!mult8(a->ld) || !mult8(a->w_stride) || !mult8(a->grad_x_stride) || a->ld < a->vocab || a->w_stride < a->dim ||
+      a->grad_x_stride < a->dim)
+    return fail(MI_ERR_STRIDE, "row strides must be multiples of 8 elements and hold a row");
+  // per-lane row offsets inside a slab are 32-bit
+  if (a->ld > (1 << 22) || a->w_stride > (1 << 22)) return fail(MI_ERR_STRIDE, "row stride beyond 2^22 elements");
+  const long long tiles = (((long long)a->tokens + 255) / 256) * (((long long)a->dim + 255) / 256);
+  const int pairs = ((a->vocab + 63) / 64 + 1) / 2;
+  if (a->n_split < 1 || a->n_split > pairs || tiles * a->n_split > 65536)
+    return fail(MI_ERR_SHAPE, "n_split %d: 1 to %d, and no more than 65536 partial tiles", a->n_split, pairs);
+  if (a->workspace_bytes < mi::xent_gradx_bytes(a->tokens, a->dim, a->n_split))
+    return fail(MI_ERR_WORKSPACE, "workspace of %zu bytes needed", mi::xent_gradx_bytes(a->tokens, a->dim, a->n_split));
+  mi::XentGradXParams p;
+  p.dlogits = a->dlogits; p.w = a->w; p.gx = a->grad_x; p.part = static_cast<float*>(a->workspace);
+  p.dl_ld = a->ld; p.w_st = a->w_stride; p.gx_ld = a->grad_x_stride;
+  p.T = a->tokens; p.D = a->dim; p.N = a->vocab;
+  p.tiles_t = (a->tokens + 255) / 256; p.tiles_d = (a->dim + 255) / 256; p.n_split = a->n_split;
+  return launch_status(mi::launch_xent_gradx(p, a->dtype, static_cast<hipStream_t>(stream)), "mi_xent_grad_x");
+}
+
 int mi_transpose16(const void* src, int64_t rows, int64_t cols, int64_t ld_src, void* dst, int64_t ld_dst, void* stream) {
   if (rows < 0 || cols < 0) return fail(MI_ERR_SHAPE, "rows %lld and cols %lld must not be negative", (long long)rows, (long long)cols);
   if (rows == 0 || cols == 0) return MI_OK;

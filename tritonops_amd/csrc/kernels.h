@@ -118,6 +118,16 @@ struct XentParams {
   int32_t tiles_t, block_t;  // set by the launcher
 };
 
+// grad_x [T, D] = dlogits [T, N] w [N, D], fp32 sums
+struct XentGradXParams {
+  const void *dlogits, *w;
+  void* gx;
+  float* part;         // xent_gradx_bytes(): partial tiles of the n_split vocabulary ranges
+  int64_t dl_ld, w_st, gx_ld;
+  int32_t T, D, N;
+  int32_t tiles_t, tiles_d, n_split;
+};
+
 struct XentGradParams {
   void* logits;        // [rows, N] in / dlogits out, row stride ld (elements)
   const float* lse;    // [rows]
@@ -207,6 +217,9 @@ int launch_xent_fwd(const XentParams& p, int dtype, bool grad, hipStream_t s);  
 size_t xent_kept_bytes(long long tokens, long long vocab);
 int launch_xent_kept_dlogits(const XentParams& p, int dtype, hipStream_t s);
 int launch_xent_dlogits(const XentGradParams& p, int dtype, hipStream_t s);
+int xent_gradx_splits(long long tokens, long long dim, long long vocab, int num_cus);
+size_t xent_gradx_bytes(long long tokens, long long dim, int n_split);
+int launch_xent_gradx(const XentGradXParams& p, int dtype, hipStream_t s);
 // dst[c][r] = src[r][c], 16-bit elements: src [rows, cols] and dst [cols, ld_dst] with 16-byte aligned rows of
 // multiples of 8 elements, ld_dst >= rows rounded up to 64; columns of dst from `rows` up to that multiple are zeroed.
 int launch_transpose16(const void* src, int64_t rows, int64_t cols, int64_t ld_src, void* dst, int64_t ld_dst, hipStream_t s);

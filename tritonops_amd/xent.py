@@ -13,7 +13,7 @@ import weakref
 import torch
 
 from . import _lib
-from .ops import _ptr, _require_gpu, _stream
+from .ops import _num_cus, _ptr, _require_gpu, _stream
 
 _TAGS = {torch.bfloat16: _lib.MI_DTYPE_BF16, torch.float16: _lib.MI_DTYPE_F16}
 # Rows of logits that the backward materialises at a time (the reference uses
@@ -45,6 +45,12 @@ KEEP_DIM = 1024
 # (8192 x 4096 x 128256: 6.25 -> 5.34, 0.40 ms; 8192 x 1024: 1.69 -> 1.39, 0.10;
 # 4096 x 2560: 2.88 -> 2.02, 0.26, but 4096 x 1024: 1.25 -> 1.34 and 2048 x 4096:
 # 1.62 -> 1.37, 0.40).
+# Where the result has so few tiles of 256 x 256 that _SPLIT_ROUNDS times as many still
+# fit the CUs, grad_x comes from a kernel of this library that divides the vocabulary
+# (the library's product leaves the other CUs idle: 1000 x 2560 x 128256: 1083 -> 604 us,
+# 300 x 1024 x 50257: 158 -> 57, 2000 x 2048 x 32000: 392 -> 242, 64 x 4096 x 128256:
+# 472 -> 253; with 96 tiles, 2000 x 3072, 1381 -> 1407).
+_SPLIT_ROUNDS, _SPLIT_VOCAB = 3, 8192
 _TURN_ROWS, _TURN_DIM = 256, 1536
 _TURN_X_ROWS, _TURN_X_DIM = 2048, 1024
 _TURN_W_ROWS, _TURN_W_TILES = 4096, 128
@@ -281,6 +287,37 @@ def _turns_w(rows, w):
             and w.shape[1] >= _TURN_X_DIM and _can_turn(w))
 
 
+def _splits_vocab(rows, w):
+    """The ranges of the vocabulary that grad_x of a block of `rows` rows is divided into; 0: it is not."""
+    N, D = w.shape
+    if N < _SPLIT_VOCAB or not _can_turn(w) or w.stride(0) > 1 << 22 or N > (1 << 22) - 64:
+        return 0
+    lib = _lib.load()
+    cus = _num_cus(lib)
+    if -(-rows // 256) * -(-D // 256) * _SPLIT_ROUNDS > cus:
+        return 0
+    return lib.mi_xent_grad_x_splits(rows, D, N, cus)
+
+
+def _grad_x(dl, w, out, n_split):
+    """out <- dl @ w, the vocabulary in n_split ranges; False without memory for their partial sums."""
+    lib = _lib.load()
+    a = _lib.XentGradXArgs()
+    a.struct_size = C.sizeof(a)
+    a.dtype = _tag(dl)
+    a.tokens, a.dim, a.vocab, a.n_split = out.shape[0], out.shape[1], w.shape[0], n_split
+    a.dlogits, a.w, a.grad_x = _ptr(dl), _ptr(w), _ptr(out)
+    a.ld, a.w_stride, a.grad_x_stride = dl.stride(0), w.stride(0), out.shape[1]
+    a.workspace_bytes = lib.mi_xent_grad_x_workspace_bytes(a.tokens, a.dim, n_split)
+    try:
+        ws = torch.empty(a.workspace_bytes, device=dl.device, dtype=torch.uint8)
+    except torch.OutOfMemoryError:
+        return False
+    a.workspace = _ptr(ws)
+    _lib.check(lib.mi_xent_grad_x(C.byref(a), _stream()))
+    return True
+
+
 def _bwd_bytes(x, w):
     """What the backward allocates for its dlogits and products at a time."""
     rows, N = min(x.shape[0], BWD_ROWS), w.shape[0]
@@ -328,7 +365,9 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
             _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl)
         else:
             _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl, dl_t)
-        torch.mm(dl, w if w_t is None else w_t, out=grad_x[s:e])
+        n_split = _splits_vocab(e - s, w) if grad_x.is_contiguous() else 0
+        if not (n_split and _grad_x(dl, w, grad_x[s:e], n_split)):
+            torch.mm(dl, w if w_t is None else w_t, out=grad_x[s:e])
         d, v = dl.t(), xc
         if x_t is not None:
             v = _turn(xc, x_t).t()
