@@ -92,10 +92,11 @@ typedef enum mi_status {
  * items of 256 query rows on workgroups of eight wavefronts, one to a compute
  * unit, and work items of 128 rows on workgroups of four wavefronts, two to a
  * compute unit (three at head_dim 64).  MI_DENSE_FORM_AUTO lets the library
- * pick per launch from the number of work items (the short form when every
- * work item has a compute unit to itself; at head_dim 64 also where three
- * workgroups per unit outrun one); the other two values are for tests and for
- * callers who have measured their own shapes.
+ * pick per launch from the number of work items (the short form for few rounds
+ * at head_dim 128, and at head_dim 64 where three workgroups per unit outrun
+ * one; a third form, two wavefronts to 32 rows and the same bits again, when
+ * every work item has a compute unit to itself); the other two values are for
+ * tests and for callers who have measured their own shapes.
  */
 enum { MI_DENSE_FORM_AUTO = 0, MI_DENSE_FORM_256_ROWS = 1, MI_DENSE_FORM_128_ROWS = 2 };
 
