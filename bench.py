@@ -40,7 +40,7 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 _NS = "_ZN2mi12_GLOBAL__N_1"
 KERNELS = {
     "dense_causal": _NS + "12dense_kernelIDF16bLi128EEEvNS_13PrefillParamsE",
-    "c1_dense_noncausal_small": _NS + "18dense_short_kernelIDF16bLi64ELb0EEEvNS_13PrefillParamsE",
+    "c1_dense_noncausal_small": _NS + "17dense_pair_kernelIDF16bLi64EEEvNS_13PrefillParamsE",
     "gqa_decode": _NS + "21decode_splitkv_kernelIDF16bLi128ELi1ELb0EEEvNS_12DecodeParamsE",
     "block_sparse": _NS + "13sparse_kernelIDF16bLi128EEEvNS_13PrefillParamsE",
     "sparse_decode": _NS + "21decode_splitkv_kernelIDF16bLi128ELi1ELb1EEEvNS_12DecodeParamsE",
@@ -156,7 +156,8 @@ def _dense_kernel_name(D):
         return long_form
     if DENSE_FORM == "128":
         return short_form
-    return long_form + " or " + short_form   # the launcher picks the form from the number of work items
+    pair_form = _NS + "17dense_pair_kernelIDF16bLi%dEEEvNS_13PrefillParamsE" % D
+    return " or ".join((long_form, short_form, pair_form))   # the launcher picks the form from the number of work items
 
 
 def run_dense_causal(steps, warmup):
