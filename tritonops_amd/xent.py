@@ -72,6 +72,18 @@ def _tag(t):
         raise TypeError("fused cross-entropy supports bfloat16 and float16 tensors, got %s" % t.dtype)
 
 
+def _check_xw(x, w):
+    """x [T, D] and w [N, D] of one dtype on one device: the kernels take w's type from x."""
+    if x.ndim != 2 or w.ndim != 2:
+        raise ValueError("x and w must be 2D tensors.")
+    if x.shape[1] != w.shape[1]:
+        raise ValueError("x has %d columns, w has %d" % (x.shape[1], w.shape[1]))
+    if w.dtype != x.dtype:
+        raise TypeError("x and w must share one dtype (got %s and %s)" % (x.dtype, w.dtype))
+    if w.device != x.device:
+        raise ValueError("x and w must be on one device (got %s and %s)" % (x.device, w.device))
+
+
 def _pad_dim(t, mult=128):
     """Rows as the kernel wants them: unit inner stride, 16-byte aligned, row
     stride a multiple of 8 and the inner size a multiple of 128 (zero columns
@@ -139,13 +151,8 @@ def _fwd(x, w, y, keep):
     """(loss, lse, kept): kept is the logits for _kept_dlogits, or None; `keep`:
     False never, True where there is memory for them, None within the budget."""
     _require_gpu(x, w, y)
+    _check_xw(x, w)
     lib = _lib.load()
-    if x.ndim != 2 or w.ndim != 2:
-        raise ValueError("x and w must be 2D tensors.")
-    if x.shape[1] != w.shape[1]:
-        raise ValueError("x has %d columns, w has %d" % (x.shape[1], w.shape[1]))
-    if w.dtype != x.dtype:
-        raise TypeError("x and w must share one dtype")
     T, N = x.shape[0], w.shape[0]
     y = _labels(y, T)
     xp, wp = _pad_dim(x), _pad_dim(w)
@@ -197,6 +204,7 @@ def cross_entropy_dlogits(x, w, y, lse, dloss):
     accumulators (replaces the logits GEMM + element-wise kernel of
     cross_entropy.py:374, :185-266, which round the logits to x's dtype first)."""
     _require_gpu(x, w, y, lse, dloss)
+    _check_xw(x, w)
     return _dlogits(x, w, y, lse, dloss, torch.empty((x.shape[0], w.shape[0]), device=x.device, dtype=x.dtype))
 
 
@@ -251,8 +259,8 @@ def _kept_dlogits(kept, first, y, lse, dloss, N, dl, dl_t=None):
 
 
 def _can_turn(t):
-    """Whether mi_transpose16 takes t (2-D, 16-bit)."""
-    return (t.stride(1) == 1 and t.shape[1] % 8 == 0 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1]
+    """Whether mi_transpose16 takes t (2-D)."""
+    return (t.element_size() == 2 and t.stride(1) == 1 and t.shape[1] % 8 == 0 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1]
             and t.data_ptr() % 16 == 0)
 
 
@@ -338,6 +346,7 @@ def cross_entropy_fused_bwd(grad_o, x, w, y, lse, rows_per_block=None):
 
 def _bwd(grad_o, x, w, y, lse, kept, step):
     _require_gpu(grad_o, x, w, y, lse)
+    _check_xw(x, w)
     T = x.shape[0]
     y = _labels(y, T)
     g = grad_o.reshape(-1).to(torch.float32).contiguous()
