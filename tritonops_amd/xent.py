@@ -361,36 +361,39 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
             w_t = _turn(w, w_t)[:, :w.shape[0]].t()
     for s in range(0, T, step):
         e = min(s + step, T)
-        xc = x[s:e]
-        dl = _dlogits_rows(e - s, w.shape[0], x)
-        turn_x, turn_dl = _turns_x(e - s, xc)
-        x_t = _room_turned(xc) if turn_x else None
-        dl_t = _room_turned(dl) if turn_dl and x_t is not None else None
-        if kept is None:
-            _dlogits(xc, w, y[s:e], lse[s:e], g[s:e], dl)
-            if dl_t is not None:  # (rows of dlogits are padded to whole pieces of 8, see _dlogits_rows)
-                _turn(dl.as_strided((e - s, dl_t.shape[0]), dl.stride()), dl_t)
-        elif dl_t is None:
-            _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl)
-        else:
-            _kept_dlogits(kept, s, y[s:e], lse[s:e], g[s:e], w.shape[0], dl, dl_t)
-        n_split = _splits_vocab(e - s, w) if grad_x.is_contiguous() else 0
-        if not (n_split and _grad_x(dl, w, grad_x[s:e], n_split)):
-            torch.mm(dl, w if w_t is None else w_t, out=grad_x[s:e])
-        d, v = dl.t(), xc
-        if x_t is not None:
-            v = _turn(xc, x_t).t()
-            if dl_t is None:
-                v = v[:e - s]
-            else:  # (the columns behind the rows are zeros in both)
-                d = dl_t[:w.shape[0]]
-        if grad_w is None:
-            grad_w = torch.mm(d, v)
-        else:
-            grad_w.addmm_(d, v)
+        grad_w = _block_gradients(x[s:e], w, w_t, y[s:e], lse[s:e], g[s:e], kept, s, grad_x[s:e], grad_w)
     if grad_w is None:
         grad_w = torch.zeros_like(w)
     return grad_x, grad_w
+
+
+def _block_gradients(x, w, w_t, y, lse, g, kept, first, grad_x, grad_w):
+    """grad_x of a block of rows, the first of which is row `first`, and grad_w with the block's part
+    added.  (A function of its own: its dlogits and copies are freed before the next block's are made.)"""
+    rows, N = x.shape[0], w.shape[0]
+    dl = _dlogits_rows(rows, N, x)
+    turn_x, turn_dl = _turns_x(rows, x)
+    x_t = _room_turned(x) if turn_x else None
+    dl_t = _room_turned(dl) if turn_dl and x_t is not None else None
+    if kept is None:
+        _dlogits(x, w, y, lse, g, dl)
+        if dl_t is not None:  # (rows of dlogits are padded to whole pieces of 8, see _dlogits_rows)
+            _turn(dl.as_strided((rows, dl_t.shape[0]), dl.stride()), dl_t)
+    elif dl_t is None:
+        _kept_dlogits(kept, first, y, lse, g, N, dl)
+    else:
+        _kept_dlogits(kept, first, y, lse, g, N, dl, dl_t)
+    n_split = _splits_vocab(rows, w) if grad_x.is_contiguous() else 0
+    if not (n_split and _grad_x(dl, w, grad_x, n_split)):
+        torch.mm(dl, w if w_t is None else w_t, out=grad_x)
+    d, v = dl.t(), x
+    if x_t is not None:
+        v = _turn(x, x_t).t()
+        if dl_t is None:
+            v = v[:rows]
+        else:  # (the columns behind the rows are zeros in both)
+            d = dl_t[:N]
+    return torch.mm(d, v) if grad_w is None else grad_w.addmm_(d, v)
 
 
 def _saved_hooks_set():
