@@ -66,3 +66,56 @@ def test_a_block_is_freed_before_the_next(on_cpu, monkeypatch, D):
     grads = xent._bwd(go, x, w, y, lse, None, 300)
     assert len(alive) == (6 if D == 1536 else 2)   # dlogits, x and dlogits turned, twice; or dlogits alone
     _check(grads, go, x, w, y)
+
+
+# the copies of the weights, of x and of the dlogits, and grad_w, which is allocated while they are held
+@pytest.mark.parametrize("fails", ["w", "x", "dlogits", "grad_w"])
+@pytest.mark.parametrize("step", [300, 600], ids=["blocks", "one_block"])
+def test_without_memory_for_the_copies_the_products_run_as_they_are(on_cpu, monkeypatch, fails, step):
+    go, x, w, y, lse = _problem(600, 1536, 72)
+    monkeypatch.setattr(xent, "_TURN_W_ROWS", 256)
+    monkeypatch.setattr(xent, "_TURN_W_TILES", 1)
+    room, mm, held = xent._room_turned, torch.mm, []
+
+    def out_of_memory():
+        raise torch.OutOfMemoryError("no memory")
+
+    def empty(t):
+        if tuple(t.shape) == {"w": (72, 1536), "x": (step, 1536), "dlogits": (step, 72)}.get(fails):
+            out_of_memory()
+        t = room(t)
+        held.append(weakref.ref(t.untyped_storage()))
+        return t
+
+    def product(a, b, out=None):
+        if fails == "grad_w" and out is None and any(r() is not None for r in held):
+            out_of_memory()
+        return mm(a, b) if out is None else mm(a, b, out=out)
+
+    monkeypatch.setattr(xent, "_room_turned", empty)
+    monkeypatch.setattr(xent.torch, "mm", product)
+    grads = xent._bwd(go, x, w, y, lse, None, step)
+    assert held or fails == "w"
+    _check(grads, go, x, w, y)
+    assert all(r() is None for r in held)
+
+
+def test_copies_take_a_quarter_of_the_free_memory(on_cpu, monkeypatch):
+    go, x, w, y, lse = _problem(600, 1536, 72)
+    made = []
+    room = xent._room_turned
+    monkeypatch.setattr(xent, "_room_turned", lambda t: made.append(t.shape) or room(t))
+    monkeypatch.setattr(xent.torch.cuda, "is_current_stream_capturing", lambda: False)
+    need = 4 * 600 * (1536 + 72) * 2
+
+    def run(free):
+        made.clear()
+        monkeypatch.setattr(xent, "_free_bytes", lambda device: free)
+        _check(xent._bwd(go, x, w, y, lse, None, 600), go, x, w, y)
+        return len(made)
+
+    assert run(0) == 2                                   # a few MB are not asked about
+    monkeypatch.setattr(xent, "KEEP_UNASKED", need // 4 - 1)
+    assert run(need) == 2 and run(need - 1) == 0
+    monkeypatch.setattr(xent.torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert run(0) == 2                                   # (its program has run the same before)

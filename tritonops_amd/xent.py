@@ -265,12 +265,8 @@ def _can_turn(t):
 
 
 def _room_turned(t):
-    """Room for the transpose of t [r, c]: [c rounded up to 8, r rounded up to 64], or
-    None without memory for it."""
-    try:
-        return torch.empty((-(-t.shape[1] // 8) * 8, -(-t.shape[0] // 64) * 64), device=t.device, dtype=t.dtype)
-    except torch.OutOfMemoryError:
-        return None
+    """Room for the transpose of t [r, c]: [c rounded up to 8, r rounded up to 64]."""
+    return torch.empty((-(-t.shape[1] // 8) * 8, -(-t.shape[0] // 64) * 64), device=t.device, dtype=t.dtype)
 
 
 def _turn(t, out):
@@ -326,15 +322,26 @@ def _grad_x(dl, w, out, n_split):
     return True
 
 
+def _copy_bytes(rows, x, w):
+    """What the operands that blocks of `rows` rows take the other way round occupy."""
+    turn_x, turn_dl = _turns_x(rows, x)
+    n = rows * (turn_x * x.shape[1] + turn_dl * w.shape[0]) + _turns_w(rows, w) * w.numel()
+    return n * x.element_size()
+
+
+def _makes_copies(rows, x, w):
+    """Whether blocks of `rows` rows take operands the other way round: where the rules above say so
+    and, from KEEP_UNASKED bytes on, the copies take at most a quarter of the free memory."""
+    n = _copy_bytes(rows, x, w)
+    if n <= KEEP_UNASKED or torch.cuda.is_current_stream_capturing():   # (as in _alloc_kept)
+        return n > 0
+    return 4 * n <= _free_bytes(x.device)
+
+
 def _bwd_bytes(x, w):
     """What the backward allocates for its dlogits and products at a time."""
-    rows, N = min(x.shape[0], BWD_ROWS), w.shape[0]
-    n = rows * N
-    turn_x, turn_dl = _turns_x(rows, x)
-    n += rows * (turn_x * x.shape[1] + turn_dl * N)
-    if _turns_w(rows, w):
-        n += w.numel()
-    return n * x.element_size()
+    rows = min(x.shape[0], BWD_ROWS)
+    return rows * w.shape[0] * x.element_size() + _copy_bytes(rows, x, w)
 
 
 def cross_entropy_fused_bwd(grad_o, x, w, y, lse, rows_per_block=None):
@@ -353,28 +360,37 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
     lse = lse.contiguous()
     if kept is not None and step % _KEPT_ROWS:
         step = max(step - step % _KEPT_ROWS, _KEPT_ROWS)
+    if _makes_copies(min(T, step), x, w):
+        try:
+            return _gradients(x, w, y, lse, g, kept, step, True)
+        except torch.OutOfMemoryError:
+            pass   # (whichever allocation it was, the copies are gone with the frames that held them)
+    return _gradients(x, w, y, lse, g, kept, step, False)
+
+
+def _gradients(x, w, y, lse, g, kept, step, copies):
+    """_bwd in blocks of `step` rows; `copies`: with operands the other way round where _turns_x and
+    _turns_w say so."""
     grad_x = torch.empty_like(x)
     grad_w = w_t = None
-    if _turns_w(min(T, step), w):
-        w_t = _room_turned(w)
-        if w_t is not None:
-            w_t = _turn(w, w_t)[:, :w.shape[0]].t()
-    for s in range(0, T, step):
-        e = min(s + step, T)
-        grad_w = _block_gradients(x[s:e], w, w_t, y[s:e], lse[s:e], g[s:e], kept, s, grad_x[s:e], grad_w)
+    if copies and _turns_w(min(x.shape[0], step), w):
+        w_t = _turn(w, _room_turned(w))[:, :w.shape[0]].t()
+    for s in range(0, x.shape[0], step):
+        r = slice(s, min(s + step, x.shape[0]))
+        grad_w = _block_gradients(x[r], w, w_t, y[r], lse[r], g[r], kept, s, copies, grad_x[r], grad_w)
     if grad_w is None:
         grad_w = torch.zeros_like(w)
     return grad_x, grad_w
 
 
-def _block_gradients(x, w, w_t, y, lse, g, kept, first, grad_x, grad_w):
+def _block_gradients(x, w, w_t, y, lse, g, kept, first, copies, grad_x, grad_w):
     """grad_x of a block of rows, the first of which is row `first`, and grad_w with the block's part
     added.  (A function of its own: its dlogits and copies are freed before the next block's are made.)"""
     rows, N = x.shape[0], w.shape[0]
     dl = _dlogits_rows(rows, N, x)
-    turn_x, turn_dl = _turns_x(rows, x)
+    turn_x, turn_dl = _turns_x(rows, x) if copies else (False, False)
     x_t = _room_turned(x) if turn_x else None
-    dl_t = _room_turned(dl) if turn_dl and x_t is not None else None
+    dl_t = _room_turned(dl) if turn_dl else None
     if kept is None:
         _dlogits(x, w, y, lse, g, dl)
         if dl_t is not None:  # (rows of dlogits are padded to whole pieces of 8, see _dlogits_rows)
@@ -446,9 +462,14 @@ def cross_entropy_fused_triton(x, w, y, *, keep_logits=None):
 
     `keep_logits`: whether the fp32 logits (4 bytes each) stay in memory from the
     forward to the backward, which then does not compute them again; loss and
-    gradients are the same bits either way.  None: where that is the faster way and
-    KEEP_BYTES and the free memory allow it.  False: never, no more memory than the
-    reference's scheme takes.  True: always where the allocation succeeds."""
+    gradients are the same bits either way (but for the order of the gradients' fp32
+    sums where memory is so short that one of the two backwards goes without its
+    copies, see below).  None: where that is the faster way and KEEP_BYTES and the
+    free memory allow it.  False: never.  True: always where the allocation succeeds.
+
+    The backward holds BWD_ROWS rows of dlogits at a time and, where its products are
+    faster for it and a quarter of the free memory is enough, transposed copies of
+    these and of its x and w; if an allocation fails with them it goes without."""
     if keep_logits is None:
         keep_logits = None if _keeps_logits(x, w) else False
     return CrossEntropyFusedFunction.apply(x, w, y, keep_logits)
