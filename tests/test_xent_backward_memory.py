@@ -119,3 +119,16 @@ def test_copies_take_a_quarter_of_the_free_memory(on_cpu, monkeypatch):
     assert run(need) == 2 and run(need - 1) == 0
     monkeypatch.setattr(xent.torch.cuda, "is_current_stream_capturing", lambda: True)
     assert run(0) == 2                                   # (its program has run the same before)
+
+
+def test_the_bytes_asked_for_cover_what_is_allocated(monkeypatch):
+    """Dlogits, copies and the partial sums of a divided vocabulary (fp32 tiles of 256 x 256)."""
+    monkeypatch.setattr(xent, "_num_cus", lambda lib: 256)
+
+    def asked(T, D, N):
+        return xent._bwd_bytes(torch.empty((T, D), dtype=torch.bfloat16), torch.empty((N, D), dtype=torch.bfloat16))
+
+    assert asked(40, 1024, 300) == 40 * 300 * 2                    # a small vocabulary is not divided
+    n_split = xent._lib.load().mi_xent_grad_x_splits(300, 1536, 8192, 256)
+    assert n_split > 1
+    assert asked(300, 1536, 8192) == 300 * 8192 * 2 + 300 * (1536 + 8192) * 2 + 2 * 6 * n_split * 65536 * 4

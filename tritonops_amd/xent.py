@@ -341,7 +341,9 @@ def _makes_copies(rows, x, w):
 def _bwd_bytes(x, w):
     """What the backward allocates for its dlogits and products at a time."""
     rows = min(x.shape[0], BWD_ROWS)
-    return rows * w.shape[0] * x.element_size() + _copy_bytes(rows, x, w)
+    n_split = _splits_vocab(rows, w)
+    split = _lib.load().mi_xent_grad_x_workspace_bytes(rows, w.shape[1], n_split) if n_split else 0
+    return rows * w.shape[0] * x.element_size() + _copy_bytes(rows, x, w) + split
 
 
 def cross_entropy_fused_bwd(grad_o, x, w, y, lse, rows_per_block=None):
