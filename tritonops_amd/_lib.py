@@ -5,6 +5,8 @@ if it has not been built (python -m tritonops_amd.build) loading raises.
 """
 import ctypes as C
 import os
+import sys
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmi_attn.so")
@@ -239,16 +241,32 @@ def load():
 _native = None
 
 
+class _GeneralWay:
+    """In the place of the native calls: answers none of them, as they answer a call
+    whose form they do not know, so that every call goes the general way."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def native():
-    """The native host calls (csrc/host_calls.cpp), loaded behind the library."""
+    """The native host calls (csrc/host_calls.cpp), loaded behind the library.  They are
+    tied to the Python and the torch they were built with and only save host time: where
+    they cannot be used, everything runs on the library alone, with one warning."""
     global _native
     if _native is None:
         load()
+        import torch
+        here = (str(torch.__version__), "%d.%d" % sys.version_info[:2])
         try:
             from . import _native as module
-        except ImportError as e:
-            raise ImportError("tritonops_amd/_native.so is missing or does not load (%s): build it with "
-                              "`python -m tritonops_amd.build`" % e) from e
+            why = "was built for torch %s and Python %s" % module.built_for if module.built_for != here else None
+        except (ImportError, AttributeError) as e:
+            why = "is missing or does not load (%s)" % e
+        if why is not None:
+            warnings.warn("tritonops_amd/_native.so %s: calls take up to 12 us longer on the host; build it with "
+                          "`python -m tritonops_amd.build`" % why, RuntimeWarning, stacklevel=2)
+            module = _GeneralWay()
         _native = module
     return _native
 

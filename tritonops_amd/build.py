@@ -53,6 +53,7 @@ def _native_object():
     obj = os.path.join(OBJ_DIR, "host_calls.o")
     include = cpp_extension.include_paths() + [sysconfig.get_paths()["include"]]
     cmd = [CXX, "-O2", "-std=c++17", "-fPIC", "-Wall", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+           '-DMI_TORCH_VERSION="%s"' % torch.__version__, '-DMI_PYTHON_VERSION="%d.%d"' % sys.version_info[:2],
            *("-isystem" + i for i in include), "-c", NATIVE_SRC, "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

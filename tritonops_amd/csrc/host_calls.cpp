@@ -534,4 +534,16 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+// built_for: the versions of torch and Python whose headers this was compiled with; the loader compares them
+// with those it runs under before anything is called.
+PyMODINIT_FUNC PyInit__native(void) {
+  PyObject* m = PyModule_Create(&module);
+  if (!m) return nullptr;
+  PyObject* v = Py_BuildValue("(ss)", MI_TORCH_VERSION, MI_PYTHON_VERSION);
+  if (!v || PyModule_AddObject(m, "built_for", v) < 0) {
+    Py_XDECREF(v);
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}
