@@ -217,10 +217,15 @@ def dense_form(form):
         _dense_form.value = before
 
 
+def _native_lengths(cu_seq_lens):
+    """Whether the native calls know a cu_seq_lens of this type (any other is converted on the general way)."""
+    return cu_seq_lens is None or cu_seq_lens.dtype == torch.int32
+
+
 def _native_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse, bhsd):
     """(o, lse) of a plain call in native code, or None (host_calls.cpp); with `bhsd`
     all tensors are [X, H, S, D], without it [X, S, H, D]."""
-    if not q.is_cuda or q.dim() != 4:
+    if not q.is_cuda or q.dim() != 4 or not _native_lengths(cu_seq_lens):
         return None
     max_len, rows = _cu_launch(cu_seq_lens, max_seq_len, q.shape[1])
     return _outputs(_lib.native().dense_fwd(q, k, v, cu_seq_lens, max_len, rows, scale_log2, causal, want_lse, bhsd,
@@ -297,7 +302,7 @@ def _general_fwd(q, k, v, cu_seq_lens, scale_log2, causal, max_seq_len, want_lse
 def _dense_bwd(q, k, v, o, do, lse, cu_seq_lens, scale_log2, causal, max_seq_len):
     """q, k, v, o, do as [X, S, H, D] views, lse [X, S, H] (see _fill_qkvo).
     Returns dq, dk, dv shaped and laid out like q, k, v."""
-    if q.is_cuda and q.dim() == 4:
+    if q.is_cuda and q.dim() == 4 and _native_lengths(cu_seq_lens):
         max_len, rows = _cu_launch(cu_seq_lens, max_seq_len, q.shape[1])
         out = _outputs(_lib.native().dense_bwd(q, k, v, o, do, lse, cu_seq_lens, max_len, rows, scale_log2, causal,
                                                *_here()))
@@ -484,8 +489,10 @@ def flash_attn_sparse_triton(q, k, v, cu_seqlens, softmax_scale=None, local_wind
     `csr_strides`); diagonal blocks are masked causally per token.
     A query with no allowed key gets o = 0 and lse = -inf.
     """
-    if q.is_cuda and q.dim() == 4 and q.shape[-1] in _HEAD_DIMS and q.numel() != 0:
-        packed = cu_seqlens is not None
+    lists = None
+    packed = cu_seqlens is not None
+    if q.is_cuda and q.dim() == 4 and q.shape[-1] in _HEAD_DIMS and q.numel() != 0 and _native_lengths(cu_seqlens) \
+            and (not packed or q.is_contiguous()):
         max_len, rows = _cu_launch(cu_seqlens, max_seq_len, q.shape[1])
         lists = _sparse_lists(q.shape[-1], max_len if packed else q.shape[2], local_window_size, global_window_size,
                               block_mask, row_ptr, col_idx, csr_strides, q.device)
@@ -495,7 +502,7 @@ def flash_attn_sparse_triton(q, k, v, cu_seqlens, softmax_scale=None, local_wind
         if out is not None:
             return out
     return _general_sparse(q, k, v, cu_seqlens, softmax_scale, local_window_size, global_window_size, block_mask,
-                           row_ptr, col_idx, csr_strides, max_seq_len)
+                           row_ptr, col_idx, csr_strides, max_seq_len, lists)
 
 
 def _sparse_lists(D, max_len, local_window_size, global_window_size, block_mask, row_ptr, col_idx, csr_strides, device):
@@ -525,8 +532,8 @@ def _sparse_lists(D, max_len, local_window_size, global_window_size, block_mask,
 
 
 def _general_sparse(q, k, v, cu_seqlens, softmax_scale, local_window_size, global_window_size, block_mask, row_ptr,
-                    col_idx, csr_strides, max_seq_len):
-    """flash_attn_sparse_triton for every form of its arguments."""
+                    col_idx, csr_strides, max_seq_len, lists=None):
+    """flash_attn_sparse_triton for every form of its arguments; `lists`: what _sparse_lists gives for them."""
     if cu_seqlens is not None:
         _check_qkv(q, k, v)
     else:
@@ -566,8 +573,8 @@ def _general_sparse(q, k, v, cu_seqlens, softmax_scale, local_window_size, globa
         qv, kv, vv, ov, lv = (t.transpose(1, 2) for t in (q, k, v, o, lse))
         batch = X
     scale = (D ** -0.5 if softmax_scale is None else float(softmax_scale)) * LOG2E
-    row_ptr, col_idx, csr_strides, wl, wg = _sparse_lists(D, max_len, local_window_size, global_window_size, block_mask,
-                                                          row_ptr, col_idx, csr_strides, q.device)
+    row_ptr, col_idx, csr_strides, wl, wg = lists or _sparse_lists(
+        D, max_len, local_window_size, global_window_size, block_mask, row_ptr, col_idx, csr_strides, q.device)
     if q.numel() == 0:
         return o, lse
     a = _lib.AttnSparseArgs()
@@ -592,7 +599,7 @@ def _decode(q, k, v, cu_seq_lens, seq_lens, scale, max_seq_len, split_tokens, re
             block_idx=None, block_cnt=None, bi_strides=(0, 0), max_blocks=0, split_blocks=0,
             window=(-1, -1), include_last=False, kv_layout="batched", page_table=None, page_size=0,
             window_form=False):
-    if q.is_cuda and (max_seq_len is None or max_seq_len >= 0) \
+    if q.is_cuda and (max_seq_len is None or max_seq_len >= 0) and _native_lengths(cu_seq_lens) \
             and (block_idx is None or tuple(bi_strides) == block_idx.stride()[:2]):
         listed = window_form or block_idx is not None
         out = _outputs(_lib.native().decode(
