@@ -1617,7 +1617,7 @@ constexpr int kPairLdsBytes = 2 * kPairStages * kShortTileKeys * SwizzledFrags<D
 //
 // The output wavefronts, which have fewer instructions to issue, load the tiles
 // into a ring of eight stages: tile p + 6 is requested at the top of position p into
-// the stage of tile p - 2, whose V was read in position p - 1; at the top of
+// the stage of tile p - 2, whose V was read in position p - 2; at the top of
 // position h tiles up to h + 2 have landed and up to three may still fly.
 template <typename T, int D>
 __global__ void __launch_bounds__(kShortRows * 4) dense_pair_kernel(const PrefillParams p) {
