@@ -132,3 +132,21 @@ def test_the_bytes_asked_for_cover_what_is_allocated(monkeypatch):
     n_split = xent._lib.load().mi_xent_grad_x_splits(300, 1536, 8192, 256)
     assert n_split > 1
     assert asked(300, 1536, 8192) == 300 * 8192 * 2 + 300 * (1536 + 8192) * 2 + 2 * 6 * n_split * 65536 * 4
+
+
+def test_without_memory_for_the_partial_sums_the_library_multiplies(on_cpu, monkeypatch):
+    go, x, w, y, lse = _problem(90, 136, 200)
+    asked = []
+
+    def empty(*size, dtype=None, **kw):
+        if dtype == torch.uint8:
+            asked.append(size)
+            raise torch.OutOfMemoryError("no memory")
+        return torch_empty(*size, dtype=dtype, **kw)
+
+    torch_empty = torch.empty
+    monkeypatch.setattr(xent.torch, "empty", empty)
+    monkeypatch.setattr(xent, "_splits_vocab", lambda rows, w: 2)
+    grads = xent._bwd(go, x, w, y, lse, None, 90)
+    assert asked == [(xent._lib.load().mi_xent_grad_x_workspace_bytes(90, 136, 2),)]
+    _check(grads, go, x, w, y)
