@@ -108,15 +108,23 @@ def test_copies_take_a_quarter_of_the_free_memory(on_cpu, monkeypatch):
     monkeypatch.setattr(xent.torch.cuda, "is_current_stream_capturing", lambda: False)
     need = 4 * 600 * (1536 + 72) * 2
 
-    def run(free):
+    def kept_dlogits(kept, first, y, lse, g, N, dl, dl_t=None):
+        xent._dlogits(x, w, y, lse, g, dl)
+        if dl_t is not None:
+            xent._turn(dl, dl_t)
+
+    def run(free, kept=None):
         made.clear()
         monkeypatch.setattr(xent, "_free_bytes", lambda device: free)
-        _check(xent._bwd(go, x, w, y, lse, None, 600), go, x, w, y)
+        _check(xent._bwd(go, x, w, y, lse, kept, 768), go, x, w, y)
         return len(made)
+
+    monkeypatch.setattr(xent, "_kept_dlogits", kept_dlogits)
 
     assert run(0) == 2                                   # a few MB are not asked about
     monkeypatch.setattr(xent, "KEEP_UNASKED", need // 4 - 1)
     assert run(need) == 2 and run(need - 1) == 0
+    assert run(0, object()) == 2                         # the forward asked for them along with the logits it kept
     monkeypatch.setattr(xent.torch.cuda, "is_current_stream_capturing", lambda: True)
     assert run(0) == 2                                   # (its program has run the same before)
 

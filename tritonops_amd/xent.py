@@ -329,11 +329,13 @@ def _copy_bytes(rows, x, w):
     return n * x.element_size()
 
 
-def _makes_copies(rows, x, w):
+def _makes_copies(rows, x, w, kept):
     """Whether blocks of `rows` rows take operands the other way round: where the rules above say so
-    and, from KEEP_UNASKED bytes on, the copies take at most a quarter of the free memory."""
+    and, from KEEP_UNASKED bytes on, the copies take at most a quarter of the free memory.  (With
+    kept logits that is not asked again, 25 us on a busy device: the forward has asked for the
+    copies along with them, unless its caller wanted them kept whatever is free.)"""
     n = _copy_bytes(rows, x, w)
-    if n <= KEEP_UNASKED or torch.cuda.is_current_stream_capturing():   # (as in _alloc_kept)
+    if kept is not None or n <= KEEP_UNASKED or torch.cuda.is_current_stream_capturing():   # (as in _alloc_kept)
         return n > 0
     return 4 * n <= _free_bytes(x.device)
 
@@ -362,7 +364,7 @@ def _bwd(grad_o, x, w, y, lse, kept, step):
     lse = lse.contiguous()
     if kept is not None and step % _KEPT_ROWS:
         step = max(step - step % _KEPT_ROWS, _KEPT_ROWS)
-    if _makes_copies(min(T, step), x, w):
+    if _makes_copies(min(T, step), x, w, kept):
         try:
             return _gradients(x, w, y, lse, g, kept, step, True)
         except torch.OutOfMemoryError:
@@ -471,7 +473,8 @@ def cross_entropy_fused_triton(x, w, y, *, keep_logits=None):
 
     The backward holds BWD_ROWS rows of dlogits at a time and, where its products are
     faster for it and a quarter of the free memory is enough, transposed copies of
-    these and of its x and w; if an allocation fails with them it goes without."""
+    these and of its x and w (which keep_logits=True asks for whatever is free); if an
+    allocation fails with them it goes without."""
     if keep_logits is None:
         keep_logits = None if _keeps_logits(x, w) else False
     return CrossEntropyFusedFunction.apply(x, w, y, keep_logits)
