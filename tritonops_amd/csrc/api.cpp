@@ -706,7 +706,11 @@ int mi_decode_choose_split(int batch, int heads_kv, int max_seqlen, int num_cus)
   // 2048 -> 1024: 92 -> 79; 64 x 2048 to 8192 of 16384, 2 kv-heads 2048 -> 1024:
   // 90 -> 71.  Over 175 calls of 1 to 64 sequences, bounds 64 to 131072, 2 to 16
   // kv-heads, 12 % less in the mean.  (Beyond 2048 tokens nothing is gained, and
-  // chunks of no power of two are slower than either neighbour.)
+  // chunks of no power of two are slower than either neighbour.)  Other chunks are
+  // other bits, 2.5e-3 apart in bf16: the probabilities, rounded to 16 bits in
+  // either case, are rounded against other reference points.  Error against 64
+  // bits over 45 calls of those ranges, the function above -> this one: 0.978 of it
+  // in the mean (0.93 to 1.03), e.g. 2.291e-3 -> 2.259e-3 for 2 x 6000 to 8000.
   if (batch <= 0 || heads_kv <= 0 || max_seqlen <= 0) return 64;
   if (num_cus <= 0) num_cus = 256;
   const long long work = (long long)batch * heads_kv * max_seqlen;  // tokens x kv-heads
