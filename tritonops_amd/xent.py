@@ -120,10 +120,11 @@ def _free_bytes(device):
     return torch.cuda.mem_get_info(device)[0] + reserved - used
 
 
-def _alloc_kept(T, N, device, bwd_bytes, always):
-    """Room for the logits of [T, N], or None: where the automatic choice (not
+def _alloc_kept(x, w, always):
+    """Room for the logits of x w^T, or None: where the automatic choice (not
     `always`) finds too many of them alive or too little memory free for them and
-    the `bwd_bytes` of the backward, and where the allocation fails."""
+    what the backward allocates, and where the allocation fails."""
+    T, N, device = x.shape[0], w.shape[0], x.device
     nbytes = _lib.load().mi_xent_kept_bytes(T, N)
     token = object()
     with _kept_lock:
@@ -133,7 +134,7 @@ def _alloc_kept(T, N, device, bwd_bytes, always):
                 return None
             # (a capture repeats what its program ran before it, and its pool is not in these figures)
             if live > KEEP_UNASKED and not torch.cuda.is_current_stream_capturing() \
-                    and 4 * (nbytes + bwd_bytes) > _free_bytes(device):
+                    and 4 * (nbytes + _bwd_bytes(x, w)) > _free_bytes(device):
                 return None
         _kept_live[token] = (device, nbytes)
     try:
@@ -172,7 +173,7 @@ def _fwd(x, w, y, keep):
     a.workspace, a.workspace_bytes = _ptr(ws), nbytes
     kept = None
     if keep is not False and T and N:
-        kept = _alloc_kept(T, N, x.device, _bwd_bytes(x, w), bool(keep))
+        kept = _alloc_kept(x, w, bool(keep))
     if kept is None:
         _lib.check(lib.mi_xent_fwd(C.byref(a), _stream()))
     else:
@@ -330,12 +331,14 @@ def _copy_bytes(rows, x, w):
 
 
 def _makes_copies(rows, x, w, kept):
-    """Whether blocks of `rows` rows take operands the other way round: where the rules above say so
-    and, from KEEP_UNASKED bytes on, the copies take at most a quarter of the free memory.  (With
+    """Whether blocks of `rows` rows may take operands the other way round where the rules above say so:
+    from KEEP_UNASKED bytes on, the copies take at most a quarter of the free memory.  (With
     kept logits that is not asked again, 25 us on a busy device: the forward has asked for the
     copies along with them, unless its caller wanted them kept whatever is free.)"""
+    if kept is not None:
+        return True
     n = _copy_bytes(rows, x, w)
-    if kept is not None or n <= KEEP_UNASKED or torch.cuda.is_current_stream_capturing():   # (as in _alloc_kept)
+    if n <= KEEP_UNASKED or torch.cuda.is_current_stream_capturing():   # (as in _alloc_kept)
         return n > 0
     return 4 * n <= _free_bytes(x.device)
 
