@@ -132,6 +132,11 @@ int mi_attn_fwd(const mi_attn_fwd_args *args, void *stream);
  * summed inside the kernel).  Addressing modes, causal flag and scale as in
  * mi_attn_fwd.  The workspace holds
  * Delta = rowsum(o * dout) in fp32.  Two launches on `stream`.
+ * A workspace of MI_ATTN_BWD_QUEUE_BYTES more than mi_attn_bwd_workspace_bytes()
+ * lets the second launch deal its work out at run time, which is faster where a
+ * GPU has few items of uneven length (one call's workspace must not be used by
+ * another call that may run at the same time, with or without it); the results
+ * are the same bits.
  * total_rows as in mi_attn_fwd: with a value > 0 (packed form) the rows of dq,
  * dk and dv that belong to no sequence are zero-filled by one more launch.
  */
@@ -161,6 +166,7 @@ typedef struct mi_attn_bwd_args {
   int32_t total_rows;                /* packed: rows of dq/dk/dv to cover, or 0 */
 } mi_attn_bwd_args;
 
+#define MI_ATTN_BWD_QUEUE_BYTES 640
 size_t mi_attn_bwd_workspace_bytes(const mi_attn_bwd_args *args);
 int mi_attn_bwd(const mi_attn_bwd_args *args, void *stream);
 

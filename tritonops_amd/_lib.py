@@ -15,6 +15,7 @@ MI_ATTN_ABI_VERSION = 8
 MI_DECODE_STATIC_SCRATCH_BYTES = 32 << 20
 MI_KV_BATCHED, MI_KV_PACKED, MI_KV_PAGED = 0, 1, 2
 MI_ATTN_BLOCK = 64
+MI_ATTN_BWD_QUEUE_BYTES = 640
 MI_DENSE_FORM_AUTO, MI_DENSE_FORM_256_ROWS, MI_DENSE_FORM_128_ROWS = 0, 1, 2
 MI_DTYPE_F32 = 2
 MI_DTYPE_BF16 = 0

@@ -465,6 +465,8 @@ int mi_xent_dlogits(const mi_xent_grad_args* a, void* stream) {
   return launch_status(mi::launch_xent_dlogits(p, a->dtype, static_cast<hipStream_t>(stream)), "mi_xent_dlogits");
 }
 
+static_assert(MI_ATTN_BWD_QUEUE_BYTES >= mi::kBwdQueueBytes + 127, "queues on a 128-byte boundary");
+
 int mi_attn_bwd_validate(const mi_attn_bwd_args* a) {
   if (!a) return fail(MI_ERR_NULL_POINTER, "args is NULL");
   if (a->struct_size != sizeof(mi_attn_bwd_args))
@@ -532,6 +534,9 @@ int mi_attn_bwd(const mi_attn_bwd_args* a, void* stream) {
   std::memset(&p, 0, sizeof(p));
   p.q = a->q; p.k = a->k; p.v = a->v; p.o = a->o; p.dout = a->dout; p.lse = a->lse;
   p.delta = static_cast<float*>(a->workspace);
+  const size_t queue_at = (mi_attn_bwd_workspace_bytes(a) + 127) / 128 * 128;   // behind Delta, where there is room
+  if (a->workspace_bytes >= queue_at + mi::kBwdQueueBytes)
+    p.queue = reinterpret_cast<int32_t*>(static_cast<char*>(a->workspace) + queue_at);
   p.dq = a->dq; p.dk = a->dk; p.dv = a->dv;
   p.q_sb = a->q_stride_b; p.q_ss = a->q_stride_s; p.q_sh = a->q_stride_h;
   p.k_sb = a->k_stride_b; p.k_ss = a->k_stride_s; p.k_sh = a->k_stride_h;

@@ -29,6 +29,7 @@
 // the accumulating product; its A operand is a streamed tile read through the
 // transposing LDS load.  Every streamed tile uses one layout that serves both
 // the row-fragment read and the transposing read (UniFrags).
+#include <algorithm>
 #include <type_traits>
 
 #include "item_order.h"
@@ -489,11 +490,12 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
 // rounded to the storage dtype (the operand of dV; the reference forms dS from
 // the fp32 P, :578): the score wave works one streamed tile AHEAD of the grad
 // wave, so the barrier that ends a tile step is the only synchronisation.
-template <typename T, int D>
-__device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, const int hr, const int rt, const int wave) {
+template <typename T, int D, int NP, typename Next>
+__device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, const int hr, const int rt, const int wave,
+                                              Next&& take_next) {
   using G = RowGeom<D>;
   using F = UniFrags<D>;
-  constexpr int NP = 4, BM = 32 * NP, TN = 64, NS = kBwdStages;
+  constexpr int BM = 32 * NP, TN = 64, NS = kBwdStages;
   static_assert(NS == 3, "stage reuse below assumes three stages");
   constexpr int TILEB = TN * F::ROWB;
   constexpr int STAGEB = 2 * TILEB + 1024;
@@ -503,8 +505,15 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   constexpr uint32_t PSLOT = NP * 2 * 2048;
 
   const int lane = opaque_lane();
-  const int pr = wave & 3;            // 32-row group of the item
-  const bool grad = wave >= 4;        // role of this wave
+  constexpr bool kLoaders = NP == 2;  // waves 4 to 7 send the loads and do nothing else
+  const int pr = wave & (NP - 1);             // 32-row group of the item
+  const bool grad = (wave & (2 * NP - 1)) >= NP;  // role of this wave
+  const bool loader = kLoaders && wave >= 4;
+  const bool sends = kLoaders ? loader : !grad;
+  const int lw = wave & 3;            // which of the four senders
+  // The wavefront that takes the workgroup's next unit, during the last step, in which it has nothing else to do
+  // (at the start of an item the choice would be made before anyone knows who will be done first).
+  constexpr int kTaker = kLoaders ? 7 : 3;
 
   const int gqa = p.hq / p.hkv;
   int len;
@@ -519,7 +528,10 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   }
   const int64_t bsel = p.cu ? 0 : b;
   const int r0 = rt * BM;
-  if (rt < 0 || r0 >= len) return;
+  if (rt < 0 || r0 >= len) {
+    if (wave == kTaker) take_next();
+    return;
+  }
 
   F fr;
   const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd);
@@ -556,6 +568,11 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   // straight-line code: a branch around it would end the basic block and let
   // the compiler move the arithmetic that is meant to sit behind the MFMAs.
   auto dma_masked = [&](uint64_t mask, uint64_t base, uint32_t off, uint32_t slab, auto wide_c) __attribute__((always_inline)) {
+    if (kLoaders) {
+      mask = uniform64(mask);
+      base = uniform64(base);
+      slab = (uint32_t)__builtin_amdgcn_readfirstlane(slab);
+    }
     if (decltype(wide_c)::value)
       asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 exec, %0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
                    : : "s"(mask), "v"(off), "s"(base), "s"(slab) : "memory");
@@ -574,36 +591,36 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   const int64_t pitch0 = p.q_ss * 2, pitch1 = p.do_ss * 2;
   const char* h0 = reinterpret_cast<const char*>(reinterpret_cast<const T*>(p.q) + bsel * p.q_sb + (start + j0 * TN) * p.q_ss + hr * gqa * p.q_sh);
   const char* h1 = reinterpret_cast<const char*>(reinterpret_cast<const T*>(p.dout) + bsel * p.do_sb + (start + j0 * TN) * p.do_ss + hr * gqa * p.do_sh);
-  const char* hl = wave == 0
+  const char* hl = lw == 0
       ? reinterpret_cast<const char*>(p.lse + bsel * p.lse_sb + (start + j0 * TN) * p.lse_ss + hr * gqa * p.lse_sh)
       : reinterpret_cast<const char*>(p.delta + (int64_t)b * p.dl_sb + (int64_t)hr * gqa * p.dl_sh + j0 * TN);
-  const int64_t pitchl = wave == 0 ? p.lse_ss * 4 : 4;
+  const int64_t pitchl = lw == 0 ? p.lse_ss * 4 : 4;
   uint64_t a0 = uniform64((uint64_t)(uintptr_t)h0), a1 = uniform64((uint64_t)(uintptr_t)h1), al = uniform64((uint64_t)(uintptr_t)hl);
   const uint64_t step0 = uniform64((uint64_t)(TN * pitch0)), step1 = uniform64((uint64_t)(TN * pitch1));
   const uint64_t stepl = uniform64((uint64_t)(TN * pitchl));
   const uint64_t wrap0 = uniform64((uint64_t)(p.q_sh * 2 - (int64_t)(nj - 1) * TN * pitch0));
   const uint64_t wrap1 = uniform64((uint64_t)(p.do_sh * 2 - (int64_t)(nj - 1) * TN * pitch1));
-  const uint64_t wrapl = uniform64((uint64_t)((wave == 0 ? p.lse_sh * 4 : p.dl_sh * 4) - (int64_t)(nj - 1) * TN * pitchl));
+  const uint64_t wrapl = uniform64((uint64_t)((lw == 0 ? p.lse_sh * 4 : p.dl_sh * 4) - (int64_t)(nj - 1) * TN * pitchl));
   // The four score wavefronts send the loads (the grad wavefronts carry more
   // arithmetic per tile): wave pr sends slabs pr, pr + 4, pr + 8, pr + 12 of
   // the Q tile and of the dO tile (1 KiB = four rows each).  The swizzle of a
   // lane's chunk depends on the slab only through slab % 4, so one lane offset
   // per tensor serves all four slabs; the slab moves the scalar base.
-  constexpr int kSlabs = TN / RPI / NP;      // slabs per tensor, tile and score wave
+  constexpr int kSlabs = TN / RPI / 4;      // slabs per tensor, tile and score wave
   constexpr int kDrips = 2 * kSlabs;
   static_assert(kDrips == 8, "compute_fast() places eight loads");
   uint32_t off0, off1;
   uint64_t lane_mask;
   {
-    const int r = RPI * pr + drow;
+    const int r = RPI * lw + drow;
     const int c = dslot ^ F::swz(r);
     off0 = (uint32_t)r * (uint32_t)pitch0 + c * 16;
     off1 = (uint32_t)r * (uint32_t)pitch1 + c * 16;
     lane_mask = __builtin_amdgcn_ballot_w64(G::NCH == 16 || c < G::NCH);
   }
-  const uint64_t slab0 = uniform64((uint64_t)(NP * RPI * pitch0)), slab1 = uniform64((uint64_t)(NP * RPI * pitch1));
+  const uint64_t slab0 = uniform64((uint64_t)(4 * RPI * pitch0)), slab1 = uniform64((uint64_t)(4 * RPI * pitch1));
   const uint32_t lv_off = (uint32_t)lane * (uint32_t)pitchl;
-  const uint64_t lv_mask = wave < 2 ? ~0ull : 0ull;
+  const uint64_t lv_mask = lw < 2 ? ~0ull : 0ull;
   int iss_left = nj;        // tiles of the current head still to request
   int iss_s0 = j0 * TN;     // first row of the next request
   int iss_st = 0;           // its stage
@@ -619,12 +636,12 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
       drip_on = ~0ull;
     } else {
       drip_on = 0;
-      if (grad) return;
+      if (!sends) return;
       const int last = len - 1 - iss_s0;  // >= 0
       const int ln = opaque_lane();
 #pragma unroll
       for (int t = 0; t < kSlabs; ++t) {
-        const int inst = pr + NP * t;
+        const int inst = lw + 4 * t;
         const int r = RPI * inst + ln / F::SLOTS;
         const int c = (ln % F::SLOTS) ^ F::swz(r);
         const int64_t rr = min(r, last);
@@ -636,9 +653,9 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
                        : : "v"((const char*)a1 + rr * pitch1 + c * 16), "s"(slab + TILEB) : "memory");
         }
       }
-      if (wave < 2) {
+      if (lw < 2) {
         const int64_t rr = min(ln, last);
-        const uint32_t slab = (uint32_t)__builtin_amdgcn_readfirstlane(iss_base + 2 * TILEB + (wave == 0 ? 0 : 256));
+        const uint32_t slab = (uint32_t)__builtin_amdgcn_readfirstlane(iss_base + 2 * TILEB + (lw == 0 ? 0 : 256));
         asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
                      : : "v"((const char*)al + rr * pitchl), "s"(slab) : "memory");
       }
@@ -647,15 +664,15 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   // load k of a request (score waves): k & 1 = tensor, k >> 1 = slab
   auto drip = [&](int k) __attribute__((always_inline)) {
     const int t = k >> 1;
-    const int inst = pr + NP * t;
+    const int inst = lw + 4 * t;
     if (k & 1)
       dma_masked(drip_on & lane_mask, a1 + t * slab1, off1, iss_base + TILEB + inst * 1024, ic<1>{});
     else
       dma_masked(drip_on & lane_mask, a0 + t * slab0, off0, iss_base + inst * 1024, ic<1>{});
-    if (k == 0) dma_masked(drip_on & lv_mask, al, lv_off, iss_base + 2 * TILEB + (wave == 0 ? 0 : 256), ic<0>{});
+    if (k == 0) dma_masked(drip_on & lv_mask, al, lv_off, iss_base + 2 * TILEB + (lw == 0 ? 0 : 256), ic<0>{});
   };
   auto drip_all = [&]() __attribute__((always_inline)) {
-    if (grad) return;
+    if (!sends) return;
 #pragma unroll
     for (int k = 0; k < kDrips; ++k) drip(k);
   };
@@ -806,7 +823,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
         constexpr int nx = st + kPrefetch;
         f[st % kPrefetch] = nx < K ? fr.rows(0, 0, nx) : fr.rows(0, 1, nx - K);
         side_reads(ic<st>{});
-        if (!grad)
+        if (!grad && !kLoaders)
           static_for<0, 4>([&](auto n_c) __attribute__((always_inline)) {
             if (st == drip_slice(decltype(n_c)::value)) drip(decltype(n_c)::value);
           });
@@ -827,7 +844,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
           W0[i] = pair(S0, lv[0], pp[0], i);
           asm volatile("" : "+v"(W0[i]));  // computed here, behind this MFMA
         }
-        if (!grad)
+        if (!grad && !kLoaders)
           static_for<0, 4>([&](auto n_c) __attribute__((always_inline)) {
             if (st == drip_slice(decltype(n_c)::value)) drip(4 + decltype(n_c)::value);
           });
@@ -873,7 +890,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   auto compute_slow = [&](auto role_c) __attribute__((always_inline)) {
     constexpr bool grad = decltype(role_c)::value != 0;
     const int s0 = cmp_s0;
-    drip_all();
+    if (!kLoaders) drip_all();
 #pragma unroll
     for (int sb = 0; sb < 2; ++sb) {
       const int sblk = s0 + 32 * sb;
@@ -987,7 +1004,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   auto run = [&](auto role_c) __attribute__((always_inline)) {
     constexpr bool gr = decltype(role_c)::value != 0;
     auto step = [&](auto fast_c) __attribute__((always_inline)) {
-      const bool more = req_left > 0;
+      const bool more = !kLoaders && req_left > 0;
       if (more) request();
       if (decltype(fast_c)::value)
         compute_fast(role_c);
@@ -999,7 +1016,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
       sync_step();
     };
     if (gr) {  // step 0: nothing to work on yet
-      if (req_left > 0) {
+      if (!kLoaders && req_left > 0) {
         request();
         drip_all();
         advance();
@@ -1012,12 +1029,27 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
       for (int jj = n_pre; jj < nj - n_post; ++jj) step(ic<1>{});
       for (int jj = nj - n_post; jj < nj; ++jj) step(ic<0>{});
     }
-    if (!gr) sync_step();  // the grad waves' last tile
+    if (!gr) {  // the grad waves' last tile
+      if (wave == kTaker) take_next();
+      sync_step();
+    }
   };
-  if (!grad)
+  if (loader) {
+    for (int i = 0; i <= n_stream; ++i) {
+      if (i == n_stream && wave == kTaker) take_next();
+      if (req_left > 0) {
+        request();
+        drip_all();
+        advance();
+      }
+      --req_left;
+      sync_step();
+    }
+  } else if (!grad) {
     run(ic<0>{});
-  else
+  } else {
     run(ic<1>{});
+  }
 
   // ---- epilogue: dV from the score waves, dK from the grad waves
   const float oscale = grad ? p.scale_nat : 1.f;
@@ -1026,6 +1058,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
   const int64_t o_ss = grad ? p.dk_ss : p.dv_ss;
   const int ln = opaque_lane();
   unsigned char* stg = smem_bwd + wave * 32 * OROWB;
+  if (loader) return;
 #pragma unroll
   for (int db = 0; db < G::NDB; ++db)
 #pragma unroll
@@ -1036,7 +1069,7 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
       w[1] = (int)Elem<T>::pack2(acc[db][4 * g + 2] * oscale, acc[db][4 * g + 3] * oscale);
       *reinterpret_cast<i32x2*>(stg + (ln & 31) * OROWB + d * 2) = w;
     }
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wavefront reads only what it has staged itself)
 #pragma unroll
   for (int i = 0; i < (32 * G::NCH + 63) / 64; ++i) {
     const int idx = ln + 64 * i;
@@ -1083,17 +1116,218 @@ __device__ __forceinline__ void walk_items(const BwdParams& p, const int n_items
 constexpr uint32_t kDqLds = kBwdStages * (2 * 64 * 256 + 1024);
 constexpr uint32_t kDkdvLds = kDqLds + 2 * 4 * 2 * 2048;  // tile ring + P exchange
 
+// The units of work of the dK + dV launch, dealt out at run time.
+//
+// An item of 128 keys is worked on whole (eight wavefronts in their two roles, two
+// to a SIMD), or as two halves of 64 keys (four wavefronts with a SIMD each, the
+// other four send the loads).  What bounds a launch of few items is the chain of
+// query tiles of its longest item: 1.23 us a tile, 0.80 in a half; with every CU
+// at work a tile takes 1.9 to 2.0 us (matrix pipes at the power limit) and the two
+// halves 1.18 times as long as the whole.  So the longest items are halved, as many
+// as shorten the launch, and a workgroup takes the next unit, longest first, when
+// it is done (in the fixed order two rounds of whole items left the busiest
+// workgroup with 1.3 times the mean).  Rows meet their tiles in the same order
+// either way: the results are the same bits.  dK + dV, fixed whole items -> this,
+// head_dim 128: 1000 tokens, 4 kv-heads of 4 94 -> 68 us; 2048, 2 of 8 315 -> 216;
+// 4096, 8 of 4 352 -> 292; 16384, 2 of 4 1362 -> 1137; five of 517 to 3400, 8 of 4
+// 384 -> 332; 8192, 8 of 4 (two even rounds, none halved) 967 -> 954.  Looking the
+// units up costs a launch 3 us: eight of 512, 8 of 1 20 -> 24.
+// Cost model, in hundredths of a microsecond, of n tiles:
+constexpr int kFullTile = 175, kHalfTile = 100, kUnitFixed = 700;
+static_assert(kFullTile * 4 == kHalfTile * 7, "key_units_before() orders the units by 4 : 7");
+constexpr int kMaxLevels = 512;      // tiles of 128 keys of the longest sequence
+static_assert(kMaxLevels < 1024, "plan_key_units() packs a level into ten bits");
+// Items per workgroup from which the fixed order is even enough (one sequence of 8192, 16 heads of their own, two
+// rounds: 128 us in either) and keeps neighbours together in an L2.
+constexpr int kDealtRounds = 4;
+
+// In LDS, behind the tiles and the P exchange.
+struct KeyPlan {
+  int list[3 * kMaxRounds];          // fixed order: items of this workgroup
+  int at_or_above[kMaxLevels + 1];  // (sequence, tile) pairs on level t and above; level: tiles counted from the sequence's end
+  int weight[kMaxLevels + 1];       // the same, pairs weighted with their level + 1
+  int tiles[kLevelMaxBatch];
+  int top;                           // levels, rounded up to a wavefront's lanes; at_or_above[top] = 0
+  int split_from, pairs, dealt;      // levels that are halved; (sequence, tile or half) pairs; whether units are dealt at run time
+  int next[2];                       // unit of the next round, by parity
+};
+
+typedef __attribute__((address_space(3))) KeyPlan LdsKeyPlan;
+typedef __attribute__((address_space(3))) int lds_int;
+
+// Units run from the longest to the shortest: pairs that stand before level t's.
+__device__ __forceinline__ int key_units_before(const LdsKeyPlan& k, const int t) {
+  const int T = k.split_from;
+  if (t >= T) {   // halves of level t: behind the whole items that cost more, 7 (t' + 1) > 4 (t + 1)
+    const int first = min(4 * (t + 1) / 7, T);
+    return 2 * k.at_or_above[t + 1] + k.at_or_above[first] - k.at_or_above[T];
+  }
+  const int first = max((7 * (t + 1) + 3) / 4 - 1, T);
+  return k.at_or_above[t + 1] - k.at_or_above[T] + 2 * k.at_or_above[min(first, k.top)];
+}
+
+// By one wavefront: the levels, and which of them are halved.  The estimate that is
+// minimised is the longer of the longest unit and the mean load plus a quarter of a mean unit.
+__device__ __forceinline__ void plan_key_units(LdsKeyPlan& k, const BwdParams& p, const int grid) {
+  const int lane = threadIdx.x & 63;
+  int tiles = 0;
+  if (lane < p.batch) {
+    const int len = p.cu ? min(p.cu[lane + 1] - p.cu[lane], p.max_seqlen) : p.max_seqlen;
+    tiles = len > 0 ? (len + 127) / 128 : 0;
+  }
+  k.tiles[lane] = tiles;
+  int levels = 0;
+  for (int b = 0; b < p.batch; ++b) levels = max(levels, __builtin_amdgcn_readlane(tiles, b));
+  const int top = (levels + 63) / 64 * 64;
+  int above = 0, above_w = 0;        // all pairs, all weights
+  for (int b = 0; b < p.batch; ++b) {
+    const int all = __builtin_amdgcn_readlane(tiles, b);
+    above += all;
+    above_w += all * (all + 1) / 2;
+  }
+  for (int t = lane; t <= top; t += 64) {
+    int n = 0, w = 0;
+    for (int b = 0; b < p.batch; ++b) {
+      const int all = __builtin_amdgcn_readlane(tiles, b);
+      if (all > t) n += all - t, w += (all * (all + 1) - t * (t + 1)) / 2;
+    }
+    k.at_or_above[t] = n;
+    k.weight[t] = w;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // lanes read what other lanes have written
+  const int gqa = p.hq / p.hkv;
+  const float unit = 2.f * gqa;      // tiles of 64 queries of a level-0 item
+  int T = levels;                    // halved from here on
+  if (p.causal) {
+    // (the estimate and the level in one word, the larger level among equals: one reduction)
+    uint32_t best = ~0u;
+    for (int base = 0; base <= levels; base += 64) {
+      const int t = base + lane;     // candidate
+      if (t <= levels) {
+        const float a = (float)k.at_or_above[t], w = (float)k.weight[t];
+        const float whole = (float)above - a, units = whole + 2.f * a;
+        const float total = (float)p.hkv * (2.f * (kHalfTile * unit * w + kUnitFixed * a) +
+                                            kFullTile * unit * ((float)above_w - w) + kUnitFixed * whole);
+        float longest = t > 0 ? kFullTile * unit * t + kUnitFixed : 0.f;
+        if (t < levels) longest = fmaxf(longest, kHalfTile * unit * levels + kUnitFixed);
+        float est = total / (float)grid;
+        if (units * (float)p.hkv > (float)grid) est += 0.25f * total / (units * (float)p.hkv);
+        est = fmaxf(est, longest);
+        best = min(best, (__builtin_bit_cast(uint32_t, est) & ~1023u) | (uint32_t)(1023 - t));
+      }
+    }
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, m, 64));
+    T = 1023 - (int)(best & 1023u);
+  } else if (2 * above * p.hkv <= grid) {
+    T = 0;                           // (every item of a sequence is as long as the next: all of them or none)
+  }
+  T = __builtin_amdgcn_readfirstlane(T);
+  if (lane == 0) {
+    k.top = top;
+    k.split_from = T;
+    k.pairs = above + k.at_or_above[T];
+    k.dealt = (p.causal ? above * p.hkv < kDealtRounds * grid : T == 0);
+  }
+}
+
+// Unit u: sequence, kv-head, tile of 128 keys (-1: behind the last unit) and half (-1: a whole item).
+struct KeyUnit {
+  int b, kvh, rt, half;
+};
+__device__ __forceinline__ KeyUnit key_unit(const LdsKeyPlan& k, const int hkv, const int u) {
+  KeyUnit it = {0, 0, -1, -1};
+  const int pair = __builtin_amdgcn_readfirstlane((int)((uint32_t)u / (uint32_t)hkv));
+  const int T = __builtin_amdgcn_readfirstlane(k.split_from), top = __builtin_amdgcn_readfirstlane(k.top);
+  const int lane = threadIdx.x & 63;
+  for (int base = 0; base < top; base += 64) {
+    const int t = base + lane;
+    const int n = pair - key_units_before(k, t);
+    const bool here = n >= 0 && n < (t >= T ? 2 : 1) * (k.at_or_above[t] - k.at_or_above[t + 1]);
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(here);
+    if (hit) {
+      const int at = __builtin_ctzll(hit);
+      const int level = base + at;
+      int seq = __builtin_amdgcn_readlane(n, at);
+      if (level >= T) {
+        it.half = seq & 1;
+        seq >>= 1;
+      }
+      const int all = k.tiles[lane];
+      const uint64_t live = __builtin_amdgcn_ballot_w64(all > level);
+      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(live >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)live, 0));
+      it.b = __builtin_ctzll(__builtin_amdgcn_ballot_w64(all > level && rank == seq));
+      it.kvh = u - pair * hkv;
+      it.rt = __builtin_amdgcn_readlane(all, it.b) - 1 - level;
+      break;
+    }
+  }
+  return it;
+}
+
+// Eight queues (workgroup ids go round-robin to the 8 XCDs): with the kv-head running
+// fastest an XCD keeps to its kv-heads, whose queries and gradients its L2 then holds,
+// whenever the head counts are multiples of eight.
 template <typename T, int D>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt) {
-  walk_items<128, true, kDkdvLds>(p, n_items, p.hkv, p.hkv, n_rt, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
-    bwd_dkdv_item<T, D>(p, b, hr, rt, wave);
-  });
+  LdsKeyPlan& k = *(LdsKeyPlan*)(uintptr_t)((uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd) + kDkdvLds);
+  const int grid = gridDim.x;
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int queues = (grid & 7) == 0 ? 8 : 1;
+  const int queue = queues == 8 ? blockIdx.x & 7 : 0;
+  const int first = queues == 8 ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
+  bool dealt = false;
+  if (p.queue) {
+    if (wave == 0) plan_key_units(k, p, grid);
+    __syncthreads();
+    dealt = __builtin_amdgcn_readfirstlane(k.dealt);
+  }
+  if (!dealt) {
+    if (wave == 0) {
+      const ItemId ids = items_of_rounds<128, true>(p.cu, p.batch, p.max_seqlen, n_rt, p.hkv, p.hkv, p.by_level, n_items, grid);
+      k.list[threadIdx.x] = ids.t;
+      k.list[kMaxRounds + threadIdx.x] = ids.b;
+      k.list[2 * kMaxRounds + threadIdx.x] = ids.h;
+    }
+    __syncthreads();
+  }
+  const int n_rounds = (n_items + grid - 1) / grid;
+  int unit = first * queues + queue;
+  for (int round = 0;; ++round) {
+    int b, h, rt, half = -1;
+    if (dealt) {
+      if (round > 0) unit = __builtin_amdgcn_readfirstlane(k.next[round & 1]);
+      const KeyUnit it = key_unit(k, p.hkv, unit);   // (every wavefront by itself)
+      if (it.rt < 0) break;
+      b = it.b;
+      h = it.kvh;
+      rt = it.rt;
+      half = it.half;
+    } else {
+      if (round == n_rounds) break;
+      rt = __builtin_amdgcn_readfirstlane(k.list[round]);
+      b = __builtin_amdgcn_readfirstlane(k.list[kMaxRounds + round]);
+      h = __builtin_amdgcn_readfirstlane(k.list[2 * kMaxRounds + round]);
+    }
+    auto take_next = [&]() __attribute__((always_inline)) {
+      if (dealt && (threadIdx.x & 63) == 0) {
+        const int n = __hip_atomic_fetch_add(p.queue + 16 * queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        k.next[(round + 1) & 1] = (n + grid / queues) * queues + queue;
+      }
+    };
+    if (half >= 0)
+      bwd_dkdv_item<T, D, 2>(p, b, h, 2 * rt + half, wave, take_next);
+    else
+      bwd_dkdv_item<T, D, 4>(p, b, h, rt, wave, take_next);
+    __syncthreads();  // the next item's tiles overwrite the staging area
+  }
 }
 
 template <typename T, int D>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 bwd_dq_kernel(const BwdParams p, const int n_items) {
+  if (blockIdx.x == 0 && threadIdx.x < 8 && p.queue) p.queue[16 * threadIdx.x] = 0;  // for the dK + dV kernel, which runs after this one
   walk_items<256, false, kDqLds>(p, n_items, p.hq, p.hkv, p.n_rtiles, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
     bwd_dq_item<T, D>(p, b, hr, rt, wave);
   });
@@ -1117,14 +1351,17 @@ int launch_dq(const BwdParams& p0, hipStream_t s) {
 template <typename T, int D>
 int launch_dkdv(const BwdParams& p0, hipStream_t s) {
   BwdParams p = p0;
-  constexpr size_t lds = kDkdvLds + kListBytes;
+  constexpr size_t lds = kDkdvLds + sizeof(KeyPlan);
   static_assert(kDqLds >= 8 * 32 * (D * 2 + 16), "epilogue staging must fit");
   auto kern = bwd_dkdv_kernel<T, D>;
   static LdsLimitOnce lds_once;
   if (const int e = raise_lds_limit(lds_once, reinterpret_cast<const void*>(kern), (int)lds)) return e;
   const int n_rt = (p.max_seqlen + 127) / 128;
   const long long items = (long long)n_rt * p.hkv * p.batch;
-  const long long grid = persistent_grid(items, device_cu_count());  // one workgroup per CU is resident (LDS)
+  const int cus = device_cu_count();
+  long long grid = persistent_grid(items, cus);  // one workgroup per CU is resident (LDS)
+  if (p.batch > kLevelMaxBatch || n_rt > kMaxLevels || (!p.cu && items >= kDealtRounds * (long long)cus)) p.queue = nullptr;
+  if (p.queue && items <= cus) grid = std::min((2 * items + 7) / 8 * 8, (long long)cus);  // each half a workgroup of its own
   p.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items, n_rt);
   return (int)hipGetLastError();

@@ -322,8 +322,8 @@ PyObject* dense_bwd(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     a.dq = dq.data_ptr();
     a.dk = dk.data_ptr();
     a.dv = dv.data_ptr();
-    a.workspace_bytes = mi_attn_bwd_workspace_bytes(&a);
-    ws = at::empty({(int64_t)std::max<size_t>(a.workspace_bytes, 16)}, q.options().dtype(at::kByte));
+    a.workspace_bytes = mi_attn_bwd_workspace_bytes(&a) + MI_ATTN_BWD_QUEUE_BYTES;
+    ws = at::empty({(int64_t)a.workspace_bytes}, q.options().dtype(at::kByte));
     a.workspace = ws.data_ptr();
     rc = mi_attn_bwd(&a, stream);
   }

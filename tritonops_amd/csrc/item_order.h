@@ -17,7 +17,9 @@
 // being known on the host.  The keys of the backward pass (128 rows to an item):
 // 1.61 -> 1.33 times the mean with 8 kv-heads, where 536 items make two rounds
 // and a few items of a third and the longest one alone is 1.2 times the mean,
-// 1.57 -> 1.09 with 32.
+// 1.57 -> 1.09 with 32.  (Launches of fewer than four rounds of these deal their
+// items, or halves of them, out at run time where they are given a place to count
+// in: bwd.hip.)
 //
 // The window walk's items cost t + 1 tiles only until the local window is filled
 // and a band each from there; numbered by level (always: what the unit order would

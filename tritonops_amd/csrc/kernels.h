@@ -68,6 +68,7 @@ struct BwdParams {
   const void *q, *k, *v, *o, *dout;
   const float* lse;  // base-2 row log-sum-exp of the forward pass
   float* delta;      // workspace [batch][hq][max_seqlen] fp32
+  int32_t* queue;    // workspace, kBwdQueueBytes: units taken so far from each of eight queues, 64 bytes apart (null: none)
   void *dq, *dk, *dv;
   int64_t q_sb, q_ss, q_sh;
   int64_t k_sb, k_ss, k_sh;
@@ -195,6 +196,7 @@ int launch_decode_merge(const DecodeParams& p, int dtype, int head_dim, hipStrea
 // device (hipError_t as int; no allocation).
 constexpr unsigned kDecodeScratchBytes = 32u << 20;
 int decode_static_scratch(void** ptr);
+constexpr size_t kBwdQueueBytes = 8 * 64;
 // the dQ kernel (which also writes Delta), then the dK + dV kernel
 int launch_attn_bwd(const BwdParams& p, int dtype, int head_dim, hipStream_t s);
 // RMSNorm.  x_dtype: 0 bf16, 1 f16, 2 f32; w_dtype: x_dtype or 2.  `vec`: rows

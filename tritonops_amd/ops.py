@@ -356,8 +356,8 @@ def _general_bwd(q, k, v, o, do, lse, cu_seq_lens, scale_log2, causal, max_seq_l
     a.heads_q, a.heads_kv, a.head_dim = Hq, k.shape[2], D
     a.causal = 1 if causal else 0
     a.scale_log2 = float(scale_log2)
-    nbytes = lib.mi_attn_bwd_workspace_bytes(C.byref(a))
-    ws = torch.empty(max(nbytes, 16), device=q.device, dtype=torch.uint8)
+    nbytes = lib.mi_attn_bwd_workspace_bytes(C.byref(a)) + _lib.MI_ATTN_BWD_QUEUE_BYTES
+    ws = torch.empty(nbytes, device=q.device, dtype=torch.uint8)
     a.workspace, a.workspace_bytes = _ptr(ws), nbytes
     _lib.check(lib.mi_attn_bwd(C.byref(a), _stream()))
     return dq, dk, dv
