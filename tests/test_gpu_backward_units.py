@@ -48,3 +48,25 @@ def test_dealt_units_equal_fixed_order(lens, Hq, Hkv, D, dt, causal, monkeypatch
     for name, a, b, c in zip(("dq", "dk", "dv"), dealt, again, fixed):
         assert torch.isfinite(c).all(), name
         assert torch.equal(a, c) and torch.equal(b, c), name
+
+
+@pytest.mark.parametrize("lens,H,D,dt,causal", [
+    ([127, 128, 129, 255, 256, 257, 383, 1, 0, 65], 40, 128, torch.bfloat16, True),
+    ([2100], 64, 96, torch.float16, True),
+    ([500, 300], 70, 64, torch.bfloat16, False),
+])
+def test_query_items_of_128_rows_equal_those_of_256(lens, H, D, dt, causal):
+    """Many heads at once have the long items, one head at a time the short ones."""
+    import tritonops_amd as ta
+    from tritonops_amd import ops
+
+    cu, T = cu_from(torch.tensor(lens, dtype=torch.int32)).cuda(), sum(lens)
+    q, k, v, do = (randn((1, T, H, D), 1 + i, dt).cuda() for i in range(4))
+    sm = D ** -0.5 * ta.LOG2E
+    o, lse = ops._general_fwd(q, k, v, cu, sm, causal, None, True, False)
+    grads = ops._general_bwd(q, k, v, o, do, lse, cu, sm, causal, None)
+    for h in range(0, H, 7):
+        p = slice(h, h + 1)
+        want = ops._general_bwd(q[:, :, p], k[:, :, p], v[:, :, p], o[:, :, p], do[:, :, p], lse[:, :, p], cu, sm, causal, None)
+        for name, a, b in zip(("dq", "dk", "dv"), grads, want):
+            assert torch.equal(a[:, :, p], b), (name, h)

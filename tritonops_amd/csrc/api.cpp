@@ -550,7 +550,6 @@ int mi_attn_bwd(const mi_attn_bwd_args* a, void* stream) {
   p.dl_sh = a->max_seqlen; p.dl_sb = (int64_t)a->heads_q * a->max_seqlen;
   p.cu = a->cu_seqlens;
   p.batch = a->batch; p.hq = a->heads_q; p.hkv = a->heads_kv; p.max_seqlen = a->max_seqlen;
-  p.n_rtiles = (a->max_seqlen + 255) / 256;
   p.causal = a->causal;
   p.scale = a->scale_log2;
   p.scale_nat = a->scale_log2 * 0.6931471805599453f;

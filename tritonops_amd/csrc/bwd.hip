@@ -119,15 +119,20 @@ constexpr int kBwdStages = 3;  // streamed tile pairs resident in LDS (4 measure
 
 // dQ: resident q, do rows; streams K, V.
 //   S^T = K Q^T,  dP^T = V dO^T,  dS = P o (dP - Delta),  dQ^T += K^T dS^T
-template <typename T, int D>
+// NW wavefronts of 32 rows each: eight, two to a SIMD, or (launches of few items,
+// see launch_all) four, while the other four send the loads.  A row meets its keys
+// in the same order in both: the results are the same bits.
+template <typename T, int D, int NW>
 __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, const int hr, const int rt, const int wave) {
   using G = RowGeom<D>;
   using F = UniFrags<D>;
-  constexpr int NW = 8, BM = 32 * NW, TN = 64, NS = kBwdStages;
+  constexpr int BM = 32 * NW, TN = 64, NS = kBwdStages;
+  constexpr bool kLoaders = NW == 4;              // wavefronts 4 to 7 send the loads and do nothing else
+  constexpr int NL = kLoaders ? 4 : 8;            // wavefronts that send loads
   constexpr int TILEB = TN * F::ROWB;             // one streamed tile
   constexpr int STAGEB = 2 * TILEB + 1024;        // tile 0, tile 1, lse[64] and delta[64] (fp32)
   constexpr int RPI = 1024 / F::ROWB;             // tile rows per direct-to-LDS instruction
-  constexpr int IPW = TN / RPI / NW;              // such instructions per tile and wave
+  constexpr int IPW = TN / RPI / NL;              // such instructions per tile and wave
   constexpr int IPT = 2 * IPW;                    // loads per streamed tile and wave
   constexpr int OROWB = D * 2 + 16;               // epilogue staging row
 
@@ -155,7 +160,9 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
   F fr;
   const uint32_t lds0 = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd);
   fr.init(lane, lds0);
-  const int r0w = r0 + 32 * wave;
+  const bool loader = kLoaders && wave >= NW;
+  const int lw = wave & (NL - 1);               // which of the senders
+  const int r0w = r0 + 32 * (wave & (NW - 1));
   const int rrow = r0w + fr.lq;                 // resident row of this lane
   const int rclamp = min(rrow, len - 1);
 
@@ -179,7 +186,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
     for (int i = 0; i < 8; ++i) delta_l += (float)oe[i] * (float)de[i];
   }
   delta_l += __shfl_xor(delta_l, 32);
-  if (fr.lh == 0 && rrow < len) p.delta[(int64_t)b * p.dl_sb + (int64_t)hr * p.dl_sh + rrow] = delta_l;
+  if (fr.lh == 0 && rrow < len && !loader) p.delta[(int64_t)b * p.dl_sb + (int64_t)hr * p.dl_sh + rrow] = delta_l;
   const float lse_l = p.lse[bsel * p.lse_sb + (start + rclamp) * p.lse_ss + hr * p.lse_sh];
 
   f32x16 acc[G::NDB];
@@ -200,6 +207,11 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
   // a load of the lanes in `mask` in straight-line code (all lanes are active
   // and control flow is wave-uniform here: exec is restored to all ones)
   auto dma_masked = [&](uint64_t mask, uint64_t base, uint32_t off, uint32_t slab) __attribute__((always_inline)) {
+    if (kLoaders) {
+      mask = uniform64(mask);
+      base = uniform64(base);
+      slab = (uint32_t)__builtin_amdgcn_readfirstlane(slab);
+    }
     asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 exec, %0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"
                  : : "s"(mask), "v"(off), "s"(base), "s"(slab) : "memory");
   };
@@ -214,17 +226,17 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
   const char* h1 = reinterpret_cast<const char*>(reinterpret_cast<const T*>(p.v) + bsel * p.v_sb + start * p.v_ss + hs * p.v_sh);
   uint64_t a0 = uniform64((uint64_t)(uintptr_t)h0), a1 = uniform64((uint64_t)(uintptr_t)h1);
   const uint64_t step0 = uniform64((uint64_t)(TN * pitch0)), step1 = uniform64((uint64_t)(TN * pitch1));
-  const uint64_t slab0 = uniform64((uint64_t)(NW * RPI * pitch0)), slab1 = uniform64((uint64_t)(NW * RPI * pitch1));
+  const uint64_t slab0 = uniform64((uint64_t)(NL * RPI * pitch0)), slab1 = uniform64((uint64_t)(NL * RPI * pitch1));
   uint32_t off0, off1;
   uint64_t lane_mask;
   {
-    const int r = RPI * wave + drow;
+    const int r = RPI * lw + drow;
     const int c = dslot ^ F::swz(r);
     off0 = (uint32_t)r * (uint32_t)pitch0 + c * 16;
     off1 = (uint32_t)r * (uint32_t)pitch1 + c * 16;
     lane_mask = __builtin_amdgcn_ballot_w64(G::NCH == 16 || c < G::NCH);
   }
-  static_assert(IPT == 4, "compute_fast() places four loads");
+  static_assert(kLoaders || IPT == 4, "compute_fast() places four loads");
   int iss_s0 = 0;            // first row of the next request
   int iss_st = 0;            // its stage
   uint32_t iss_base = lds0;  // and the stage's LDS address
@@ -240,7 +252,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
       const int last = len - 1 - iss_s0;  // >= 0
 #pragma unroll
       for (int t = 0; t < IPW; ++t) {
-        const int inst = wave + NW * t;
+        const int inst = lw + NL * t;
         const int r = RPI * inst + drow;
         const int c = dslot ^ F::swz(r);
         const int64_t rr = min(r, last);
@@ -257,7 +269,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
   // load k of a request: k & 1 = tensor, k >> 1 = slab
   auto drip = [&](int k) __attribute__((always_inline)) {
     const int t = k >> 1;
-    const int inst = wave + NW * t;
+    const int inst = lw + NL * t;
     if (k & 1)
       dma_masked(drip_on & lane_mask, a1 + t * slab1, off1, iss_base + TILEB + inst * 1024);
     else
@@ -336,7 +348,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
       constexpr int st = decltype(st_c)::value;
       S = Elem<T>::mfma(f[st % kPrefetch], Xf[st], S);
       if (st + kPrefetch < NSTEP) f[st % kPrefetch] = frag(st + kPrefetch);
-      if (sb == 0 && !masked)
+      if (sb == 0 && !masked && !kLoaders)
         static_for<0, IPT>([&](auto n_c) __attribute__((always_inline)) {
           if (st == drip_slice(decltype(n_c)::value)) drip(decltype(n_c)::value);
         });
@@ -398,7 +410,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
   };
   // a tile on the diagonal or at the sequence end
   auto compute_slow = [&](int s0) __attribute__((always_inline)) {
-    drip_all();
+    if (!kLoaders) drip_all();
     bool f_ready = false;
     if (s0 < len && !(causal && s0 > r0w + 31)) {
       block(ic<0>{}, ic<1>{}, s0, false);
@@ -411,7 +423,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
   // into the stage that tile u - 1 has left
 #pragma unroll
   for (int u = 0; u < NS - 1; ++u)
-    if (u < n_stream) {
+    if (u < n_stream && (!kLoaders || loader)) {
       request();
       drip_all();
       advance();
@@ -427,7 +439,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
   int n_fast = min(n_stream, len / TN);
   if (causal) n_fast = min(n_fast, (r0w + 1) / TN);
   auto step = [&](auto fast_c, int u) __attribute__((always_inline)) {
-    const bool refill = u + NS - 1 < n_stream;
+    const bool refill = !kLoaders && u + NS - 1 < n_stream;
     if (refill) request();
     if (decltype(fast_c)::value)
       compute_fast(u * TN);
@@ -443,6 +455,22 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
       __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     __syncthreads();
   };
+  if (loader) {
+    for (int u = 0; u < n_stream; ++u) {
+      const bool refill = u + NS - 1 < n_stream;
+      if (refill) {
+        request();
+        drip_all();
+        advance();
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(IPT));
+      } else {
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+      }
+      __syncthreads();
+    }
+    __syncthreads();
+    return;
+  }
   for (int u = 0; u < n_fast; ++u) step(ic<1>{}, u);
   for (int u = n_fast; u < n_stream; ++u) step(ic<0>{}, u);
   __builtin_amdgcn_s_setprio(0);
@@ -463,7 +491,7 @@ __device__ __forceinline__ void bwd_dq_item(const BwdParams& p, const int b, con
       w[1] = (int)Elem<T>::pack2(acc[db][4 * g + 2] * oscale, acc[db][4 * g + 3] * oscale);
       *reinterpret_cast<i32x2*>(stage + fr.lq * OROWB + d * 2) = w;
     }
-  __syncthreads();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (a wavefront reads only what it has staged itself)
 #pragma unroll
   for (int i = 0; i < (32 * G::NCH + 63) / 64; ++i) {
     const int idx = lane + 64 * i;
@@ -1324,27 +1352,28 @@ bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt) {
   }
 }
 
-template <typename T, int D>
+template <typename T, int D, int NW>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
-bwd_dq_kernel(const BwdParams p, const int n_items) {
+bwd_dq_kernel(const BwdParams p, const int n_items, const int n_rt) {
   if (blockIdx.x == 0 && threadIdx.x < 8 && p.queue) p.queue[16 * threadIdx.x] = 0;  // for the dK + dV kernel, which runs after this one
-  walk_items<256, false, kDqLds>(p, n_items, p.hq, p.hkv, p.n_rtiles, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
-    bwd_dq_item<T, D>(p, b, hr, rt, wave);
+  walk_items<32 * NW, false, kDqLds>(p, n_items, p.hq, p.hkv, n_rt, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
+    bwd_dq_item<T, D, NW>(p, b, hr, rt, wave);
   });
 }
 
-template <typename T, int D>
+template <typename T, int D, int NW>
 int launch_dq(const BwdParams& p0, hipStream_t s) {
   BwdParams p = p0;
   constexpr size_t lds = kDqLds + kListBytes;
   static_assert(kDqLds >= 8 * 32 * (D * 2 + 16), "epilogue staging must fit the tile ring");
-  auto kern = bwd_dq_kernel<T, D>;
+  auto kern = bwd_dq_kernel<T, D, NW>;
   static LdsLimitOnce lds_once;
   if (const int e = raise_lds_limit(lds_once, reinterpret_cast<const void*>(kern), (int)lds)) return e;
-  const long long items = (long long)p.n_rtiles * p.hq * p.batch;
+  const int n_rt = (p.max_seqlen + 32 * NW - 1) / (32 * NW);
+  const long long items = (long long)n_rt * p.hq * p.batch;
   const long long grid = persistent_grid(items, device_cu_count());  // one workgroup per CU is resident (LDS)
   p.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items, n_rt);
   return (int)hipGetLastError();
 }
 
@@ -1369,9 +1398,16 @@ int launch_dkdv(const BwdParams& p0, hipStream_t s) {
 
 template <typename T, int D>
 int launch_all(const BwdParams& p, hipStream_t s) {
-  // dQ first: it also writes Delta, which the dK + dV kernel reads
+  // dQ first: it also writes Delta, which the dK + dV kernel reads.
+  // Items of 128 queries, a wavefront to a SIMD, where they are at most one round of workgroups, or two of a causal
+  // call (its second round is of short items): a tile of 64 keys then takes 1.5 instead of 2.1 us, and the longest
+  // chain bounds the launch.  256 -> 128 rows, head_dim 128: 1000 tokens, 16 heads 40 -> 29 us; 2048, 32 heads (two
+  // rounds) 82 -> 66; 4096, 16 heads 135 -> 108; 8192, 8 heads 255 -> 195; eight of 512, 8 heads 28 -> 23; head_dim 64,
+  // 2400, 16 heads 56 -> 36.  Beyond: three of 300 to 1100, 32 heads (2.3 rounds) 48 -> 57, 4096, 32 heads (four) 191 -> 208.
   int rc;
-  if ((rc = launch_dq<T, D>(p, s))) return rc;
+  const long long halves = (long long)((p.max_seqlen + 127) / 128) * p.hq * p.batch;
+  const bool few = halves <= (p.causal ? 2 : 1) * (long long)device_cu_count();
+  if ((rc = few ? launch_dq<T, D, 4>(p, s) : launch_dq<T, D, 8>(p, s))) return rc;
   return launch_dkdv<T, D>(p, s);
 }
 

@@ -82,7 +82,6 @@ struct BwdParams {
   int64_t dl_sb, dl_sh;
   const int32_t* cu;  // null => batched
   int32_t batch, hq, hkv, max_seqlen;
-  int32_t n_rtiles;   // ceil(max_seqlen / 256): resident tiles of the dQ kernel
   int32_t by_level;   // items numbered by level (item_order.h; set by the launcher)
   int32_t causal;
   float scale;        // log2 domain
