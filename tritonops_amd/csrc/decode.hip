@@ -78,6 +78,20 @@ __device__ __forceinline__ void lds_barrier() {
   }
 }
 
+// A word at a wave-uniform address of memory that no kernel of the launch writes
+// (lengths, block lists, page tables), through the scalar cache.  As an ordinary
+// load it goes the way of the K/V tiles, whose loads retire in order: the wait for
+// one page number or list entry then waits for every tile that is in flight: pass 1
+// of 8 sequences of 4k to 8k tokens in pages of 64, 8 kv-heads of 128, 38.5 -> 35.2 us
+// (32 of them 143 -> 135, contiguous 135), lists of 64 blocks, 4 sequences, 15.9 -> 14.4.
+__device__ __forceinline__ int scalar_word(const int32_t* a) {
+  typedef __attribute__((address_space(4))) const int32_t c_int32;
+  const uint64_t u = (uint64_t)(uintptr_t)a;
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)u);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  return *(c_int32*)(((uint64_t)hi << 32) | lo);
+}
+
 // One work item: chunk `split` of (sequence b, kv-head kvh) for the 32 query
 // heads of the group that start at head g0 of it (slice kvs % gslices; a group
 // of up to 32 heads is one slice).
@@ -89,7 +103,7 @@ __device__ __forceinline__ void lds_barrier() {
 // is the bound), and the output needs no merge between wavefronts.
 template <typename T, int D, int NW, bool LIST>
 __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char* smem, const int split, const int kvs,
-                                            const int b) {
+                                            const int b, const int len) {
   const int kvh = kvs / p.gslices;
   const int g0 = (kvs % p.gslices) * 32;
   using G = RowGeom<D>;
@@ -105,7 +119,6 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
   unsigned char* sK = smem;
   unsigned char* sV = smem + NW * KTILEB;
 
-  const int len = p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
   const int gqa_all = p.hq / p.hkv;
   const int gqa = min(32, gqa_all - g0);  // query heads of this slice
   constexpr bool sparse = LIST;
@@ -123,7 +136,7 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
       wlist = window_list(len, p.win_global, p.win_local);
       cnt = min(wlist.cnt, p.max_blocks);
     } else {
-      cnt = p.block_cnt ? min(p.block_cnt[b * p.hkv + kvh], p.max_blocks) : p.max_blocks;
+      cnt = p.block_cnt ? min(scalar_word(p.block_cnt + b * p.hkv + kvh), p.max_blocks) : p.max_blocks;
     }
     const int total = cnt + p.add_last;  // the implicit last block sits behind the list
     b0 = split * p.split_blocks;
@@ -141,29 +154,19 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
   auto tile_base = [&](int i) -> int {
     if (!sparse) return t_begin + i * kDecTile;
     const int e = i >> 1;
-    const int blk = e < n_listed ? (derived ? wlist.block(b0 + e) : blist[e]) : last_blk;
+    const int blk = e < n_listed ? (derived ? wlist.block(b0 + e) : scalar_word(blist + e)) : last_blk;
     if (p.add_last && e < n_listed && blk == last_blk) return -1;
     return blk * 64 + (i & 1) * kDecTile;
   };
 
   // Start of this sequence's rows: batch stride, row offset cu[b] of a packed
   // buffer, or (paged) the pool itself with the page looked up per tile.
-  const int64_t seq0 = p.kv_layout == 1 ? (int64_t)p.cu[b] : 0;
+  const int64_t seq0 = p.kv_layout == 1 ? (int64_t)scalar_word(p.cu + b) : 0;
   const int64_t bsel = p.kv_layout == 0 ? b : 0;
   const T* kp = reinterpret_cast<const T*>(p.k) + bsel * p.k_sb + seq0 * p.k_ss + kvh * p.k_sh;
   const T* vp = reinterpret_cast<const T*>(p.v) + bsel * p.v_sb + seq0 * p.v_ss + kvh * p.v_sh;
   const bool paged = p.kv_layout == 2;
   const int32_t* ptab = paged ? p.page_table + b * p.pt_sb : nullptr;
-  // Paged: a 32-token tile never straddles a page (page_size % 32 == 0).  The
-  // returned element offset moves token `tb` of the flat addressing below onto
-  // its place in the physical page.
-  auto page_shift = [&](int tb, int64_t page_stride, int64_t row_stride) -> int64_t {
-    if (!paged) return 0;
-    const int lp = tb / p.page_size;
-    const int64_t phys = ptab[lp];
-    return phys * page_stride - (int64_t)lp * p.page_size * row_stride;
-  };
-
   F lc;
   lc.init(lane);
 
@@ -252,8 +255,15 @@ __device__ __forceinline__ void decode_item(const DecodeParams& p, unsigned char
   auto tile_src = [&](int base) __attribute__((always_inline)) -> TileSrc {
     const int tb = addr_base(base);
     TileSrc t;
-    t.k = uniform64((uint64_t)(uintptr_t)(kp + page_shift(tb, p.k_sb, p.k_ss) + (int64_t)tb * p.k_ss));
-    t.v = uniform64((uint64_t)(uintptr_t)(vp + page_shift(tb, p.v_sb, p.v_ss) + (int64_t)tb * p.v_ss));
+    int64_t page = 0;
+    int row = tb;
+    if (paged) {   // a 32-token tile never straddles a page (page_size % 32 == 0)
+      const int lp = tb / p.page_size;
+      page = scalar_word(ptab + lp);
+      row = tb - lp * p.page_size;
+    }
+    t.k = uniform64((uint64_t)(uintptr_t)(kp + page * p.k_sb + (int64_t)row * p.k_ss));
+    t.v = uniform64((uint64_t)(uintptr_t)(vp + page * p.v_sb + (int64_t)row * p.v_ss));
     t.row_max = len - 1 - tb;
     return t;
   };
@@ -370,15 +380,16 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)
 decode_splitkv_kernel(const DecodeParams p) {
   __shared__ __attribute__((aligned(16))) unsigned char smem[NW * wave_lds<D>()];
   if constexpr (LIST) {
-    decode_item<T, D, NW, true>(p, smem, blockIdx.x, blockIdx.y, blockIdx.z);
+    const int b = blockIdx.z;
+    const int len = p.seq_lens ? scalar_word(p.seq_lens + b) : scalar_word(p.cu + b + 1) - scalar_word(p.cu + b);
+    decode_item<T, D, NW, true>(p, smem, blockIdx.x, blockIdx.y, b, len);
     return;
   }
   const int lane = threadIdx.x & 63;
-  auto chunks_of = [&](int b) -> int {
-    if (b >= p.batch) return 0;
-    const int len = p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
-    return len > 0 ? min((len - 1) / p.split_tokens + 1, p.n_splits) : 0;
+  auto len_of = [&](int b) -> int {
+    return b >= p.batch ? 0 : p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
   };
+  auto chunks_of = [&](int len) -> int { return len > 0 ? min((len - 1) / p.split_tokens + 1, p.n_splits) : 0; };
   auto chunks_up_to = [&](int n) __attribute__((always_inline)) -> int {  // inclusive scan over the lanes
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -388,18 +399,20 @@ decode_splitkv_kernel(const DecodeParams p) {
     return n;
   };
   // the first 64 sequences, which most batches end within: looked at once
-  const int n_first = chunks_of(lane);
+  const int len_first = len_of(lane);
+  const int n_first = chunks_of(len_first);
   const int incl_first = chunks_up_to(n_first);
   const uint32_t kv_slices = p.hkv * p.gslices;  // (kv-head, 32-head slice of its group) pairs
   // (every item has a slot of at least 64 floats in the workspace: ids stay far below 2^32)
   for (uint32_t g = blockIdx.x;; g += gridDim.x) {
     const int t = (int)(g / kv_slices), kvs = (int)(g % kv_slices);
     // the sequence that owns live chunk t, and the number of its first chunk
-    int b = -1, first = 0;
+    int b = -1, first = 0, len = 0;
     for (int b0 = 0, seen = 0; b0 < p.batch; b0 += 64) {
-      int n = n_first, incl = incl_first;
+      int n = n_first, incl = incl_first, own = len_first;
       if (b0 != 0) {
-        n = chunks_of(b0 + lane);
+        own = len_of(b0 + lane);
+        n = chunks_of(own);
         incl = chunks_up_to(n);
       }
       const int before = seen + incl - n;  // live chunks ahead of this lane's sequence
@@ -408,12 +421,13 @@ decode_splitkv_kernel(const DecodeParams p) {
         const int at = __builtin_ctzll(hit);
         b = b0 + at;
         first = __builtin_amdgcn_readlane(before, at);
+        len = __builtin_amdgcn_readlane(own, at);
         break;
       }
       seen += __builtin_amdgcn_readlane(incl, 63);
     }
     if (b < 0) return;  // behind the last live chunk
-    decode_item<T, D, NW, false>(p, smem, t - first, kvs, b);
+    decode_item<T, D, NW, false>(p, smem, t - first, kvs, b, len);
   }
 }
 
