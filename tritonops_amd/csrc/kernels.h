@@ -115,7 +115,7 @@ struct XentParams {
   int32_t T, D, N;
   int32_t y_is_i64;
   int32_t n_split;           // vocabulary ranges (xent_choose_splits)
-  int32_t tiles_t, block_t;  // set by the launcher
+  int32_t tiles_t;           // set by the launcher
 };
 
 // grad_x [T, D] = dlogits [T, N] w [N, D], fp32 sums

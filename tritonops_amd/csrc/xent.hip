@@ -23,9 +23,15 @@
 // at the end and the workgroup writes one partial (lse, target logit) per token
 // and vocabulary range.  A second kernel merges the ranges.
 //
-// Workgroup ids are dealt round-robin to the 8 XCDs; the id is remapped so
-// that the 32 workgroups that run together on one XCD form a block of token
-// tiles x vocabulary ranges and share their slabs in that XCD's L2.
+// Workgroup ids are dealt round-robin to the 8 XCDs.  Token tiles are taken in
+// panels of up to eight, nearly equal in width; within a panel the tiles of a
+// vocabulary range follow each other, and every XCD is given an eighth of this
+// order: the 32 workgroups that run together on it form a block of tiles x ranges
+// and share their slabs in its L2, and no XCD has more of them than another.
+// (In whole blocks of 8 tiles x 4 ranges, a count of tiles that is no multiple of
+// eight left some XCDs with two rounds of workgroups and others with half a one:
+// 2876 tokens x 2560 x 64000 1769 -> 988 us, 6646 x 1024 x 64000 1893 -> 1260,
+// 1292 x 1024 x 64000 364 -> 220, keeping the logits; 8192 x 4096 x 128256 as before.)
 #include <type_traits>
 
 #include "kernels.h"
@@ -86,15 +92,16 @@ __global__ void __launch_bounds__(512) xent_gemm_kernel(const XentParams p) {
   // ---- workgroup id -> (token tile, vocabulary range)
   int t_tile, split;
   {
-    const int id = blockIdx.x;
-    const int xcd = id & 7, slot = id >> 3;
-    const int L = ((slot >> 5) << 8) + (xcd << 5) + (slot & 31);
-    const int bt = p.block_t, bs = 32 / p.block_t;  // block shape, bt a power of two
-    const int blocks_t = (p.tiles_t + bt - 1) / bt;
-    const int blk = L >> 5, in = L & 31;
-    t_tile = (blk % blocks_t) * bt + (in & (bt - 1));
-    split = (blk / blocks_t) * bs + in / bt;
-    if (t_tile >= p.tiles_t || split >= p.n_split) return;
+    const int per_xcd = gridDim.x >> 3;
+    const int at = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    const int panels = (p.tiles_t + 7) >> 3, base = p.tiles_t / panels, wider = p.tiles_t % panels;
+    const int in_wider = wider * (base + 1) * p.n_split;   // workgroups of the panels that are a tile wider
+    const bool w = at < in_wider;
+    const int width = w ? base + 1 : base, rest = w ? at : at - in_wider;
+    const int panel = rest / (width * p.n_split), in = rest % (width * p.n_split);
+    t_tile = (w ? 0 : wider * (base + 1)) + panel * width + in % width;
+    split = in / width;
+    if (t_tile >= p.tiles_t) return;
   }
   const int t0 = t_tile * kXTileT;
   // vocabulary tiles of this range
@@ -656,10 +663,7 @@ int launch_gemm(const XentParams& p, unsigned grid, hipStream_t s) {
 int launch_xent_fwd(const XentParams& p0, int dtype, bool grad, hipStream_t s) {
   XentParams p = p0;
   p.tiles_t = (p.T + kXTileT - 1) / kXTileT;
-  p.block_t = p.tiles_t >= 8 ? 8 : p.tiles_t >= 4 ? 4 : p.tiles_t >= 2 ? 2 : 1;
-  const int bs = 32 / p.block_t;
-  const long long blocks = (long long)((p.tiles_t + p.block_t - 1) / p.block_t) * ((p.n_split + bs - 1) / bs);
-  const unsigned grid = (unsigned)((blocks * 32 + 255) / 256 * 256);
+  const unsigned grid = (unsigned)(((long long)p.tiles_t * p.n_split + 7) / 8 * 8);
   int rc;
   if (dtype == 0)
     rc = grad     ? launch_gemm<__bf16, false, true>(p, grid, s)
