@@ -496,22 +496,33 @@ __global__ void __launch_bounds__(512) xent_gemm_kernel(const XentParams p) {
   }
 }
 
-// lse[t] = log sum over the ranges of exp(lse_part), loss[t] = lse[t] - target logit
+// lse[t] = log sum over the ranges of exp(lse_part), loss[t] = lse[t] - target logit.
+// A wavefront to a token (a thread that walks the ranges of its token by
+// itself waits for memory at every one: 205 tokens, 256 ranges
+// 77 -> 4.4 us, 500, 128 ranges 53 -> 4.6).
 __global__ void __launch_bounds__(256) xent_combine_kernel(const XentParams p) {
-  const int t = blockIdx.x * 256 + threadIdx.x;
+  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (t >= p.T) return;
   const float* lp = p.lse_part + (int64_t)t * p.n_split;
   const float* tp = p.tgt_part + (int64_t)t * p.n_split;
-  float M = -INFINITY;
-  for (int s = 0; s < p.n_split; ++s) M = fmaxf(M, lp[s]);
-  float sum = 0.f, tg = 0.f;
-  for (int s = 0; s < p.n_split; ++s) {
-    sum += exp2f((lp[s] - M) * kLog2e);
+  float M = -INFINITY, sum = 0.f, tg = 0.f;
+  for (int s = lane; s < p.n_split; s += 64) {
+    M = fmaxf(M, lp[s]);
     tg += tp[s];
   }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) M = fmaxf(M, __shfl_xor(M, m, 64));
+  for (int s = lane; s < p.n_split; s += 64) sum += exp2f((lp[s] - M) * kLog2e);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    sum += __shfl_xor(sum, m, 64);
+    tg += __shfl_xor(tg, m, 64);
+  }
   const float lse = M + log2f(sum) * kLn2;
-  p.lse[t] = lse;
-  p.loss[t] = lse - tg;
+  if (lane == 0) {
+    p.lse[t] = lse;
+    p.loss[t] = lse - tg;
+  }
 }
 
 // In place over a [rows, N] block of logits: g = do[t] (exp(logit - lse[t]) - [n == y[t]]).
@@ -674,7 +685,7 @@ int launch_xent_fwd(const XentParams& p0, int dtype, bool grad, hipStream_t s) {
          : p.kept ? launch_gemm<_Float16, true, false>(p, grid, s)
                   : launch_gemm<_Float16, false, false>(p, grid, s);
   if (rc || grad) return rc;
-  hipLaunchKernelGGL(xent_combine_kernel, dim3((unsigned)((p.T + 255) / 256)), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(xent_combine_kernel, dim3((unsigned)((p.T + 3) / 4)), dim3(256), 0, s, p);
   return (int)hipGetLastError();
 }
 
