@@ -509,6 +509,9 @@ typedef struct mi_xent_grad_x_args {
 } mi_xent_grad_x_args;
 
 int mi_xent_grad_x_splits(int64_t tokens, int64_t dim, int64_t vocab, int num_cus);
+/* the same where the result has tiles enough but fills the chip in uneven rounds;
+ * 0: a library product is likely to be faster                               */
+int mi_xent_grad_x_uneven_splits(int64_t tokens, int64_t dim, int64_t vocab, int num_cus);
 size_t mi_xent_grad_x_workspace_bytes(int64_t tokens, int64_t dim, int n_split);
 int mi_xent_grad_x(const mi_xent_grad_x_args *args, void *stream);
 

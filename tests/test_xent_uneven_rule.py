@@ -1,0 +1,25 @@
+"""Where grad_x of many tiles is divided over the vocabulary: the rule's edges."""
+
+import pytest
+
+from tritonops_amd import _lib
+
+
+@pytest.mark.parametrize("tokens,dim,vocab,used", [
+    (2876, 4096, 128256, True),
+    (4100, 2560, 50257, True),
+    (2876, 4096, 32000, False),     # small vocabulary
+    (3072, 4096, 128256, False),    # a multiple of 512
+    (3001, 4096, 128256, False),    # fills one up
+    (6200, 2560, 128256, False),    # 250 of 256 places
+    (1800, 4096, 128256, False),    # 256 narrow tiles
+    (0, 4096, 128256, False),
+    (2876, 0, 128256, False),
+])
+def test_which_results_are_divided(tokens, dim, vocab, used):
+    lib = _lib.load()
+    s = lib.mi_xent_grad_x_uneven_splits(tokens, dim, vocab, 256)
+    assert (s > 0) == used
+    if used:  # the partial sums are no larger than the 16-bit dlogits
+        assert s * tokens * dim * 4 <= tokens * vocab * 2
+        assert lib.mi_xent_grad_x_workspace_bytes(tokens, dim, s) > 0

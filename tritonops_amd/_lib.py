@@ -184,6 +184,7 @@ EXPORTS = {
     "mi_xent_kept_dlogits": (C.c_int, [C.POINTER(XentBwdArgs), _vp, _vp]),
     "mi_xent_kept_dlogits_both": (C.c_int, [C.POINTER(XentBwdArgs), _vp, _vp, _i64, _vp]),
     "mi_xent_grad_x_splits": (C.c_int, [_i64, _i64, _i64, C.c_int]),
+    "mi_xent_grad_x_uneven_splits": (C.c_int, [_i64, _i64, _i64, C.c_int]),
     "mi_xent_grad_x_workspace_bytes": (_sz, [_i64, _i64, C.c_int]),
     "mi_xent_grad_x": (C.c_int, [C.POINTER(XentGradXArgs), _vp]),
     "mi_transpose16": (C.c_int, [_vp, _i64, _i64, _i64, _vp, _i64, _vp]),

@@ -368,6 +368,9 @@ int mi_xent_grad_x_splits(int64_t tokens, int64_t dim, int64_t vocab, int num_cu
   return mi::xent_gradx_splits(tokens, dim, vocab, num_cus);
 }
 
+int mi_xent_grad_x_uneven_splits(int64_t tokens, int64_t dim, int64_t vocab, int num_cus) {
+  return mi::xent_gradx_uneven_splits(tokens, dim, vocab, num_cus);
+}
 size_t mi_xent_grad_x_workspace_bytes(int64_t tokens, int64_t dim, int n_split) {
   return tokens <= 0 || dim <= 0 || n_split <= 0 ? 0 : mi::xent_gradx_bytes(tokens, dim, n_split);
 }

@@ -219,6 +219,7 @@ size_t xent_kept_bytes(long long tokens, long long vocab);
 int launch_xent_kept_dlogits(const XentParams& p, int dtype, hipStream_t s);
 int launch_xent_dlogits(const XentGradParams& p, int dtype, hipStream_t s);
 int xent_gradx_splits(long long tokens, long long dim, long long vocab, int num_cus);
+int xent_gradx_uneven_splits(long long tokens, long long dim, long long vocab, int num_cus);
 size_t xent_gradx_bytes(long long tokens, long long dim, int n_split);
 int launch_xent_gradx(const XentGradXParams& p, int dtype, hipStream_t s);
 // dst[c][r] = src[r][c], 16-bit elements: src [rows, cols] and dst [cols, ld_dst] with 16-byte aligned rows of

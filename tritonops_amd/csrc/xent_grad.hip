@@ -1,6 +1,6 @@
 // grad_x = dlogits w of the fused cross-entropy for gfx950, where the result is
-// too small for its tiles to fill the chip: the vocabulary, which is summed over,
-// is divided among workgroups.
+// too small for its tiles to fill the chip, or fills it in uneven rounds: the
+// vocabulary, which is summed over, is divided among workgroups.
 //
 // A result of T x D has T D / 65536 tiles of 256 x 256 for 256 CUs (1000 x 2560:
 // 40), and the library's product, one workgroup to a tile, takes as long as one
@@ -254,25 +254,64 @@ int launch_t(const XentGradXParams& p, hipStream_t s) {
 
 }  // namespace
 
-// Ranges of the vocabulary: as many as make the estimate of the time least, a
-// round of workgroups being one per CU, a step 1.65 us and a partial result 8
-// bytes of traffic; 0 where the vocabulary is less than a step.
-int xent_gradx_splits(long long tokens, long long dim, long long vocab, int num_cus) {
-  if (tokens <= 0 || dim <= 0 || vocab < kStepN) return 0;
-  if (num_cus <= 0) num_cus = 256;
+namespace {
+// Ranges of the vocabulary that make the estimate of the time least, a round of
+// workgroups being one per CU, a step 1.65 us and a partial result 8 bytes of
+// traffic: the estimate in us and the ranges (at most `most`).
+double best_splits(long long tokens, long long dim, long long vocab, int num_cus, long long most, int* splits) {
   const long long tiles = ((tokens + 255) / 256) * ((dim + 255) / 256);
   const long long pairs = ((vocab + kStepN - 1) / kStepN + 1) / 2;
-  long long best = 1;
   double least = 0.0;
-  for (long long s = 1; s <= pairs && s <= 256 && s * tiles <= 65536; ++s) {
+  *splits = 1;
+  for (long long s = 1; s <= pairs && s <= most && s * tiles <= 65536; ++s) {
     const double rounds = (double)((tiles * s + num_cus - 1) / num_cus);
     const double us = rounds * (double)((pairs + s - 1) / s) * 2 * 1.65 + (double)s * tokens * dim * 8 / 4.5e6;
     if (s == 1 || us < least) {
       least = us;
-      best = s;
+      *splits = (int)s;
     }
   }
-  return (int)best;
+  return least;
+}
+}  // namespace
+
+// Ranges of the vocabulary for a result too small for its tiles to fill the chip;
+// 0 where the vocabulary is less than a step.
+int xent_gradx_splits(long long tokens, long long dim, long long vocab, int num_cus) {
+  if (tokens <= 0 || dim <= 0 || vocab < kStepN) return 0;
+  int s;
+  best_splits(tokens, dim, vocab, num_cus > 0 ? num_cus : 256, 256, &s);
+  return s;
+}
+
+// The same for a result with tiles enough, or 0 where the library's product is
+// left to it.  The library has products at 1.0 to 1.05 times the time of the matrix
+// rate where its tiles of 256 x 256 or 256 x 128 fill whole rounds of the chip to
+// 96 %, and for token counts that fill up a multiple of 512 to 3 %; elsewhere it
+// mostly takes 1.3 to 1.9 times that time, and ranges of the vocabulary even the rounds
+// out.  Library (with w the other way round where that is the rule) -> this, us, at
+// 50257 / 128256 words: 1292 x 4096 741 -> 578 / 1905 -> 1380; 2876 x 2048 799 ->
+// 563 / 2021 -> 1328; 2876 x 4096 1515 -> 1058 / 3891 -> 2599; 3700 x 3072 1520 ->
+// 1039 / 3986 -> 2587; 4100 x 2560 1550 -> 936 / 4054 -> 2289; 4700 x 4096 3109 ->
+// 1783 / 8188 -> 4290.  The mean of 16 token counts from 1292 to 7777 that the rule
+// takes, at 1024 to 4096 columns and 50257 to 128256 words, is 1.45 times as fast;
+// 5 of 160 lose (3900 x 3072 x 50257 929 -> 1056, 4900 x 2048 x 50257 840 -> 894).  Not
+// taken: 6000 x 2048 x 50257 943, here 1057; 6200 x 2560 x 50257 (250 tiles) 1080,
+// here 1280; vocabularies of 32000, where one in five loses (4700 x 2560 594, here
+// 711).  A step of 64 takes the library 1.52 us a round of wide tiles and 0.80 of
+// narrow ones at best; the partial sums are at most as large as the dlogits.
+int xent_gradx_uneven_splits(long long tokens, long long dim, long long vocab, int num_cus) {
+  if (tokens <= 0 || dim <= 0 || vocab < 40000) return 0;
+  if ((512 - tokens % 512) % 512 * 100 <= 3 * tokens) return 0;
+  if (num_cus <= 0) num_cus = 256;
+  const long long tiles = ((tokens + 255) / 256) * ((dim + 255) / 256);
+  const long long wide_rounds = (tiles + num_cus - 1) / num_cus, narrow_rounds = (2 * tiles + num_cus - 1) / num_cus;
+  if (100 * tiles >= 96 * wide_rounds * num_cus || 200 * tiles >= 96 * narrow_rounds * num_cus) return 0;
+  const double steps = (double)((vocab + kStepN - 1) / kStepN);
+  const double wide = 1.52 * steps * (double)wide_rounds, narrow = 0.80 * steps * (double)narrow_rounds;
+  int s;
+  const double us = best_splits(tokens, dim, vocab, num_cus, vocab / (2 * dim), &s);
+  return us > 0.0 && us <= 1.2 * (wide < narrow ? wide : narrow) ? s : 0;
 }
 
 size_t xent_gradx_bytes(long long tokens, long long dim, int n_split) {

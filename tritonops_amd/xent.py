@@ -49,7 +49,8 @@ KEEP_DIM = 1024
 # fit the CUs, grad_x comes from a kernel of this library that divides the vocabulary
 # (the library's product leaves the other CUs idle: 1000 x 2560 x 128256: 1083 -> 604 us,
 # 300 x 1024 x 50257: 158 -> 57, 2000 x 2048 x 32000: 392 -> 242, 64 x 4096 x 128256:
-# 472 -> 253; with 96 tiles, 2000 x 3072, 1381 -> 1407).
+# 472 -> 253; with 96 tiles, 2000 x 3072, 1381 -> 1407), and from 96 tiles on where the
+# library's rounds of the chip are likely to be uneven (mi_xent_grad_x_uneven_splits).
 _SPLIT_ROUNDS, _SPLIT_VOCAB = 3, 8192
 _TURN_ROWS, _TURN_DIM = 256, 1536
 _TURN_X_ROWS, _TURN_X_DIM = 2048, 1024
@@ -288,7 +289,7 @@ def _turns_x(rows, x):
 
 def _turns_w(rows, w):
     """Whether grad_x of a block of `rows` rows sums over a contiguous vocabulary."""
-    return (rows >= _TURN_W_ROWS and -(-rows // 256) * -(-w.shape[1] // 256) >= _TURN_W_TILES
+    return (not _splits_vocab(rows, w) and rows >= _TURN_W_ROWS and -(-rows // 256) * -(-w.shape[1] // 256) >= _TURN_W_TILES
             and w.shape[1] >= _TURN_X_DIM and _can_turn(w))
 
 
@@ -300,7 +301,7 @@ def _splits_vocab(rows, w):
     lib = _lib.load()
     cus = _num_cus(lib)
     if -(-rows // 256) * -(-D // 256) * _SPLIT_ROUNDS > cus:
-        return 0
+        return lib.mi_xent_grad_x_uneven_splits(rows, D, N, cus)
     return lib.mi_xent_grad_x_splits(rows, D, N, cus)
 
 
