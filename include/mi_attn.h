@@ -490,7 +490,8 @@ int mi_xent_kept_dlogits(const mi_xent_bwd_args *args, const void *kept, void *s
 int mi_xent_kept_dlogits_both(const mi_xent_bwd_args *args, const void *kept, void *dlogits_t, int64_t ld_t, void *stream);
 
 /* grad_x [tokens, dim] = dlogits [tokens, vocab] w [vocab, dim], fp32 sums, for
- * results too small to fill the chip with their tiles: the vocabulary is divided
+ * results too small to fill the chip with their tiles, or that fill it in uneven
+ * rounds: the vocabulary is divided
  * into n_split ranges (mi_xent_grad_x_splits picks their number), whose fp32
  * partial tiles go to the workspace and are added up in order.  All bases 16-byte
  * aligned, all strides multiples of 8 elements, ld and w_stride up to 2^22;

@@ -37,7 +37,9 @@ KEEP_DIM = 1024
 # grad_w = dlogits^T x: a transposed x costs little, a second copy of the dlogits, written
 # along with the first, 0.55 us per million.  Both from _TURN_ROWS rows and _TURN_DIM
 # columns on (product before -> after, cost: 8192 x 4096 x 128256: 7.85 -> 5.55, 0.61 ms;
-# 4096 x 2560 x 128256: 2.49 -> 1.90, 0.29; 1000 x 2560 x 50304: 302 -> 249, 29 us), with
+# 4096 x 2560 x 128256: 2.49 -> 1.90, 0.29; 1000 x 2560 x 50304: 302 -> 249, 29 us; forward
+# and both gradients, 100 x 2048 x 32000: 171 -> 165, 205 x 2048 x 128256: 669 -> 623, 150 x
+# 4096 x 50257: 528 -> 469, but 64 x 2048 x 32000: 148 -> 149), with
 # fewer columns the copy costs what it saves (4096 x 1024 x 128256: 1.07 -> 0.82, 0.29 ms)
 # and x alone is turned, from _TURN_X_ROWS rows on (1.07 -> 0.94; 1000 rows: 329 -> 332 us).
 # grad_x = dlogits w: a transposed w costs the same whatever the number of rows: from
@@ -52,7 +54,7 @@ KEEP_DIM = 1024
 # 472 -> 253; with 96 tiles, 2000 x 3072, 1381 -> 1407), and from 96 tiles on where the
 # library's rounds of the chip are likely to be uneven (mi_xent_grad_x_uneven_splits).
 _SPLIT_ROUNDS, _SPLIT_VOCAB = 3, 8192
-_TURN_ROWS, _TURN_DIM = 256, 1536
+_TURN_ROWS, _TURN_DIM = 96, 1536
 _TURN_X_ROWS, _TURN_X_DIM = 2048, 1024
 _TURN_W_ROWS, _TURN_W_TILES = 4096, 128
 # From KEEP_UNASKED bytes in all on, the memory is asked first: kept logits and what the
@@ -287,9 +289,9 @@ def _turns_x(rows, x):
     return both or (rows >= _TURN_X_ROWS and x.shape[1] >= _TURN_X_DIM), both
 
 
-def _turns_w(rows, w):
+def _turns_w(rows, w, may_split=True):
     """Whether grad_x of a block of `rows` rows sums over a contiguous vocabulary."""
-    return (not _splits_vocab(rows, w) and rows >= _TURN_W_ROWS and -(-rows // 256) * -(-w.shape[1] // 256) >= _TURN_W_TILES
+    return (not (may_split and _splits_vocab(rows, w)) and rows >= _TURN_W_ROWS and -(-rows // 256) * -(-w.shape[1] // 256) >= _TURN_W_TILES
             and w.shape[1] >= _TURN_X_DIM and _can_turn(w))
 
 
@@ -381,7 +383,7 @@ def _gradients(x, w, y, lse, g, kept, step, copies):
     _turns_w say so."""
     grad_x = torch.empty_like(x)
     grad_w = w_t = None
-    if copies and _turns_w(min(x.shape[0], step), w):
+    if copies and _turns_w(min(x.shape[0], step), w, grad_x.is_contiguous()):
         w_t = _turn(w, _room_turned(w))[:, :w.shape[0]].t()
     for s in range(0, x.shape[0], step):
         r = slice(s, min(s + step, x.shape[0]))
