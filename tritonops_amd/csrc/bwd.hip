@@ -1293,6 +1293,19 @@ __device__ __forceinline__ KeyUnit key_unit(const LdsKeyPlan& k, const int hkv, 
   return it;
 }
 
+// The kernel's parameters as its argument segment holds them, asked for again by
+// every item.  Kept across the items they are spilled to vector registers, lane by
+// lane (two forms of the item in one kernel: 168 of them, 73 this way), and come back
+// by several hundred v_readlane at every item boundary: dK + dV in the fixed order,
+// 40 sequences of 700 tokens, 8 heads of their own, 153.7 -> 145.6 us; eight of 512
+// 22.0 -> 20.8; one item 11.4 -> 9.8.
+__device__ __forceinline__ const BwdParams& fresh_params() {
+  typedef __attribute__((address_space(4))) const BwdParams c_params;
+  c_params* a = (c_params*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(a));
+  return *(const BwdParams*)a;
+}
+
 // Eight queues (workgroup ids go round-robin to the 8 XCDs): with the kv-head running
 // fastest an XCD keeps to its kv-heads, whose queries and gradients its L2 then holds,
 // whenever the head counts are multiples of eight.
@@ -1337,6 +1350,7 @@ bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt) {
       rt = __builtin_amdgcn_readfirstlane(k.list[round]);
       b = __builtin_amdgcn_readfirstlane(k.list[kMaxRounds + round]);
       h = __builtin_amdgcn_readfirstlane(k.list[2 * kMaxRounds + round]);
+      if (rt < 0) continue;   // (a round without an item)
     }
     auto take_next = [&]() __attribute__((always_inline)) {
       if (dealt && (threadIdx.x & 63) == 0) {
@@ -1345,9 +1359,9 @@ bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt) {
       }
     };
     if (half >= 0)
-      bwd_dkdv_item<T, D, 2>(p, b, h, 2 * rt + half, wave, take_next);
+      bwd_dkdv_item<T, D, 2>(fresh_params(), b, h, 2 * rt + half, wave, take_next);
     else
-      bwd_dkdv_item<T, D, 4>(p, b, h, rt, wave, take_next);
+      bwd_dkdv_item<T, D, 4>(fresh_params(), b, h, rt, wave, take_next);
     __syncthreads();  // the next item's tiles overwrite the staging area
   }
 }
