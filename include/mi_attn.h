@@ -168,6 +168,8 @@ typedef struct mi_attn_bwd_args {
 
 #define MI_ATTN_BWD_QUEUE_BYTES 640
 size_t mi_attn_bwd_workspace_bytes(const mi_attn_bwd_args *args);
+/* queries in a work item of the first launch (dq; the results are the same bits) */
+int mi_attn_bwd_query_rows(int max_seqlen, int batch, int heads_q, int causal, int num_cus);
 int mi_attn_bwd(const mi_attn_bwd_args *args, void *stream);
 
 /* ------------------------------------------------------------------------- */

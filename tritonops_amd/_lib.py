@@ -173,6 +173,7 @@ EXPORTS = {
     "mi_attn_fwd_blocksparse": (C.c_int, [C.POINTER(AttnSparseArgs), _vp]),
     "mi_attn_bwd": (C.c_int, [C.POINTER(AttnBwdArgs), _vp]),
     "mi_attn_bwd_workspace_bytes": (_sz, [C.POINTER(AttnBwdArgs)]),
+    "mi_attn_bwd_query_rows": (C.c_int, [C.c_int] * 5),
     "mi_attn_bwd_validate": (C.c_int, [C.POINTER(AttnBwdArgs)]),
     "mi_rmsnorm_fwd": (C.c_int, [C.POINTER(RmsNormArgs), _vp]),
     "mi_rmsnorm_bwd": (C.c_int, [C.POINTER(RmsNormArgs), _vp]),

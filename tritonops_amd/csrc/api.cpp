@@ -468,6 +468,10 @@ int mi_xent_dlogits(const mi_xent_grad_args* a, void* stream) {
   return launch_status(mi::launch_xent_dlogits(p, a->dtype, static_cast<hipStream_t>(stream)), "mi_xent_dlogits");
 }
 
+int mi_attn_bwd_query_rows(int max_seqlen, int batch, int heads_q, int causal, int num_cus) {
+  return mi::bwd_dq_short_items(max_seqlen, batch, heads_q, causal != 0, num_cus) ? 128 : 256;
+}
+
 static_assert(MI_ATTN_BWD_QUEUE_BYTES >= mi::kBwdQueueBytes + 127, "queues on a 128-byte boundary");
 
 int mi_attn_bwd_validate(const mi_attn_bwd_args* a) {

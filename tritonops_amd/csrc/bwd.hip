@@ -1412,20 +1412,30 @@ int launch_dkdv(const BwdParams& p0, hipStream_t s) {
 
 template <typename T, int D>
 int launch_all(const BwdParams& p, hipStream_t s) {
-  // dQ first: it also writes Delta, which the dK + dV kernel reads.
-  // Items of 128 queries, a wavefront to a SIMD, where they are at most one round of workgroups, or two of a causal
-  // call (its second round is of short items): a tile of 64 keys then takes 1.5 instead of 2.1 us, and the longest
-  // chain bounds the launch.  256 -> 128 rows, head_dim 128: 1000 tokens, 16 heads 40 -> 29 us; 2048, 32 heads (two
-  // rounds) 82 -> 66; 4096, 16 heads 135 -> 108; 8192, 8 heads 255 -> 195; eight of 512, 8 heads 28 -> 23; head_dim 64,
-  // 2400, 16 heads 56 -> 36.  Beyond: three of 300 to 1100, 32 heads (2.3 rounds) 48 -> 57, 4096, 32 heads (four) 191 -> 208.
-  int rc;
-  const long long halves = (long long)((p.max_seqlen + 127) / 128) * p.hq * p.batch;
-  const bool few = halves <= (p.causal ? 2 : 1) * (long long)device_cu_count();
-  if ((rc = few ? launch_dq<T, D, 4>(p, s) : launch_dq<T, D, 8>(p, s))) return rc;
+  // dQ first: it also writes Delta, which the dK + dV kernel reads
+  const bool short_items = bwd_dq_short_items(p.max_seqlen, p.batch, p.hq, p.causal, device_cu_count());
+  if (const int rc = short_items ? launch_dq<T, D, 4>(p, s) : launch_dq<T, D, 8>(p, s)) return rc;
   return launch_dkdv<T, D>(p, s);
 }
 
 }  // namespace
+
+// dQ's items of 128 queries, a wavefront to a SIMD, in place of 256, where a launch has few of them: a tile of 64
+// keys then takes 1.5 instead of 2.1 us, and the longest chain bounds the launch.  In one round of workgroups they
+// are never slower from 129 tokens on (1000 tokens, 16 heads 40 -> 29 us; 4096, 8 heads 135 -> 108); up to 128 both
+// forms have the same items, which eight wavefronts load sooner than four (128 tokens, 16 to 256 items, 1.3 to 1.8
+// us).  In the two rounds of a causal call, the second of short items, the gain of 0.53 us a tile of the longest
+// chain has to pay for what 256 rows do without: the second round's boundary and the order of the items by
+// level, 0.05 us per (sequence, tile) pair of a head.  2048, 32 heads 82 -> 66; 4096, 16 heads 135 -> 108; three of 1354, 8
+// heads 92 -> 79 with dK + dV; but 64 of 256, 4 heads, dQ alone 26 -> 43, 24 of 384, 4 heads 24 -> 32, 40 of 700,
+// 2 heads 35 -> 50.  Of 163 measured launches of two rounds this takes 54, 1.10 times as fast in the mean with dK +
+// dV, one of them 3 % slower (six of 1105, 8 heads); 42 it leaves would gain 2 to 21 %.  Beyond two rounds: 4096, 32 heads (four) 191 -> 208.
+bool bwd_dq_short_items(int max_seqlen, int batch, int heads_q, bool causal, int num_cus) {
+  if (num_cus <= 0) num_cus = 256;
+  const long long pairs = (long long)((max_seqlen + 127) / 128) * batch, items = pairs * heads_q;
+  if (max_seqlen <= 128 || items > (causal ? 2 : 1) * (long long)num_cus) return false;
+  return items <= num_cus || 53LL * ((max_seqlen + 63) / 64) >= 120 + 5 * pairs + 300 * items / num_cus;
+}
 
 int launch_attn_bwd(const BwdParams& p, int dtype, int head_dim, hipStream_t s) {
   if (dtype == 0) {

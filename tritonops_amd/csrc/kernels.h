@@ -196,6 +196,7 @@ int launch_decode_merge(const DecodeParams& p, int dtype, int head_dim, hipStrea
 constexpr unsigned kDecodeScratchBytes = 32u << 20;
 int decode_static_scratch(void** ptr);
 constexpr size_t kBwdQueueBytes = 8 * 64;
+bool bwd_dq_short_items(int max_seqlen, int batch, int heads_q, bool causal, int num_cus);
 // the dQ kernel (which also writes Delta), then the dK + dV kernel
 int launch_attn_bwd(const BwdParams& p, int dtype, int head_dim, hipStream_t s);
 // RMSNorm.  x_dtype: 0 bf16, 1 f16, 2 f32; w_dtype: x_dtype or 2.  `vec`: rows
