@@ -50,6 +50,46 @@ def test_dealt_units_equal_fixed_order(lens, Hq, Hkv, D, dt, causal, monkeypatch
         assert torch.equal(a, c) and torch.equal(b, c), name
 
 
+@pytest.mark.parametrize("lens,Hq,Hkv,causal", [(c[0], c[1], c[2], c[5]) for c in CASES] + [
+    ([60] * 64, 2, 2, True), ([128] * 32, 4, 4, True), ([512] * 8, 8, 8, True), ([1024] * 2, 16, 16, True),  # halves gain too little
+    ([65] * 3, 8, 1, True), ([64] * 3, 8, 1, True), ([512] * 4, 8, 8, True), ([512] * 8, 16, 16, True),
+    ([300, 700, 20], 6, 6, True), ((2, 500), 8, 8, True), ((1, 4096), 8, 2, False), ([3000] * 43, 4, 1, True),
+    ([R.randint(0, 900) for _ in range(37)], 12, 6, True), ([R.randint(0, 5000) for _ in range(6)], 4, 2, True),
+])
+def test_units_taken_at_run_time(lens, Hq, Hkv, causal, monkeypatch):
+    """The counters after a call: a workgroup takes another unit for each that it works on, so their sum is the
+    number of units of the plan (which levels are halved with it), and zero in the fixed order."""
+    import tritonops_amd as ta
+    from tests.key_units import MAX_BATCH, MAX_LEVELS, Plan
+    from tritonops_amd import _lib, ops
+
+    if isinstance(lens, tuple):
+        cu, shape, lens = None, lens, [lens[1]] * lens[0]
+    else:
+        cu, shape = cu_from(torch.tensor(lens, dtype=torch.int32)).cuda(), (1, sum(lens))
+    q, k, v, do = (randn((*shape, h, 64), 1 + i, torch.bfloat16).cuda() for i, h in enumerate((Hq, Hkv, Hkv, Hq)))
+    o, lse = ops._general_fwd(q, k, v, cu, 0.125 * ta.LOG2E, causal, None, True, False)
+    made = []
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: made.append(empty(*a, **kw)) or made[-1])
+    ops._general_bwd(q, k, v, o, do, lse, cu, 0.125 * ta.LOG2E, causal, None)
+    torch.cuda.synchronize()
+    ws = [t for t in made if t.dtype == torch.uint8]
+    assert len(ws) == 1 and ws[0].data_ptr() % 128 == 0
+    delta = -(-4 * len(lens) * Hq * max(lens) // 128) * 128
+    assert ws[0].numel() >= delta + 512
+    taken = ws[0][delta:delta + 512].view(torch.int32)[::16].cpu()
+    cus = _lib.load().mi_device_cu_count()
+    if len(lens) > MAX_BATCH or -(-max(lens) // 128) > MAX_LEVELS:
+        want = 0
+    else:
+        # (a launch of few items has two workgroups to each)
+        items = -(-max(lens) // 128) * len(lens) * Hkv
+        p = Plan(lens, Hq, Hkv, causal, min(-(-2 * items // 8) * 8, cus) if items <= cus else cus)
+        want = p.units() if p.dealt else 0
+    assert int(taken.sum()) == want, taken
+
+
 @pytest.mark.parametrize("lens,H,D,dt,causal", [
     ([127, 128, 129, 255, 256, 257, 383, 1, 0, 65], 40, 128, torch.bfloat16, True),
     ([2100], 64, 96, torch.float16, True),

@@ -1158,8 +1158,7 @@ constexpr uint32_t kDkdvLds = kDqLds + 2 * 4 * 2 * 2048;  // tile ring + P excha
 // either way: the results are the same bits.  dK + dV, fixed whole items -> this,
 // head_dim 128: 1000 tokens, 4 kv-heads of 4 94 -> 68 us; 2048, 2 of 8 315 -> 216;
 // 4096, 8 of 4 352 -> 292; 16384, 2 of 4 1362 -> 1137; five of 517 to 3400, 8 of 4
-// 384 -> 332; 8192, 8 of 4 (two even rounds, none halved) 967 -> 954.  Looking the
-// units up costs a launch 3 us: eight of 512, 8 of 1 20 -> 24.
+// 384 -> 332; 8192, 8 of 4 (two even rounds, none halved) 967 -> 954.
 // Cost model, in hundredths of a microsecond, of n tiles:
 constexpr int kFullTile = 175, kHalfTile = 100, kUnitFixed = 700;
 static_assert(kFullTile * 4 == kHalfTile * 7, "key_units_before() orders the units by 4 : 7");
@@ -1168,6 +1167,8 @@ static_assert(kMaxLevels < 1024, "plan_key_units() packs a level into ten bits")
 // Items per workgroup from which the fixed order is even enough (one sequence of 8192, 16 heads of their own, two
 // rounds: 128 us in either) and keeps neighbours together in an L2.
 constexpr int kDealtRounds = 4;
+// In one round: tiles of the longest chain, and how much of it has to be idle (plan_key_units()).
+constexpr int kHalvedTiles = 7, kHalvedIdle = 160;
 
 // In LDS, behind the tiles and the P exchange.
 struct KeyPlan {
@@ -1176,7 +1177,7 @@ struct KeyPlan {
   int weight[kMaxLevels + 1];       // the same, pairs weighted with their level + 1
   int tiles[kLevelMaxBatch];
   int top;                           // levels, rounded up to a wavefront's lanes; at_or_above[top] = 0
-  int split_from, pairs, dealt;      // levels that are halved; (sequence, tile or half) pairs; whether units are dealt at run time
+  int split_from, dealt;             // first of the levels that are halved; whether units are dealt at run time
   int next[2];                       // unit of the next round, by parity
 };
 
@@ -1194,38 +1195,74 @@ __device__ __forceinline__ int key_units_before(const LdsKeyPlan& k, const int t
   return k.at_or_above[t + 1] - k.at_or_above[T] + 2 * k.at_or_above[min(first, k.top)];
 }
 
-// By one wavefront: the levels, and which of them are halved.  The estimate that is
-// minimised is the longer of the longest unit and the mean load plus a quarter of a mean unit.
+// By one wavefront: whether the units are dealt out, and then the levels and which of them are halved.  The
+// estimate that is minimised is the longer of the longest unit and the mean load plus a quarter of a mean unit.
+//
+// What this costs is 2.3 us of the launch whatever the number of sequences (looked through one after another they
+// cost another 0.17 us each: 64 of 60 tokens, 2 heads, dK + dV 24.0 -> 12.9).  Where every whole item has a workgroup
+// to itself only the halves can pay for it, and only where workgroups are idle for much of the longest item: from
+// a chain of seven tiles on, where the mean load is 1.6 us less than six tenths of the longest item.  With dQ, whole
+// items -> this: chains of four tiles 30.2 -> 30.4 us, of eight 40.2 -> 38.5, of sixteen 58.2 -> 53.0; with every CU at
+// work, two of 1024, 16 heads (mean 0.65) 62.7 -> 64.7; eight of 77 to 512, 8 heads (0.53, a chain of eight)
+// 43.8 -> 45.8; 40 of 700, one kv-head of 8 (0.56, of 96) 254.8 -> 253.8; one of 4096, 8 of 4 (0.52) 540 -> 483.
 __device__ __forceinline__ void plan_key_units(LdsKeyPlan& k, const BwdParams& p, const int grid) {
   const int lane = threadIdx.x & 63;
-  int tiles = 0;
-  if (lane < p.batch) {
-    const int len = p.cu ? min(p.cu[lane + 1] - p.cu[lane], p.max_seqlen) : p.max_seqlen;
-    tiles = len > 0 ? (len + 127) / 128 : 0;
+  int tokens = 0;
+  if (lane < p.batch) tokens = max(p.cu ? min(p.cu[lane + 1] - p.cu[lane], p.max_seqlen) : p.max_seqlen, 0);
+  const int tiles = (tokens + 127) / 128;
+  int most = tokens, all = tiles, all_w = tiles * (tiles + 1) / 2;   // tokens of the longest; pairs, and their weights
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    most = max(most, __shfl_xor(most, m, 64));
+    all += __shfl_xor(all, m, 64);
+    all_w += __shfl_xor(all_w, m, 64);
   }
-  k.tiles[lane] = tiles;
-  int levels = 0;
-  for (int b = 0; b < p.batch; ++b) levels = max(levels, __builtin_amdgcn_readlane(tiles, b));
+  most = __builtin_amdgcn_readfirstlane(most);
+  all = __builtin_amdgcn_readfirstlane(all);
+  all_w = __builtin_amdgcn_readfirstlane(all_w);
+  const int levels = (most + 127) / 128;   // of the longest sequence
+  const float unit = 2.f * (p.hq / p.hkv);   // tiles of 64 queries of a level-0 item
+  const bool one_round = all * p.hkv <= grid;
+  const float whole_item = kFullTile * unit * levels + kUnitFixed;   // the longest
+  bool dealt = all * p.hkv < kDealtRounds * grid;
+  if (!p.causal) dealt = 2 * all * p.hkv <= grid;   // (every item of a sequence is as long as the next: all of them are halved or none)
+  if (one_round) {
+    const float mean = (float)p.hkv * (kFullTile * unit * all_w + kUnitFixed * all) / (float)grid;
+    dealt = dealt && unit * levels >= kHalvedTiles && most > 64;   // (up to 64 tokens the second half has no keys)
+    if (p.causal) dealt = dealt && mean + kHalvedIdle <= 0.6f * whole_item;
+  }
+  if (lane == 0) k.dealt = dealt;
+  if (!dealt) return;
+
+  // from the last level down: sequences that reach a level, and the sums over it and the levels above
   const int top = (levels + 63) / 64 * 64;
-  int above = 0, above_w = 0;        // all pairs, all weights
-  for (int b = 0; b < p.batch; ++b) {
-    const int all = __builtin_amdgcn_readlane(tiles, b);
-    above += all;
-    above_w += all * (all + 1) / 2;
-  }
-  for (int t = lane; t <= top; t += 64) {
-    int n = 0, w = 0;
-    for (int b = 0; b < p.batch; ++b) {
-      const int all = __builtin_amdgcn_readlane(tiles, b);
-      if (all > t) n += all - t, w += (all * (all + 1) - t * (t + 1)) / 2;
+  for (int t = lane; t <= top; t += 64) k.weight[t] = 0;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // lanes read and add to what other lanes have written
+  __hip_atomic_fetch_add(&k.weight[tiles], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+  k.tiles[lane] = tiles;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  auto from_here_on = [&](int v) __attribute__((always_inline)) -> int {   // sum over this lane and those behind it
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int o = __shfl_down(v, d, 64);
+      v += lane + d < 64 ? o : 0;
     }
+    return v;
+  };
+  int reach = __builtin_amdgcn_readfirstlane(k.weight[top]), above = 0, above_w = 0;
+  if (lane == 0) k.at_or_above[top] = k.weight[top] = 0;
+  for (int base = top - 64; base >= 0; base -= 64) {
+    const int t = base + lane, ends = k.weight[t];
+    const int at_least = reach + from_here_on(ends);        // sequences of t tiles and more
+    const int n = above + from_here_on(at_least - ends), w = above_w + from_here_on((t + 1) * (at_least - ends));
     k.at_or_above[t] = n;
     k.weight[t] = w;
+    reach = __builtin_amdgcn_readfirstlane(at_least);
+    above = __builtin_amdgcn_readfirstlane(n);
+    above_w = __builtin_amdgcn_readfirstlane(w);
   }
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // lanes read what other lanes have written
-  const int gqa = p.hq / p.hkv;
-  const float unit = 2.f * gqa;      // tiles of 64 queries of a level-0 item
-  int T = levels;                    // halved from here on
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  int T = 0;                         // halved from here on
   if (p.causal) {
     // (the estimate and the level in one word, the larger level among equals: one reduction)
     uint32_t best = ~0u;
@@ -1246,16 +1283,11 @@ __device__ __forceinline__ void plan_key_units(LdsKeyPlan& k, const BwdParams& p
     }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) best = min(best, (uint32_t)__shfl_xor((int)best, m, 64));
-    T = 1023 - (int)(best & 1023u);
-  } else if (2 * above * p.hkv <= grid) {
-    T = 0;                           // (every item of a sequence is as long as the next: all of them or none)
+    T = __builtin_amdgcn_readfirstlane(1023 - (int)(best & 1023u));
   }
-  T = __builtin_amdgcn_readfirstlane(T);
   if (lane == 0) {
     k.top = top;
     k.split_from = T;
-    k.pairs = above + k.at_or_above[T];
-    k.dealt = (p.causal ? above * p.hkv < kDealtRounds * grid : T == 0);
   }
 }
 
@@ -1404,6 +1436,7 @@ int launch_dkdv(const BwdParams& p0, hipStream_t s) {
   const int cus = device_cu_count();
   long long grid = persistent_grid(items, cus);  // one workgroup per CU is resident (LDS)
   if (p.batch > kLevelMaxBatch || n_rt > kMaxLevels || (!p.cu && items >= kDealtRounds * (long long)cus)) p.queue = nullptr;
+  if (items <= cus && (2 * (p.hq / p.hkv) * n_rt < kHalvedTiles || p.max_seqlen <= 64)) p.queue = nullptr;   // (as plan_key_units() would say)
   if (p.queue && items <= cus) grid = std::min((2 * items + 7) / 8 * 8, (long long)cus);  // each half a workgroup of its own
   p.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
   hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items, n_rt);
