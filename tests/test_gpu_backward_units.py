@@ -26,6 +26,7 @@ CASES = [
     ((3, 150), 3, 1, 96, torch.float16, False),
     ((8, 1000), 64, 64, 64, torch.bfloat16, False),                                                # no mask, many items: fixed order
     ([66000], 1, 1, 64, torch.bfloat16, True),                                                     # more levels than the plan holds
+    ([8192] + [100] * 63, 8, 8, 64, torch.bfloat16, True),                                         # ids for two generations of workgroups
 ]
 
 
@@ -55,6 +56,7 @@ def test_dealt_units_equal_fixed_order(lens, Hq, Hkv, D, dt, causal, monkeypatch
     ([65] * 3, 8, 1, True), ([64] * 3, 8, 1, True), ([512] * 4, 8, 8, True), ([512] * 8, 16, 16, True),
     ([300, 700, 20], 6, 6, True), ((2, 500), 8, 8, True), ((1, 4096), 8, 2, False), ([3000] * 43, 4, 1, True),
     ([R.randint(0, 900) for _ in range(37)], 12, 6, True), ([R.randint(0, 5000) for _ in range(6)], 4, 2, True),
+    ([4096] + [100] * 63, 16, 16, True),   # two generations by the ids, four rounds of one by the items that exist
 ])
 def test_units_taken_at_run_time(lens, Hq, Hkv, causal, monkeypatch):
     """The counters after a call: a workgroup takes another unit for each that it works on, so their sum is the

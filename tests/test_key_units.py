@@ -34,7 +34,7 @@ def test_every_unit_once_and_the_longest_first():
 
 # of CASES, in their order: dealt, halved levels out of all levels; None: more sequences or levels than the plan holds
 PLANS = [(True, (1, 2)), (True, (2, 27)), (True, (11, 32)), (True, (0, 67)), (True, (0, 6)), None, (True, (8, 8)),
-         (False, None), (True, (7, 16)), (True, (2, 2)), (False, None), None]
+         (False, None), (True, (7, 16)), (True, (2, 2)), (False, None), None, (True, (0, 64))]
 
 
 @pytest.mark.parametrize("case,want", list(zip(CASES, PLANS)))
@@ -58,6 +58,7 @@ def test_plans_of_the_device_test(case, want):
     ([512] * 8, 32, 8, False), ([4096], 32, 8, True), ([2048], 16, 2, True),
     ([512] * 8, 16, 16, True),                                                                                  # more than a round
     ([3000] * 43, 4, 1, False), ([3000] * 42, 4, 1, True),                                                      # four rounds
+    ([4096] + [100] * 63, 16, 16, False), ([4096] + [100] * 63, 10, 10, True),
 ])
 def test_which_launches_deal_their_units(lens, heads, heads_kv, dealt):
     assert Plan(lens, heads, heads_kv).dealt == dealt

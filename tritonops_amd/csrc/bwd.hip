@@ -1205,7 +1205,7 @@ __device__ __forceinline__ int key_units_before(const LdsKeyPlan& k, const int t
 // items -> this: chains of four tiles 30.2 -> 30.4 us, of eight 40.2 -> 38.5, of sixteen 58.2 -> 53.0; with every CU at
 // work, two of 1024, 16 heads (mean 0.65) 62.7 -> 64.7; eight of 77 to 512, 8 heads (0.53, a chain of eight)
 // 43.8 -> 45.8; 40 of 700, one kv-head of 8 (0.56, of 96) 254.8 -> 253.8; one of 4096, 8 of 4 (0.52) 540 -> 483.
-__device__ __forceinline__ void plan_key_units(LdsKeyPlan& k, const BwdParams& p, const int grid) {
+__device__ __forceinline__ void plan_key_units(LdsKeyPlan& k, const BwdParams& p, const int workers) {
   const int lane = threadIdx.x & 63;
   int tokens = 0;
   if (lane < p.batch) tokens = max(p.cu ? min(p.cu[lane + 1] - p.cu[lane], p.max_seqlen) : p.max_seqlen, 0);
@@ -1222,12 +1222,12 @@ __device__ __forceinline__ void plan_key_units(LdsKeyPlan& k, const BwdParams& p
   all_w = __builtin_amdgcn_readfirstlane(all_w);
   const int levels = (most + 127) / 128;   // of the longest sequence
   const float unit = 2.f * (p.hq / p.hkv);   // tiles of 64 queries of a level-0 item
-  const bool one_round = all * p.hkv <= grid;
+  const bool one_round = all * p.hkv <= workers;
   const float whole_item = kFullTile * unit * levels + kUnitFixed;   // the longest
-  bool dealt = all * p.hkv < kDealtRounds * grid;
-  if (!p.causal) dealt = 2 * all * p.hkv <= grid;   // (every item of a sequence is as long as the next: all of them are halved or none)
+  bool dealt = all * p.hkv < kDealtRounds * workers;
+  if (!p.causal) dealt = 2 * all * p.hkv <= workers;   // (every item of a sequence is as long as the next: all of them are halved or none)
   if (one_round) {
-    const float mean = (float)p.hkv * (kFullTile * unit * all_w + kUnitFixed * all) / (float)grid;
+    const float mean = (float)p.hkv * (kFullTile * unit * all_w + kUnitFixed * all) / (float)workers;
     dealt = dealt && unit * levels >= kHalvedTiles && most > 64;   // (up to 64 tokens the second half has no keys)
     if (p.causal) dealt = dealt && mean + kHalvedIdle <= 0.6f * whole_item;
   }
@@ -1275,8 +1275,8 @@ __device__ __forceinline__ void plan_key_units(LdsKeyPlan& k, const BwdParams& p
                                             kFullTile * unit * ((float)above_w - w) + kUnitFixed * whole);
         float longest = t > 0 ? kFullTile * unit * t + kUnitFixed : 0.f;
         if (t < levels) longest = fmaxf(longest, kHalfTile * unit * levels + kUnitFixed);
-        float est = total / (float)grid;
-        if (units * (float)p.hkv > (float)grid) est += 0.25f * total / (units * (float)p.hkv);
+        float est = total / (float)workers;
+        if (units * (float)p.hkv > (float)workers) est += 0.25f * total / (units * (float)p.hkv);
         est = fmaxf(est, longest);
         best = min(best, (__builtin_bit_cast(uint32_t, est) & ~1023u) | (uint32_t)(1023 - t));
       }
@@ -1343,18 +1343,22 @@ __device__ __forceinline__ const BwdParams& fresh_params() {
 // whenever the head counts are multiples of eight.
 template <typename T, int D>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
-bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt) {
+bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt, const int resident) {
   LdsKeyPlan& k = *(LdsKeyPlan*)(uintptr_t)((uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd) + kDkdvLds);
   const int grid = gridDim.x;
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  const int queues = (grid & 7) == 0 ? 8 : 1;
+  // Units are dealt to the workgroups that run at once.  Where the ids of a ragged batch make several generations of
+  // them (persistent_grid()), the others would come to units that were meant to be first when the queues are empty.
+  const int workers = min(grid, resident);
+  const int queues = (workers & 7) == 0 ? 8 : 1;
   const int queue = queues == 8 ? blockIdx.x & 7 : 0;
   const int first = queues == 8 ? (int)(blockIdx.x >> 3) : (int)blockIdx.x;
   bool dealt = false;
   if (p.queue) {
-    if (wave == 0) plan_key_units(k, p, grid);
+    if (wave == 0) plan_key_units(k, p, workers);
     __syncthreads();
     dealt = __builtin_amdgcn_readfirstlane(k.dealt);
+    if (dealt && (int)blockIdx.x >= workers) return;
   }
   if (!dealt) {
     if (wave == 0) {
@@ -1387,7 +1391,7 @@ bwd_dkdv_kernel(const BwdParams p, const int n_items, const int n_rt) {
     auto take_next = [&]() __attribute__((always_inline)) {
       if (dealt && (threadIdx.x & 63) == 0) {
         const int n = __hip_atomic_fetch_add(p.queue + 16 * queue, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        k.next[(round + 1) & 1] = (n + grid / queues) * queues + queue;
+        k.next[(round + 1) & 1] = (n + workers / queues) * queues + queue;
       }
     };
     if (half >= 0)
@@ -1439,7 +1443,7 @@ int launch_dkdv(const BwdParams& p0, hipStream_t s) {
   if (items <= cus && (2 * (p.hq / p.hkv) * n_rt < kHalvedTiles || p.max_seqlen <= 64)) p.queue = nullptr;   // (as plan_key_units() would say)
   if (p.queue && items <= cus) grid = std::min((2 * items + 7) / 8 * 8, (long long)cus);  // each half a workgroup of its own
   p.by_level = number_by_level(p.cu, p.causal, p.batch, items, grid);
-  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items, n_rt);
+  hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(512), lds, s, p, (int)items, n_rt, cus);
   return (int)hipGetLastError();
 }
 
