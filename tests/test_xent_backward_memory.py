@@ -142,6 +142,28 @@ def test_the_bytes_asked_for_cover_what_is_allocated(monkeypatch):
     assert asked(300, 1536, 8192) == 300 * 8192 * 2 + 300 * (1536 + 8192) * 2 + 2 * 6 * n_split * 65536 * 4
 
 
+@pytest.mark.parametrize("layout", ["rows", "columns", "padded_rows"])
+def test_weights_are_turned_where_the_layout_of_grad_x_keeps_the_vocabulary_whole(on_cpu, monkeypatch, layout):
+    """The divided product writes whole rows of grad_x, which has x's strides: where it cannot, w is turned as the
+    rules say, and its copy is in what the memory is asked for."""
+    go, x, w, y, lse = _problem(600, 1536, 72)
+    x = {"rows": x, "columns": x.t().contiguous().t(), "padded_rows": torch.cat((x, x), 1)[:, :1536]}[layout]
+    whole = layout == "columns"
+    assert torch.empty_like(x).is_contiguous() is not whole
+    monkeypatch.setattr(xent, "_TURN_W_ROWS", 256)
+    monkeypatch.setattr(xent, "_TURN_W_TILES", 1)
+    monkeypatch.setattr(xent, "_splits_vocab", lambda rows, w: 2)
+    divided, made = [], []
+    room = xent._room_turned
+    monkeypatch.setattr(xent, "_room_turned", lambda t: made.append(tuple(t.shape)) or room(t))
+    monkeypatch.setattr(xent, "_grad_x", lambda dl, w, out, n: divided.append(n) or out.copy_(dl.double() @ w.double()) is out)
+    _check(xent._bwd(go, x, w, y, lse, None, 600), go, x, w, y)
+    assert (made, divided) == (([(72, 1536)], []) if whole else ([(600, 1536), (600, 72)], [2]))
+    assert xent._copy_bytes(600, x, w) == 2 * sum(a * b for a, b in made)
+    split = 0 if whole else xent._lib.load().mi_xent_grad_x_workspace_bytes(600, 1536, 2)
+    assert xent._bwd_bytes(x, w) == 2 * 600 * 72 + xent._copy_bytes(600, x, w) + split
+
+
 def test_without_memory_for_the_partial_sums_the_library_multiplies(on_cpu, monkeypatch):
     go, x, w, y, lse = _problem(90, 136, 200)
     asked = []

@@ -289,10 +289,17 @@ def _turns_x(rows, x):
     return both or (rows >= _TURN_X_ROWS and x.shape[1] >= _TURN_X_DIM), both
 
 
-def _turns_w(rows, w, may_split=True):
+def _turns_w(rows, x, w):
     """Whether grad_x of a block of `rows` rows sums over a contiguous vocabulary."""
-    return (not (may_split and _splits_vocab(rows, w)) and rows >= _TURN_W_ROWS and -(-rows // 256) * -(-w.shape[1] // 256) >= _TURN_W_TILES
-            and w.shape[1] >= _TURN_X_DIM and _can_turn(w))
+    return (rows >= _TURN_W_ROWS and -(-rows // 256) * -(-w.shape[1] // 256) >= _TURN_W_TILES
+            and w.shape[1] >= _TURN_X_DIM and _can_turn(w) and not _splits(rows, x, w))
+
+
+def _splits(rows, x, w):
+    """_splits_vocab, for a grad_x with the strides that it takes from x: the kernel writes whole rows."""
+    if not (x.is_contiguous() or torch.empty_like(x, device="meta").is_contiguous()):
+        return 0
+    return _splits_vocab(rows, w)
 
 
 def _splits_vocab(rows, w):
@@ -329,7 +336,7 @@ def _grad_x(dl, w, out, n_split):
 def _copy_bytes(rows, x, w):
     """What the operands that blocks of `rows` rows take the other way round occupy."""
     turn_x, turn_dl = _turns_x(rows, x)
-    n = rows * (turn_x * x.shape[1] + turn_dl * w.shape[0]) + _turns_w(rows, w) * w.numel()
+    n = rows * (turn_x * x.shape[1] + turn_dl * w.shape[0]) + _turns_w(rows, x, w) * w.numel()
     return n * x.element_size()
 
 
@@ -349,7 +356,7 @@ def _makes_copies(rows, x, w, kept):
 def _bwd_bytes(x, w):
     """What the backward allocates for its dlogits and products at a time."""
     rows = min(x.shape[0], BWD_ROWS)
-    n_split = _splits_vocab(rows, w)
+    n_split = _splits(rows, x, w)
     split = _lib.load().mi_xent_grad_x_workspace_bytes(rows, w.shape[1], n_split) if n_split else 0
     return rows * w.shape[0] * x.element_size() + _copy_bytes(rows, x, w) + split
 
@@ -383,7 +390,7 @@ def _gradients(x, w, y, lse, g, kept, step, copies):
     _turns_w say so."""
     grad_x = torch.empty_like(x)
     grad_w = w_t = None
-    if copies and _turns_w(min(x.shape[0], step), w, grad_x.is_contiguous()):
+    if copies and _turns_w(min(x.shape[0], step), x, w):
         w_t = _turn(w, _room_turned(w))[:, :w.shape[0]].t()
     for s in range(0, x.shape[0], step):
         r = slice(s, min(s + step, x.shape[0]))
