@@ -23,3 +23,17 @@ def test_which_results_are_divided(tokens, dim, vocab, used):
     if used:  # the partial sums are no larger than the 16-bit dlogits
         assert s * tokens * dim * 4 <= tokens * vocab * 2
         assert lib.mi_xent_grad_x_workspace_bytes(tokens, dim, s) > 0
+
+
+def test_partial_sums_are_no_larger_than_the_dlogits():
+    """As the workspace holds them, in whole tiles of 256 x 256: token counts and columns a little past a tile among
+    them (1548 x 3136 x 50257 had 8 ranges, 1.23 times the dlogits)."""
+    lib = _lib.load()
+    some = 0
+    for tokens in (1292, 1548, 1793, 2049, 2876, 4100, 5121, 7777):
+        for dim in (1032, 2048, 2312, 2568, 3136, 4096, 5128):
+            for vocab in (40000, 50257, 128256):
+                s = lib.mi_xent_grad_x_uneven_splits(tokens, dim, vocab, 256)
+                some += s > 1
+                assert lib.mi_xent_grad_x_workspace_bytes(tokens, dim, s) <= 2 * tokens * vocab, (tokens, dim, vocab, s)
+    assert some > 20

@@ -310,8 +310,9 @@ int xent_gradx_uneven_splits(long long tokens, long long dim, long long vocab, i
   const double steps = (double)((vocab + kStepN - 1) / kStepN);
   const double wide = 1.52 * steps * (double)wide_rounds, narrow = 0.80 * steps * (double)narrow_rounds;
   int s;
-  const double us = best_splits(tokens, dim, vocab, num_cus, vocab / (2 * dim), &s);
-  return us > 0.0 && us <= 1.2 * (wide < narrow ? wide : narrow) ? s : 0;
+  const long long most = 2 * tokens * vocab / (long long)xent_gradx_bytes(tokens, dim, 1);
+  const double us = best_splits(tokens, dim, vocab, num_cus, most, &s);
+  return most > 0 && us <= 1.2 * (wide < narrow ? wide : narrow) ? s : 0;
 }
 
 size_t xent_gradx_bytes(long long tokens, long long dim, int n_split) {
