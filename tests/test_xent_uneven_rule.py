@@ -15,9 +15,9 @@ from tritonops_amd import _lib
     (1800, 4096, 128256, False),    # 256 narrow tiles
     (3900, 3072, 50257, False), (3851, 3072, 50257, False), (5959, 2048, 44032, False), (4646, 2560, 40000, False),  # one round of tiles of 192
     (3353, 3072, 50257, False), (4900, 2048, 50257, False),                                          # of 160
-    (2898, 2048, 44032, False),                                                                      # of 192 x 128
+    (2898, 2048, 44032, False), (1929, 3072, 64000, False),                                          # of 192 x 128
     (2574, 3072, 40000, False), (3200, 2560, 48000, False), (6430, 2560, 40000, False),              # of 128 x 256, and two of them
-    (6448, 2048, 42000, True), (1585, 4096, 42000, True),
+    (6448, 2048, 42000, True), (1292, 4096, 50257, True), (2876, 2048, 50257, True), (1585, 4096, 42000, True),
     (0, 4096, 128256, False),
     (2876, 0, 128256, False),
 ])
