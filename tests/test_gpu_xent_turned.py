@@ -152,3 +152,41 @@ def test_gradients(monkeypatch, T, D, N, block):
     # dlogits rounded to bf16 once (2^-9 relative each, independent) and the result once: 2^-8 of the norm with room
     for a, want in zip(got[0], xo.linear_cross_entropy_backward(go, x, w, y)):
         assert (a.cpu().double() - want).norm() <= 2.0 ** -8 * want.norm()
+
+
+# several rounds of workgroups of the divided grad_x, whose rule wants more tiles than a third of the CUs and a large
+# vocabulary; from 4096 rows on w would otherwise be turned
+@pytest.mark.parametrize("T,D,N", [(1292, 4096, 50257), (2876, 2048, 50257), (4100, 2560, 40003)])
+def test_gradients_with_uneven_rounds(monkeypatch, T, D, N):
+    import tritonops_amd as ta
+    from tritonops_amd import xent
+
+    lib = _lib.load()
+    n_split = lib.mi_xent_grad_x_uneven_splits(T, D, N, lib.mi_device_cu_count())
+    assert n_split > 1
+    divided, turned = [], []
+    grad_x, turn = xent._grad_x, xent._turn
+    monkeypatch.setattr(xent, "_grad_x", lambda dl, w, out, n: divided.append(n) or grad_x(dl, w, out, n))
+    monkeypatch.setattr(xent, "_turn", lambda t, out: turned.append(t.shape[0]) or turn(t, out))
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn((T, D), generator=g, device="cuda").bfloat16()
+    w = (torch.randn((N, D), generator=g, device="cuda") * 3 * D ** -0.5).bfloat16()
+    y = torch.randint(0, N, (T,), generator=g, device="cuda")
+    go = torch.rand(T, generator=g, device="cuda") + 0.5
+    got = []
+    for keep in (True, False):
+        xg, wg = x.clone().requires_grad_(True), w.clone().requires_grad_(True)
+        loss = ta.CrossEntropyFusedFunction.apply(xg, wg, y, keep)
+        got.append(torch.autograd.grad(loss, (xg, wg), go))
+    assert divided == [n_split] * 2 and N not in turned
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    some = torch.randperm(T, generator=g, device="cuda")[:300].sort().values   # rows; the last tile is in part behind them
+    some[-1] = T - 1
+    p = torch.softmax(x[some].double() @ w.double().t(), 1)
+    p[torch.arange(len(some), device="cuda"), y[some]] -= 1
+    want = (p * go[some, None]) @ w.double()
+    # as in test_gradients: the dlogits are rounded to bf16 once and so is the result
+    assert ((got[0][0][some].double() - want).norm() <= 2.0 ** -8 * want.norm()).item()
+    worst = (got[0][0][some].double() - want).norm(dim=1) / want.norm(dim=1)
+    assert (worst <= 2.0 ** -7).all().item()   # (of a single row: its few large dlogits carry their rounding whole)
