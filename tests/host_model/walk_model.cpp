@@ -44,7 +44,7 @@
 #include <vector>
 
 static int g_fail = 0;
-// 0: the kernels' protocols as they are.  1..24: one deliberate mistake each; the
+// 0: the kernels' protocols as they are.  1..25: one deliberate mistake each; the
 // run must then fail (tests/test_host_model.py checks that it does), which is
 // what shows that the checks below can tell a broken protocol from a sound one.
 static int g_mut = 0;
@@ -1050,6 +1050,22 @@ static void test(std::mt19937& rng) {
       for (int c = 0; c < n_splits; ++c)
         for (int kvs = 0; kvs < kv_slices; ++kvs)
           CHECK(written[((size_t)b * n_splits + c) * kv_slices + kvs] == (c < nvalid), "slot %d of sequence %d (%d of %d are merged)", c, b, nvalid, n_splits);
+      // slots that are asked for: a few before their number is known, the others up to the last one written
+      const int batch_of = 32, ahead = g_mut == 25 ? batch_of : 4;
+      if (n_splits <= 256) {
+        std::vector<unsigned char> asked(n_splits, 0);
+        for (int i = 0; i < ahead; ++i) asked[std::min(i, n_splits - 1)] = 1;
+        if (nvalid > ahead)
+          for (int i = ahead; i < batch_of; ++i) asked[std::min(i, nvalid - 1)] = 1;
+        for (int c0 = batch_of; c0 < nvalid; c0 += batch_of)
+          for (int i = 0; i < batch_of; ++i) asked[std::min(c0 + i, nvalid - 1)] = 1;
+        int idle = 0;
+        for (int c = 0; c < n_splits; ++c) {
+          CHECK(c >= nvalid || asked[c], "slot %d of sequence %d (%d of %d) is not asked for", c, b, nvalid, n_splits);
+          idle += c >= nvalid && asked[c];
+        }
+        CHECK(idle <= 4, "%d slots of sequence %d that nobody wrote are read (%d of %d are merged)", idle, b, nvalid, n_splits);
+      }
       if (g_fail) return;
     }
     ++cases;

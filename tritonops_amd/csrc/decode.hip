@@ -442,14 +442,19 @@ decode_splitkv_kernel(const DecodeParams p) {
 // of the chunk.
 //
 // NE > 0 (at most 64 NE slots): every wavefront forms all weights, NE to a lane, which
-// are read out of its lanes, and the log-sum-exps and the first slots are requested
-// before it is known how many of them pass 1 wrote (those behind are memory of the
-// workspace that is not looked at): the length, the log-sum-exps and the partial
-// results wait for memory once instead of one after another, with no barrier; slots
-// behind are requested a batch ahead.  The same sums in the same order as the
-// general form.  Merge alone, 32 heads of 128: two sequences of 32 slots 5.2 -> 4.2
-// us (a launch of nothing takes 4), 64 of 5 6.0 -> 4.6, one of 128 7.3 -> 6.0.
-constexpr int kMergeThreads = 128, kMergeBatch = 32;
+// are read out of its lanes, and the log-sum-exps and the first kMergeAhead slots are
+// requested before it is known how many of them pass 1 wrote (the length comes through
+// the scalar cache meanwhile); the others as soon as it is, and a batch ahead.  No
+// barrier, the same sums in the same order as the general form.  Merge alone, 32 heads
+// of 128: two sequences of 32 slots 5.2 -> 4.3 us (a launch of nothing takes 4), 64 of 5
+// 6.0 -> 4.6, one of 128 7.3 -> 6.0.
+// Asking for a whole batch ahead, 0.2 us faster where all of it was written, reads up to
+// 32 slots a row of what nobody wrote under a bound far above the lengths, and pass 1 of
+// the call after it pays for the caches: both passes, four sequences of 250 to 1000
+// tokens of 65536 49.7 us, with 4 ahead 45.2, 8 45.4, 16 47.2, none 45.8; 128 of 25 to
+// 100 of 32768 23.4, 19.7, 20.4, 23.0, 20.6.  A list without counts of its own has as
+// many slots as the launch says: all are asked for at once (64 blocks 19.4 -> 19.1).
+constexpr int kMergeThreads = 128, kMergeBatch = 32, kMergeAhead = 4;
 template <typename T, int NE>
 __global__ void __launch_bounds__(kMergeThreads)
 decode_merge_kernel(const DecodeParams p, int D) {
@@ -461,16 +466,23 @@ decode_merge_kernel(const DecodeParams p, int D) {
   const float* pl = p.part_lse + slot0;
   const float* po = p.part_o + slot0 * D + min(d, D - 1);
   float part[2][NE ? kMergeBatch : 1], e[NE ? NE : 1];
-  auto request = [&](float (&x)[NE ? kMergeBatch : 1], int c0) __attribute__((always_inline)) {
+  // slots [first, kMergeBatch) of the batch at c0; those behind `last` read it once more
+  auto request = [&](float (&x)[NE ? kMergeBatch : 1], int c0, auto first, int last) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < kMergeBatch; ++i) x[i] = po[(int64_t)min(c0 + i, p.n_splits - 1) * D];
+    for (int i = first; i < kMergeBatch; ++i) x[i] = po[(int64_t)min(c0 + i, last) * D];
   };
+  const bool known = p.list_mode == 1 && !p.block_cnt;   // how many slots there are, without a look at memory
   if constexpr (NE > 0) {
 #pragma unroll
     for (int k = 0; k < NE; ++k) e[k] = pl[min(64 * k + (d & 63), p.n_splits - 1)];
-    request(part[0], 0);
+    if (known) {
+      request(part[0], 0, std::integral_constant<int, 0>{}, p.n_splits - 1);
+    } else {
+#pragma unroll
+      for (int i = 0; i < kMergeAhead; ++i) part[0][i] = po[(int64_t)min(i, p.n_splits - 1) * D];
+    }
   }
-  const int len = p.seq_lens ? p.seq_lens[b] : p.cu[b + 1] - p.cu[b];
+  const int len = p.seq_lens ? scalar_word(p.seq_lens + b) : scalar_word(p.cu + b + 1) - scalar_word(p.cu + b);
   int nvalid;  // slots that pass 1 wrote
   if (p.list_mode != 0) {
     const int kvh = h / (p.hq / p.hkv);
@@ -478,7 +490,7 @@ decode_merge_kernel(const DecodeParams p, int D) {
     if (p.list_mode == 2)
       cnt = min(window_list(len, p.win_global, p.win_local).cnt, p.max_blocks);
     else
-      cnt = p.block_cnt ? min(p.block_cnt[b * p.hkv + kvh], p.max_blocks) : p.max_blocks;
+      cnt = p.block_cnt ? min(scalar_word(p.block_cnt + b * p.hkv + kvh), p.max_blocks) : p.max_blocks;
     nvalid = (cnt + p.add_last + p.split_blocks - 1) / p.split_blocks;
   } else {
     nvalid = len > 0 ? (len - 1) / p.split_tokens + 1 : 0;
@@ -487,6 +499,7 @@ decode_merge_kernel(const DecodeParams p, int D) {
 
   float M = -INFINITY, den = 0.f, acc = 0.f;
   if constexpr (NE > 0) {
+    if (!known && nvalid > kMergeAhead) request(part[0], 0, std::integral_constant<int, kMergeAhead>{}, nvalid - 1);
 #pragma unroll
     for (int k = 0; k < NE; ++k) {
       e[k] = 64 * k + (d & 63) < nvalid ? e[k] : -INFINITY;
@@ -500,7 +513,7 @@ decode_merge_kernel(const DecodeParams p, int D) {
     for (int c0 = 0; c0 < 64 * NE; c0 += kMergeBatch) {
       if (c0 >= nvalid) break;
       float(&x)[kMergeBatch] = part[(c0 / kMergeBatch) & 1];
-      if (c0 + kMergeBatch < nvalid) request(part[(c0 / kMergeBatch + 1) & 1], c0 + kMergeBatch);
+      if (c0 + kMergeBatch < nvalid) request(part[(c0 / kMergeBatch + 1) & 1], c0 + kMergeBatch, std::integral_constant<int, 0>{}, nvalid - 1);
 #pragma unroll
       for (int i = 0; i < kMergeBatch; ++i) {
         const bool live = c0 + i < nvalid;
