@@ -1113,17 +1113,16 @@ __device__ __forceinline__ void bwd_dkdv_item(const BwdParams& p, const int b, c
 // walking the work items of its rounds (a fresh 512-thread workgroup with this
 // much LDS starts several microseconds after its predecessor ends; order of the
 // items: item_order.h).  The ids are kept in LDS behind the tiles (`LIST`): held
-// in registers across the items they cost the dK + dV kernel spills inside its
-// tile loop.
+// in registers across the items they are spilled.
 constexpr int kListBytes = 3 * kMaxRounds * 4;
-template <int ROWS, bool FROM_END, uint32_t LIST, typename Item>
+template <int ROWS, uint32_t LIST, typename Item>
 __device__ __forceinline__ void walk_items(const BwdParams& p, const int n_items, const int heads, const int heads_kv,
                                            const int n_rt, Item&& item) {
   typedef __attribute__((address_space(3))) int lds_int;
   lds_int* list = (lds_int*)(uintptr_t)((uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd) + LIST);
   const int grid = gridDim.x;
   if (threadIdx.x < kMaxRounds) {
-    const ItemId ids = items_of_rounds<ROWS, FROM_END>(p.cu, p.batch, p.max_seqlen, n_rt, heads, heads_kv,
+    const ItemId ids = items_of_rounds<ROWS, false>(p.cu, p.batch, p.max_seqlen, n_rt, heads, heads_kv,
                                                        p.by_level, n_items, grid);
     list[threadIdx.x] = ids.t;
     list[kMaxRounds + threadIdx.x] = ids.b;
@@ -1182,7 +1181,6 @@ struct KeyPlan {
 };
 
 typedef __attribute__((address_space(3))) KeyPlan LdsKeyPlan;
-typedef __attribute__((address_space(3))) int lds_int;
 
 // Units run from the longest to the shortest: pairs that stand before level t's.
 __device__ __forceinline__ int key_units_before(const LdsKeyPlan& k, const int t) {
@@ -1196,7 +1194,10 @@ __device__ __forceinline__ int key_units_before(const LdsKeyPlan& k, const int t
 }
 
 // By one wavefront: whether the units are dealt out, and then the levels and which of them are halved.  The
-// estimate that is minimised is the longer of the longest unit and the mean load plus a quarter of a mean unit.
+// estimate that is minimised is the longer of the longest unit and the mean load plus a quarter of a mean unit.  It
+// is no schedule: against every level, or every twelfth of them, as the first that is halved, dQ with dK + dV took
+// within 3 % of the best for ten of thirteen sizes, and 3.3 (six of 1500, 4 kv-heads of 8), 4.6 (4096, 8 of 4: 483 us,
+// all halved 461) and 5.7 % more (40 of 700, one of 8) for the others; unhalved 4096 took 537.
 //
 // What this costs is 2.3 us of the launch whatever the number of sequences (looked through one after another they
 // cost another 0.17 us each: 64 of 60 tokens, 2 heads, dK + dV 24.0 -> 12.9).  Where every whole item has a workgroup
@@ -1406,7 +1407,7 @@ template <typename T, int D, int NW>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 bwd_dq_kernel(const BwdParams p, const int n_items, const int n_rt) {
   if (blockIdx.x == 0 && threadIdx.x < 8 && p.queue) p.queue[16 * threadIdx.x] = 0;  // for the dK + dV kernel, which runs after this one
-  walk_items<32 * NW, false, kDqLds>(p, n_items, p.hq, p.hkv, n_rt, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
+  walk_items<32 * NW, kDqLds>(p, n_items, p.hq, p.hkv, n_rt, [&](int b, int hr, int rt, int wave) __attribute__((always_inline)) {
     bwd_dq_item<T, D, NW>(p, b, hr, rt, wave);
   });
 }

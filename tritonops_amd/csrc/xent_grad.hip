@@ -284,27 +284,27 @@ int xent_gradx_splits(long long tokens, long long dim, long long vocab, int num_
   return s;
 }
 
-// The same for a result with tiles enough, or 0 where the library's product is
-// left to it.  The library has products at 1.0 to 1.2 times the time of the matrix
-// rate where one of its tile shapes fills whole rounds of the chip (the large ones
-// any number of rounds, those with a side of 192 or 160 a single one, 192 x 128 exactly) and for token
-// counts that fill up a multiple of 512 to 3 %; elsewhere it mostly takes 1.3 to 1.9
-// times that time, and ranges of the vocabulary even the rounds out.  Library
-// (with w the other way round where that is the rule) -> this, us, at
+// The same for a result with tiles enough, or 0 where the library's product is left
+// to it.  The library has products at 1.0 to 1.2 times the time of the matrix rate
+// where one of its tile shapes fills whole rounds of the chip (the large ones any
+// number of rounds, those with a side of 192 or 160 a single one, 192 x 128 exactly)
+// and for token counts that fill up a multiple of 512 to 3 %; elsewhere it mostly
+// takes 1.3 to 1.9 times that time, and ranges of the vocabulary even the rounds
+// out.  Library (with w the other way round where that is the rule) -> this, us, at
 // 50257 / 128256 words: 1292 x 4096 741 -> 578 / 1905 -> 1380; 2876 x 2048 799 ->
 // 563 / 2021 -> 1328; 2876 x 4096 1515 -> 1058 / 3891 -> 2599; 3700 x 3072 1520 ->
 // 1039 / 3986 -> 2587; 4100 x 2560 1550 -> 936 / 4054 -> 2289; 4700 x 4096 3109 ->
 // 1783 / 8188 -> 4290.  Of 757 sizes that the rule takes, drawn from 1000 to 8000
 // tokens, 1024 to 5120 columns and ten vocabularies from 40000 to 128256 words, five
-// lose (4, 4, 10, 12 and 12 %, the last 2394 x 2560 x 48000 519 -> 583) and all are 1.39
-// times as fast in the mean.  With the shapes 256 x 256 and half of it alone it took
-// 50 of 406 sizes more, 35 of which lost up to 20 % (6430 x 2560 x 40000, 128 x 256 in two
-// rounds, 1141, here 1365; 3900 x 3072 x 50257, 256 x 192 in one, 966, here 1077).
-// Not taken either: 6200 x 2560 x 50257 (250 tiles) 1080, here 1280; vocabularies of
-// 32000, where one in five loses (4700 x 2560 594, here 711; nothing was measured
-// between 32000 and 40000).  All of it describes the library that this was measured
-// with.  A step of 64 takes it 1.52 us a round of wide tiles and 0.80 of
-// narrow ones at best; the partial sums are at most as large as the dlogits.
+// lose (4, 4, 10, 12 and 12 %, the last 2394 x 2560 x 48000 519 -> 583) and all are
+// 1.39 times as fast in the mean.  With the shapes 256 x 256 and half of it alone it
+// took 50 of 406 sizes more, 35 of which lost up to 20 % (6430 x 2560 x 40000, 128 x
+// 256 in two rounds, 1141, here 1365; 3900 x 3072 x 50257, 256 x 192 in one, 966,
+// here 1077). Not taken either: 6200 x 2560 x 50257 (250 tiles) 1080, here 1280;
+// vocabularies of 32000, where one in five loses (4700 x 2560 594, here 711; nothing
+// was measured between 32000 and 40000).  All of it describes the library that this
+// was measured with.  A step of 64 takes it 1.52 us a round of wide tiles and 0.80
+// of narrow ones at best; the partial sums are at most as large as the dlogits.
 int xent_gradx_uneven_splits(long long tokens, long long dim, long long vocab, int num_cus) {
   if (tokens <= 0 || dim <= 0 || vocab < 40000) return 0;
   if ((512 - tokens % 512) % 512 * 100 <= 3 * tokens) return 0;
