@@ -46,7 +46,7 @@ KERNELS = {
     "sparse_decode": _NS + "21decode_splitkv_kernelIDF16bLi128ELi1ELb1EEEvNS_12DecodeParamsE",
     "dense_causal_bwd": " + ".join(_NS + n for n in (
         "13bwd_dq_kernelIDF16bLi128ELi8EEEvNS_9BwdParamsEii",
-        "15bwd_dkdv_kernelIDF16bLi128EEEvNS_9BwdParamsEii")),
+        "15bwd_dkdv_kernelIDF16bLi128EEEvNS_9BwdParamsEiii")),
     "rmsnorm": " + ".join(_NS + n for n in (
         "18rms_fwd_vec_kernelIDF16bfLi2ELi256ELb1EEEvNS_9RmsParamsE",
         "18rms_bwd_vec_kernelIDF16bfLi2ELi256ELb1EEEvNS_9RmsParamsE",
