@@ -44,7 +44,7 @@
 #include <vector>
 
 static int g_fail = 0;
-// 0: the kernels' protocols as they are.  1..25: one deliberate mistake each; the
+// 0: the kernels' protocols as they are.  1..26: one deliberate mistake each; the
 // run must then fail (tests/test_host_model.py checks that it does), which is
 // what shows that the checks below can tell a broken protocol from a sound one.
 static int g_mut = 0;
@@ -203,6 +203,37 @@ static std::vector<ItemId> items(const Launch& L, int wg, int block) {
           }
           at += own;
         }
+      if (block == 1) {   // the same pair found level by level: its place among the sequences that reach the level
+        uint32_t lo = 0, hi = 0;
+        int k = 0, t = -1, before = 0;
+        for (int level = L.n_tiles - 1; level >= 0 && n >= before; --level) {
+          uint64_t live = 0;
+          for (int seq = 0; seq < L.batch; ++seq) live |= (uint64_t)(L.tiles(seq) > level) << seq;
+          const int own = __builtin_popcountll(live);
+          if (n < before + own) {
+            lo = (uint32_t)live;
+            hi = (uint32_t)(live >> 32);
+            k = n - before;
+            t = level;
+          }
+          before += own;
+        }
+        const int in_lo = __builtin_popcount(lo);
+        const bool upper = k >= in_lo;
+        uint32_t m = upper ? hi : lo;
+        k -= upper && g_mut != 26 ? in_lo : 0;
+        int b = upper ? 32 : 0;
+        for (int w = 16; w >= 1; w >>= 1) {
+          const int c = __builtin_popcount(m & ((1u << w) - 1));
+          const bool above = k >= c;
+          k -= above ? c : 0;
+          b += above ? w : 0;
+          m = above ? m >> w : m;
+        }
+        if (t < 0) b = 0;
+        if (L.from_end && t >= 0 && b < L.batch) t = L.tiles(b) - 1 - t;
+        CHECK(b == it.b && t == it.t, "pair %d: (sequence %d, tile %d) by levels, (%d, %d) one by one", n, b, t, it.b, it.t);
+      }
       uint32_t member, kvh;
       divmod(small, r, L.heads_kv, member, kvh);
       it.h = (int)(kvh * group + member);
@@ -1206,7 +1237,7 @@ int main(int argc, char** argv) {
   std::mt19937 rng(12345);
   // (a mistake that sits in another part is not looked for in these two, which take longest)
   const auto in = [](std::initializer_list<int> parts) { return std::find(parts.begin(), parts.end(), g_mut) != parts.end(); };
-  if (in({0, 7, 16, 17, 18, 19, 24})) order::test(rng);
+  if (in({0, 7, 16, 17, 18, 19, 24, 26})) order::test(rng);
   if (in({0, 1, 2, 3, 4, 8, 11, 12})) dense::test(rng);
   sparse::test(rng);
   softmax::test(rng);

@@ -43,6 +43,7 @@ MISTAKES = {
     22: "decode: no barrier between the last reads of a step and the next step's stores",
     23: "decode: the refill behind a store fetches the next step again",
     24: "choice of the order: odd rounds are sampled as if they ran forward",
+    26: "level order: a sequence of the upper 32 is counted from the first of the lower",
     25: "decode: the merge asks for a whole batch of slots before it knows how many were written",
 }
 

@@ -1122,7 +1122,7 @@ __device__ __forceinline__ void walk_items(const BwdParams& p, const int n_items
   lds_int* list = (lds_int*)(uintptr_t)((uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)smem_bwd) + LIST);
   const int grid = gridDim.x;
   if (threadIdx.x < kMaxRounds) {
-    const ItemId ids = items_of_rounds<ROWS, false>(p.cu, p.batch, p.max_seqlen, n_rt, heads, heads_kv,
+    const ItemId ids = items_of_rounds<ROWS, false, kLevelWorth, true>(p.cu, p.batch, p.max_seqlen, n_rt, heads, heads_kv,
                                                        p.by_level, n_items, grid);
     list[threadIdx.x] = ids.t;
     list[kMaxRounds + threadIdx.x] = ids.b;
@@ -1463,16 +1463,16 @@ int launch_all(const BwdParams& p, hipStream_t s) {
 // are never slower from 129 tokens on (1000 tokens, 16 heads 40 -> 29 us; 4096, 8 heads 135 -> 108); up to 128 both
 // forms have the same items, which eight wavefronts load sooner than four (128 tokens, 16 to 256 items, 1.3 to 1.8
 // us).  In the two rounds of a causal call, the second of short items, the gain of 0.53 us a tile of the longest
-// chain has to pay for what 256 rows do without: the second round's boundary and the order of the items by
-// level, 0.05 us per (sequence, tile) pair of a head.  2048, 32 heads 82 -> 66; 4096, 16 heads 135 -> 108; three of 1354, 8
-// heads 92 -> 79 with dK + dV; but 64 of 256, 4 heads, dQ alone 26 -> 43, 24 of 384, 4 heads 24 -> 32, 40 of 700,
-// 2 heads 35 -> 50.  Of 163 measured launches of two rounds this takes 54, 1.10 times as fast in the mean with dK +
-// dV, one of them 3 % slower (six of 1105, 8 heads); 42 it leaves would gain 2 to 21 %.  Beyond two rounds: 4096, 32 heads (four) 191 -> 208.
+// chain has to pay for the second round's boundary, 3.5 us where both are full.  2048, 32 heads 82 -> 66; 4096, 16
+// heads 135 -> 108; with dK + dV three of 1354, 8 heads 91 -> 79, but 64 of 256, 4 heads 59 -> 69, 24 of 384, 4 heads
+// 48 -> 54.  Of 211 measured launches of two rounds this takes 106, 1.10 times as fast in the mean with dK + dV,
+// three of them 1.5 to 2 % slower; 25 of those it leaves would gain 2 to 17 %.  Beyond two rounds: 4096, 32 heads (four)
+// 191 -> 208.
 bool bwd_dq_short_items(int max_seqlen, int batch, int heads_q, bool causal, int num_cus) {
   if (num_cus <= 0) num_cus = 256;
-  const long long pairs = (long long)((max_seqlen + 127) / 128) * batch, items = pairs * heads_q;
+  const long long items = (long long)((max_seqlen + 127) / 128) * batch * heads_q;
   if (max_seqlen <= 128 || items > (causal ? 2 : 1) * (long long)num_cus) return false;
-  return items <= num_cus || 53LL * ((max_seqlen + 63) / 64) >= 120 + 5 * pairs + 300 * items / num_cus;
+  return items <= num_cus || 53LL * ((max_seqlen + 63) / 64) >= 120 + 350 * items / num_cus;
 }
 
 int launch_attn_bwd(const BwdParams& p, int dtype, int head_dim, hipStream_t s) {

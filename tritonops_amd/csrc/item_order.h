@@ -106,7 +106,12 @@ inline long long persistent_grid(long long items, long long resident) {
 // which every later query streams past), else the last.  heads_kv: heads per
 // sequence that share nothing (units); heads / heads_kv items of a unit run
 // side by side on each of its tiles.
-template <int ROWS, bool FROM_END, int WORTH = kLevelWorth>
+//
+// BY_LEVELS: where levels are taken one at a time a pair is found level by level, with
+// the sequences of a level as bits of a mask, instead of pair by pair, 0.05 us each
+// (64 sequences of 926 tokens, one head, dQ in two rounds of 128-row items with dK + dV
+// 120 -> 89 us).  The other kernels' search is as it was.
+template <int ROWS, bool FROM_END, int WORTH = kLevelWorth, bool BY_LEVELS = false>
 __device__ __forceinline__ ItemId items_of_rounds(const int32_t* cu, const int batch, const int max_seqlen,
                                                   const int n_tiles, const int heads, const int heads_kv,
                                                   const bool level_order, const int n_items, const int grid) {
@@ -201,6 +206,39 @@ __device__ __forceinline__ ItemId items_of_rounds(const int32_t* cu, const int b
       divmod(bid, (uint32_t)heads, pair, r);
       const int n = any ? (int)pair : -1;  // (sequence, tile) pair in the order below
       int at = 0;                                             // pairs before the ones being looked at
+      if (BY_LEVELS && block == 1) {
+        uint32_t lo = 0, hi = 0;   // sequences of the level that the pair lies on
+        int k = 0;                 // and which of them it is
+        for (int t = n_tiles - 1; t >= 0; --t) {
+          const uint64_t live = __builtin_amdgcn_ballot_w64(tiles > t);
+          const int own = __builtin_popcountll(live);
+          if (n >= at && n < at + own) {
+            lo = (uint32_t)live;
+            hi = (uint32_t)(live >> 32);
+            k = n - at;
+            it.t = t;
+          }
+          at += own;
+          if (__builtin_amdgcn_ballot_w64(n >= at) == 0) break;
+        }
+        // the bit of the mask that has k set ones before it
+        const int in_lo = __popc(lo);
+        const bool upper = k >= in_lo;
+        uint32_t m = upper ? hi : lo;
+        k -= upper ? in_lo : 0;
+        it.b = upper ? 32 : 0;
+#pragma unroll
+        for (int w = 16; w >= 1; w >>= 1) {
+          const int c = __popc(m & ((1u << w) - 1));
+          const bool above = k >= c;
+          k -= above ? c : 0;
+          it.b += above ? w : 0;
+          m = above ? m >> w : m;
+        }
+        if (it.t < 0) it.b = 0;
+        const int all = __shfl(tiles, it.b, 64);
+        if (FROM_END && it.t >= 0) it.t = all - 1 - it.t;
+      } else
       for (int first = (n_tiles - 1) / block * block; first >= 0; first -= block) {
         uint64_t live = __builtin_amdgcn_ballot_w64(tiles > first);
         while (live) {
